@@ -2,8 +2,8 @@
 //
 // The reference keeps the derived CRT tables as literals (src/common/crt_tables.hpp:19-112);
 // here only the moduli list is data and everything else is computed once from closed forms:
-// M = prod m_s, floor(M/2), M/m_s, (M/m_s)^-1 mod m_s and the CRT basis Q_s = inv_s * M/m_s mod M
-// (Q_s = 1 mod m_s, 0 mod m_t for t != s), so that x = sum_s (x mod m_s) Q_s (mod M).
+// M = prod m_s, floor(M/2) and, per group of three moduli, the group sum's multipliers E_s and the
+// basis R_g (CrtSet).
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -39,13 +39,13 @@ uint64_t div_small(const Big& a, uint64_t m, Big& q) {
     return (uint64_t)rem;
 }
 
-void to16(const Big& a, uint32_t out[kLimbs]) {
-    for (int j = 0; j < kLimbs; ++j) out[j] = (uint32_t)((a.d[j / 4] >> (16 * (j % 4))) & 0xffffu);
+void to32(const Big& a, uint32_t out[kWords]) {
+    for (int j = 0; j < kWords; ++j) out[j] = (uint32_t)(a.d[j / 2] >> (32 * (j % 2)));
 }
 
-int bitlen(const Big& a) {
-    for (int i = 3; i >= 0; --i)
-        if (a.d[i]) return 64 * i + (64 - __builtin_clzll(a.d[i]));
+uint64_t inverse_mod(uint64_t r, uint64_t m) {
+    for (uint64_t c = 1; c < m; ++c)
+        if ((r * c) % m == 1) return c;
     return 0;
 }
 
@@ -58,47 +58,49 @@ CrtTables build_tables() {
         Big M;
         M.d[0] = 1;
         for (int s = 0; s < S; ++s) mul_small(M, kModuli[s]);
-        Big half;
-        for (int i = 0; i < 4; ++i) half.d[i] = (M.d[i] >> 1) | (i < 3 ? (M.d[i + 1] << 63) : 0);
-        to16(M, cs.M16);
-        // X = sum_s r_s Q_s with r_s < 256: X/M < 20 * 256.  X mod M in {floor(M/2), floor(M/2)+1}
-        // puts X/M within 1/(2M) of a half integer; the device estimates X/M from X's top limbs
-        // (wl[l] = 2^(16 l)/M) to within 1e-10, so anything closer to 1/2 than this threshold is
-        // re-checked exactly.
-        double Md = 0.0;
-        for (int i = 3; i >= 0; --i) Md = Md * 18446744073709551616.0 + (double)M.d[i];
-        cs.qthr = 0.5 - 2.0 / Md - 1e-9;
-        for (int l = 0; l < kLimbs; ++l) cs.wl[l] = std::ldexp(1.0, 16 * l) / Md;
-        to16(half, cs.Mhalf16);
-        std::memcpy(cs.M64, M.d, 32);
-        std::memcpy(cs.Mhalf64, half.d, 32);
-        // sum_s r_s * Q_s < S * 256 * M: limbs needed for that bound
-        cs.nlimbs = (bitlen(M) + 8 + 5 + 15) / 16 + 1;
-        if (cs.nlimbs > kLimbs) cs.nlimbs = kLimbs;
-        for (int s = 0; s < S; ++s) {
-            const uint64_t m = kModuli[s];
-            Big q;
-            div_small(M, m, q);
-            Big qq;
-            uint64_t r = div_small(q, m, qq);
-            uint64_t inv = 0;
-            for (uint64_t c = 1; c < m; ++c)
-                if ((r * c) % m == 1) {
-                    inv = c;
-                    break;
-                }
-            // Q_s = inv * (M/m_s) mod M = inv * (M/m_s) - k M with k = floor(inv * (M/m_s) / M)
-            //     = floor(inv / m_s) = 0 since inv < m_s: Q_s = inv * (M/m_s) exactly.
-            Big Q = q;
-            mul_small(Q, inv);
-            to16(Q, cs.Q16[s]);
-            cs.m[s] = (uint32_t)m;
-            cs.inv[s] = (uint32_t)inv;
-            cs.rcp[s] = 1.0 / (double)m;
+        Big half, neg;
+        uint64_t carry = 1;
+        for (int i = 0; i < 4; ++i) {
+            half.d[i] = (M.d[i] >> 1) | (i < 3 ? (M.d[i + 1] << 63) : 0);
+            neg.d[i] = ~M.d[i] + carry;
+            carry = carry && neg.d[i] == 0;
         }
-        for (int s = 0; s < S; ++s)
-            for (int l = 0; l < 2 * kLimbs; ++l)
-                cs.Q8x4[s / 4][l] |= ((cs.Q16[s][l / 2] >> (8 * (l % 2))) & 0xffu) << (8 * (s % 4));
+        to32(M, cs.M32);
+        to32(half, cs.Mhalf32);
+        to32(neg, cs.Mneg);
+        std::memcpy(cs.M64, M.d, 32);
+        uint64_t err = 0;  // bound of 2^32 X/M - sum_g u_g F_g: each F_g is short by less than one
+        for (int g = 0; 3 * g < S; ++g) {
+            const int s0 = 3 * g, s1 = s0 + 3 < S ? s0 + 3 : S;
+            uint64_t P = 1, w = 0;
+            for (int s = s0; s < s1; ++s) P *= kModuli[s];
+            Big MP = M;  // M / P_g
+            for (int s = s0; s < s1; ++s) {
+                Big q;
+                div_small(MP, kModuli[s], q);
+                MP = q;
+            }
+            for (int s = s0; s < s1; ++s) {
+                const uint64_t m = kModuli[s], e = P / m;
+                Big q, qq;
+                div_small(M, m, q);
+                // w = ((M/m_s) mod m_s)^-1 mod m_s, combined over the group by the CRT mod P
+                const uint64_t a = inverse_mod(div_small(q, m, qq), m);
+                w = (w + a * inverse_mod(e % m, m) % m * e) % P;
+                cs.E[s] = (uint32_t)e;
+                cs.m[s] = (uint32_t)m;
+                cs.rcp[s] = 1.0 / (double)m;
+                err += (m - 1) * e;
+            }
+            Big R = MP;
+            mul_small(R, w);
+            to32(R, cs.R[g]);
+            cs.F[g] = (uint32_t)((w << 32) / P);
+        }
+        // Largest residue that maps to a positive value: floor(M/2) - 1, so X/M + 1/2 may come
+        // within 1/(2M) of the next integer without reaching it (see crt_words).
+        err += 2 + (M.d[1] || M.d[2] || M.d[3] ? 0 : (uint64_t(1) << 31) / M.d[0]);
+        cs.amb = (uint32_t)((uint64_t(1) << 32) - err);
     }
     return t;
 }

@@ -4,12 +4,11 @@
 // The reference sums c_s * (M/m_s) modulo M, c_s = (C_s mod m_s) * (M/m_s)^-1 mod m_s, in u64
 // (S <= 7) or four u64 limbs (S > 7), maps acc >= floor(M/2) to -(M - acc), converts limb by limb
 // (to_double_256) and scales by 2^-(shift_A[i] + shift_B[j]).  The value it converts is the fixed
-// integer C mod M, so any exact method gives the same double.  Here, with r_s = C_s mod m_s and the
-// CRT basis Q_s = (M/m_s)^-1 mod m_s * (M/m_s): X = sum_s r_s Q_s accumulated without reduction in
-// 16-bit limbs held in 32-bit registers (from blocked digits: one v_dot4_u32_u8 per four terms
-// and byte of a limb; from INT32 planes: one v_mad_u32_u24 per limb and term), the quotient
-// q = round(sum_s r_s Q_s/M) from an FP64 dot product, Y = X - q*M by signed limb arithmetic, an
-// exact range check only when q was ambiguous, then the reference's limb-wise conversion.
+// integer C mod M, so any exact method gives the same double.  Here the digits c_s = C_s mod m_s are
+// combined in groups of three moduli into X = C (mod M) in 32-bit words, the quotient
+// q = floor(X/M + 1/2) comes from a 32-bit fixed-point sum of the same groups, Y = X - q*M in one
+// carry pass, an exact range check only when q was ambiguous, then the reference's limb-wise
+// conversion (crt_value, recon_core.hpp).
 //
 // Scheme I group reconstruction (step4_reconstruction.hpp:21-49): C = 0, then
 // C = fma(T_g, scale_g, C) for g = 2..S+1 ascending, from the GEMM's blocked INT32 planes
@@ -51,7 +50,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int s = 0; s < S; ++s)
         c[s] = (uint32_t)crt_digit(Ct[s * MN + idx], (double)cs->m[s], cs->rcp[s]);
-    const double f = crt_value<S>(c, cs);
+    const double f = crt_value<S>(c, 0, cs);
     Cout[idx] = ldexp(f, -(shA[row] + shB[col]));
 }
 

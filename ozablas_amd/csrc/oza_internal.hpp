@@ -50,24 +50,26 @@ constexpr int bitlen_M(int S) {
 }
 static_assert(bitlen_M(8) == 63 && bitlen_M(16) == 124 && bitlen_M(20) == 153, "moduli products");
 
-// Per-S CRT constants used by the kernels.  Big integers are little-endian 16-bit limbs held
-// in 32-bit words so that c * limb (c < 2^8) and sums of up to 20 such products fit in 32 bits.
-constexpr int kLimbs = 12;  // 192 bits: M < 2^153, sum c_s*(M/m_s) < 20*2^8*M < 2^166
+// Per-S CRT constants used by the kernels.  Big integers are little-endian 32-bit words.
+//
+// The moduli s = 0..S-1 are taken in groups of three, g = s / 3 (the last one may be shorter), with
+// P_g the product of a group's moduli (< 2^24).  With the group sums
+//   u_g = sum_{s in g} c_s (P_g / m_s)            (24-bit operands, u_g < 3 * 2^24)
+// and the constants R_g = w_g (M / P_g), w_g < P_g with w_g (M / m_s) = 1 mod m_s for every s in g,
+//   X = sum_g u_g R_g = C (mod M)   whenever   c_s = C mod m_s for all s.
+constexpr int kWords = 5;                          // 160 bits: M < 2^153 and a sign
+constexpr int kGroups = (kMaxSlices + 2) / 3;
 struct CrtSet {
     int S;
-    int nlimbs;                       // limbs actually used for this S
-    uint32_t M16[kLimbs];             // M = prod m_s
-    uint32_t Mhalf16[kLimbs];         // floor(M/2)
-    uint32_t Q16[kMaxSlices][kLimbs];  // Q_s = ((M/m_s)^-1 mod m_s) * (M/m_s) mod M
-    // Byte k of Q8x4[j][l] = 8-bit limb l of Q_{4j+k} (0 past S): operand of v_dot4_u32_u8
-    // against four digits of one element.
-    uint32_t Q8x4[kMaxSlices / 4][2 * kLimbs];
+    uint32_t E[kMaxSlices];           // P_g / m_s (< 2^16; 1 in a group of one)
+    uint32_t F[kGroups];              // floor(2^32 R_g / M) = floor(2^32 w_g / P_g)
+    uint32_t amb;                     // fractional part of the quotient estimate from which on it may be one short
+    uint32_t R[kGroups][kWords];
+    uint32_t Mneg[kWords];            // 2^160 - M
+    uint32_t M32[kWords], Mhalf32[kWords];  // M and floor(M/2)
     uint32_t m[kMaxSlices];
-    uint32_t inv[kMaxSlices];         // (M/m_s)^-1 mod m_s
     double rcp[kMaxSlices];           // 1/m_s rounded
-    double wl[kLimbs];                // 2^(16 l) / M rounded (quotient estimate from limbs)
-    double qthr;                      // |frac - 1/2| below 1/M + margin: quotient may be ambiguous
-    uint64_t M64[4], Mhalf64[4];      // the same, 64-bit limbs
+    uint64_t M64[4];                  // M in 64-bit words
 };
 
 // All S = 1..20, computed on the host from the moduli (closed forms).

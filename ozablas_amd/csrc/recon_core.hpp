@@ -12,144 +12,89 @@ namespace core {
 template <int S>
 struct CrtShape {
     static constexpr int BITS = bitlen_M(S);
-    static constexpr int LP = (BITS + 15) / 16;               // limbs of M / m_s
-    static constexpr int NL = (BITS + 5 + 8 + 15) / 16 + 1;   // accumulator limbs + sign spare
-    static_assert(NL <= kLimbs, "limb budget");
+    static constexpr int G = (S + 2) / 3;            // groups of three moduli
+    static constexpr int LR = (BITS + 31) / 32;      // words of R_g
+    static constexpr int L = (BITS + 1 + 31) / 32;   // words of the signed Y, |Y| < 0.56 M
+    static_assert(L <= kWords, "word budget");
 };
 
-template <int NL>
-__device__ __forceinline__ void propagate(int32_t (&y)[NL]) {
+// Byte b of w (b a compile-time constant: a byte select of the 24-bit multiply that uses it).
+__device__ __forceinline__ uint32_t byte_of(uint32_t w, int b) { return (w >> (8 * b)) & 0xffu; }
+
+// Adds k * v to Y, words modulo 2^(32 L), k = +1 or -1.
+template <int L, bool SUB>
+__device__ __forceinline__ void add_words(uint32_t (&y)[L], const uint32_t* __restrict__ v) {
+    uint32_t carry = SUB ? 1 : 0;
 #pragma unroll
-    for (int l = 0; l < NL - 1; ++l) {
-        const int32_t c = y[l] >> 16;  // arithmetic shift: floor division
-        y[l] -= c * 65536;
-        y[l + 1] += c;
-    }
+    for (int l = 0; l < L; ++l) y[l] = __builtin_addc(y[l], SUB ? ~v[l] : v[l], carry, &carry);
 }
 
-// X = sum_s c_s Q_s in LP unpropagated 16-bit limbs (each < S * 255 * 65535 < 2^28.4), one
-// v_mad_u32_u24 per limb and term.
+// Signed reconstruction of one element from its digits, byte b of w[s] = c_s, as the reference's
+// double.  With the groups of CrtSet:
+//   X = sum_g u_g R_g in LR 64-bit columns (u_g < 2^25.4, at most 7 groups: every column < 2^61);
+//   q estimates floor(X/M + 1/2) from h = 2^31 + sum_g u_g F_g, which is short of 2^32 (X/M + 1/2)
+//     by less than sum_g u_g: q is that floor, or one less when the fraction of h is at or above
+//     cs->amb (sum of the u_g bounds from the top, with a margin of 1/(2M));
+//   Y = X - q M: the columns get q times the words of 2^160 - M, then one carry pass.
+// The reference maps X mod M >= floor(M/2) to X mod M - M.  Away from the ambiguous fractions that
+// is the Y above (|Y| < M/2, M odd); at them the exact comparison with floor(M/2) decides.
+// What bounds it: VALU issue and the digits' and C's bytes about equally (every instruction here, the
+// 64-bit multiply-add included, issues in four cycles per wave).  Groups of three, because u_g must
+// fit the 32-bit operand of the multiply-add: three digits then cost 3 byte-select multiplies, one
+// three-way add and LR multiply-adds.  16-bit limbs of X by v_dot4_u32_u8 (18 limbs at S = 17, five
+// dot products each, a carry and a sign pass over every limb) took 239 instructions per element and
+// 1.26 ms for the 512-GEMM batch's step 4 against 0.99 ms here (156 per element at S = 17, the
+// ambiguous path included).
 template <int S>
-__device__ __forceinline__ void crt_limbs(const uint32_t (&c)[S], const CrtSet* __restrict__ cs,
-                                          int32_t (&y)[CrtShape<S>::NL]) {
-    constexpr int LP = CrtShape<S>::LP, NL = CrtShape<S>::NL;
+__device__ __forceinline__ double crt_value(const uint32_t (&w)[S], int b, const CrtSet* __restrict__ cs) {
+    constexpr int G = CrtShape<S>::G, LR = CrtShape<S>::LR, L = CrtShape<S>::L;
+    uint64_t col[L];
+    uint64_t h = 1ull << 31;
 #pragma unroll
-    for (int l = 0; l < NL; ++l) y[l] = 0;
+    for (int l = 0; l < L; ++l) col[l] = 0;
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
+    for (int g = 0; g < G; ++g) {
+        uint32_t u = __umul24(byte_of(w[3 * g], b), cs->E[3 * g]);
+        if (3 * g + 1 < S) u += __umul24(byte_of(w[3 * g + 1], b), cs->E[3 * g + 1]);
+        if (3 * g + 2 < S) u += __umul24(byte_of(w[3 * g + 2], b), cs->E[3 * g + 2]);
+        h += (uint64_t)u * cs->F[g];
 #pragma unroll
-        for (int l = 0; l < LP; ++l) y[l] = (int32_t)__umul24(c[s], cs->Q16[s][l]) + y[l];
+        for (int l = 0; l < LR; ++l) col[l] += (uint64_t)u * cs->R[g][l];
     }
-}
-
-// The same limbs from digits packed four moduli to a word (byte k of P[j] = c_{4j+k}, 0 past S):
-// the sums against the low and high bytes of each 16-bit limb of Q_s by v_dot4_u32_u8 (four
-// products and the add in one instruction; each sum < S * 255^2 < 2^21), then lo + 256 hi, which
-// is crt_limbs' limb exactly.
-template <int S>
-__device__ __forceinline__ void crt_limbs_packed(const uint32_t (&P)[(S + 3) / 4], const CrtSet* __restrict__ cs,
-                                                 int32_t (&y)[CrtShape<S>::NL]) {
-    constexpr int LP = CrtShape<S>::LP, NL = CrtShape<S>::NL, NJ = (S + 3) / 4;
-    uint32_t b8[2 * LP];  // byte-limb sums; one table row (contiguous) per group of four moduli
+    const uint32_t q = (uint32_t)(h >> 32);
+    uint32_t y[L];
+    uint32_t carry = 0;
 #pragma unroll
-    for (int l = 0; l < 2 * LP; ++l) b8[l] = 0;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-#pragma unroll
-        for (int l = 0; l < 2 * LP; ++l) b8[l] = __builtin_amdgcn_udot4(P[j], cs->Q8x4[j][l], b8[l], false);
+    for (int l = 0; l < L; ++l) {
+        col[l] += (uint64_t)q * cs->Mneg[l];
+        y[l] = l == 0 ? (uint32_t)col[0]
+                      : __builtin_addc((uint32_t)col[l], (uint32_t)(col[l > 0 ? l - 1 : 0] >> 32), carry, &carry);
     }
+    if (__builtin_expect((uint32_t)h >= cs->amb, 0)) {
+        uint32_t d[L];
 #pragma unroll
-    for (int l = 0; l < LP; ++l) y[l] = (int32_t)(b8[2 * l] + (b8[2 * l + 1] << 8));
-#pragma unroll
-    for (int l = LP; l < NL; ++l) y[l] = 0;
-}
-
-// Signed reconstruction of one element from the limbs of X = sum_s c_s Q_s (crt_limbs or
-// crt_limbs_packed), returned as the reference's double.
-//   q = round(X/M), with X/M estimated from the top min(LP, 5) limbs: the limbs below contribute
-//     < 2^-50 and the FP64 sum errs by < 2^-38 (X/M < 20 * 256), inside the 1e-9 margin of qthr;
-//   Y = X - qM.  When X/M is clearly inside (q - 1/2, q + 1/2), Y has the sign of qf - q except
-//     when |Y| is below the estimate's error; |Y| is formed by negating the limbs before the one
-//     carry pass, and a negative top limb afterwards (the rare wrong guess) flips it back.
-//     Otherwise the exact comparisons against floor(M/2) decide (the reference's mapping of
-//     X mod M >= floor(M/2) to negative).
-template <int S>
-__device__ __forceinline__ double crt_finish(int32_t (&y)[CrtShape<S>::NL], const CrtSet* __restrict__ cs) {
-    constexpr int LP = CrtShape<S>::LP, NL = CrtShape<S>::NL;
-    constexpr int LQ = LP < 5 ? LP : 5;
-    double qf = 0.0;
-#pragma unroll
-    for (int l = LP - 1; l >= LP - LQ; --l) qf = fma((double)y[l], cs->wl[l], qf);
-    const double q = rint(qf);
-    const int32_t qi = (int32_t)q;
-#pragma unroll
-    for (int l = 0; l < LP; ++l) y[l] += __mul24(-qi, (int32_t)cs->M16[l]);  // 0 <= qi < 2^13, M16 < 2^16
-    bool neg;
-    if (fabs(qf - q) > cs->qthr) {
-        propagate<NL>(y);
-        // Bring Y into [-(floor(M/2)+1), floor(M/2)-1] exactly.
-        int32_t d[NL];
-#pragma unroll
-        for (int l = 0; l < NL; ++l) d[l] = y[l] - (int32_t)(l < kLimbs ? cs->Mhalf16[l] : 0);
-        propagate<NL>(d);
-        if (d[NL - 1] >= 0) {
-#pragma unroll
-            for (int l = 0; l < NL; ++l) y[l] -= (int32_t)cs->M16[l];
-            propagate<NL>(y);
-        } else {
-#pragma unroll
-            for (int l = 0; l < NL; ++l) d[l] = y[l] + (int32_t)cs->Mhalf16[l] + (l == 0 ? 1 : 0);
-            propagate<NL>(d);
-            if (d[NL - 1] < 0) {
-#pragma unroll
-                for (int l = 0; l < NL; ++l) y[l] += (int32_t)cs->M16[l];
-                propagate<NL>(y);
-            }
-        }
-        neg = y[NL - 1] < 0;
-        if (neg) {
-#pragma unroll
-            for (int l = 0; l < NL; ++l) y[l] = -y[l];
-            propagate<NL>(y);
-        }
-    } else {
-        neg = qf < q;
-        if (neg) {
-#pragma unroll
-            for (int l = 0; l < NL; ++l) y[l] = -y[l];
-        }
-        propagate<NL>(y);
-        if (y[NL - 1] < 0) {
-            neg = !neg;
-#pragma unroll
-            for (int l = 0; l < NL; ++l) y[l] = -y[l];
-            propagate<NL>(y);
-        }
+        for (int l = 0; l < L; ++l) d[l] = y[l];
+        add_words<L, true>(d, cs->Mhalf32);
+        if ((int32_t)d[L - 1] >= 0) add_words<L, true>(y, cs->M32);
     }
-    // to_double_256 (crt_math.hpp:73-80) on the 32-bit words w of |Y| (16-bit limbs in pairs): the
-    // 64-bit word d_i = w[2i+1] 2^32 + w[2i] converted with one rounding, as one fma of its exact
-    // halves, already scaled by its power of two 2^(64 i) (exact); then the reference's additions in
-    // its order (0 + RN(d0) is RN(d0); the word d3 is zero).
-    uint32_t w[6];
+    // |Y| and the sign
+    const uint32_t neg = (uint32_t)((int32_t)y[L - 1] >> 31);
+    carry = neg & 1u;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        const uint32_t lo = 2 * k < NL ? (uint32_t)y[2 * k] : 0u;
-        const uint32_t hi = 2 * k + 1 < NL ? (uint32_t)y[2 * k + 1] : 0u;
-        w[k] = lo | (hi << 16);
+    for (int l = 0; l < L; ++l) y[l] = __builtin_addc(y[l] ^ neg, 0u, carry, &carry);
+    // to_double_256 (crt_math.hpp:73-80): the 64-bit word d_i = y[2i+1] 2^32 + y[2i] converted with one
+    // rounding, as one fma of its exact halves, already scaled by its power of two 2^(64 i) (exact);
+    // then the reference's additions in its order (0 + RN(d0) is RN(d0); the word d3 is zero).
+    double f = (double)y[0];
+    if (L > 1) f = fma((double)y[L > 1 ? 1 : 0], 0x1p32, f);
+    if (L > 2) {
+        double d1 = (double)y[L > 2 ? 2 : 0] * 0x1p64;
+        if (L > 3) d1 = fma((double)y[L > 3 ? 3 : 0], 0x1p96, d1);
+        f = f + d1;
     }
-    const double d0 = fma((double)w[1], 0x1p32, (double)w[0]);
-    const double d1 = fma((double)w[3], 0x1p96, (double)w[2] * 0x1p64);
-    const double d2 = fma((double)w[5], 0x1p160, (double)w[4] * 0x1p128);
-    double f = d0 + d1;
-    f = f + d2;
-    return (neg && f != 0.0) ? -f : f;  // Y = 0 is +0 as in the reference
-}
-
-template <int S>
-__device__ __forceinline__ double crt_value(const uint32_t (&c)[S], const CrtSet* __restrict__ cs) {
-    int32_t y[CrtShape<S>::NL];
-    crt_limbs<S>(c, cs, y);
-    return crt_finish<S>(y, cs);
+    if (L > 4) f = f + (double)y[L > 4 ? 4 : 0] * 0x1p128;
+    // Y = 0 is +0 as in the reference: neg is 0 there
+    return __longlong_as_double(__double_as_longlong(f) ^ ((int64_t)((uint64_t)(neg & 0x80000000u) << 32)));
 }
 
 // C[row * ldc + col] = alpha * x + beta * C[...] as fma(alpha, x, beta * C); beta == 0 does not
@@ -175,31 +120,15 @@ __device__ __forceinline__ void recon_digits_block(const uint8_t* __restrict__ d
     const int64_t row0 = R * 32 + 8 * wd + 4 * (lane >> 5);
     if (col >= N || row0 >= M) return;
     const uint8_t* base = dg + ((R * (Np >> 5) + Q) << 10) + t * 4;
-    constexpr int NJ = (S + 3) / 4;
-    uint32_t w[4 * NJ];
+    uint32_t w[S];
 #pragma unroll
-    for (int s = 0; s < 4 * NJ; ++s) w[s] = s < S ? *reinterpret_cast<const uint32_t*>(base + s * plane) : 0u;
+    for (int s = 0; s < S; ++s) w[s] = *reinterpret_cast<const uint32_t*>(base + s * plane);
     const int32_t sb = shB[col];
-    // Not unrolled: the CRT tables are then re-read through the scalar cache for each element
-    // instead of being held in (spilled) scalar registers across all four.
-#pragma unroll 1
+#pragma unroll
     for (int b = 0; b < 4; ++b) {
         const int64_t row = row0 + b;
         if (row < M) {
-            // Element b's digits, four moduli to a word: byte b of w[4j..4j+3] (v_perm_b32 byte
-            // selectors: 0-3 pick from the second source, 4-7 from the first, 0x0c gives zero).
-            const uint32_t pick = 0x0c0c0000u | ((4u + b) << 8) | (uint32_t)b;
-            uint32_t P[NJ];
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                const uint32_t lo = __builtin_amdgcn_perm(w[4 * j + 1], w[4 * j], pick);
-                const uint32_t hi = __builtin_amdgcn_perm(w[4 * j + 3], w[4 * j + 2], pick);
-                P[j] = lo | (hi << 16);
-            }
-            int32_t y[CrtShape<S>::NL];
-            crt_limbs_packed<S>(P, cs, y);
-            const double f = crt_finish<S>(y, cs);
-            const double x = ldexp(f, -(shA[row] + sb));
+            const double x = ldexp(crt_value<S>(w, b, cs), -(shA[row] + sb));
             if (PLAIN) Cout[row * ldc + col] = x;
             else store_c(Cout, row * ldc + col, x, alpha, beta);
         }
