@@ -120,8 +120,7 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
         uint8_t* plane;  // digit plane of modulus s (a partial plane for splits j > 0)
         int64_t Kp, Np, M, N;
         int tm, tn, k0, KT;  // K steps [k0, k0 + KT) of BK bytes
-        uint32_t m;
-        double rcp;
+        uint32_t m, minv, bias;
     };
     constexpr int kSteps128 = 128 / C::BK;  // K steps per 128-byte K block
     auto decode = [&](int64_t wi) {
@@ -147,7 +146,8 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
         t.plane = (j == 0 ? P.dg : P.dgp + (int64_t)(j - 1) * P.S * plane) + (int64_t)s * plane;
         const auto& cs = as_constant(g.crt)->set[P.S - 1];
         t.m = cs.m[s];
-        t.rcp = cs.rcp[s];
+        t.minv = cs.minv[s];
+        t.bias = cs.bias[s];
         return t;
     };
     Item cur = decode(w);
@@ -169,10 +169,10 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
                             (real ? nxt.k0 + j : cur.k0 + cur.KT - 1) * C::BK};
         };
         v16i acc[C::FM][C::FN];
-        zero_acc<C>(acc);
+        fill_acc<C>(acc, (int)cur.bias);
         mainloop_chain<C>(acc, smem, base, cur.KT, own_of(cur), tail);
         store_digits<C, true, true>(acc, cur.plane, cur.Np, (int64_t)cur.tm * C::BM + wm * C::WTM,
-                                    (int64_t)cur.tn * C::BN + wn * C::WTN, cur.M, cur.N, cur.m, cur.rcp, lane);
+                                    (int64_t)cur.tn * C::BN + wn * C::WTN, cur.M, cur.N, cur.m, cur.minv, lane);
         if (!more) break;
         // the epilogue's stores are drained by the next item's first stage wait
         base = (base + cur.KT) & 1;

@@ -6,8 +6,8 @@
 // v_mfma_i32_32x32x32_i8 fragments with exact INT32 accumulation (mainloop in igemm_core.hpp).
 //
 //   Scheme II (reference: rocblas_gemm_strided_batched_ex, src/hip/pipeline.hip:237-245):
-//     one launch covers every (tile, modulus); the epilogue reduces C_s to the CRT digit
-//     c_s = C_s mod m_s and stores it as one byte (layout below), or stores
+//     one launch covers every (tile, modulus); the epilogue reduces C_s to its CRT digit
+//     modulo m_s (stored_digit) and stores it as one byte (layout below), or stores
 //     the raw INT32 C_s planes in the reference's [s][M][N] layout.
 //   Scheme I (reference: rocblas_gemm_ex loop, pipeline.hip:110-135): one launch covers every
 //     (group g, tile); the pairs of group g = s + t accumulate into one INT32 fragment set and
@@ -87,7 +87,7 @@ struct S2Args {
     int S, KT, tiles_m, tiles_n;
     int tm0;               // first tile row: the launch covers tile rows [tm0, tm0 + tiles_m)
     void* out;             // digits or int32 planes
-    const CrtSet* crt;     // device copy (m, rcp used)
+    const CrtSet* crt;     // device copy (m, minv, bias used)
     unsigned* queue;       // 8 work counters, zero at launch (dynamic order), or null (static order)
     int split, kts;        // K parts and K steps per part (SPLIT only)
 };
@@ -113,8 +113,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         int s, tm, tn, j, k0, KT;
         const int8_t* a;
         const int8_t* b;
-        uint32_t m;
-        double rcp;
+        uint32_t m, minv, bias;
     };
     auto decode = [&](int64_t wi) {
         Item t;
@@ -136,7 +135,8 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         t.b = p.B + (int64_t)t.s * p.Np * p.Kp + (int64_t)t.tn * C::BN * p.Kp;
         // scalar loads: counted by lgkmcnt, so the epilogue does not wait for the direct loads
         t.m = as_constant(p.crt)->m[t.s];
-        t.rcp = as_constant(p.crt)->rcp[t.s];
+        t.minv = as_constant(p.crt)->minv[t.s];
+        t.bias = as_constant(p.crt)->bias[t.s];
         return t;
     };
     Item cur = decode(c.w);
@@ -156,7 +156,8 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
                             (real ? nxt.k0 + j : cur.k0 + cur.KT - 1) * C::BK};
         };
         v16i acc[C::FM][C::FN];
-        zero_acc<C>(acc);
+        if (DIGITS) fill_acc<C>(acc, (int)cur.bias);
+        else zero_acc<C>(acc);
         mainloop_chain<C>(acc, smem, base, cur.KT, own_of(cur), tail);
         // The item after next (dynamic order).  Only thread 0's ticket is used, so the other lanes
         // leave it unset: a value merged from both paths would be copied as soon as the atomic
@@ -167,7 +168,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         if (DIGITS) {
             uint8_t* plane = reinterpret_cast<uint8_t*>(p.out) + ((int64_t)cur.j * p.S + s) * p.Mp * p.Np;
             store_digits<C, false>(acc, plane, p.Np, (int64_t)tm * C::BM + wm * C::WTM, (int64_t)tn * C::BN + wn * C::WTN,
-                                   p.M, p.N, cur.m, cur.rcp, lane);
+                                   p.M, p.N, cur.m, cur.minv, lane);
         } else {
             int32_t* o = reinterpret_cast<int32_t*>(p.out) + (int64_t)s * p.M * p.N;
 #pragma unroll

@@ -1,7 +1,8 @@
 """The integer steps of Scheme II's reconstruction (crt_value, ozablas_amd/csrc/recon_core.hpp, with the
 constants of crt_host.cpp), transcribed: group sums u_g, the quotient estimate with its ambiguous
 fractions, and Y = X - q M, against the definition (X mod M, minus M from floor(M/2) on), with every
-intermediate inside the width the device holds it in.  Host only; the device code is checked bit
+intermediate inside the width the device holds it in; and the stored digit of an INT32 product
+(stored_digit, oza_device.hpp).  Host only; the device code is checked bit
 for bit by the GPU parity tests."""
 import random
 
@@ -19,7 +20,7 @@ def tables(moduli):
         for m in ms:
             P *= m
         E = [P // m for m in ms]
-        w = sum(pow(M // m, -1, m) * pow(e, -1, m) * e for m, e in zip(ms, E)) % P
+        w = sum(-2 ** 32 * pow(M // m, -1, m) * pow(e, -1, m) * e for m, e in zip(ms, E)) % P
         err += sum((m - 1) * e for m, e in zip(ms, E))
         groups.append((s0, E, w * (M // P), (w << 32) // P))
     err += 2 + (0 if M >> 64 else (1 << 31) // M)
@@ -61,4 +62,16 @@ def test_grouped_crt(orc, S):
     xs += [rng.randrange(int(0.43 * M), int(0.57 * M) + 1) % M for _ in range(400)]  # the ambiguous fractions
     for x in xs:
         want = x - M if x >= half else x
-        assert value([x % m for m in moduli], M, groups, amb, limbs) == want, (S, x)
+        assert value([-x * pow(2, -32, m) % m for m in moduli], M, groups, amb, limbs) == want, (S, x)
+
+
+def test_stored_digit(orc):
+    top = 137438 * 125 ** 2  # the largest |C_s| of an accepted K
+    rng = random.Random(7)
+    for m in (int(m) for m in orc.moduli()):
+        minv, bias = pow(m, -1, 1 << 32), -(-2 ** 31 // m) * m
+        vs = [0, 1, -1, m, -m, top, -top, top - m, m - top] + [rng.randint(-top, top) for _ in range(3000)]
+        for v in vs:
+            u = v + bias
+            assert 0 <= u < 1 << 32
+            assert (u * minv % (1 << 32)) * m >> 32 == -v * pow(2, -32, m) % m, (m, v)
