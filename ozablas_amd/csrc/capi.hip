@@ -326,13 +326,24 @@ static int enqueue_pipeline(int scheme, oza_ctx ctx, size_t M, size_t N, size_t 
     if (t) ev = ctx->ev;
     else if (ctx->ring_on && ctx->ring_n < oza_context::kRing) ev = ctx->ring + 5 * ctx->ring_n++;
     if (ev) OZA_HIP(hipEventRecord(ev[0], st), "event");
-    if (scheme == 2) {
-        const int kp = scheme2_kparam(S, K);
-        OZA_HIP(launch_stats(d, A, B, kp, shA, shB, st, ctx->queue_dev, 8 * oza_context::kMaxBands),
-                "step 1 launch");
+    const int beta = scheme == 1 ? scheme1_beta(K) : 0;
+    const int kp = scheme == 2 ? scheme2_kparam(S, K) : 0;
+    const int nqueue = 8 * oza_context::kMaxBands;
+    if (one_pass(d)) {  // short K: one launch, counted as step 2
         if (ev) OZA_HIP(hipEventRecord(ev[1], st), "event");
-        OZA_HIP(launch_slice_s2(d, A, B, shA, shB, Asl, Bsl, st), "step 2 launch");
-        if (ev) OZA_HIP(hipEventRecord(ev[2], st), "event");
+        OZA_HIP(launch_one_pass(scheme, d, scheme == 1 ? beta : kp, A, B, shA, shB, Asl, Bsl, st, ctx->queue_dev,
+                                nqueue),
+                "step 2 launch");
+    } else {
+        OZA_HIP(launch_stats(d, A, B, kp, shA, shB, st, ctx->queue_dev, nqueue), "step 1 launch");
+        if (ev) OZA_HIP(hipEventRecord(ev[1], st), "event");
+        if (scheme == 2)
+            OZA_HIP(launch_slice_s2(d, A, B, shA, shB, Asl, Bsl, st, core::residue_words(kp)), "step 2 launch");
+        else
+            OZA_HIP(launch_slice_s1(d, beta, A, B, shA, shB, Asl, Bsl, st), "step 2 launch");
+    }
+    if (ev) OZA_HIP(hipEventRecord(ev[2], st), "event");
+    if (scheme == 2) {
         const int nb = pipeline_bands(ctx, 2, d);
         if (nb > 1) {
             if (int r = enqueue_banded(ctx, 2, d, nb, Asl, Bsl, Ctc, shA, shB, C, ev ? ev[3] : nullptr)) return r;
@@ -347,12 +358,6 @@ static int enqueue_pipeline(int scheme, oza_ctx ctx, size_t M, size_t N, size_t 
                     "step 4 launch");
         }
     } else {
-        const int sbeta = scheme1_beta(K);
-        OZA_HIP(launch_stats(d, A, B, 0, shA, shB, st, ctx->queue_dev, 8 * oza_context::kMaxBands),
-                "step 1 launch");
-        if (ev) OZA_HIP(hipEventRecord(ev[1], st), "event");
-        OZA_HIP(launch_slice_s1(d, sbeta, A, B, shA, shB, Asl, Bsl, st), "step 2 launch");
-        if (ev) OZA_HIP(hipEventRecord(ev[2], st), "event");
         const int nb = pipeline_bands(ctx, 1, d);
         if (nb > 1) {
             if (int r = enqueue_banded(ctx, 1, d, nb, Asl, Bsl, Ctc, shA, shB, C, ev ? ev[3] : nullptr)) return r;
@@ -360,7 +365,7 @@ static int enqueue_pipeline(int scheme, oza_ctx ctx, size_t M, size_t N, size_t 
             OZA_HIP(launch_igemm_s1_blocked(d, Asl, Bsl, static_cast<int32_t*>(Ctc), st, ctx->queue_dev),
                     "step 3 launch");
             if (ev) OZA_HIP(hipEventRecord(ev[3], st), "event");
-            OZA_HIP(launch_recon_s1_blocked(d, sbeta, static_cast<const int32_t*>(Ctc), shA, shB, C, st),
+            OZA_HIP(launch_recon_s1_blocked(d, beta, static_cast<const int32_t*>(Ctc), shA, shB, C, st),
                     "step 4 launch");
         }
     }
@@ -582,7 +587,7 @@ int oza_stage2_slices(oza_ctx ctx, int scheme, size_t M, size_t N, size_t K, int
     OZA_STAGE_PROLOGUE(scheme)
     const Operand a{A, (int64_t)K, true}, b{B, (int64_t)N, false};
     if (scheme == 2)
-        OZA_HIP(launch_slice_s2(d, a, b, shA, shB, Asl, Bsl, st), "step 2 launch");
+        OZA_HIP(launch_slice_s2(d, a, b, shA, shB, Asl, Bsl, st, 3), "step 2 launch");  // the caller's shifts
     else
         OZA_HIP(launch_slice_s1(d, scheme1_beta(K), a, b, shA, shB, Asl, Bsl, st), "step 2 launch");
     return OZA_SUCCESS;

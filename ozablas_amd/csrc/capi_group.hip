@@ -395,7 +395,7 @@ int build_plan(const GroupModel& model, int n, const size_t* M, const size_t* N,
     for (int i = 0; i < n; ++i) {
         GroupProblem& P = out.probs[i];
         P.kparam = scheme2_kparam(P.S, (size_t)P.K);
-        P.wide = P.kparam > 72 ? 1 : 0;  // residue split limit, as in the single-problem slicing
+        P.words = core::residue_words(P.kparam);
         const core::StatShape h = core::stat_shape(P.M, P.N, P.K);
         P.chunksA = h.chunksA;
         P.nblkA = h.nblkA;
@@ -491,7 +491,7 @@ hipError_t enqueue_plan(const DevPlan& d, const CrtTables* crt, hipStream_t st, 
     L.probs = d.probs;
     L.ptrs = d.ptrs;
     L.crt = crt;
-    L.rc = core::make_residue_consts(kMaxSlices);
+    L.rc = core::make_residue_consts();
     L.gemm_share = gemm_share;
     hipError_t e = hipSuccess;
     auto stage = [&](int s) {

@@ -28,7 +28,7 @@ struct GroupProblem {
     int8_t* Bsl;                  // [S][Np][Kp] fragment-tiled
     uint8_t* dg;                  // [S][Mp][Np] blocked digits
     uint8_t* dgp;                 // [split - 1][S][Mp][Np] partial digits of splits 1.. (split > 1)
-    int32_t S, kparam, wide, tile;
+    int32_t S, kparam, words, tile;  // words: 32-bit words per scaled value (residue_words)
     int32_t tiles_m, tiles_n;
     int32_t split, kbs;           // K splits of the GEMM (1: none), 128-byte K blocks per split
     int64_t chunksA, nblkA, colblkB, nblkB;  // step-1 blocks of A and B

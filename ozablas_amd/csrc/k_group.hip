@@ -57,34 +57,44 @@ __global__ void __launch_bounds__(256) k_group_finalize(GroupLaunch g) {
 }
 
 // Steps 1 and 2 of A in one pass for problems with short K (fused_s2_A_block).
+template <int ND>
+__device__ __forceinline__ void group_fuse_a(const GroupProblem& P, const double* A, const ResidueConsts& rc,
+                                             int64_t blk, uint32_t* s_key, int32_t* s_shift) {
+    fused_s2_A_block<ND>(A, P.K, P.M, P.K, P.Mp, P.Kp, P.kparam, P.S, rc, P.shA, P.Asl, blk, s_key, s_shift);
+}
+
 __global__ void __launch_bounds__(kFuseThreads) k_group_fuse_a(GroupLaunch g) {
     __shared__ uint32_t s_key[kFuseThreads];
     __shared__ int32_t s_shift[128];
     const GItem it = g.items[blockIdx.x];
     const GroupProblem& P = g.probs[it.prob];
     const GroupPtrs q = g.ptrs[it.prob];
-    if (P.wide)
-        fused_s2_A_block<true>(q.A, P.K, P.M, P.K, P.Mp, P.Kp, P.kparam, P.S, g.rc, P.shA, P.Asl, it.local, s_key,
-                               s_shift);
-    else
-        fused_s2_A_block<false>(q.A, P.K, P.M, P.K, P.Mp, P.Kp, P.kparam, P.S, g.rc, P.shA, P.Asl, it.local, s_key,
-                                s_shift);
+    switch (P.words) {  // uniform per workgroup
+        case 1: group_fuse_a<1>(P, q.A, g.rc, it.local, s_key, s_shift); break;
+        case 2: group_fuse_a<2>(P, q.A, g.rc, it.local, s_key, s_shift); break;
+        default: group_fuse_a<3>(P, q.A, g.rc, it.local, s_key, s_shift); break;
+    }
+}
+
+template <int ND>
+__device__ __forceinline__ void group_slice(const GroupProblem& P, const GroupPtrs& q, const ResidueConsts& rc,
+                                            int64_t l) {
+    const int64_t kb = P.Kp / 128;
+    const bool is_a = l < P.slA;
+    if (!is_a) l -= P.slA;
+    const int64_t bx = l / kb, by = l - bx * kb;
+    if (is_a) slice_s2_A_block<ND, true>(q.A, P.K, P.shA, P.M, P.K, P.Mp, P.Kp, P.S, rc, P.Asl, bx, by);
+    else slice_s2_B_block<ND, true>(q.B, P.N, P.shB, P.K, P.N, P.Np, P.Kp, P.S, rc, P.Bsl, bx, by);
 }
 
 __global__ void __launch_bounds__(kSliceThreads) k_group_slice(GroupLaunch g) {
     const GItem it = g.items[blockIdx.x];
     const GroupProblem& P = g.probs[it.prob];
     const GroupPtrs q = g.ptrs[it.prob];
-    const int64_t kb = P.Kp / 128;
-    if (it.local < P.slA) {
-        const int64_t bx = it.local / kb, by = it.local - bx * kb;
-        if (P.wide) slice_s2_A_block<true, true>(q.A, P.K, P.shA, P.M, P.K, P.Mp, P.Kp, P.S, g.rc, P.Asl, bx, by);
-        else slice_s2_A_block<false, true>(q.A, P.K, P.shA, P.M, P.K, P.Mp, P.Kp, P.S, g.rc, P.Asl, bx, by);
-    } else {
-        const int64_t l = it.local - P.slA;
-        const int64_t bx = l / kb, by = l - bx * kb;
-        if (P.wide) slice_s2_B_block<true, true>(q.B, P.N, P.shB, P.K, P.N, P.Np, P.Kp, P.S, g.rc, P.Bsl, bx, by);
-        else slice_s2_B_block<false, true>(q.B, P.N, P.shB, P.K, P.N, P.Np, P.Kp, P.S, g.rc, P.Bsl, bx, by);
+    switch (P.words) {  // uniform per workgroup
+        case 1: group_slice<1>(P, q, g.rc, it.local); break;
+        case 2: group_slice<2>(P, q, g.rc, it.local); break;
+        default: group_slice<3>(P, q, g.rc, it.local); break;
     }
 }
 

@@ -3,7 +3,7 @@
 // Scheme II (reference: src/pipeline/step2_slicing.hpp:29-38, 110-206): x = ldexp(a, shift),
 // t = rint(x) (round-half-even, which is what both the reference's llrint fast path and its
 // rint/fmod heavy path round to), residue r_s = symmetric residue of t mod m_s.  Any exact
-// method yields the same bytes; sym_residue uses two FMAs per modulus.
+// method yields the same bytes; sym_residue works on t as one to three 32-bit words.
 //
 // Scheme I (reference: step2_slicing.hpp:20-25, 44-100): the reference's exact sequence of
 // FP64 operations, sigma = 0.75 * 2^(E+1-beta+53-beta*s), a_s = (a + sigma) - sigma,
@@ -16,6 +16,8 @@
 // a wave's 64 units form contiguous runs of the tiled layout.
 #pragma clang fp contract(off)
 
+#include <algorithm>
+
 #include "slice_core.hpp"
 
 namespace oza {
@@ -23,18 +25,51 @@ namespace {
 
 using namespace core;
 
+// Blocks a one-pass launch aims for by dealing a row block's planes to several blocks: one per CU.
+// 1024^3, S = 16 (128 row blocks): 53 us per call undivided, 46 us in two parts, 48 in four, 55 in eight.
+constexpr int64_t kPassTargetBlocks = 256;
+
 // Blocks [0, a.nblk) slice operand a into its planes, the rest operand b.
-template <bool WIDE>
+template <int ND>
 __global__ void __launch_bounds__(kSliceThreads)
     k_slice_s2(SliceOp a, SliceOp b, int64_t K, int64_t Kp, int S, ResidueConsts rc) {
-    if ((int64_t)blockIdx.x < a.nblk) slice_s2_op_block<WIDE>(a, K, Kp, S, rc, blockIdx.x);
-    else slice_s2_op_block<WIDE>(b, K, Kp, S, rc, (int64_t)blockIdx.x - a.nblk);
+    if ((int64_t)blockIdx.x < a.nblk) slice_s2_op_block<ND>(a, K, Kp, S, rc, blockIdx.x);
+    else slice_s2_op_block<ND>(b, K, Kp, S, rc, (int64_t)blockIdx.x - a.nblk);
 }
 
 __global__ void __launch_bounds__(kSliceThreads)
     k_slice_s1(SliceOp a, SliceOp b, int64_t K, int64_t Kp, int S, int beta) {
     if ((int64_t)blockIdx.x < a.nblk) slice_s1_op_block(a, K, Kp, S, beta, blockIdx.x);
     else slice_s1_op_block(b, K, Kp, S, beta, (int64_t)blockIdx.x - a.nblk);
+}
+
+// Steps 1 and 2 of both operands in one launch (pass_block).  Block b -> part and row block: sets of 8
+// consecutive row blocks (of operand 0, then operand 1), each set's parts after one another.
+template <int ND, int NU>
+__global__ void __launch_bounds__(kPassThreads) k_pass(PassArgs g, ResidueConsts rc) {
+    __shared__ uint32_t s_key[kPassThreads];
+    __shared__ int32_t s_shift[64];
+    if (blockIdx.x == 0 && (int)threadIdx.x < g.nzero) g.zero[threadIdx.x] = 0;
+    const int64_t set = blockIdx.x / (8 * g.parts);
+    const int in = (int)(blockIdx.x - set * 8 * g.parts);
+    const int part = in >> 3;
+    int64_t rb = set * 8 + (in & 7);
+    const int w = rb >= g.op[0].nrow;
+    if (w) rb -= g.op[0].nrow;
+    const PassOp& o = g.op[w];
+    if (rb >= o.nrow) return;  // past the last set's row blocks (whole block)
+    if (o.kcontig) pass_block<ND, NU, true>(o, g, rc, rb, part, s_key, s_shift);
+    else pass_block<ND, NU, false>(o, g, rc, rb, part, s_key, s_shift);
+}
+
+template <int ND>
+hipError_t launch_pass_words(const PassArgs& g, const ResidueConsts& rc, unsigned grid, hipStream_t st) {
+    switch (pass_units(g.Kp)) {
+        case 1: k_pass<ND, 1><<<grid, kPassThreads, 0, st>>>(g, rc); break;
+        case 2: k_pass<ND, 2><<<grid, kPassThreads, 0, st>>>(g, rc); break;
+        default: k_pass<ND, 4><<<grid, kPassThreads, 0, st>>>(g, rc); break;
+    }
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------- unpack to planar layout
@@ -63,17 +98,16 @@ __global__ void k_unpack_B(const int8_t* __restrict__ in, int64_t K, int64_t N, 
 }  // namespace
 
 hipError_t launch_slice_s2(const Dims& d, const Operand& A, const Operand& B, const int32_t* shift_A,
-                           const int32_t* shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st) {
-    const ResidueConsts rc = make_residue_consts(d.S);
-    // |t| <= 2^kparam.  Up to kparam = 72 the two-part split alone is exact (|v| < 2^48, see
-    // sym_residue); above it the high part is first reduced mod m (WIDE, exact for |t| < 2^80, which
-    // covers K_param's largest value, 75 at S = 20 and K <= 2: test_stage2_tiny_K_wide_residues).
-    const bool wide = scheme2_kparam(d.S, (size_t)d.K) > 72;
+                           const int32_t* shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st, int words) {
+    const ResidueConsts rc = make_residue_consts();
     const SliceOp a = make_slice_op(A.p, d.M, d.Mp, A.ld, A.kcontig, d.Kp, shift_A, A_sl);
     const SliceOp b = make_slice_op(B.p, d.N, d.Np, B.ld, B.kcontig, d.Kp, shift_B, B_sl);
     const unsigned grid = (unsigned)(a.nblk + b.nblk);
-    if (wide) k_slice_s2<true><<<grid, kSliceThreads, 0, st>>>(a, b, d.K, d.Kp, d.S, rc);
-    else k_slice_s2<false><<<grid, kSliceThreads, 0, st>>>(a, b, d.K, d.Kp, d.S, rc);
+    switch (words) {
+        case 1: k_slice_s2<1><<<grid, kSliceThreads, 0, st>>>(a, b, d.K, d.Kp, d.S, rc); break;
+        case 2: k_slice_s2<2><<<grid, kSliceThreads, 0, st>>>(a, b, d.K, d.Kp, d.S, rc); break;
+        default: k_slice_s2<3><<<grid, kSliceThreads, 0, st>>>(a, b, d.K, d.Kp, d.S, rc); break;
+    }
     return hipGetLastError();
 }
 
@@ -83,6 +117,38 @@ hipError_t launch_slice_s1(const Dims& d, int beta, const Operand& A, const Oper
     const SliceOp b = make_slice_op(B.p, d.N, d.Np, B.ld, B.kcontig, d.Kp, shift_B, B_sl);
     k_slice_s1<<<(unsigned)(a.nblk + b.nblk), kSliceThreads, 0, st>>>(a, b, d.K, d.Kp, d.S, beta);
     return hipGetLastError();
+}
+
+bool one_pass(const Dims& d) { return d.Kp <= kPassMaxKp; }
+
+hipError_t launch_one_pass(int scheme, const Dims& d, int offset, const Operand& A, const Operand& B, int32_t* shift_A,
+                           int32_t* shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st, uint32_t* zero, int nzero) {
+    PassArgs g;
+    g.K = d.K;
+    g.Kp = d.Kp;
+    g.S = d.S;
+    g.R = pass_rows(d.Kp);
+    g.offset = offset;
+    g.zero = zero;
+    g.nzero = nzero;
+    if (nzero > kPassThreads) return hipErrorInvalidValue;
+    auto op = [&](const Operand& X, int64_t rows, int64_t rows_p, int32_t* shift, int8_t* out) {
+        return PassOp{X.p, rows, rows_p, X.ld, X.kcontig, shift, out, ((rows + 31) / 32 * 32 + g.R - 1) / g.R};
+    };
+    g.op[0] = op(A, d.M, d.Mp, shift_A, A_sl);
+    g.op[1] = op(B, d.N, d.Np, shift_B, B_sl);
+    const int64_t nrow = g.op[0].nrow + g.op[1].nrow;
+    g.parts = 1;
+    while (2 * g.parts <= std::min(d.S, 8) && nrow * g.parts < kPassTargetBlocks) g.parts *= 2;
+    const int64_t grid = (nrow + 7) / 8 * 8 * g.parts;
+    if (grid * kPassThreads > (int64_t)UINT32_MAX) return hipErrorInvalidValue;
+    const ResidueConsts rc = make_residue_consts();
+    if (scheme == 1) return launch_pass_words<0>(g, rc, (unsigned)grid, st);
+    switch (residue_words(offset)) {
+        case 1: return launch_pass_words<1>(g, rc, (unsigned)grid, st);
+        case 2: return launch_pass_words<2>(g, rc, (unsigned)grid, st);
+        default: return launch_pass_words<3>(g, rc, (unsigned)grid, st);
+    }
 }
 
 hipError_t launch_unpack_A(const Dims& d, const int8_t* A_sl, int8_t* out, hipStream_t st) {

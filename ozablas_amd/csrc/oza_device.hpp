@@ -28,6 +28,34 @@ __host__ __device__ __forceinline__ int exp_from_key(uint32_t key) {
     return be - 1022;
 }
 
+// The largest exponent key of 16 values.  Finite values' keys are their high words without the sign;
+// anything else is rare and takes the exact form.
+constexpr uint32_t kNonFinite = 0x7ff00000u;
+__device__ __forceinline__ uint32_t high16(const double (&a)[16]) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+        m = max(m, (uint32_t)((uint64_t)__double_as_longlong(a[j]) >> 32) & 0x7fffffffu);
+    return m;
+}
+__device__ __forceinline__ uint32_t exp_key16(const double (&a)[16]) {
+    uint32_t m = high16(a);
+    if (m >= kNonFinite) {
+        m = 0;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) m = max(m, exp_key(a[j]));
+    }
+    return m;
+}
+// Infinities and NaNs have residue 0 for every modulus.
+__device__ __forceinline__ void drop_non_finite(double (&a)[16]) {
+    if (high16(a) >= kNonFinite) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            if (((uint64_t)__double_as_longlong(a[j]) >> 32 & kNonFinite) == kNonFinite) a[j] = 0.0;
+    }
+}
+
 // Wave-wide max of a 32-bit unsigned value: DPP within each 16-lane row (quad permutes,
 // half-row and row mirrors), then two cross-row exchanges.  All 64 lanes must be active.
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
@@ -40,25 +68,35 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
     return v;
 }
 
-// ---- Scheme II residues ------------------------------------------------------------------------
-// Symmetric residue of an integer-valued double t (|t| < 2^80) modulo an odd m < 256, in
-// [-(m-1)/2, (m-1)/2].  t is split exactly as t = th * 2^32 + tl (tl in [0, 2^32)); then
-// v = th * (2^32 mod m) + tl is exact (|v| < 2^57 ... in practice < 2^46) and congruent to t.
-// rint(v / m) is the nearest integer to v/m: the exact quotient is at least 1/(2m) away from a
-// half-integer and the product v * rcp(m) errs by far less, so r = v - m * rint(v * rcp) is the
-// symmetric residue itself, computed exactly by one FMA.
-struct SplitInt {
-    double th, tl;
-};
-__device__ __forceinline__ SplitInt split32(double t) {
-    const double th = floor(t * 0x1p-32);
-    const double tl = fma(-th, 0x1p32, t);
-    return {th, tl};
+// ---- Scheme II residues and digits ---------------------------------------------------------------
+// Integer-valued t, |t| <= 2^(32 ND - 2), as the ND 32-bit words of t + 2^(32 ND - 1) (word 0 lowest).
+template <int ND>
+__device__ __forceinline__ void int_words(double t, uint32_t (&w)[ND]) {
+    static_assert(ND >= 1 && ND <= 3, "one to three words");
+#pragma unroll
+    for (int n = 0; n + 1 < ND; ++n) {  // exact: t has at most 53 bits, so t - floor(t 2^-32) 2^32 < 2^32 does too
+        const double top = floor(t * 0x1p-32);
+        w[n] = (uint32_t)fma(-top, 0x1p32, t);
+        t = top;
+    }
+    w[ND - 1] = (uint32_t)(int)t;
+    w[ND - 1] ^= 0x80000000u;
 }
-__device__ __forceinline__ int sym_residue(SplitInt t, double m, double rcp, double c32) {
-    const double v = fma(t.th, c32, t.tl);
-    const double q = rint(v * rcp);
-    return (int)fma(-q, m, v);
+
+// Symmetric residue of t mod an odd m < 256, in [-(m-1)/2, (m-1)/2], from t's words: d, the sum of the
+// 4 ND bytes times wt (byte k of wt[n] = -2^32 2^(8(4n+k)) mod m) plus init, which takes the words'
+// bias off, is congruent to -2^32 t and below 2^20.  With p = d m^-1 mod 2^32 taken as a signed number,
+// p m = r 2^32 + d for r = floor(p m / 2^32), so r is congruent to -2^-32 d = t, and |p| <= 2^31
+// bounds r to the symmetric range: r + d / 2^32 = p m / 2^32 is in [-m/2, m/2) and d < 2^31 / m keeps
+// r > -m/2.  ND + 2 full-rate integer operations against five in FP64 (fma, multiply, rint, fma,
+// convert), on ND registers per value instead of four.
+template <int ND>
+__device__ __forceinline__ int sym_residue(const uint32_t (&w)[ND], const uint32_t (&wt)[ND], uint32_t init, uint32_t m,
+                                           uint32_t minv) {
+    uint32_t d = init;
+#pragma unroll
+    for (int n = 0; n < ND; ++n) d = __builtin_amdgcn_udot4(w[n], wt[n], d, false);
+    return __mulhi((int)(d * minv), (int)m);
 }
 
 // Stored digit of an INT32 product v (K 125^2 < 2^31): d = -2^-32 v mod m, in [0, m).  u = v + bias, with

@@ -121,11 +121,17 @@ hipError_t launch_scale_c(const OutC& c, int64_t M, int64_t N, hipStream_t st);
 hipError_t launch_stats(const Dims& d, const Operand& A, const Operand& B, int32_t offset, int32_t* shift_A,
                         int32_t* shift_B, hipStream_t st, uint32_t* zero = nullptr, int64_t nzero = 0);
 
-// Step 2.
+// Step 2.  words: 32-bit words per scaled value, |rint(2^shift a)| <= 2^(32 words - 2)
+// (core::residue_words(K_param) with step 1's shifts).
 hipError_t launch_slice_s2(const Dims& d, const Operand& A, const Operand& B, const int32_t* shift_A,
-                           const int32_t* shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st);
+                           const int32_t* shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st, int words);
 hipError_t launch_slice_s1(const Dims& d, int beta, const Operand& A, const Operand& B, const int32_t* shift_A,
                            const int32_t* shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st);
+// Steps 1 and 2 in one launch, for shapes with one_pass(d): offset is K_param (scheme 2) or beta
+// (scheme 1); zero / nzero as in launch_stats.
+bool one_pass(const Dims& d);
+hipError_t launch_one_pass(int scheme, const Dims& d, int offset, const Operand& A, const Operand& B, int32_t* shift_A,
+                           int32_t* shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st, uint32_t* zero, int nzero);
 // Unpack product-layout operand planes to the reference's planar layout [s][rows][cols].
 hipError_t launch_unpack_A(const Dims& d, const int8_t* A_sl, int8_t* out, hipStream_t st);
 hipError_t launch_unpack_B(const Dims& d, const int8_t* B_sl, int8_t* out, hipStream_t st);

@@ -12,46 +12,91 @@ namespace core {
 
 constexpr int kSliceThreads = 256;
 
+// Constants of sym_residue: byte weights per word, the word bias' share, m and m^-1 mod 2^32.
 struct ResidueConsts {
-    double m[kMaxSlices];
-    double rcp[kMaxSlices];
-    double c32[kMaxSlices];  // 2^32 mod m
+    uint32_t wt[kMaxSlices][3];
+    uint32_t init[kMaxSlices][3];  // by word count - 1
+    uint32_t m[kMaxSlices], minv[kMaxSlices];
 };
 
-inline ResidueConsts make_residue_consts(int S) {
+inline ResidueConsts make_residue_consts() {
     ResidueConsts rc;
     for (int s = 0; s < kMaxSlices; ++s) {
-        const uint32_t m = kModuli[s];
-        rc.m[s] = (double)m;
-        rc.rcp[s] = 1.0 / (double)m;
-        rc.c32[s] = (double)((uint64_t(1) << 32) % m);
+        const uint64_t m = kModuli[s];
+        uint64_t p = (uint64_t(1) << 32) % m;  // 2^32 2^(8 i) mod m
+        const uint64_t p256 = 256 % m;
+        uint64_t w[13];
+        for (int i = 0; i < 13; ++i) {
+            w[i] = p;
+            p = p * p256 % m;
+        }
+        for (int n = 0; n < 3; ++n) {
+            rc.wt[s][n] = 0;
+            for (int k = 0; k < 4; ++k) rc.wt[s][n] |= (uint32_t)((m - w[4 * n + k]) % m) << (8 * k);
+            rc.init[s][n] = (uint32_t)(w[4 * n + 3] * 128 % m);  // 2^32 times the bias 2^(32 (n + 1) - 1)
+        }
+        uint32_t inv = 1;  // Newton: correct bits of m^-1 mod 2^32 double each time
+        for (int i = 0; i < 6; ++i) inv *= 2u - (uint32_t)m * inv;
+        rc.m[s] = (uint32_t)m;
+        rc.minv[s] = inv;
     }
-    (void)S;
     return rc;
 }
 
-// Symmetric residues of 16 split integers for one modulus, packed into 16 bytes.
-template <bool WIDE>
-__device__ __forceinline__ uint4 residues16(const SplitInt (&t)[16], double m, double rcp, double c32) {
+// Words sym_residue needs for |t| <= 2^kparam (K_param is at most 75: S = 20 and K <= 2).
+inline int residue_words(int kparam) { return kparam <= 30 ? 1 : kparam <= 62 ? 2 : 3; }
+
+template <int ND>
+struct Words16 {
+    uint32_t w[16][ND];
+};
+
+// rint(2^sh a) of 16 values as words.
+template <int ND>
+__device__ __forceinline__ void scaled_words16(const double (&a)[16], int sh, Words16<ND>& t) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) int_words<ND>(rint(ldexp(a[j], sh)), t.w[j]);
+}
+
+// Symmetric residues of 16 integers modulo m_s, packed into 16 bytes.
+template <int ND>
+__device__ __forceinline__ uint4 residues16(const Words16<ND>& t, const ResidueConsts& rc, int s) {
+    uint32_t wt[ND];
+#pragma unroll
+    for (int n = 0; n < ND; ++n) wt[n] = rc.wt[s][n];
     int r[16];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        SplitInt tj = t[j];
-        if (WIDE) {  // |t| up to 2^80: first reduce the high part modulo m (exact, |th| < 2^48)
-            const double q = rint(tj.th * rcp);
-            tj.th = fma(-q, m, tj.th);
-        }
-        r[j] = sym_residue(tj, m, rcp, c32);
-    }
+    for (int j = 0; j < 16; ++j) r[j] = sym_residue<ND>(t.w[j], wt, rc.init[s][ND - 1], rc.m[s], rc.minv[s]);
     return make_uint4(pack4_lo(r[0], r[1], r[2], r[3]), pack4_lo(r[4], r[5], r[6], r[7]),
                       pack4_lo(r[8], r[9], r[10], r[11]), pack4_lo(r[12], r[13], r[14], r[15]));
+}
+
+// 16 values of row `row` from K-byte 16c on, zero past K.  Ragged or unaligned: every load
+// unconditional (clamped index), padding zeroed after.
+__device__ __forceinline__ void load_row16(const double* __restrict__ A, int64_t lda, int64_t row, int64_t k0,
+                                           int64_t K, double (&a)[16]) {
+    const double* p = A + row * lda + k0;
+    if (k0 + 16 <= K && ((reinterpret_cast<uintptr_t>(p) & 15) == 0)) {
+#pragma unroll
+        for (int j = 0; j < 16; j += 2) {
+            const double2 v = *reinterpret_cast<const double2*>(p + j);
+            a[j] = v.x;
+            a[j + 1] = v.y;
+        }
+    } else {
+        const double* row_p = A + row * lda;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) a[j] = row_p[min(k0 + j, K - 1)];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) a[j] = k0 + j < K ? a[j] : 0.0;
+    }
 }
 
 // ---------------------------------------------------------------- Scheme II, K-contiguous rows
 // Operand element (row, k) at A[row * lda + k] (the reference's A; also op(B) = B^T stored N x K).
 // Block = 32 rows x 128 K; thread = row (tid % 32), 16-byte K chunk (tid / 32).  The 64 lanes of a
 // wave cover one whole 1 KiB fragment block.
-template <bool WIDE, bool NT = false>
+template <int ND, bool NT = false>
 __device__ __forceinline__ void slice_s2_A_block(const double* __restrict__ A, int64_t lda,
                                                  const int32_t* __restrict__ shift, int64_t M, int64_t K, int64_t Mp,
                                                  int64_t Kp, int S, const ResidueConsts& rc, int8_t* __restrict__ out,
@@ -59,35 +104,19 @@ __device__ __forceinline__ void slice_s2_A_block(const double* __restrict__ A, i
     const int64_t row = bx * 32 + (threadIdx.x & 31);
     const int64_t c = by * 8 + (threadIdx.x >> 5);
     const int64_t k0 = c * 16;
-    SplitInt t[16];
+    Words16<ND> t;
     if (row < M) {
-        const int sh = shift[row];
-        const double* p = A + row * lda + k0;
         double a[16];
-        if (k0 + 16 <= K && ((reinterpret_cast<uintptr_t>(p) & 15) == 0)) {
-#pragma unroll
-            for (int j = 0; j < 16; j += 2) {
-                const double2 v = *reinterpret_cast<const double2*>(p + j);
-                a[j] = v.x;
-                a[j + 1] = v.y;
-            }
-        } else {  // ragged or unaligned: every load unconditional (clamped index), padding zeroed after
-            const double* row_p = A + row * lda;
-#pragma unroll
-            for (int j = 0; j < 16; ++j) a[j] = row_p[min(k0 + j, K - 1)];
-#pragma unroll
-            for (int j = 0; j < 16; ++j) a[j] = k0 + j < K ? a[j] : 0.0;
-        }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) t[j] = split32(rint(ldexp(a[j], sh)));
+        load_row16(A, lda, row, k0, K, a);
+        drop_non_finite(a);
+        scaled_words16(a, shift[row], t);
     } else {
-#pragma unroll
-        for (int j = 0; j < 16; ++j) t[j] = {0.0, 0.0};
+        const double zero[16] = {};
+        scaled_words16(zero, 0, t);
     }
     const int64_t plane = Mp * Kp;
     int8_t* o = out + frag_off16(row, c, Kp);
-    for (int s = 0; s < S; ++s)
-        store_unit16<NT>(o + s * plane, residues16<WIDE>(t, rc.m[s], rc.rcp[s], rc.c32[s]));
+    for (int s = 0; s < S; ++s) store_unit16<NT>(o + s * plane, residues16(t, rc, s));
 }
 
 // ---------------------------------------------------------------- Scheme II, steps 1 and 2 fused
@@ -111,28 +140,8 @@ __host__ __device__ inline int fuse_rows(int64_t Kp) {
     return r;
 }
 
-// 16 values of row `row` from K-byte 16c on, zero past K (loads as in slice_s2_A_block).
-__device__ __forceinline__ void load_row16(const double* __restrict__ A, int64_t lda, int64_t row, int64_t k0,
-                                           int64_t K, double (&a)[16]) {
-    const double* p = A + row * lda + k0;
-    if (k0 + 16 <= K && ((reinterpret_cast<uintptr_t>(p) & 15) == 0)) {
-#pragma unroll
-        for (int j = 0; j < 16; j += 2) {
-            const double2 v = *reinterpret_cast<const double2*>(p + j);
-            a[j] = v.x;
-            a[j + 1] = v.y;
-        }
-    } else {
-        const double* row_p = A + row * lda;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) a[j] = row_p[min(k0 + j, K - 1)];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) a[j] = k0 + j < K ? a[j] : 0.0;
-    }
-}
-
 // s_key: kFuseThreads words of LDS, s_shift: 128 words.
-template <bool WIDE>
+template <int ND>
 __device__ __forceinline__ void fused_s2_A_block(const double* __restrict__ A, int64_t lda, int64_t M, int64_t K,
                                                  int64_t Mp, int64_t Kp, int32_t kparam, int S,
                                                  const ResidueConsts& rc, int32_t* __restrict__ shift,
@@ -152,8 +161,8 @@ __device__ __forceinline__ void fused_s2_A_block(const double* __restrict__ A, i
         const int64_t u = t + (int64_t)kFuseThreads * i;
         if (u < nunits && row < M) {
             load_row16(A, lda, row, (u / R) * 16, K, a[i]);
-#pragma unroll
-            for (int j = 0; j < 16; ++j) key = max(key, exp_key(a[i][j]));
+            key = max(key, exp_key16(a[i]));
+            drop_non_finite(a[i]);
         } else {
 #pragma unroll
             for (int j = 0; j < 16; ++j) a[i][j] = 0.0;
@@ -176,19 +185,17 @@ __device__ __forceinline__ void fused_s2_A_block(const double* __restrict__ A, i
     for (int i = 0; i < 4; ++i) {
         const int64_t u = t + (int64_t)kFuseThreads * i;
         if (u >= nunits) break;
-        SplitInt v[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) v[j] = split32(rint(ldexp(a[i][j], sh)));
+        Words16<ND> v;
+        scaled_words16(a[i], sh, v);
         int8_t* o = out + frag_off16(row, u / R, Kp);
-        for (int s = 0; s < S; ++s)
-            store_unit16<true>(o + s * plane, residues16<WIDE>(v, rc.m[s], rc.rcp[s], rc.c32[s]));
+        for (int s = 0; s < S; ++s) store_unit16<true>(o + s * plane, residues16(v, rc, s));
     }
 }
 
 // ---------------------------------------------------------------- Scheme II, row-contiguous columns
 // Operand element (col, k) at B[k * ldb + col] (the reference's B; also op(A) = A^T stored K x M).
 // Block = 64 columns x 4 groups of 32 K rows; thread = one column, 32 consecutive k.
-template <bool WIDE, bool NT = false>
+template <int ND, bool NT = false>
 __device__ __forceinline__ void slice_s2_B_block(const double* __restrict__ B, int64_t ldb,
                                                  const int32_t* __restrict__ shift, int64_t K, int64_t N, int64_t Np,
                                                  int64_t Kp, int S, const ResidueConsts& rc, int8_t* __restrict__ out,
@@ -204,18 +211,21 @@ __device__ __forceinline__ void slice_s2_B_block(const double* __restrict__ B, i
         double a[16];
 #pragma unroll
         for (int j = 0; j < 16; ++j) a[j] = B[min(k0 + j, K - 1) * ldb + cc];
-        SplitInt t[16];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) t[j] = split32(rint(ldexp(col < N && k0 + j < K ? a[j] : 0.0, sh)));
+        for (int j = 0; j < 16; ++j) a[j] = col < N && k0 + j < K ? a[j] : 0.0;
+        drop_non_finite(a);
+        Words16<ND> t;
+        scaled_words16(a, sh, t);
         int8_t* o = out + frag_off16(col, k0 >> 4, Kp);
-        for (int s = 0; s < S; ++s)
-            store_unit16<NT>(o + s * plane, residues16<WIDE>(t, rc.m[s], rc.rcp[s], rc.c32[s]));
+        for (int s = 0; s < S; ++s) store_unit16<NT>(o + s * plane, residues16(t, rc, s));
     }
 }
 
 // ---------------------------------------------------------------- Scheme I
-// Slices of 16 values sharing one exponent e (row of A or column of B).
-__device__ __forceinline__ void slice_s1_16(double (&a)[16], int e, int beta, int S, int8_t* o, int64_t plane) {
+// Slices of 16 values sharing one exponent e (row of A or column of B); slices below s0 are formed (each
+// takes its part off the values) but not stored.
+__device__ __forceinline__ void slice_s1_16(double (&a)[16], int e, int beta, int S, int8_t* o, int64_t plane,
+                                            int s0 = 0) {
 #pragma clang fp contract(off)  // every operation rounds where the reference's does
     const double scale = ldexp(1.0, e + 1 - beta);
     const double inv_scale = ldexp(1.0, -(e + 1 - beta));
@@ -232,9 +242,10 @@ __device__ __forceinline__ void slice_s1_16(double (&a)[16], int e, int beta, in
             r[j] = (int)scaled;
             a[j] = a[j] - a_s;
         }
-        *reinterpret_cast<uint4*>(o + s * plane) =
-            make_uint4(pack4_lo(r[0], r[1], r[2], r[3]), pack4_lo(r[4], r[5], r[6], r[7]),
-                       pack4_lo(r[8], r[9], r[10], r[11]), pack4_lo(r[12], r[13], r[14], r[15]));
+        if (s >= s0)
+            *reinterpret_cast<uint4*>(o + s * plane) =
+                make_uint4(pack4_lo(r[0], r[1], r[2], r[3]), pack4_lo(r[4], r[5], r[6], r[7]),
+                           pack4_lo(r[8], r[9], r[10], r[11]), pack4_lo(r[12], r[13], r[14], r[15]));
     }
 }
 
@@ -248,22 +259,8 @@ __device__ __forceinline__ void slice_s1_A_block(const double* __restrict__ A, i
     int8_t* o = out + frag_off16(row, c, Kp);
     if (row < M) {
         const int e = -neg_exp[row];
-        const double* p = A + row * lda + k0;
         double a[16];
-        if (k0 + 16 <= K && ((reinterpret_cast<uintptr_t>(p) & 15) == 0)) {
-#pragma unroll
-            for (int j = 0; j < 16; j += 2) {
-                const double2 v = *reinterpret_cast<const double2*>(p + j);
-                a[j] = v.x;
-                a[j + 1] = v.y;
-            }
-        } else {  // ragged or unaligned: every load unconditional (clamped index), padding zeroed after
-            const double* row_p = A + row * lda;
-#pragma unroll
-            for (int j = 0; j < 16; ++j) a[j] = row_p[min(k0 + j, K - 1)];
-#pragma unroll
-            for (int j = 0; j < 16; ++j) a[j] = k0 + j < K ? a[j] : 0.0;
-        }
+        load_row16(A, lda, row, k0, K, a);
         slice_s1_16(a, e, beta, S, o, Mp * Kp);
     } else {
         for (int s = 0; s < S; ++s) *reinterpret_cast<uint4*>(o + s * Mp * Kp) = make_uint4(0, 0, 0, 0);
@@ -324,13 +321,13 @@ inline SliceOp make_slice_op(const double* p, int64_t rows, int64_t rows_p, int6
     return o;
 }
 
-template <bool WIDE>
+template <int ND>
 __device__ __forceinline__ void slice_s2_op_block(const SliceOp& o, int64_t K, int64_t Kp, int S,
                                                   const ResidueConsts& rc, int64_t blk) {
     const int64_t kb = Kp / 128;
     const int64_t bx = blk / kb, by = blk - bx * kb;
-    if (o.kcontig) slice_s2_A_block<WIDE>(o.p, o.ld, o.shift, o.rows, K, o.rows_p, Kp, S, rc, o.out, bx, by);
-    else slice_s2_B_block<WIDE>(o.p, o.ld, o.shift, K, o.rows, o.rows_p, Kp, S, rc, o.out, bx, by);
+    if (o.kcontig) slice_s2_A_block<ND>(o.p, o.ld, o.shift, o.rows, K, o.rows_p, Kp, S, rc, o.out, bx, by);
+    else slice_s2_B_block<ND>(o.p, o.ld, o.shift, K, o.rows, o.rows_p, Kp, S, rc, o.out, bx, by);
 }
 
 __device__ __forceinline__ void slice_s1_op_block(const SliceOp& o, int64_t K, int64_t Kp, int S, int beta,
@@ -339,6 +336,117 @@ __device__ __forceinline__ void slice_s1_op_block(const SliceOp& o, int64_t K, i
     const int64_t bx = blk / kb, by = blk - bx * kb;
     if (o.kcontig) slice_s1_A_block(o.p, o.ld, o.shift, o.rows, K, o.rows_p, Kp, S, beta, o.out, bx, by);
     else slice_s1_B_block(o.p, o.ld, o.shift, K, o.rows, o.rows_p, Kp, S, beta, o.out, bx, by);
+}
+
+// ---------------------------------------------------------------- steps 1 and 2 in one pass, both operands
+// Single calls with Kp <= kPassMaxKp: a block of 256 threads holds R whole rows (columns of a
+// row-contiguous operand) in registers, takes their exponent maxima, writes the shifts and then the
+// slices of the values it still holds.  Unit u = (row u % R, 16-byte K chunk u / R) of the block; thread t
+// takes units t + 256 i, i < NU, all of row t % R.  With R = 16 a wave reads a row-contiguous operand
+// in 128-byte runs and writes 256-byte runs of a fragment block; R grows to 64 for short K so that the
+// threads have units.  Values and results are those of the separate kernels.
+// A block's planes may be dealt to `parts` blocks that each read the rows again (part j stores planes
+// [S j / parts, S (j + 1) / parts), part 0 the shifts): more blocks for small operands, whose second
+// reads come from the XCD's L2 (the parts of a row block are 8 block indices apart, on one XCD).
+// Small calls are bound by launches (4.7 us of stream time each) and latency: this takes the place of
+// four launches (keys cleared, maxima, keys to shifts, slices).  256^3, S = 4: 23.9 -> 15.0 us per call;
+// 1024^3, S = 16: 59.6 -> 46.2 us; 777 x 1501 x 1003, S = 14: 70.7 -> 64.4 us.  With Kp up to 2048 in
+// 512-thread blocks (one per CU at 242 registers, nothing to hide its load latency) the launch took 37 us
+// at 2048^3 where the two kernels take 39.
+constexpr int64_t kPassMaxKp = 1024;
+constexpr int kPassThreads = 256;
+
+inline int pass_units(int64_t Kp) { return Kp <= 256 ? 1 : Kp <= 512 ? 2 : 4; }
+inline int pass_rows(int64_t Kp) {
+    int r = 64;
+    while (r > 16 && r * (Kp / 16) > kPassThreads * pass_units(Kp)) r >>= 1;
+    return r;
+}
+
+struct PassOp {
+    const double* p;
+    int64_t rows, rows_p, ld;
+    int32_t kcontig;
+    int32_t* shift;
+    int8_t* out;
+    int64_t nrow;  // row blocks
+};
+
+struct PassArgs {
+    PassOp op[2];
+    int64_t K, Kp;
+    int S, R, parts, offset;  // offset: K_param (Scheme II) or beta (Scheme I)
+    uint32_t* zero;           // words cleared by the first block (the GEMM's work counters)
+    int nzero;
+};
+
+// ND: words per value (Scheme II), or 0 for Scheme I.
+template <int ND, int NU, bool KC>
+__device__ __forceinline__ void pass_block(const PassOp& o, const PassArgs& g, const ResidueConsts& rc, int64_t rb,
+                                           int part, uint32_t* s_key, int32_t* s_shift) {
+    const int R = g.R;
+    const int t = threadIdx.x;
+    const int rl = t & (R - 1), c0 = t / R, cstep = kPassThreads / R;
+    const int64_t row = rb * R + rl;
+    const int U = (int)(g.Kp / 16);
+    double a[NU][16];
+    uint32_t key = 0;
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+        const int c = c0 + i * cstep;
+        if (c < U && row < o.rows) {
+            const int64_t k0 = (int64_t)c * 16;
+            if (KC) {
+                load_row16(o.p, o.ld, row, k0, g.K, a[i]);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 16; ++j) a[i][j] = o.p[min(k0 + j, g.K - 1) * o.ld + row];
+#pragma unroll
+                for (int j = 0; j < 16; ++j) a[i][j] = k0 + j < g.K ? a[i][j] : 0.0;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) a[i][j] = 0.0;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+        key = max(key, exp_key16(a[i]));
+        if (ND > 0) drop_non_finite(a[i]);
+    }
+    for (int d = R; d < 64; d <<= 1) key = max(key, (uint32_t)__shfl_xor((int)key, d));
+    if ((t & 63) < R) s_key[(t >> 6) * 64 + (t & 63)] = key;
+    __syncthreads();
+    if (t < R) {
+        uint32_t k = 0;
+#pragma unroll
+        for (int w = 0; w < kPassThreads / 64; ++w) k = max(k, s_key[w * 64 + t]);
+        const int32_t sh = (ND == 0 ? 0 : g.offset) - exp_from_key(k);  // key_to_shift
+        s_shift[t] = sh;
+        if (part == 0 && row < o.rows) o.shift[row] = sh;
+    }
+    __syncthreads();
+    if (row >= (o.rows + 31) / 32 * 32) return;  // the planes' blocks past the last logical row stay unwritten
+    const int sh = s_shift[rl];
+    const int64_t plane = o.rows_p * g.Kp;
+    const int s0 = g.S * part / g.parts, s1 = g.S * (part + 1) / g.parts;
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+        const int c = c0 + i * cstep;
+        if (c >= U) break;
+        int8_t* out = o.out + frag_off16(row, c, g.Kp);
+        if constexpr (ND == 0) {
+            if (row < o.rows) {
+                slice_s1_16(a[i], -sh, g.offset, s1, out, plane, s0);
+            } else {
+                for (int s = s0; s < s1; ++s) *reinterpret_cast<uint4*>(out + s * plane) = make_uint4(0, 0, 0, 0);
+            }
+        } else {
+            Words16<ND> v;
+            scaled_words16(a[i], sh, v);
+            for (int s = s0; s < s1; ++s) store_unit16<false>(out + s * plane, residues16(v, rc, s));
+        }
+    }
 }
 
 }  // namespace core
