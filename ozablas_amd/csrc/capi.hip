@@ -335,12 +335,13 @@ static int enqueue_pipeline(int scheme, oza_ctx ctx, size_t M, size_t N, size_t 
                                 nqueue),
                 "step 2 launch");
     } else {
-        OZA_HIP(launch_stats(d, A, B, kp, shA, shB, st, ctx->queue_dev, nqueue), "step 1 launch");
+        Shifts sh[2];
+        OZA_HIP(launch_stats_parts(d, A, B, kp, shA, shB, Ctc, sh, st, ctx->queue_dev, nqueue), "step 1 launch");
         if (ev) OZA_HIP(hipEventRecord(ev[1], st), "event");
         if (scheme == 2)
-            OZA_HIP(launch_slice_s2(d, A, B, shA, shB, Asl, Bsl, st, core::residue_words(kp)), "step 2 launch");
+            OZA_HIP(launch_slice_s2(d, A, B, sh[0], sh[1], Asl, Bsl, st, core::residue_words(kp)), "step 2 launch");
         else
-            OZA_HIP(launch_slice_s1(d, beta, A, B, shA, shB, Asl, Bsl, st), "step 2 launch");
+            OZA_HIP(launch_slice_s1(d, beta, A, B, sh[0], sh[1], Asl, Bsl, st), "step 2 launch");
     }
     if (ev) OZA_HIP(hipEventRecord(ev[2], st), "event");
     if (scheme == 2) {
@@ -586,10 +587,11 @@ int oza_stage2_slices(oza_ctx ctx, int scheme, size_t M, size_t N, size_t K, int
                       const double* B, const int32_t* shA, const int32_t* shB, int8_t* Asl, int8_t* Bsl) {
     OZA_STAGE_PROLOGUE(scheme)
     const Operand a{A, (int64_t)K, true}, b{B, (int64_t)N, false};
+    const Shifts sa{const_cast<int32_t*>(shA)}, sb{const_cast<int32_t*>(shB)};  // read only
     if (scheme == 2)
-        OZA_HIP(launch_slice_s2(d, a, b, shA, shB, Asl, Bsl, st, 3), "step 2 launch");  // the caller's shifts
+        OZA_HIP(launch_slice_s2(d, a, b, sa, sb, Asl, Bsl, st, 3), "step 2 launch");  // the caller's shifts
     else
-        OZA_HIP(launch_slice_s1(d, scheme1_beta(K), a, b, shA, shB, Asl, Bsl, st), "step 2 launch");
+        OZA_HIP(launch_slice_s1(d, scheme1_beta(K), a, b, sa, sb, Asl, Bsl, st), "step 2 launch");
     return OZA_SUCCESS;
 }
 

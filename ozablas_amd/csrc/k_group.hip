@@ -83,8 +83,8 @@ __device__ __forceinline__ void group_slice(const GroupProblem& P, const GroupPt
     const bool is_a = l < P.slA;
     if (!is_a) l -= P.slA;
     const int64_t bx = l / kb, by = l - bx * kb;
-    if (is_a) slice_s2_A_block<ND, true>(q.A, P.K, P.shA, P.M, P.K, P.Mp, P.Kp, P.S, rc, P.Asl, bx, by);
-    else slice_s2_B_block<ND, true>(q.B, P.N, P.shB, P.K, P.N, P.Np, P.Kp, P.S, rc, P.Bsl, bx, by);
+    if (is_a) slice_s2_A_block<ND, true>(q.A, P.K, Shifts{P.shA}, P.M, P.K, P.Mp, P.Kp, P.S, rc, P.Asl, bx, by);
+    else slice_s2_B_block<ND, true>(q.B, P.N, Shifts{P.shB}, P.K, P.N, P.Np, P.Kp, P.S, rc, P.Bsl, bx, by);
 }
 
 __global__ void __launch_bounds__(kSliceThreads) k_group_slice(GroupLaunch g) {

@@ -28,6 +28,7 @@ using namespace core;
 // Blocks a one-pass launch aims for by dealing a row block's planes to several blocks: one per CU.
 // 1024^3, S = 16 (128 row blocks): 53 us per call undivided, 46 us in two parts, 48 in four, 55 in eight.
 constexpr int64_t kPassTargetBlocks = 256;
+constexpr int64_t kPassResident = 512;
 
 // Blocks [0, a.nblk) slice operand a into its planes, the rest operand b.
 template <int ND>
@@ -97,8 +98,8 @@ __global__ void k_unpack_B(const int8_t* __restrict__ in, int64_t K, int64_t N, 
 
 }  // namespace
 
-hipError_t launch_slice_s2(const Dims& d, const Operand& A, const Operand& B, const int32_t* shift_A,
-                           const int32_t* shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st, int words) {
+hipError_t launch_slice_s2(const Dims& d, const Operand& A, const Operand& B, const Shifts& shift_A,
+                           const Shifts& shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st, int words) {
     const ResidueConsts rc = make_residue_consts();
     const SliceOp a = make_slice_op(A.p, d.M, d.Mp, A.ld, A.kcontig, d.Kp, shift_A, A_sl);
     const SliceOp b = make_slice_op(B.p, d.N, d.Np, B.ld, B.kcontig, d.Kp, shift_B, B_sl);
@@ -111,15 +112,24 @@ hipError_t launch_slice_s2(const Dims& d, const Operand& A, const Operand& B, co
     return hipGetLastError();
 }
 
-hipError_t launch_slice_s1(const Dims& d, int beta, const Operand& A, const Operand& B, const int32_t* shift_A,
-                           const int32_t* shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st) {
+hipError_t launch_slice_s1(const Dims& d, int beta, const Operand& A, const Operand& B, const Shifts& shift_A,
+                           const Shifts& shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st) {
     const SliceOp a = make_slice_op(A.p, d.M, d.Mp, A.ld, A.kcontig, d.Kp, shift_A, A_sl);
     const SliceOp b = make_slice_op(B.p, d.N, d.Np, B.ld, B.kcontig, d.Kp, shift_B, B_sl);
     k_slice_s1<<<(unsigned)(a.nblk + b.nblk), kSliceThreads, 0, st>>>(a, b, d.K, d.Kp, d.S, beta);
     return hipGetLastError();
 }
 
-bool one_pass(const Dims& d) { return d.Kp <= kPassMaxKp; }
+// Not when a second round of the resident blocks (two per CU at four units per thread) would hold a few
+// blocks only, which take as long as a full one: 200 x 8000 x 900, S = 16 (514 row blocks) 125 us in one
+// pass, 112 us in two kernels; 5000 x 4000 x 1000 (563) 518 against 523, 1000 x 6000 x 1000 (438) 179
+// against 188.
+bool one_pass(const Dims& d) {
+    if (d.Kp > kPassMaxKp) return false;
+    const int R = pass_rows(d.Kp);
+    const int64_t over = pass_row_blocks(d.M, R) + pass_row_blocks(d.N, R) - kPassResident;
+    return !(pass_units(d.Kp) == 4 && over > 0 && over < kPassResident / 16);
+}
 
 hipError_t launch_one_pass(int scheme, const Dims& d, int offset, const Operand& A, const Operand& B, int32_t* shift_A,
                            int32_t* shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st, uint32_t* zero, int nzero) {
@@ -133,7 +143,7 @@ hipError_t launch_one_pass(int scheme, const Dims& d, int offset, const Operand&
     g.nzero = nzero;
     if (nzero > kPassThreads) return hipErrorInvalidValue;
     auto op = [&](const Operand& X, int64_t rows, int64_t rows_p, int32_t* shift, int8_t* out) {
-        return PassOp{X.p, rows, rows_p, X.ld, X.kcontig, shift, out, ((rows + 31) / 32 * 32 + g.R - 1) / g.R};
+        return PassOp{X.p, rows, rows_p, X.ld, X.kcontig, shift, out, pass_row_blocks(rows, g.R)};
     };
     g.op[0] = op(A, d.M, d.Mp, shift_A, A_sl);
     g.op[1] = op(B, d.N, d.Np, shift_B, B_sl);

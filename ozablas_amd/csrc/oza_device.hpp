@@ -28,28 +28,29 @@ __host__ __device__ __forceinline__ int exp_from_key(uint32_t key) {
     return be - 1022;
 }
 
-// The largest exponent key of 16 values.  Finite values' keys are their high words without the sign;
+// The largest exponent key of N values.  Finite values' keys are their high words without the sign;
 // anything else is rare and takes the exact form.
 constexpr uint32_t kNonFinite = 0x7ff00000u;
-__device__ __forceinline__ uint32_t high16(const double (&a)[16]) {
+template <int N>
+__device__ __forceinline__ uint32_t max_high(const double (&a)[N]) {
     uint32_t m = 0;
 #pragma unroll
-    for (int j = 0; j < 16; ++j)
-        m = max(m, (uint32_t)((uint64_t)__double_as_longlong(a[j]) >> 32) & 0x7fffffffu);
+    for (int j = 0; j < N; ++j) m = max(m, (uint32_t)((uint64_t)__double_as_longlong(a[j]) >> 32) & 0x7fffffffu);
     return m;
 }
-__device__ __forceinline__ uint32_t exp_key16(const double (&a)[16]) {
-    uint32_t m = high16(a);
+template <int N>
+__device__ __forceinline__ uint32_t max_key(const double (&a)[N]) {
+    uint32_t m = max_high(a);
     if (m >= kNonFinite) {
         m = 0;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) m = max(m, exp_key(a[j]));
+        for (int j = 0; j < N; ++j) m = max(m, exp_key(a[j]));
     }
     return m;
 }
 // Infinities and NaNs have residue 0 for every modulus.
 __device__ __forceinline__ void drop_non_finite(double (&a)[16]) {
-    if (high16(a) >= kNonFinite) {
+    if (max_high(a) >= kNonFinite) {
 #pragma unroll
         for (int j = 0; j < 16; ++j)
             if (((uint64_t)__double_as_longlong(a[j]) >> 32 & kNonFinite) == kNonFinite) a[j] = 0.0;

@@ -116,19 +116,34 @@ struct OutC {
 hipError_t launch_scale_c(const OutC& c, int64_t M, int64_t N, hipStream_t st);
 
 // Step 1: shift_A[i] = offset - E_i, shift_B[j] = offset - F_j.
-// The key-clearing launch also clears `nzero` words at `zero` (may be null): the work counters
-// of the calls' step-3 GEMMs.
 hipError_t launch_stats(const Dims& d, const Operand& A, const Operand& B, int32_t offset, int32_t* shift_A,
-                        int32_t* shift_B, hipStream_t st, uint32_t* zero = nullptr, int64_t nzero = 0);
+                        int32_t* shift_B, hipStream_t st);
+
+// Where a slicing block finds its rows' shifts: in `shift`, or (part != null) from step 1's partial
+// maxima, `parts` (at most kStatParts) planes of `rows` exponent keys, whose maximum it turns into
+// offset - exponent and stores in `shift`.
+constexpr int kStatParts = 32;
+struct Shifts {
+    int32_t* shift;
+    const uint32_t* part;
+    int32_t parts, offset;
+    int64_t rows;
+};
+// Step 1 into partial maxima at `scratch`, at most 128 (M + N) bytes (the digit planes hold S Mp Np, with
+// Mp and Np at least 256); out: the shifts for step 2.  The launch also clears nzero words at `zero` (the
+// work counters of the call's step-3 GEMMs).
+hipError_t launch_stats_parts(const Dims& d, const Operand& A, const Operand& B, int32_t offset, int32_t* shift_A,
+                              int32_t* shift_B, void* scratch, Shifts out[2], hipStream_t st, uint32_t* zero,
+                              int nzero);
 
 // Step 2.  words: 32-bit words per scaled value, |rint(2^shift a)| <= 2^(32 words - 2)
 // (core::residue_words(K_param) with step 1's shifts).
-hipError_t launch_slice_s2(const Dims& d, const Operand& A, const Operand& B, const int32_t* shift_A,
-                           const int32_t* shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st, int words);
-hipError_t launch_slice_s1(const Dims& d, int beta, const Operand& A, const Operand& B, const int32_t* shift_A,
-                           const int32_t* shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st);
+hipError_t launch_slice_s2(const Dims& d, const Operand& A, const Operand& B, const Shifts& shift_A,
+                           const Shifts& shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st, int words);
+hipError_t launch_slice_s1(const Dims& d, int beta, const Operand& A, const Operand& B, const Shifts& shift_A,
+                           const Shifts& shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st);
 // Steps 1 and 2 in one launch, for shapes with one_pass(d): offset is K_param (scheme 2) or beta
-// (scheme 1); zero / nzero as in launch_stats.
+// (scheme 1); zero / nzero as in launch_stats_parts.
 bool one_pass(const Dims& d);
 hipError_t launch_one_pass(int scheme, const Dims& d, int offset, const Operand& A, const Operand& B, int32_t* shift_A,
                            int32_t* shift_B, int8_t* A_sl, int8_t* B_sl, hipStream_t st, uint32_t* zero, int nzero);

@@ -92,28 +92,48 @@ __device__ __forceinline__ void load_row16(const double* __restrict__ A, int64_t
     }
 }
 
+// The shift of row r for a block of 256 threads, 256 / G of them (consecutive, the same rows) in each of
+// its G groups.  Every thread of the block calls it; 0 past the last row.  From partial maxima, the
+// block with `store` also writes the shift.
+template <int G>
+__device__ __forceinline__ int shift_of_row(const Shifts& s, int64_t r, int64_t rows, bool store) {
+    if (!s.part) return r < rows ? s.shift[r] : 0;
+    constexpr int T = kSliceThreads / G;
+    __shared__ uint32_t s_key[kSliceThreads];
+    const int g = threadIdx.x / T;
+    const int64_t rr = min(r, rows - 1);
+    uint32_t v[kStatParts / G], key = 0;
+#pragma unroll
+    for (int i = 0; i < kStatParts / G; ++i) v[i] = s.part[(int64_t)min(g + i * G, s.parts - 1) * s.rows + rr];
+#pragma unroll
+    for (int i = 0; i < kStatParts / G; ++i) key = max(key, v[i]);
+    s_key[threadIdx.x] = key;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < G; ++i) key = max(key, s_key[i * T + threadIdx.x % T]);
+    const int sh = s.offset - exp_from_key(key);
+    if (store && g == 0 && r < rows) s.shift[r] = sh;
+    return r < rows ? sh : 0;
+}
+
 // ---------------------------------------------------------------- Scheme II, K-contiguous rows
 // Operand element (row, k) at A[row * lda + k] (the reference's A; also op(B) = B^T stored N x K).
 // Block = 32 rows x 128 K; thread = row (tid % 32), 16-byte K chunk (tid / 32).  The 64 lanes of a
 // wave cover one whole 1 KiB fragment block.
 template <int ND, bool NT = false>
 __device__ __forceinline__ void slice_s2_A_block(const double* __restrict__ A, int64_t lda,
-                                                 const int32_t* __restrict__ shift, int64_t M, int64_t K, int64_t Mp,
-                                                 int64_t Kp, int S, const ResidueConsts& rc, int8_t* __restrict__ out,
-                                                 int64_t bx, int64_t by) {
+                                                 const Shifts& shift, int64_t M, int64_t K, int64_t Mp, int64_t Kp,
+                                                 int S, const ResidueConsts& rc, int8_t* __restrict__ out, int64_t bx,
+                                                 int64_t by) {
     const int64_t row = bx * 32 + (threadIdx.x & 31);
     const int64_t c = by * 8 + (threadIdx.x >> 5);
     const int64_t k0 = c * 16;
+    double a[16] = {};
+    if (row < M) load_row16(A, lda, row, k0, K, a);
+    const int sh = shift_of_row<8>(shift, row, M, by == 0);
+    drop_non_finite(a);
     Words16<ND> t;
-    if (row < M) {
-        double a[16];
-        load_row16(A, lda, row, k0, K, a);
-        drop_non_finite(a);
-        scaled_words16(a, shift[row], t);
-    } else {
-        const double zero[16] = {};
-        scaled_words16(zero, 0, t);
-    }
+    scaled_words16(a, sh, t);
     const int64_t plane = Mp * Kp;
     int8_t* o = out + frag_off16(row, c, Kp);
     for (int s = 0; s < S; ++s) store_unit16<NT>(o + s * plane, residues16(t, rc, s));
@@ -161,7 +181,7 @@ __device__ __forceinline__ void fused_s2_A_block(const double* __restrict__ A, i
         const int64_t u = t + (int64_t)kFuseThreads * i;
         if (u < nunits && row < M) {
             load_row16(A, lda, row, (u / R) * 16, K, a[i]);
-            key = max(key, exp_key16(a[i]));
+            key = max(key, max_key(a[i]));
             drop_non_finite(a[i]);
         } else {
 #pragma unroll
@@ -197,13 +217,13 @@ __device__ __forceinline__ void fused_s2_A_block(const double* __restrict__ A, i
 // Block = 64 columns x 4 groups of 32 K rows; thread = one column, 32 consecutive k.
 template <int ND, bool NT = false>
 __device__ __forceinline__ void slice_s2_B_block(const double* __restrict__ B, int64_t ldb,
-                                                 const int32_t* __restrict__ shift, int64_t K, int64_t N, int64_t Np,
-                                                 int64_t Kp, int S, const ResidueConsts& rc, int8_t* __restrict__ out,
-                                                 int64_t bx, int64_t by) {
+                                                 const Shifts& shift, int64_t K, int64_t N, int64_t Np, int64_t Kp,
+                                                 int S, const ResidueConsts& rc, int8_t* __restrict__ out, int64_t bx,
+                                                 int64_t by) {
     const int64_t col = bx * 64 + (threadIdx.x & 63);
     const int64_t kbase = by * 128 + (threadIdx.x >> 6) * 32;
     const int64_t plane = Np * Kp;
-    const int sh = col < N ? shift[col] : 0;
+    const int sh = shift_of_row<4>(shift, col, N, by == 0);
     const int64_t cc = min(col, N - 1);  // clamped: every load unconditional, padding zeroed after
 #pragma unroll 1
     for (int half = 0; half < 2; ++half) {
@@ -250,17 +270,16 @@ __device__ __forceinline__ void slice_s1_16(double (&a)[16], int e, int beta, in
 }
 
 __device__ __forceinline__ void slice_s1_A_block(const double* __restrict__ A, int64_t lda,
-                                                 const int32_t* __restrict__ neg_exp, int64_t M, int64_t K, int64_t Mp,
-                                                 int64_t Kp, int S, int beta, int8_t* __restrict__ out, int64_t bx,
-                                                 int64_t by) {
+                                                 const Shifts& neg_exp, int64_t M, int64_t K, int64_t Mp, int64_t Kp,
+                                                 int S, int beta, int8_t* __restrict__ out, int64_t bx, int64_t by) {
     const int64_t row = bx * 32 + (threadIdx.x & 31);
     const int64_t c = by * 8 + (threadIdx.x >> 5);
     const int64_t k0 = c * 16;
     int8_t* o = out + frag_off16(row, c, Kp);
+    double a[16];
+    if (row < M) load_row16(A, lda, row, k0, K, a);
+    const int e = -shift_of_row<8>(neg_exp, row, M, by == 0);
     if (row < M) {
-        const int e = -neg_exp[row];
-        double a[16];
-        load_row16(A, lda, row, k0, K, a);
         slice_s1_16(a, e, beta, S, o, Mp * Kp);
     } else {
         for (int s = 0; s < S; ++s) *reinterpret_cast<uint4*>(o + s * Mp * Kp) = make_uint4(0, 0, 0, 0);
@@ -268,18 +287,17 @@ __device__ __forceinline__ void slice_s1_A_block(const double* __restrict__ A, i
 }
 
 __device__ __forceinline__ void slice_s1_B_block(const double* __restrict__ B, int64_t ldb,
-                                                 const int32_t* __restrict__ neg_exp, int64_t K, int64_t N, int64_t Np,
-                                                 int64_t Kp, int S, int beta, int8_t* __restrict__ out, int64_t bx,
-                                                 int64_t by) {
+                                                 const Shifts& neg_exp, int64_t K, int64_t N, int64_t Np, int64_t Kp,
+                                                 int S, int beta, int8_t* __restrict__ out, int64_t bx, int64_t by) {
     const int64_t col = bx * 64 + (threadIdx.x & 63);
     const int64_t kbase = by * 128 + (threadIdx.x >> 6) * 32;
     const int64_t plane = Np * Kp;
+    const int e = -shift_of_row<4>(neg_exp, col, N, by == 0);
 #pragma unroll 1
     for (int half = 0; half < 2; ++half) {
         const int64_t k0 = kbase + half * 16;
         int8_t* o = out + frag_off16(col, k0 >> 4, Kp);
         if (col < N) {
-            const int e = -neg_exp[col];
             double a[16];  // every load unconditional (clamped index), padding zeroed after
 #pragma unroll
             for (int j = 0; j < 16; ++j) a[j] = B[min(k0 + j, K - 1) * ldb + col];
@@ -301,13 +319,13 @@ struct SliceOp {
     const double* p;
     int64_t rows, rows_p, ld;
     int32_t kcontig;
-    const int32_t* shift;
+    Shifts shift;
     int8_t* out;
     int64_t nblk;
 };
 
 inline SliceOp make_slice_op(const double* p, int64_t rows, int64_t rows_p, int64_t ld, bool kcontig,
-                             int64_t Kp, const int32_t* shift, int8_t* out) {
+                             int64_t Kp, const Shifts& shift, int8_t* out) {
     SliceOp o;
     o.p = p;
     o.rows = rows;
@@ -362,6 +380,8 @@ inline int pass_rows(int64_t Kp) {
     while (r > 16 && r * (Kp / 16) > kPassThreads * pass_units(Kp)) r >>= 1;
     return r;
 }
+// Row blocks of an operand: the rows its planes hold, whole 32-row fragment blocks.
+inline int64_t pass_row_blocks(int64_t rows, int R) { return ((rows + 31) / 32 * 32 + R - 1) / R; }
 
 struct PassOp {
     const double* p;
@@ -411,7 +431,7 @@ __device__ __forceinline__ void pass_block(const PassOp& o, const PassArgs& g, c
     }
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
-        key = max(key, exp_key16(a[i]));
+        key = max(key, max_key(a[i]));
         if (ND > 0) drop_non_finite(a[i]);
     }
     for (int d = R; d < 64; d <<= 1) key = max(key, (uint32_t)__shfl_xor((int)key, d));

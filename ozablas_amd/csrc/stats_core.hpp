@@ -5,6 +5,7 @@
 
 #include "oza_device.hpp"
 #include "oza_internal.hpp"
+#include "slice_core.hpp"
 
 namespace oza {
 namespace core {
@@ -165,6 +166,125 @@ __device__ __forceinline__ void stats_op_block(const StatOp& o, int64_t K, int64
     } else {
         if (o.vec) stats_B_block<true>(o.p, K, o.rows, o.ld, o.colblk, o.keys, blk, o.rowsB);
         else stats_B_block<false>(o.p, K, o.rows, o.ld, o.colblk, o.keys, blk, o.rowsB);
+    }
+}
+
+// ---------------------------------------------------------------- partial maxima without atomics
+// Step 1 of a single call: `parts` (at most kStatParts) planes of `rows` exponent keys, plane p the
+// maxima over the p-th run of `step` K values; the slicing kernel takes the maximum over the planes.
+// No keys to clear before and none to convert after: two launches less per call, 10 us of stream time
+// (2048^3, S = 6: 115.4 -> 109.7 us per call; 512 x 512 x 32768, S = 14: 338 -> 331).  K-contiguous rows: a wave per (row, run of at least 4096 values).
+// Row-contiguous: a block of 256 threads covers 2 ct columns, a thread two adjacent columns of every
+// (256 / ct)-th row of the run, kStatUnroll rows in flight, and the row groups meet in LDS.  ct = 64 (a
+// wave reads 1 KiB of one row); 16 for few rows, so that there are blocks for every CU.
+struct PartOp {
+    const double* p;
+    int64_t rows, ld;
+    int32_t kcontig, vec, ct, parts;
+    int64_t step, colblk, nblk;
+    uint32_t* out;
+};
+
+inline PartOp make_part_op(const double* p, int64_t rows, int64_t K, int64_t ld, bool kcontig, uint32_t* out) {
+    PartOp o;
+    o.p = p;
+    o.rows = rows;
+    o.ld = ld;
+    o.kcontig = kcontig;
+    o.vec = (ld % 2 == 0) && ((reinterpret_cast<uintptr_t>(p) & 15) == 0) && (!kcontig || K % 2 == 0);
+    o.ct = rows >= 1024 ? 64 : 16;
+    const int64_t unit = kcontig ? kRowChunk : (kStatThreads / o.ct) * kStatUnroll;
+    const int64_t units = (K + unit - 1) / unit;
+    o.step = (units + kStatParts - 1) / kStatParts * unit;
+    o.parts = (int32_t)((K + o.step - 1) / o.step);
+    o.colblk = (rows + 2 * o.ct - 1) / (2 * o.ct);
+    o.nblk = kcontig ? (rows * o.parts + 3) / 4 : o.colblk * o.parts;
+    o.out = out;
+    return o;
+}
+
+template <bool VEC>
+__device__ __forceinline__ void part_rows_block(const PartOp& o, int64_t K, int64_t blk) {
+    const int64_t w = blk * (kStatThreads / 64) + (threadIdx.x >> 6);
+    if (w >= o.rows * o.parts) return;  // whole wave leaves together
+    const int64_t row = w / o.parts, part = w - row * o.parts;
+    const int lane = threadIdx.x & 63;
+    const double* p = o.p + row * o.ld;
+    const int64_t c0 = part * o.step, c1 = min(K, c0 + o.step);
+    // indices past the end are clamped to the last element of the run, which is read again
+    uint32_t key = 0;
+    if (VEC) {
+        for (int64_t c = c0 + 2 * lane; c < c1; c += 128 * kStatUnroll) {
+            double v[2 * kStatUnroll];
+#pragma unroll
+            for (int u = 0; u < kStatUnroll; ++u) {
+                const double2 x = load_stream2(p + min(c + 128 * u, c1 - 2));
+                v[2 * u] = x.x;
+                v[2 * u + 1] = x.y;
+            }
+            key = max(key, max_key(v));
+        }
+    } else {
+        for (int64_t c = c0 + lane; c < c1; c += 64 * kStatUnroll) {
+            double v[kStatUnroll];
+#pragma unroll
+            for (int u = 0; u < kStatUnroll; ++u) v[u] = load_stream(p + min(c + 64 * u, c1 - 1));
+            key = max(key, max_key(v));
+        }
+    }
+    key = wave_max_u32(key);
+    if (lane == 0) o.out[part * o.rows + row] = key;
+}
+
+// s_key: 2 * kStatThreads words of LDS.
+template <bool VEC>
+__device__ __forceinline__ void part_cols_block(const PartOp& o, int64_t K, int64_t blk, uint32_t* s_key) {
+    const int64_t part = blk / o.colblk, cb = blk - part * o.colblk;
+    const int ct = o.ct, groups = kStatThreads / ct;
+    const int cg = threadIdx.x & (ct - 1), rg = threadIdx.x / ct;
+    const int64_t c = min(cb * (2 * ct) + 2 * cg, o.rows - 1);  // columns past the last one read it again
+    const int64_t c2 = min(c + 1, o.rows - 1);
+    const bool pair = VEC && c2 > c;
+    const int64_t r0 = part * o.step, r1 = min(K, r0 + o.step);
+    uint32_t k0 = 0, k1 = 0;
+    for (int64_t r = r0 + rg; r < r1; r += (int64_t)groups * kStatUnroll) {
+        double x[kStatUnroll], y[kStatUnroll];
+        if (pair) {
+#pragma unroll
+            for (int u = 0; u < kStatUnroll; ++u) {
+                const double2 v = load_stream2(o.p + min(r + u * groups, r1 - 1) * o.ld + c);
+                x[u] = v.x;
+                y[u] = v.y;
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < kStatUnroll; ++u) {
+                const int64_t rr = min(r + u * groups, r1 - 1) * o.ld;
+                x[u] = o.p[rr + c];
+                y[u] = o.p[rr + c2];
+            }
+        }
+        k0 = max(k0, max_key(x));
+        k1 = max(k1, max_key(y));
+    }
+    s_key[rg * 2 * ct + 2 * cg] = k0;
+    s_key[rg * 2 * ct + 2 * cg + 1] = k1;
+    __syncthreads();
+    const int64_t col = cb * (2 * ct) + threadIdx.x;
+    if ((int)threadIdx.x < 2 * ct && col < o.rows) {
+        uint32_t k = 0;
+        for (int g = 0; g < groups; ++g) k = max(k, s_key[g * 2 * ct + threadIdx.x]);
+        o.out[part * o.rows + col] = k;
+    }
+}
+
+__device__ __forceinline__ void part_op_block(const PartOp& o, int64_t K, int64_t blk, uint32_t* s_key) {
+    if (o.kcontig) {
+        if (o.vec) part_rows_block<true>(o, K, blk);
+        else part_rows_block<false>(o, K, blk);
+    } else {
+        if (o.vec) part_cols_block<true>(o, K, blk, s_key);
+        else part_cols_block<false>(o, K, blk, s_key);
     }
 }
 
