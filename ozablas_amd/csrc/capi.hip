@@ -287,7 +287,7 @@ static int enqueue_banded(oza_ctx ctx, int scheme, const Dims& d, int nb, const 
     for (int b = 0; b < nb; ++b) {
         const int t0 = (int)((int64_t)tm * b / nb), t1 = (int)((int64_t)tm * (b + 1) / nb);
         if (scheme == 2)
-            OZA_HIP(launch_igemm_s2(d, Asl, Bsl, S2Out::Digits, Ctc, cs, st, t0, t1 - t0, ctx->queue_dev + 8 * b),
+            OZA_HIP(launch_igemm_s2(d, Asl, Bsl, S2Out::Digits, Ctc, cs, st, t0, t1 - t0),
                     "step 3 launch");
         else
             OZA_HIP(launch_igemm_s1_blocked(d, Asl, Bsl, static_cast<int32_t*>(Ctc), st, ctx->queue_dev + 8 * b, t0,
@@ -351,7 +351,7 @@ static int enqueue_pipeline(int scheme, oza_ctx ctx, size_t M, size_t N, size_t 
         } else {
             // Few tiles and a long K: the K steps run in parts (partial digits summed mod m_s)
             const int split = scheme2_single_split(M, N, K, S);
-            OZA_HIP(launch_igemm_s2(d, Asl, Bsl, S2Out::Digits, Ctc, crt_for(ctx, S), st, 0, -1, ctx->queue_dev, split),
+            OZA_HIP(launch_igemm_s2(d, Asl, Bsl, S2Out::Digits, Ctc, crt_for(ctx, S), st, 0, -1, split),
                     "step 3 launch");
             OZA_HIP(launch_digits_reduce(d, static_cast<uint8_t*>(Ctc), split, crt_for(ctx, S), st), "step 3 launch");
             if (ev) OZA_HIP(hipEventRecord(ev[3], st), "event");

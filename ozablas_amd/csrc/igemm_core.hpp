@@ -156,9 +156,16 @@ __device__ __forceinline__ void interleave_hint_last() {
 //     Scheme I -3 % against no priorities; priority 1 over all MFMA sections gave -2.4 % (Scheme
 //     II), over the first k-step only +4 %.
 //
+//   The first wait lets LPS later operations stay outstanding: stage 1's loads, or the stores of the
+//   previous item's epilogue, which would otherwise be waited for at every item (R1 needs stage 0 only;
+//   with nit == 1 slot 1 is loaded at once, so there everything is waited for, R3).  Scheme II GEMM alone,
+//   S = 8: 4096^2 x 256 69.8 -> 64.1 us, 4096^2 x 1024 138.7 -> 137.0 us (with the static order).
+//
 //   On entry this item's stage 0 has been issued, and its stage 1 too when nit >= 2 (chain_start
 //   for a chain's first item; the previous item's last two iterations otherwise).  With nit == 1 no
 //   earlier iteration can take chain stage 1, so it is issued after the first barrier.
+//   entry() runs after the first barrier: there the caller learns the next item, which tail() and the
+//   ring need from then on.
 //   own(i) gives this item's stage i, tail(j) the next item's stage j -- or, when there is no such
 //   stage, any valid source (a refetch: nothing reads it, and the next chain start's vmcnt(0)
 //   completes it before its slot is loaded again).  Both are evaluated and one is selected, so no
@@ -177,9 +184,9 @@ __device__ __forceinline__ void chain_start(int8_t* smem, int base, int nit, Own
     }
 }
 
-template <class C, class Own, class Tail>
+template <class C, class Own, class Tail, class Entry>
 __device__ __forceinline__ void mainloop_chain(v16i (&acc)[C::FM][C::FN], int8_t* smem, int base, int nit, Own own,
-                                               Tail tail) {
+                                               Tail tail, Entry entry) {
     static_assert(C::STAGES == 2, "the chain keeps two slots");
     constexpr int KSTEPS = C::BK / 32;
     const int lane = threadIdx.x & 63;
@@ -197,10 +204,14 @@ __device__ __forceinline__ void mainloop_chain(v16i (&acc)[C::FM][C::FN], int8_t
         block_sync_lds();
     };
     Frags<C> f[2];
-    wait_vmcnt<0>();
+    // Stage 0 is the oldest of this wave's outstanding operations, and LPS loads of chain stage 1 and the
+    // previous item's stores (if any) follow it.
+    if (nit >= 2) wait_vmcnt<C::LPS>();
+    else wait_vmcnt<0>();
     lds_barrier();
-    if (nit == 1) issue(1);
     load_frags<C>(f[0], slot(0), 0, wm, wn, lane);
+    entry();
+    if (nit == 1) issue(1);
     for (int it = 0; it + 1 < nit; ++it) {
         const int8_t* cur = slot(it);
 #pragma unroll

@@ -180,11 +180,10 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
         };
         v16i acc[C::FM][C::FN];
         fill_acc<C>(acc, (int)cur.bias);
-        mainloop_chain<C>(acc, smem, base, cur.KT, own_of(cur), tail);
+        mainloop_chain<C>(acc, smem, base, cur.KT, own_of(cur), tail, [] {});
         store_digits<C, true, true>(acc, cur.plane, cur.Np, (int64_t)cur.tm * C::BM + wm * C::WTM,
                                     (int64_t)cur.tn * C::BN + wn * C::WTN, cur.M, cur.N, cur.m, cur.minv, lane);
         if (!more) break;
-        // the epilogue's stores are drained by the next item's first stage wait
         base = (base + cur.KT) & 1;
         w = w2;
         cur = nxt;

@@ -29,18 +29,133 @@ namespace {
 using namespace core;
 
 // ------------------------------------------------------------------------------------------
-// Work order of the persistent GEMMs (one workgroup per CU).  Work items are split into 8
-// contiguous runs, one per XCD (workgroup b runs on XCD b % 8):
-//   static order (queue == null): workgroup b takes positions b, b + gridDim.x, ... of the whole
-//     list (through xcd_remap for Scheme II);
-//   dynamic order (queue != null, gridDim.x a multiple of 8): the workgroups of XCD v take the
-//     positions of run v in the order they ask for them (counter queue[v]), so that the items in
-//     flight on one XCD stay neighbours and share their operand panels in L2 even when CUs drift
-//     apart.
-// A workgroup knows its next item while it works on the current one (the chain issues the next
-// item's first stages during the current item's last iterations).  With the dynamic order, thread 0
-// asks for the item after next when the current item's mainloop ends; the answer comes back during
-// the epilogue and is passed to every wave through LDS (Claims below).
+// Work order of the persistent GEMMs (one workgroup per CU).  Scheme II's items are all of one length:
+// workgroup b takes positions b, b + gridDim.x, ... of the item list through xcd_remap, so that each XCD
+// (workgroup b runs on XCD b % 8) works through a contiguous run and its tiles in flight share their
+// operand panels in L2.  Taking positions from per-XCD counters instead, to keep them neighbours when
+// CUs drift apart, fetches less (13.4 against 19.1 GB at 8192^3 unbanded) in the same time, and the
+// claim's wait costs 0.6 % (8192^3, S = 17: 8.715 against 8.667 ms; 4096^2 x 1024, S = 16: 415 against
+// 410 us).  Scheme I's items differ in length and do take them from counters (Claims below).
+// ------------------------------------------------------------------------------------------
+
+// ------------------------------------------------------------------------------------------
+// Scheme II
+// ------------------------------------------------------------------------------------------
+struct S2Args {
+    const int8_t* A;
+    const int8_t* B;
+    int64_t M, N, Mp, Np, Kp;
+    int S, KT, tiles_m, tiles_n;
+    int tm0;               // first tile row: the launch covers tile rows [tm0, tm0 + tiles_m)
+    void* out;             // digits or int32 planes
+    const CrtSet* crt;     // device copy (m, minv, bias used)
+    int split, kts;        // K parts and K steps per part (SPLIT only)
+};
+
+// Work items (modulus, tile) in logical order l = 0..total-1: modulus-major; inside a modulus,
+// tiles in groups of GM tile rows.  SPLIT: items (part j, modulus, tile), part-major, part j over
+// K steps [j kts, min((j + 1) kts, KT)), its digits into plane set j of the output.
+template <class C, bool DIGITS, bool SPLIT = false>
+__global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
+    __shared__ __attribute__((aligned(1024))) int8_t smem[C::LDS_BYTES];
+    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n, total = tiles * p.S;
+    const int64_t items = SPLIT ? total * p.split : total;
+    int64_t w = blockIdx.x;
+    if (w >= items) return;  // whole workgroup leaves together
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = wave / C::NWN, wn = wave % C::NWN;
+    struct Item {
+        int s, tm, tn, j, k0, KT;
+        const int8_t* a;
+        const int8_t* b;
+        uint32_t m, minv, bias;
+    };
+    auto decode = [&](int64_t wi) {
+        Item t;
+        int64_t l = xcd_remap(wi, items);
+        t.j = 0;
+        t.k0 = 0;
+        t.KT = p.KT;
+        if (SPLIT) {
+            t.j = (int)(l / total);
+            l -= (int64_t)t.j * total;
+            t.k0 = t.j * p.kts;
+            t.KT = min(p.kts, p.KT - t.k0);
+        }
+        t.s = (int)(l / tiles);
+        grouped_tile<C>(l - (int64_t)t.s * tiles, p.tiles_m, p.tiles_n, t.tm, t.tn);
+        t.tm += p.tm0;
+        // tile (tm, tn) starts at block-row tm*BM/32 of the fragment-tiled planes (BM*Kp bytes)
+        t.a = p.A + (int64_t)t.s * p.Mp * p.Kp + (int64_t)t.tm * C::BM * p.Kp;
+        t.b = p.B + (int64_t)t.s * p.Np * p.Kp + (int64_t)t.tn * C::BN * p.Kp;
+        // scalar loads: counted by lgkmcnt, so the epilogue does not wait for the direct loads
+        t.m = as_constant(p.crt)->m[t.s];
+        t.minv = as_constant(p.crt)->minv[t.s];
+        t.bias = as_constant(p.crt)->bias[t.s];
+        return t;
+    };
+    Item cur = decode(w);
+    auto own_of = [&](const Item& t) {
+        return [&t, &p](int i) { return StageSrc{t.a, t.b, p.Kp, (t.k0 + i) * C::BK}; };
+    };
+    chain_start<C>(smem, 0, cur.KT, own_of(cur));
+    int base = 0;  // ring slot of the current item's stage 0
+    for (;;) {
+        w += gridDim.x;
+        const bool more = w < items;
+        Item nxt = cur;
+        auto entry = [&] {
+            if (more) nxt = decode(w);
+        };
+        // The next item's stage j; past its stages, or with no next item, a refetch of this item's
+        // last stage.
+        auto tail = [&](int j) {
+            const bool real = more && j < nxt.KT;
+            return StageSrc{real ? nxt.a : cur.a, real ? nxt.b : cur.b, p.Kp,
+                            (real ? nxt.k0 + j : cur.k0 + cur.KT - 1) * C::BK};
+        };
+        v16i acc[C::FM][C::FN];
+        if (DIGITS) fill_acc<C>(acc, (int)cur.bias);
+        else zero_acc<C>(acc);
+        mainloop_chain<C>(acc, smem, base, cur.KT, own_of(cur), tail, entry);
+        const int s = cur.s, tm = cur.tm, tn = cur.tn;
+        if (DIGITS) {
+            uint8_t* plane = reinterpret_cast<uint8_t*>(p.out) + ((int64_t)cur.j * p.S + s) * p.Mp * p.Np;
+            store_digits<C, false>(acc, plane, p.Np, (int64_t)tm * C::BM + wm * C::WTM, (int64_t)tn * C::BN + wn * C::WTN,
+                                   p.M, p.N, cur.m, cur.minv, lane);
+        } else {
+            int32_t* o = reinterpret_cast<int32_t*>(p.out) + (int64_t)s * p.M * p.N;
+#pragma unroll
+            for (int fm = 0; fm < C::FM; ++fm)
+#pragma unroll
+                for (int fn = 0; fn < C::FN; ++fn) {
+                    const int64_t col = (int64_t)tn * C::BN + wn * C::WTN + fn * 32 + (lane & 31);
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) {
+                        const int64_t row = (int64_t)tm * C::BM + wm * C::WTM + fm * 32 + frag_row(j, lane);
+                        if (row < p.M && col < p.N) o[row * p.N + col] = acc[fm][fn][j];
+                    }
+                }
+        }
+        if (!more) break;
+        base = (base + cur.KT) & 1;
+        cur = nxt;
+    }
+    wait_vmcnt<0>();  // no direct load in flight into LDS when the workgroup leaves
+}
+
+// Split-K digit reduction of a single call: 4 KiB of the S digit planes per workgroup (Mp * Np is a
+// multiple of 65536, so a workgroup's bytes lie in one plane), partial sets after set 0.
+__global__ void __launch_bounds__(256) k_digits_reduce(uint8_t* dg, int64_t plane, int S, int split,
+                                                       const CrtSet* crt) {
+    const int64_t off = (int64_t)blockIdx.x * 4096 + threadIdx.x * 16;
+    const int s = (int)(off / plane);
+    const int64_t stride = (int64_t)S * plane;
+    reduce_digits16(dg, dg + stride, stride, split - 1, crt->m[s], off);
+}
+
+// ------------------------------------------------------------------------------------------
+// Scheme I
 // ------------------------------------------------------------------------------------------
 struct Claims {
     int64_t w, w1;  // positions of the current and the next item
@@ -77,136 +192,6 @@ __device__ __forceinline__ int64_t publish_claim(unsigned ticket, unsigned* s_po
     return s_pos[1];
 }
 
-// ------------------------------------------------------------------------------------------
-// Scheme II
-// ------------------------------------------------------------------------------------------
-struct S2Args {
-    const int8_t* A;
-    const int8_t* B;
-    int64_t M, N, Mp, Np, Kp;
-    int S, KT, tiles_m, tiles_n;
-    int tm0;               // first tile row: the launch covers tile rows [tm0, tm0 + tiles_m)
-    void* out;             // digits or int32 planes
-    const CrtSet* crt;     // device copy (m, minv, bias used)
-    unsigned* queue;       // 8 work counters, zero at launch (dynamic order), or null (static order)
-    int split, kts;        // K parts and K steps per part (SPLIT only)
-};
-
-// Work items (modulus, tile) in logical order l = 0..total-1: modulus-major; inside a modulus,
-// tiles in groups of GM tile rows.  SPLIT: items (part j, modulus, tile), part-major, part j over
-// K steps [j kts, min((j + 1) kts, KT)), its digits into plane set j of the output.
-template <class C, bool DIGITS, bool SPLIT = false>
-__global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
-    __shared__ __attribute__((aligned(1024))) int8_t smem[C::LDS_BYTES];
-    __shared__ unsigned s_pos[2];
-    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n, total = tiles * p.S;
-    const int64_t items = SPLIT ? total * p.split : total;
-    const bool dyn = p.queue != nullptr;
-    const int xcd = blockIdx.x & 7;
-    const int64_t run = items >> 3, run0 = (int64_t)xcd * run;
-    const int64_t nwork = dyn ? (xcd == 7 ? items - 7 * run : run) : items;  // positions to take
-    Claims c = first_claims(p.queue, xcd, s_pos);
-    if (c.w >= nwork) return;  // whole workgroup leaves together
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = wave / C::NWN, wn = wave % C::NWN;
-    struct Item {
-        int s, tm, tn, j, k0, KT;
-        const int8_t* a;
-        const int8_t* b;
-        uint32_t m, minv, bias;
-    };
-    auto decode = [&](int64_t wi) {
-        Item t;
-        int64_t l = dyn ? run0 + wi : xcd_remap(wi, items);
-        t.j = 0;
-        t.k0 = 0;
-        t.KT = p.KT;
-        if (SPLIT) {
-            t.j = (int)(l / total);
-            l -= (int64_t)t.j * total;
-            t.k0 = t.j * p.kts;
-            t.KT = min(p.kts, p.KT - t.k0);
-        }
-        t.s = (int)(l / tiles);
-        grouped_tile<C>(l - (int64_t)t.s * tiles, p.tiles_m, p.tiles_n, t.tm, t.tn);
-        t.tm += p.tm0;
-        // tile (tm, tn) starts at block-row tm*BM/32 of the fragment-tiled planes (BM*Kp bytes)
-        t.a = p.A + (int64_t)t.s * p.Mp * p.Kp + (int64_t)t.tm * C::BM * p.Kp;
-        t.b = p.B + (int64_t)t.s * p.Np * p.Kp + (int64_t)t.tn * C::BN * p.Kp;
-        // scalar loads: counted by lgkmcnt, so the epilogue does not wait for the direct loads
-        t.m = as_constant(p.crt)->m[t.s];
-        t.minv = as_constant(p.crt)->minv[t.s];
-        t.bias = as_constant(p.crt)->bias[t.s];
-        return t;
-    };
-    Item cur = decode(c.w);
-    auto own_of = [&](const Item& t) {
-        return [&t, &p](int i) { return StageSrc{t.a, t.b, p.Kp, (t.k0 + i) * C::BK}; };
-    };
-    chain_start<C>(smem, 0, cur.KT, own_of(cur));
-    int base = 0;  // ring slot of the current item's stage 0
-    for (;;) {
-        const bool more = c.w1 < nwork;
-        const Item nxt = more ? decode(c.w1) : cur;
-        // The next item's stage j; past its stages, or with no next item, a refetch of this item's
-        // last stage.
-        auto tail = [&](int j) {
-            const bool real = more && j < nxt.KT;
-            return StageSrc{real ? nxt.a : cur.a, real ? nxt.b : cur.b, p.Kp,
-                            (real ? nxt.k0 + j : cur.k0 + cur.KT - 1) * C::BK};
-        };
-        v16i acc[C::FM][C::FN];
-        if (DIGITS) fill_acc<C>(acc, (int)cur.bias);
-        else zero_acc<C>(acc);
-        mainloop_chain<C>(acc, smem, base, cur.KT, own_of(cur), tail);
-        // The item after next (dynamic order).  Only thread 0's ticket is used, so the other lanes
-        // leave it unset: a value merged from both paths would be copied as soon as the atomic
-        // returns, and the wait for it would hold the epilogue behind the next item's loads.
-        unsigned ticket;
-        if (dyn && more && threadIdx.x == 0) ticket = atomicAdd(&p.queue[xcd], 1u);
-        const int s = cur.s, tm = cur.tm, tn = cur.tn;
-        if (DIGITS) {
-            uint8_t* plane = reinterpret_cast<uint8_t*>(p.out) + ((int64_t)cur.j * p.S + s) * p.Mp * p.Np;
-            store_digits<C, false>(acc, plane, p.Np, (int64_t)tm * C::BM + wm * C::WTM, (int64_t)tn * C::BN + wn * C::WTN,
-                                   p.M, p.N, cur.m, cur.minv, lane);
-        } else {
-            int32_t* o = reinterpret_cast<int32_t*>(p.out) + (int64_t)s * p.M * p.N;
-#pragma unroll
-            for (int fm = 0; fm < C::FM; ++fm)
-#pragma unroll
-                for (int fn = 0; fn < C::FN; ++fn) {
-                    const int64_t col = (int64_t)tn * C::BN + wn * C::WTN + fn * 32 + (lane & 31);
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) {
-                        const int64_t row = (int64_t)tm * C::BM + wm * C::WTM + fm * 32 + frag_row(j, lane);
-                        if (row < p.M && col < p.N) o[row * p.N + col] = acc[fm][fn][j];
-                    }
-                }
-        }
-        if (!more) break;
-        // the epilogue's stores are drained by the next chain start's vmcnt(0)
-        const int64_t w2 = dyn ? publish_claim(ticket, s_pos) : c.w1 + gridDim.x;
-        base = (base + cur.KT) & 1;
-        c.w = c.w1;
-        c.w1 = w2;
-        cur = nxt;
-    }
-    wait_vmcnt<0>();  // no direct load in flight into LDS when the workgroup leaves
-}
-
-// Split-K digit reduction of a single call: 4 KiB of the S digit planes per workgroup (Mp * Np is a
-// multiple of 65536, so a workgroup's bytes lie in one plane), partial sets after set 0.
-__global__ void __launch_bounds__(256) k_digits_reduce(uint8_t* dg, int64_t plane, int S, int split,
-                                                       const CrtSet* crt) {
-    const int64_t off = (int64_t)blockIdx.x * 4096 + threadIdx.x * 16;
-    const int s = (int)(off / plane);
-    const int64_t stride = (int64_t)S * plane;
-    reduce_digits16(dg, dg + stride, stride, split - 1, crt->m[s], off);
-}
-
-// ------------------------------------------------------------------------------------------
-// Scheme I
-// ------------------------------------------------------------------------------------------
 struct S1Args {
     const int8_t* A;
     const int8_t* B;
@@ -261,7 +246,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1(S1Args p) {
         };
         v16i acc[C::FM][C::FN];
         zero_acc<C>(acc);
-        mainloop_chain<C>(acc, smem, base, nit, own_of(g), tail);
+        mainloop_chain<C>(acc, smem, base, nit, own_of(g), tail, [] {});
         int32_t* o = p.T + (int64_t)(g - 2) * p.M * p.N;
 #pragma unroll
         for (int fm = 0; fm < C::FM; ++fm)
@@ -338,7 +323,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1g(S1Args p) {
         };
         v16i acc[C::FM][C::FN];
         zero_acc<C>(acc);
-        mainloop_chain<C>(acc, smem, base, cur.nit, own_of(cur), tail);
+        mainloop_chain<C>(acc, smem, base, cur.nit, own_of(cur), tail, [] {});
         unsigned ticket;  // the item after next (dynamic order); thread 0's only, as in k_igemm_s2
         if (dyn && more && threadIdx.x == 0) ticket = atomicAdd(&p.queue[xcd], 1u);
         store_i32_blocked<C>(acc, p.T + (int64_t)(cur.g - 2) * p.Mp * p.Np, p.Np,
@@ -371,7 +356,7 @@ using CfgS2 = IgemmCfgS2;
 using CfgS1 = IgemmCfgS1;
 
 hipError_t launch_igemm_s2(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, S2Out mode, void* out,
-                           const CrtSet* crt_dev, hipStream_t st, int tm0, int tms, unsigned* queue, int split) {
+                           const CrtSet* crt_dev, hipStream_t st, int tm0, int tms, int split) {
     if (split < 1 || (split > 1 && mode != S2Out::Digits)) return hipErrorInvalidValue;
     S2Args p;
     p.A = A_sl;
@@ -396,10 +381,6 @@ hipError_t launch_igemm_s2(const Dims& d, const int8_t* A_sl, const int8_t* B_sl
     if (total == 0) return hipSuccess;
     unsigned grid = 0;
     if (hipError_t e = persistent_grid(total, grid)) return e;
-    // A workgroup of the dynamic order claims two positions before it starts, so with fewer than two
-    // items per workgroup the first claimants would take them all and the others none: below that,
-    // the static order (every workgroup its own positions) is the balanced one.
-    p.queue = queue && grid % 8 == 0 && total >= 2 * (int64_t)grid ? queue : nullptr;  // counters zeroed by the caller
     if (mode == S2Out::Digits && p.split > 1)
         k_igemm_s2<CfgS2, true, true><<<grid, CfgS2::NT, 0, st>>>(p);
     else if (mode == S2Out::Digits)
@@ -458,7 +439,9 @@ hipError_t launch_igemm_s1_blocked(const Dims& d, const int8_t* A_sl, const int8
     if (total == 0) return hipSuccess;
     unsigned grid = 0;
     if (hipError_t e = persistent_grid(total, grid)) return e;
-    // two positions claimed up front: dynamic order only with at least two items per workgroup
+    // A workgroup of the dynamic order claims two positions before it starts, so with fewer than two
+    // items per workgroup the first claimants would take them all and the others none: below that,
+    // the static order (every workgroup its own positions) is the balanced one.
     p.queue = queue && grid % 8 == 0 && total >= 2 * (int64_t)grid ? queue : nullptr;  // counters zeroed by the caller
     k_igemm_s1g<CfgS2><<<grid, CfgS2::NT, 0, st>>>(p);
     return hipGetLastError();
