@@ -244,9 +244,12 @@ int oza_scheme2_slices_for_accuracy(size_t K, double digits, double spread, int*
 
 // ------------------------------------------------------------------------ pipelines
 // Row bands for overlapping step 4 with step 3 (both schemes; bands of whole 256-row tiles).
-// Scheme II, automatic: the most bands (up to 4) for which every band's products still take at
-// least 8 rounds of one tile per CU and the bands' partial last rounds cost at most one round in
-// total.  Scheme I (items of g - 1 pair products, largest first): the most bands (up to 4) with at
+// Scheme II, automatic: for K >= 2048 the most bands (up to 4) for which every band's products still
+// take at least 8 rounds of one tile per CU and the bands' partial last rounds cost at most 1/32 of the
+// rounds in total.  One to four bands: 8192^2 x 2048, S = 17 (4 x 17 rounds) 2.757 to 2.655 ms,
+// 8192^3, S = 12 6.42 to 6.39 ms; but 4096^3, S = 17 (17 rounds, 18 in two bands) 1.314 to 1.352 ms in
+// two, and with short items, whose GEMM the reconstruction beside it slows by more than it hides,
+// 8192^2 x 1024 1.643 to 1.671 ms, x 512 1.12 to 1.25 ms.  Scheme I (items of g - 1 pair products, largest first): the most bands (up to 4) with at
 // least 16 pair products per CU in every band.  1 (no overlap) when none qualifies.
 static int pipeline_bands(const oza_context* ctx, int scheme, const Dims& d) {
     const int64_t tm = (d.M + kS2TileRows - 1) / kS2TileRows, tn = (d.N + kS2TileRows - 1) / kS2TileRows;
@@ -261,7 +264,7 @@ static int pipeline_bands(const oza_context* ctx, int scheme, const Dims& d) {
     auto rounds = [&](int64_t items) { return (items + cus - 1) / cus; };
     const int64_t whole = rounds(tm * tn * d.S);
     for (int nb = 4; nb >= 2; --nb) {
-        if (tm < nb) continue;
+        if (tm < nb || d.K < 2048) continue;
         int64_t sum = 0, least = INT64_MAX;
         for (int b = 0; b < nb; ++b) {
             const int64_t rows = tm * (b + 1) / nb - tm * b / nb;
@@ -269,7 +272,7 @@ static int pipeline_bands(const oza_context* ctx, int scheme, const Dims& d) {
             sum += r;
             least = std::min(least, r);
         }
-        if (least >= 8 && sum <= whole + 1) return nb;
+        if (least >= 8 && sum <= whole + whole / 32) return nb;
     }
     return 1;
 }
