@@ -25,10 +25,8 @@ namespace {
 
 using namespace core;
 
-// Blocks a one-pass launch aims for by dealing a row block's planes to several blocks: one per CU.
-// 1024^3, S = 16 (128 row blocks): 53 us per call undivided, 46 us in two parts, 48 in four, 55 in eight.
-constexpr int64_t kPassTargetBlocks = 256;
-constexpr int64_t kPassResident = 512;
+// Blocks of a one-pass launch that run at once when K is long (one 1024-thread block per CU).
+constexpr int64_t kPassResident = 256;
 
 // Blocks [0, a.nblk) slice operand a into its planes, the rest operand b.
 template <int ND>
@@ -46,9 +44,9 @@ __global__ void __launch_bounds__(kSliceThreads)
 
 // Steps 1 and 2 of both operands in one launch (pass_block).  Block b -> part and row block: sets of 8
 // consecutive row blocks (of operand 0, then operand 1), each set's parts after one another.
-template <int ND, int NU>
-__global__ void __launch_bounds__(kPassThreads) k_pass(PassArgs g, ResidueConsts rc) {
-    __shared__ uint32_t s_key[kPassThreads];
+template <int ND, int T, int NU>
+__global__ void __launch_bounds__(T) k_pass(PassArgs g, ResidueConsts rc) {
+    __shared__ uint32_t s_key[T];
     __shared__ int32_t s_shift[64];
     if (blockIdx.x == 0 && (int)threadIdx.x < g.nzero) g.zero[threadIdx.x] = 0;
     const int64_t set = blockIdx.x / (8 * g.parts);
@@ -59,16 +57,17 @@ __global__ void __launch_bounds__(kPassThreads) k_pass(PassArgs g, ResidueConsts
     if (w) rb -= g.op[0].nrow;
     const PassOp& o = g.op[w];
     if (rb >= o.nrow) return;  // past the last set's row blocks (whole block)
-    if (o.kcontig) pass_block<ND, NU, true>(o, g, rc, rb, part, s_key, s_shift);
-    else pass_block<ND, NU, false>(o, g, rc, rb, part, s_key, s_shift);
+    if (o.kcontig) pass_block<ND, T, NU, true>(o, g, rc, rb, part, s_key, s_shift);
+    else pass_block<ND, T, NU, false>(o, g, rc, rb, part, s_key, s_shift);
 }
 
 template <int ND>
 hipError_t launch_pass_words(const PassArgs& g, const ResidueConsts& rc, unsigned grid, hipStream_t st) {
-    switch (pass_units(g.Kp)) {
-        case 1: k_pass<ND, 1><<<grid, kPassThreads, 0, st>>>(g, rc); break;
-        case 2: k_pass<ND, 2><<<grid, kPassThreads, 0, st>>>(g, rc); break;
-        default: k_pass<ND, 4><<<grid, kPassThreads, 0, st>>>(g, rc); break;
+    switch (pass_threads(g.Kp) * pass_units(g.Kp)) {
+        case 256: k_pass<ND, 256, 1><<<grid, 256, 0, st>>>(g, rc); break;
+        case 512: k_pass<ND, 512, 1><<<grid, 512, 0, st>>>(g, rc); break;
+        case 1024: k_pass<ND, 1024, 1><<<grid, 1024, 0, st>>>(g, rc); break;
+        default: k_pass<ND, 1024, 2><<<grid, 1024, 0, st>>>(g, rc); break;
     }
     return hipGetLastError();
 }
@@ -120,15 +119,15 @@ hipError_t launch_slice_s1(const Dims& d, int beta, const Operand& A, const Oper
     return hipGetLastError();
 }
 
-// Not when a second round of the resident blocks (two per CU at four units per thread) would hold a few
-// blocks only, which take as long as a full one: 200 x 8000 x 900, S = 16 (514 row blocks) 125 us in one
-// pass, 112 us in two kernels; 5000 x 4000 x 1000 (563) 518 against 523, 1000 x 6000 x 1000 (438) 179
-// against 188.
+// Not when one more round of 1024-thread blocks would hold a few blocks only, which take as long as a full
+// round, unless there are many rounds: 200 x 8000 x 900, S = 16 (514 row blocks) 120 us per call in one
+// pass, 114 us in two kernels; 200 x 7800 x 900 (502) 102 against 109, 200 x 6000 x 900 (389) 88 against 93.
 bool one_pass(const Dims& d) {
     if (d.Kp > kPassMaxKp) return false;
     const int R = pass_rows(d.Kp);
-    const int64_t over = pass_row_blocks(d.M, R) + pass_row_blocks(d.N, R) - kPassResident;
-    return !(pass_units(d.Kp) == 4 && over > 0 && over < kPassResident / 16);
+    const int64_t n = pass_row_blocks(d.M, R) + pass_row_blocks(d.N, R), over = n % kPassResident;
+    return !(pass_threads(d.Kp) == 1024 && n > kPassResident && n < 4 * kPassResident && over > 0 &&
+             over < kPassResident / 8);
 }
 
 hipError_t launch_one_pass(int scheme, const Dims& d, int offset, const Operand& A, const Operand& B, int32_t* shift_A,
@@ -141,17 +140,19 @@ hipError_t launch_one_pass(int scheme, const Dims& d, int offset, const Operand&
     g.offset = offset;
     g.zero = zero;
     g.nzero = nzero;
-    if (nzero > kPassThreads) return hipErrorInvalidValue;
+    if (nzero > 256) return hipErrorInvalidValue;
     auto op = [&](const Operand& X, int64_t rows, int64_t rows_p, int32_t* shift, int8_t* out) {
         return PassOp{X.p, rows, rows_p, X.ld, X.kcontig, shift, out, pass_row_blocks(rows, g.R)};
     };
     g.op[0] = op(A, d.M, d.Mp, shift_A, A_sl);
     g.op[1] = op(B, d.N, d.Np, shift_B, B_sl);
     const int64_t nrow = g.op[0].nrow + g.op[1].nrow;
+    // Parts while the blocks still run at once: 1024^3, S = 16 (128 row blocks) 49 us per call undivided,
+    // 45 in two parts, 51 in four; 500 x 500 x 1000 (64) 39, 34 and 33; 777 x 1501 x 1003 (146) 60, 62 and 65.
     g.parts = 1;
-    while (2 * g.parts <= std::min(d.S, 8) && nrow * g.parts < kPassTargetBlocks) g.parts *= 2;
+    while (2 * g.parts <= std::min(d.S, 8) && nrow * g.parts * 2 <= kPassResident) g.parts *= 2;
     const int64_t grid = (nrow + 7) / 8 * 8 * g.parts;
-    if (grid * kPassThreads > (int64_t)UINT32_MAX) return hipErrorInvalidValue;
+    if (grid * pass_threads(d.Kp) > (int64_t)UINT32_MAX) return hipErrorInvalidValue;
     const ResidueConsts rc = make_residue_consts();
     if (scheme == 1) return launch_pass_words<0>(g, rc, (unsigned)grid, st);
     switch (residue_words(offset)) {

@@ -357,29 +357,30 @@ __device__ __forceinline__ void slice_s1_op_block(const SliceOp& o, int64_t K, i
 }
 
 // ---------------------------------------------------------------- steps 1 and 2 in one pass, both operands
-// Single calls with Kp <= kPassMaxKp: a block of 256 threads holds R whole rows (columns of a
-// row-contiguous operand) in registers, takes their exponent maxima, writes the shifts and then the
-// slices of the values it still holds.  Unit u = (row u % R, 16-byte K chunk u / R) of the block; thread t
-// takes units t + 256 i, i < NU, all of row t % R.  With R = 16 a wave reads a row-contiguous operand
-// in 128-byte runs and writes 256-byte runs of a fragment block; R grows to 64 for short K so that the
-// threads have units.  Values and results are those of the separate kernels.
+// Single calls with Kp <= kPassMaxKp: a block of T threads (pass_threads: 256, 512 or 1024 by K) holds R
+// whole rows (columns of a row-contiguous operand) in registers, takes their exponent maxima, writes
+// the shifts and then the slices of the values it still holds.  Unit u = (row u % R, 16-byte K chunk u / R)
+// of the block; thread t takes units t + T i, i < NU, all of row t % R.  With R = 16 a wave reads a
+// row-contiguous operand in 128-byte runs and writes 256-byte runs of a fragment block; R grows to 64
+// for short K so that the threads have units.  Values and results are those of the separate kernels.
 // A block's planes may be dealt to `parts` blocks that each read the rows again (part j stores planes
 // [S j / parts, S (j + 1) / parts), part 0 the shifts): more blocks for small operands, whose second
 // reads come from the XCD's L2 (the parts of a row block are 8 block indices apart, on one XCD).
 // Small calls are bound by launches (4.7 us of stream time each) and latency: this takes the place of
-// four launches (keys cleared, maxima, keys to shifts, slices).  256^3, S = 4: 23.9 -> 15.0 us per call;
-// 1024^3, S = 16: 59.6 -> 46.2 us; 777 x 1501 x 1003, S = 14: 70.7 -> 64.4 us.  With Kp up to 2048 in
-// 512-thread blocks (one per CU at 242 registers, nothing to hide its load latency) the launch took 37 us
-// at 2048^3 where the two kernels take 39.
-constexpr int64_t kPassMaxKp = 1024;
-constexpr int kPassThreads = 256;
+// two launches (four before: keys cleared, maxima, keys to shifts, slices).  One or two units per thread
+// and many threads, not four units in 256 threads (184 registers, 8 waves per CU instead of 16):
+// 2048^3, S = 6 111 us per call in two kernels, 101 in one pass (37 us for the launch with four units in 512
+// threads); 1024^3, S = 16 54 and 45; 8192^2 x 1024, S = 16 1.551 and 1.523 ms; 256^3, S = 4 24 and 15 us.
+constexpr int64_t kPassMaxKp = 2048;
 
-inline int pass_units(int64_t Kp) { return Kp <= 256 ? 1 : Kp <= 512 ? 2 : 4; }
+inline int pass_threads(int64_t Kp) { return Kp <= 256 ? 256 : Kp <= 512 ? 512 : 1024; }
+inline int pass_units(int64_t Kp) { return Kp <= 1024 ? 1 : 2; }
 inline int pass_rows(int64_t Kp) {
     int r = 64;
-    while (r > 16 && r * (Kp / 16) > kPassThreads * pass_units(Kp)) r >>= 1;
+    while (r > 16 && r * (Kp / 16) > pass_threads(Kp) * pass_units(Kp)) r >>= 1;
     return r;
 }
+
 // Row blocks of an operand: the rows its planes hold, whole 32-row fragment blocks.
 inline int64_t pass_row_blocks(int64_t rows, int R) { return ((rows + 31) / 32 * 32 + R - 1) / R; }
 
@@ -401,12 +402,12 @@ struct PassArgs {
 };
 
 // ND: words per value (Scheme II), or 0 for Scheme I.
-template <int ND, int NU, bool KC>
+template <int ND, int T, int NU, bool KC>
 __device__ __forceinline__ void pass_block(const PassOp& o, const PassArgs& g, const ResidueConsts& rc, int64_t rb,
                                            int part, uint32_t* s_key, int32_t* s_shift) {
     const int R = g.R;
     const int t = threadIdx.x;
-    const int rl = t & (R - 1), c0 = t / R, cstep = kPassThreads / R;
+    const int rl = t & (R - 1), c0 = t / R, cstep = T / R;
     const int64_t row = rb * R + rl;
     const int U = (int)(g.Kp / 16);
     double a[NU][16];
@@ -440,7 +441,7 @@ __device__ __forceinline__ void pass_block(const PassOp& o, const PassArgs& g, c
     if (t < R) {
         uint32_t k = 0;
 #pragma unroll
-        for (int w = 0; w < kPassThreads / 64; ++w) k = max(k, s_key[w * 64 + t]);
+        for (int w = 0; w < T / 64; ++w) k = max(k, s_key[w * 64 + t]);
         const int32_t sh = (ND == 0 ? 0 : g.offset) - exp_from_key(k);  // key_to_shift
         s_shift[t] = sh;
         if (part == 0 && row < o.rows) o.shift[row] = sh;

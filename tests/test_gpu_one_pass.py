@@ -1,4 +1,4 @@
-"""Steps 1 and 2 of single calls (one launch for Kp <= 1024, else partial maxima finished by the
+"""Steps 1 and 2 of single calls (one launch for Kp <= 2048, else partial maxima finished by the
 slicing kernels) against the separate kernels of the
 stage entry points and the oracle: shifts and planes byte for byte, at the edges of its unit, row-block,
 word-count and part choices, with non-finite values, and for both orientations of each operand."""
@@ -9,11 +9,11 @@ from test_gpu_parity import gen_pair, special_matrix, stage_shifts, stage_slices
 
 pytestmark = pytest.mark.gpu
 
-# K at the edges of 1, 2 and 4 units per thread and of the path; rows at the edges of 16, 32, 64; many
+# K at the edges of the thread counts, of 1 and 2 units per thread and of the path; rows at the edges of 16, 32, 64; many
 # and few row blocks (parts 1, 2, 4, 8); S at the edges of one, two and three words per value
 CASES = [(1, 1, 1, 20), (15, 17, 128, 1), (16, 33, 129, 3), (31, 64, 256, 5), (65, 48, 257, 8), (100, 63, 384, 20),
          (63, 129, 512, 10), (64, 1, 513, 17), (250, 31, 1000, 16), (33, 260, 1024, 18), (1700, 2500, 700, 9),
-         (40, 50, 1025, 12), (200, 8000, 900, 4), (1024, 33, 5001, 9), (1100, 1023, 1300, 6), (3, 70, 40000, 7)]
+         (40, 50, 1025, 12), (200, 8000, 900, 4), (1024, 33, 5001, 9), (1100, 1023, 2049, 6), (70, 1023, 1300, 6), (33, 40, 2048, 19), (130, 47, 1025, 2), (3, 70, 40000, 7)]
 
 
 @pytest.mark.parametrize("scheme", [1, 2])
