@@ -95,11 +95,12 @@ int oza_ctx_event_times(oza_ctx ctx, double sums[5], int* count);
  *   shift_A int32[M], shift_B int32[N]          (reference semantics)
  *   A_slices int8 [S][Mp][Kp], B_slices int8 [S][Np][Kp] (B transposed: K contiguous)
  *   C_tc   Scheme II: S planes of uint8 CRT digits (-2^-32 C_s mod m_s), Mp x Np each in 32 x 32 element
- *          blocks (oza_unpack_digits gives C_s mod m_s in planar layout), followed, for shapes whose GEMM runs
- *          in K parts (few tiles, long K), by the partial digits of parts 1..; Scheme I: S planes of int32 group
- *          products T_g, Mp x Np each in 32 x 32 element blocks, and at least the reference's
- *          planar int32 [S][M][N] size, which the stage entry points write
- * with Mp = roundup(M,256), Np = roundup(N,256), Kp = roundup(K,128).
+ *          blocks (oza_unpack_digits gives C_s mod m_s in planar layout); Scheme I: S planes of int32 group
+ *          products T_g, Mp x Np each in 32 x 32 element blocks (the stage entry points write the
+ *          reference's planar int32 [S][M][N] there); then room for the partial sums of tiles whose
+ *          products run in several parts along K, for shapes with few tiles
+ * with Mp = roundup(M,256), Np = roundup(N,256), Kp = roundup(K,128).  Sizes grow with each of M, N, K and
+ * slices, so buffers made for the largest of several shapes hold all of them.
  * Fails with OZA_INVALID_ARGUMENT for S outside 1..20 or K beyond exact INT32 accumulation. */
 int oza_workspace_bytes(int scheme, size_t M, size_t N, size_t K, int slices, size_t bytes[5]);
 
@@ -187,7 +188,8 @@ int oza_generate_matrix(size_t rows, size_t cols, double phi, int seed, double* 
  * and op(B) (a column-major call is the row-major product C^T = op(B)^T op(A)^T).  Otherwise each
  * entry is fma(alpha, X, beta * C) of the emulated product X; beta == 0 does not read C, and
  * alpha == 0 or K == 0 only scales C, as in BLAS.  workspace may be NULL: the context then keeps a
- * workspace of its own, grown on demand; otherwise it must hold oza_gemm_workspace_bytes.
+ * workspace of its own, grown on demand; otherwise it must hold oza_gemm_workspace_bytes (one that
+ * holds the call's planes but not its partial sums gives the same result, in whole tiles).
  * Asynchronous on the context's stream. */
 typedef enum oza_layout { OZA_ROW_MAJOR = 0, OZA_COL_MAJOR = 1 } oza_layout;
 typedef enum oza_op { OZA_OP_N = 0, OZA_OP_T = 1 } oza_op;
@@ -200,7 +202,7 @@ int oza_gemm(oza_ctx ctx, int scheme, int slices, int layout, int transA, int tr
  * hipMalloc).  Same arguments and results as oza_gemm, without the workspace: the call's shifts,
  * operand planes and digit (or group-product) planes live in one scratch array of
  * OZA_NOALLOC_SCRATCH_BYTES that the library holds on every device it runs on until the process
- * ends.  A problem whose oza_gemm_workspace_bytes exceeds that size is rejected with
+ * ends.  A problem whose shifts and planes (without partial sums) exceed that size is rejected with
  * OZA_INVALID_ARGUMENT before anything is enqueued.  All calls on one device share the array, so
  * calls that overlap on one device (two streams, two contexts, two threads) race: order them. */
 #define OZA_NOALLOC_SCRATCH_BYTES ((size_t)128 << 20)

@@ -19,17 +19,45 @@ namespace {
 // address (oza_context::scratch) is handed to kernels.
 static __device__ __align__(256) uint8_t scratch[OZA_NOALLOC_SCRATCH_BYTES];
 
-void ws_bytes(int scheme, size_t M, size_t N, size_t K, int S, size_t b[5]) {
-    const Dims d = make_dims(M, N, K, S);
+// How a call's GEMM is cut into items: by the plan of its scheme, or (split false) whole.
+struct CallPlan {
+    S2Plan s2;
+    S1Plan s1;
+};
+
+CallPlan call_plan(int scheme, const Dims& d, bool split = true) {
+    CallPlan p;
+    if (scheme == 2 && split) p.s2 = scheme2_plan(d);
+    if (scheme == 1 && split) p.s1 = scheme1_plan(d);
+    if (scheme == 1 && !split) {
+        p.s1.planes = d.S;
+        std::fill(p.s1.parts, p.s1.parts + d.S, 1);
+    }
+    return p;
+}
+
+// Buffer sizes of a call with the given plan, or (null) those that the sizing entry points report.
+void ws_bytes(int scheme, size_t M, size_t N, const Dims& d, const CallPlan* plan, size_t b[5]) {
+    const size_t S = (size_t)d.S;
     b[0] = sizeof(int32_t) * (M ? M : 1);
     b[1] = sizeof(int32_t) * (N ? N : 1);
-    b[2] = (size_t)S * d.Mp * d.Kp;
-    b[3] = (size_t)S * d.Np * d.Kp;
-    // Scheme II: uint8 digit planes, times the K split of the call (the partial digits of parts
-    // 1.. follow the S planes); Scheme I: INT32 group-product planes (both blocked, Mp x Np), and
-    // at least the reference's planar [S][M][N] INT32 size for the stage entry points.
-    b[4] = scheme == 2 ? (size_t)S * d.Mp * d.Np * (size_t)scheme2_single_split(M, N, K, S)
-                       : sizeof(int32_t) * (size_t)S * std::max((size_t)d.Mp * d.Np, (M ? M : 1) * (N ? N : 1));
+    b[2] = S * d.Mp * d.Kp;
+    b[3] = S * d.Np * d.Kp;
+    // Scheme II: uint8 digit planes, then the plan's partial tiles; Scheme I: INT32 group-product planes
+    // (blocked, Mp x Np, one per part of a group).  Scheme I's S planes also hold the reference's planar
+    // [S][M][N] INT32 of the stage entry points.
+    const size_t tiles = (size_t)(d.Mp / kS2TileRows) * (d.Np / kS2TileRows);
+    if (scheme == 2)
+        b[4] = (size_t)kTileBytes * (plan ? s2_plan_tiles(d, plan->s2) : s2_most_tiles(d));
+    else
+        b[4] = sizeof(int32_t) * std::max(kTileBytes * (plan ? plan->s1.planes * tiles : (size_t)s1_most_tiles(d)),
+                                          S * (M ? M : 1) * (N ? N : 1));
+}
+
+size_t ws_total(const size_t b[5]) {
+    size_t tot = 0;
+    for (int i = 0; i < 5; ++i) tot += (b[i] + 255) / 256 * 256;
+    return tot;
 }
 
 }  // namespace
@@ -209,7 +237,8 @@ int oza_blas_handle(oza_ctx ctx, void** handle) {
 int oza_workspace_bytes(int scheme, size_t M, size_t N, size_t K, int S, size_t bytes[5]) {
     if (!bytes) return fail(OZA_INVALID_ARGUMENT, "null output");
     if (int r = check_problem(scheme, M, N, K, S)) return r;
-    ws_bytes(scheme, M, N, K, S, bytes);
+    const Dims d = make_dims(M, N, K, S);
+    ws_bytes(scheme, M, N, d, nullptr, bytes);
     return OZA_SUCCESS;
 }
 
@@ -286,6 +315,7 @@ static int enqueue_banded(oza_ctx ctx, int scheme, const Dims& d, int nb, const 
     hipStream_t st = ctx->stream;
     const CrtSet* cs = crt_for(ctx, d.S);
     const int beta = scheme1_beta((size_t)d.K);
+    const S1Plan whole = call_plan(1, d, false).s1;
     const int tm = (int)((d.M + kS2TileRows - 1) / kS2TileRows);
     for (int b = 0; b < nb; ++b) {
         const int t0 = (int)((int64_t)tm * b / nb), t1 = (int)((int64_t)tm * (b + 1) / nb);
@@ -293,8 +323,8 @@ static int enqueue_banded(oza_ctx ctx, int scheme, const Dims& d, int nb, const 
             OZA_HIP(launch_igemm_s2(d, Asl, Bsl, S2Out::Digits, Ctc, cs, st, t0, t1 - t0),
                     "step 3 launch");
         else
-            OZA_HIP(launch_igemm_s1_blocked(d, Asl, Bsl, static_cast<int32_t*>(Ctc), st, ctx->queue_dev + 8 * b, t0,
-                                            t1 - t0),
+            OZA_HIP(launch_igemm_s1_blocked(d, Asl, Bsl, static_cast<int32_t*>(Ctc), st, whole, ctx->queue_dev + 8 * b,
+                                            t0, t1 - t0),
                     "step 3 launch");
         const int64_t row0 = (int64_t)t0 * kS2TileRows, rows = (int64_t)(t1 - t0) * kS2TileRows;
         const bool last = b + 1 == nb;
@@ -306,11 +336,11 @@ static int enqueue_banded(oza_ctx ctx, int scheme, const Dims& d, int nb, const 
             OZA_HIP(hipEventRecord(e3, st), "event");
         }
         if (scheme == 2)
-            OZA_HIP(launch_recon_s2_digits(d, static_cast<const uint8_t*>(Ctc), shA, shB, cs, C, rs, row0, rows, !last),
+            OZA_HIP(launch_recon_s2_digits(d, static_cast<uint8_t*>(Ctc), shA, shB, cs, C, rs, row0, rows, !last),
                     "step 4 launch");
         else
-            OZA_HIP(launch_recon_s1_blocked(d, beta, static_cast<const int32_t*>(Ctc), shA, shB, C, rs, row0, rows,
-                                            !last),
+            OZA_HIP(launch_recon_s1_blocked(d, beta, static_cast<int32_t*>(Ctc), shA, shB, C, rs, whole, row0,
+                                            rows, !last),
                     "step 4 launch");
     }
     OZA_HIP(hipEventRecord(ctx->join_ev, ctx->side), "event");
@@ -320,10 +350,11 @@ static int enqueue_banded(oza_ctx ctx, int scheme, const Dims& d, int nb, const 
 
 // The four steps for operands A (M logical rows), B (N logical rows) and output C.  The caller
 // has validated the arguments and made the context's device current.
-static int enqueue_pipeline(int scheme, oza_ctx ctx, size_t M, size_t N, size_t K, int S, const Operand& A,
+static int enqueue_pipeline(int scheme, oza_ctx ctx, const Dims& d, const CallPlan& plan, const Operand& A,
                             const Operand& B, const OutC& C, int32_t* shA, int32_t* shB, int8_t* Asl, int8_t* Bsl,
                             void* Ctc, oza_timings* t) {
-    const Dims d = make_dims(M, N, K, S);
+    const size_t K = (size_t)d.K;
+    const int S = d.S;
     hipStream_t st = ctx->stream;
     hipEvent_t* ev = nullptr;  // events to record this call, if any
     if (t) ev = ctx->ev;
@@ -352,13 +383,11 @@ static int enqueue_pipeline(int scheme, oza_ctx ctx, size_t M, size_t N, size_t 
         if (nb > 1) {
             if (int r = enqueue_banded(ctx, 2, d, nb, Asl, Bsl, Ctc, shA, shB, C, ev ? ev[3] : nullptr)) return r;
         } else {
-            // Few tiles and a long K: the K steps run in parts (partial digits summed mod m_s)
-            const int split = scheme2_single_split(M, N, K, S);
-            OZA_HIP(launch_igemm_s2(d, Asl, Bsl, S2Out::Digits, Ctc, crt_for(ctx, S), st, 0, -1, split),
+            OZA_HIP(launch_igemm_s2(d, Asl, Bsl, S2Out::Digits, Ctc, crt_for(ctx, S), st, 0, -1, &plan.s2),
                     "step 3 launch");
-            OZA_HIP(launch_digits_reduce(d, static_cast<uint8_t*>(Ctc), split, crt_for(ctx, S), st), "step 3 launch");
             if (ev) OZA_HIP(hipEventRecord(ev[3], st), "event");
-            OZA_HIP(launch_recon_s2_digits(d, static_cast<const uint8_t*>(Ctc), shA, shB, crt_for(ctx, S), C, st),
+            OZA_HIP(launch_recon_s2_digits(d, static_cast<uint8_t*>(Ctc), shA, shB, crt_for(ctx, S), C, st, 0, -1,
+                                           false, &plan.s2),
                     "step 4 launch");
         }
     } else {
@@ -366,10 +395,10 @@ static int enqueue_pipeline(int scheme, oza_ctx ctx, size_t M, size_t N, size_t 
         if (nb > 1) {
             if (int r = enqueue_banded(ctx, 1, d, nb, Asl, Bsl, Ctc, shA, shB, C, ev ? ev[3] : nullptr)) return r;
         } else {
-            OZA_HIP(launch_igemm_s1_blocked(d, Asl, Bsl, static_cast<int32_t*>(Ctc), st, ctx->queue_dev),
+            OZA_HIP(launch_igemm_s1_blocked(d, Asl, Bsl, static_cast<int32_t*>(Ctc), st, plan.s1, ctx->queue_dev),
                     "step 3 launch");
             if (ev) OZA_HIP(hipEventRecord(ev[3], st), "event");
-            OZA_HIP(launch_recon_s1_blocked(d, beta, static_cast<const int32_t*>(Ctc), shA, shB, C, st),
+            OZA_HIP(launch_recon_s1_blocked(d, beta, static_cast<int32_t*>(Ctc), shA, shB, C, st, plan.s1),
                     "step 4 launch");
         }
     }
@@ -396,8 +425,9 @@ static int run_pipeline(int scheme, oza_ctx ctx, size_t M, size_t N, size_t K, i
     if (!A || !B || !C || !shA || !shB || !Asl || !Bsl || !Ctc)
         return fail(OZA_INVALID_ARGUMENT, "OzaBLAS: null matrix or workspace pointer.");
     DeviceGuard g(ctx->device);
-    return enqueue_pipeline(scheme, ctx, M, N, K, S, Operand{A, (int64_t)K, true}, Operand{B, (int64_t)N, false},
-                            OutC{C, (int64_t)N, 1.0, 0.0}, shA, shB, Asl, Bsl, Ctc, t);
+    const Dims d = make_dims(M, N, K, S);
+    return enqueue_pipeline(scheme, ctx, d, call_plan(scheme, d), Operand{A, (int64_t)K, true},
+                            Operand{B, (int64_t)N, false}, OutC{C, (int64_t)N, 1.0, 0.0}, shA, shB, Asl, Bsl, Ctc, t);
 }
 
 int oza_scheme1_gemm(oza_ctx ctx, size_t M, size_t N, size_t K, int S, const double* A, const double* B, double* C,
@@ -466,10 +496,9 @@ int oza_gemm_workspace_bytes(int scheme, size_t M, size_t N, size_t K, int S, si
     if (!bytes) return fail(OZA_INVALID_ARGUMENT, "null output");
     if (int r = check_problem(scheme, M, N, K ? K : 1, S)) return r;
     size_t b[5];
-    ws_bytes(scheme, M, N, K ? K : 1, S, b);
-    size_t tot = 0;
-    for (size_t x : b) tot += (x + 255) / 256 * 256;
-    *bytes = tot;
+    const Dims d = make_dims(M, N, K ? K : 1, S);
+    ws_bytes(scheme, M, N, d, nullptr, b);
+    *bytes = ws_total(b);
     return OZA_SUCCESS;
 }
 
@@ -506,11 +535,18 @@ int oza_gemm(oza_ctx ctx, int scheme, int S, int layout, int transA, int transB,
     if (int r = check_problem(scheme, M, N, K, S)) return r;
     if (!A || !B) return fail(OZA_INVALID_ARGUMENT, "OzaBLAS: null matrix pointer.");
     size_t b[5];
-    ws_bytes(scheme, M, N, K, S, b);
-    size_t need = 0;
-    for (size_t x : b) need += (x + 255) / 256 * 256;
+    const Dims d = make_dims(M, N, K, S);
+    CallPlan plan = call_plan(scheme, d);
+    ws_bytes(scheme, M, N, d, &plan, b);
+    size_t need = ws_total(b);
+    auto unsplit = [&] {  // the same result without partial tiles
+        plan = call_plan(scheme, d, false);
+        ws_bytes(scheme, M, N, d, &plan, b);
+        need = ws_total(b);
+    };
     char* ws = static_cast<char*>(workspace);
     if (ws) {
+        if (workspace_bytes < need) unsplit();
         if (workspace_bytes < need)
             return fail(OZA_INVALID_ARGUMENT, "OzaBLAS: workspace smaller than oza_gemm_workspace_bytes.");
     } else {  // the context's own workspace, grown on demand and kept for later calls
@@ -522,12 +558,21 @@ int oza_gemm(oza_ctx ctx, int scheme, int S, int layout, int transA, int transB,
                 ctx->ws = nullptr;
                 ctx->ws_bytes = 0;
             }
-            if (hipMalloc(&ctx->ws, need) != hipSuccess) {
+            size_t most[5];  // what oza_gemm_workspace_bytes says: smaller shapes then fit too
+            ws_bytes(scheme, M, N, d, nullptr, most);
+            size_t size = ws_total(most);
+            if (hipMalloc(&ctx->ws, size) != hipSuccess) {
                 (void)hipGetLastError();
-                ctx->ws = nullptr;
-                return fail(OZA_ALLOC_FAILED, "HIP: workspace allocation of " + std::to_string(need) + " bytes failed.");
+                unsplit();
+                size = need;
+                if (hipMalloc(&ctx->ws, size) != hipSuccess) {
+                    (void)hipGetLastError();
+                    ctx->ws = nullptr;
+                    return fail(OZA_ALLOC_FAILED,
+                                "HIP: workspace allocation of " + std::to_string(need) + " bytes failed.");
+                }
             }
-            ctx->ws_bytes = need;
+            ctx->ws_bytes = size;
         }
         ws = static_cast<char*>(ctx->ws);
     }
@@ -538,7 +583,7 @@ int oza_gemm(oza_ctx ctx, int scheme, int S, int layout, int transA, int transB,
     }
     const Operand a{A, (int64_t)lda, transA == OZA_OP_N};   // op(A) rows: A rows, or A columns
     const Operand bb{B, (int64_t)ldb, transB == OZA_OP_T};  // op(B) columns: B columns, or B^T rows
-    return enqueue_pipeline(scheme, ctx, M, N, K, S, a, bb, OutC{C, (int64_t)ldc, alpha, beta},
+    return enqueue_pipeline(scheme, ctx, d, plan, a, bb, OutC{C, (int64_t)ldc, alpha, beta},
                             reinterpret_cast<int32_t*>(parts[0]), reinterpret_cast<int32_t*>(parts[1]),
                             reinterpret_cast<int8_t*>(parts[2]), reinterpret_cast<int8_t*>(parts[3]), parts[4],
                             nullptr);
@@ -553,9 +598,10 @@ int oza_gemm_noalloc(oza_ctx ctx, int scheme, int S, int layout, int transA, int
     // oza_gemm needs no workspace.  (oza_gemm repeats the argument checks.)
     if (K != 0 && alpha != 0.0 && M != 0 && N != 0 && check_problem(scheme, M, N, K, S) == OZA_SUCCESS) {
         size_t b[5];
-        ws_bytes(scheme, M, N, K, S, b);
-        size_t need = 0;
-        for (size_t x : b) need += (x + 255) / 256 * 256;
+        const Dims d = make_dims(M, N, K, S);
+        const CallPlan whole = call_plan(scheme, d, false);
+        ws_bytes(scheme, M, N, d, &whole, b);
+        const size_t need = ws_total(b);
         if (need > OZA_NOALLOC_SCRATCH_BYTES)
             return fail(OZA_INVALID_ARGUMENT, "OzaBLAS: the problem needs " + std::to_string(need) +
                                                   " bytes of workspace; oza_gemm_noalloc holds " +
@@ -653,7 +699,7 @@ int oza_stage4_s2_products(oza_ctx ctx, size_t M, size_t N, size_t K, int S, con
 int oza_stage4_s2_digits(oza_ctx ctx, size_t M, size_t N, size_t K, int S, const void* Ctc, const int32_t* shA,
                          const int32_t* shB, double* C) {
     OZA_STAGE_PROLOGUE(2)
-    OZA_HIP(launch_recon_s2_digits(d, static_cast<const uint8_t*>(Ctc), shA, shB, crt_for(ctx, S),
+    OZA_HIP(launch_recon_s2_digits(d, static_cast<uint8_t*>(const_cast<void*>(Ctc)), shA, shB, crt_for(ctx, S),
                                    OutC{C, (int64_t)N, 1.0, 0.0}, st),
             "step 4 launch");
     return OZA_SUCCESS;

@@ -5,6 +5,8 @@
 // stages through an LDS ring filled by direct global->LDS loads.
 #pragma once
 
+#include <utility>
+
 #include "oza_device.hpp"
 #include "oza_internal.hpp"
 #include "k_igemm_cfg.hpp"
@@ -18,8 +20,8 @@ namespace core {
 // fragment-tiled (frag_off16): every 1 KiB block is one 32x32 MFMA operand fragment in lane order,
 // so a wave-wide direct load copies one block contiguously from HBM/L2 into LDS and a wave reads a
 // fragment back with one contiguous, bank-conflict-free ds_read_b128.  In LDS a stage holds A blocks
-// [kb][BM/32] followed by B blocks [kb][BN/32]; wave w always loads blocks w, w + NWAVES, ... of a
-// stage, so two waves never write the same LDS bytes.
+// [BM/32][kb] followed by B blocks [BN/32][kb]; wave w always loads the same few blocks of a stage,
+// consecutive in memory and in LDS, so two waves never write the same LDS bytes.
 // ------------------------------------------------------------------------------------------
 #define OZA_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 
@@ -43,34 +45,47 @@ __device__ __forceinline__ void block_sync_lds() {
     asm volatile("" ::: "memory");
 }
 
+// Loads of one stage by one wave: LPA consecutive A blocks from `a` on and LPB B blocks from `b` on (the
+// wave's own, see wave_src).  The pointers are wave-uniform and lane * 16 is the only lane part, and the
+// instruction's offset moves both the memory and the LDS address, so a stage costs one scalar base and
+// one M0 per operand.  (With a 64-bit address per load and blocks interleaved over the waves, about 45
+// scalar and 10 vector instructions stood between a stage's barrier and its last k-step's MFMAs: Scheme I
+// 8192^3, S = 8 16.76 against 15.96 ms, 4096^3, S = 6 1.393 against 1.347 ms; Scheme II 8192^3, S = 17
+// 8.55 against 8.37 ms.)
 template <class C>
 __device__ __forceinline__ void issue_stage(int8_t* stage, const int8_t* __restrict__ a, const int8_t* __restrict__ b,
-                                            int64_t ldk, int k0, int wave, int lane) {
-    const int64_t kblocks = ldk >> 5;  // fragment blocks per block-row of a plane
-#pragma unroll
-    for (int i = 0; i < C::ABLK / C::NWAVES; ++i) {
-        const int blk = i * C::NWAVES + wave;  // = kb * (BM/32) + rb
-        const int kb = blk / (C::BM / 32), rb = blk % (C::BM / 32);
-        __builtin_amdgcn_global_load_lds(a + ((rb * kblocks + (k0 >> 5) + kb) << 10) + lane * 16,
-                                         OZA_LDS_PTR(stage + blk * 1024), 16, 0, 0);
-    }
-    int8_t* sb = stage + C::BM * C::BK;
-#pragma unroll
-    for (int i = 0; i < C::BBLK / C::NWAVES; ++i) {
-        const int blk = i * C::NWAVES + wave;
-        const int kb = blk / (C::BN / 32), rb = blk % (C::BN / 32);
-        __builtin_amdgcn_global_load_lds(b + ((rb * kblocks + (k0 >> 5) + kb) << 10) + lane * 16,
-                                         OZA_LDS_PTR(sb + blk * 1024), 16, 0, 0);
-    }
+                                            int wave, unsigned lane) {
+    const unsigned off = lane * 16;
+    int8_t* sa = stage + wave * (C::LPA * 1024);
+    int8_t* sb = stage + C::BM * C::BK + wave * (C::LPB * 1024);
+    auto load = [&]<int... I>(const int8_t* p, int8_t* l, std::integer_sequence<int, I...>) {
+        (__builtin_amdgcn_global_load_lds(p + off, OZA_LDS_PTR(l), 16, I * 1024, 0), ...);
+    };
+    load(a, sa, std::make_integer_sequence<int, C::LPA>{});
+    load(b, sb, std::make_integer_sequence<int, C::LPB>{});
 }
 
-// One K stage of a work item: its operand tiles (fragment-tiled planes of ldk K-bytes per row)
-// and the stage's first K byte.
+// Sources of one K stage for one wave.
 struct StageSrc {
     const int8_t* a;
     const int8_t* b;
-    int64_t ldk;
-    int k0;
+};
+
+// The wave's blocks of stage 0 of the operand tiles at a and b (fragment-tiled planes, ldk K-bytes per
+// row); stage i lies i * C::STEP bytes further.
+template <class C>
+__device__ __forceinline__ StageSrc wave_src(const int8_t* a, const int8_t* b, int64_t ldk, int wave) {
+    const int64_t kblocks = ldk >> 5;  // fragment blocks per block-row of a plane
+    constexpr int KB = C::KB;
+    return StageSrc{a + (((wave * C::LPA / KB) * kblocks + wave * C::LPA % KB) << 10),
+                    b + (((wave * C::LPB / KB) * kblocks + wave * C::LPB % KB) << 10)};
+}
+
+// What a wave loads after its current item's stages: the next item's stages 0 and 1 (any valid source
+// where there is no such stage: nothing reads it, and the next chain start's vmcnt(0) completes it
+// before its slot is loaded again).
+struct NextSrc {
+    StageSrc s0, s1;
 };
 
 template <class C>
@@ -84,10 +99,10 @@ __device__ __forceinline__ void load_frags(Frags<C>& f, const int8_t* stage, int
     const int8_t* sb = stage + C::BM * C::BK;
 #pragma unroll
     for (int fm = 0; fm < C::FM; ++fm)
-        f.a[fm] = *reinterpret_cast<const v4i*>(stage + ((kk * (C::BM / 32) + wm * C::FM + fm) << 10) + lane * 16);
+        f.a[fm] = *reinterpret_cast<const v4i*>(stage + (((wm * C::FM + fm) * C::KB + kk) << 10) + lane * 16);
 #pragma unroll
     for (int fn = 0; fn < C::FN; ++fn)
-        f.b[fn] = *reinterpret_cast<const v4i*>(sb + ((kk * (C::BN / 32) + wn * C::FN + fn) << 10) + lane * 16);
+        f.b[fn] = *reinterpret_cast<const v4i*>(sb + (((wn * C::FN + fn) * C::KB + kk) << 10) + lane * 16);
 }
 
 template <class C>
@@ -164,41 +179,28 @@ __device__ __forceinline__ void interleave_hint_last() {
 //   On entry this item's stage 0 has been issued, and its stage 1 too when nit >= 2 (chain_start
 //   for a chain's first item; the previous item's last two iterations otherwise).  With nit == 1 no
 //   earlier iteration can take chain stage 1, so it is issued after the first barrier.
-//   entry() runs after the first barrier: there the caller learns the next item, which tail() and the
-//   ring need from then on.
-//   own(i) gives this item's stage i, tail(j) the next item's stage j -- or, when there is no such
-//   stage, any valid source (a refetch: nothing reads it, and the next chain start's vmcnt(0)
-//   completes it before its slot is loaded again).  Both are evaluated and one is selected, so no
-//   branch separates the loads from the MFMAs they are interleaved with.
+//   `cur` is this item's stage 2 (if it has one) and step(cur) moves it on by a stage.  entry() runs after
+//   the first barrier and returns the next item's sources.  The source is selected, so no branch
+//   separates the loads from the MFMAs they are interleaved with.
 // ------------------------------------------------------------------------------------------
-template <class C, class Own>
-__device__ __forceinline__ void chain_start(int8_t* smem, int base, int nit, Own own) {
+template <class C>
+__device__ __forceinline__ void chain_start(int8_t* smem, int base, int nit, const StageSrc& s0, const StageSrc& s1) {
     static_assert(C::STAGES == 2, "the chain keeps two slots");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const StageSrc s0 = own(0);
-    issue_stage<C>(smem + (base & 1) * C::STAGE_BYTES, s0.a, s0.b, s0.ldk, s0.k0, wave, lane);
-    if (nit >= 2) {
-        const StageSrc s1 = own(1);
-        issue_stage<C>(smem + ((base + 1) & 1) * C::STAGE_BYTES, s1.a, s1.b, s1.ldk, s1.k0, wave, lane);
-    }
+    issue_stage<C>(smem + (base & 1) * C::STAGE_BYTES, s0.a, s0.b, wave, lane);
+    if (nit >= 2) issue_stage<C>(smem + ((base + 1) & 1) * C::STAGE_BYTES, s1.a, s1.b, wave, lane);
 }
 
-template <class C, class Own, class Tail, class Entry>
-__device__ __forceinline__ void mainloop_chain(v16i (&acc)[C::FM][C::FN], int8_t* smem, int base, int nit, Own own,
-                                               Tail tail, Entry entry) {
+template <class C, class Cur, class Step, class Entry>
+__device__ __forceinline__ void mainloop_chain(v16i (&acc)[C::FM][C::FN], int8_t* smem, int base, int nit, Cur cur,
+                                               Step step, Entry entry) {
     static_assert(C::STAGES == 2, "the chain keeps two slots");
     constexpr int KSTEPS = C::BK / 32;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / C::NWN, wn = wave % C::NWN;
     auto slot = [&](int i) { return smem + ((base + i) & 1) * C::STAGE_BYTES; };
-    auto issue = [&](int i) {  // chain stage i: this item's stage i, or the next item's stage i - nit
-        const StageSrc o = own(i), t = tail(i - nit);
-        const bool mine = i < nit;  // selects, not a branch: the loads stay among the MFMAs
-        issue_stage<C>(slot(i), mine ? o.a : t.a, mine ? o.b : t.b, mine ? o.ldk : t.ldk, mine ? o.k0 : t.k0, wave,
-                       lane);
-    };
     auto lds_barrier = [] {
         wait_lgkmcnt0();  // this wave's LDS reads are done
         block_sync_lds();
@@ -210,13 +212,17 @@ __device__ __forceinline__ void mainloop_chain(v16i (&acc)[C::FM][C::FN], int8_t
     else wait_vmcnt<0>();
     lds_barrier();
     load_frags<C>(f[0], slot(0), 0, wm, wn, lane);
-    entry();
-    if (nit == 1) issue(1);
+    const NextSrc nx = entry();
+    if (nit == 1) issue_stage<C>(slot(1), nx.s0.a, nx.s0.b, wave, lane);
     for (int it = 0; it + 1 < nit; ++it) {
-        const int8_t* cur = slot(it);
+        const int8_t* now = slot(it);
+        const bool own = it + 2 < nit;  // chain stage it + 2: this item's, or the next item's stage 0
+        const int8_t* pa = own ? cur.a : nx.s0.a;
+        const int8_t* pb = own ? cur.b : nx.s0.b;
+        step(cur);
 #pragma unroll
         for (int kk = 0; kk + 1 < KSTEPS; ++kk) {
-            load_frags<C>(f[(kk + 1) & 1], cur, kk + 1, wm, wn, lane);
+            load_frags<C>(f[(kk + 1) & 1], now, kk + 1, wm, wn, lane);
             mma_frags<C>(acc, f[kk & 1]);
             interleave_hint<C>();
         }
@@ -224,7 +230,7 @@ __device__ __forceinline__ void mainloop_chain(v16i (&acc)[C::FM][C::FN], int8_t
         lds_barrier();
         load_frags<C>(f[KSTEPS & 1], slot(it + 1), 0, wm, wn, lane);
         __builtin_amdgcn_s_setprio(1);
-        issue(it + 2);
+        issue_stage<C>(slot(it + 2), pa, pb, wave, lane);
         mma_frags<C>(acc, f[(KSTEPS - 1) & 1]);
         interleave_hint_last<C>();
         __builtin_amdgcn_s_setprio(0);
@@ -236,16 +242,16 @@ __device__ __forceinline__ void mainloop_chain(v16i (&acc)[C::FM][C::FN], int8_t
         }
     }
     {  // last iteration: its slot is freed at the barrier for chain stage nit + 1
-        const int8_t* cur = slot(nit - 1);
+        const int8_t* now = slot(nit - 1);
 #pragma unroll
         for (int kk = 0; kk + 1 < KSTEPS; ++kk) {
-            load_frags<C>(f[(kk + 1) & 1], cur, kk + 1, wm, wn, lane);
+            load_frags<C>(f[(kk + 1) & 1], now, kk + 1, wm, wn, lane);
             mma_frags<C>(acc, f[kk & 1]);
             interleave_hint<C>();
         }
         lds_barrier();
         __builtin_amdgcn_s_setprio(1);
-        issue(nit + 1);
+        issue_stage<C>(slot(nit + 1), nx.s1.a, nx.s1.b, wave, lane);
         mma_frags<C>(acc, f[(KSTEPS - 1) & 1]);
         __builtin_amdgcn_s_setprio(0);
     }

@@ -122,13 +122,12 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
     __shared__ __attribute__((aligned(1024))) int8_t smem[C::LDS_BYTES];
     int64_t w = blockIdx.x;
     if (w >= g.n) return;  // whole workgroup leaves together
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / C::NWN, wn = wave % C::NWN;
     struct Item {
-        const int8_t* a;
-        const int8_t* b;
+        StageSrc src;    // this wave's blocks of stage 0
         uint8_t* plane;  // digit plane of modulus s (a partial plane for splits j > 0)
-        int64_t Kp, Np, M, N;
+        int64_t Np, M, N;
         int tm, tn, k0, KT;  // K steps [k0, k0 + KT) of BK bytes
         uint32_t m, minv, bias;
     };
@@ -144,14 +143,14 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
         const uint32_t rest = local - j * per_split;
         const int s = (int)(rest / tiles);
         grouped_tile<C>((int64_t)(rest - (uint32_t)s * tiles), P.tiles_m, P.tiles_n, t.tm, t.tn);
-        t.Kp = P.Kp;
         t.Np = P.Np;
         t.M = P.M;
         t.N = P.N;
         t.k0 = (int)j * P.kbs * kSteps128;
         t.KT = min(P.kbs * kSteps128, (int)(P.Kp / C::BK) - t.k0);
-        t.a = P.Asl + (int64_t)s * P.Mp * P.Kp + (int64_t)t.tm * C::BM * P.Kp;
-        t.b = P.Bsl + (int64_t)s * P.Np * P.Kp + (int64_t)t.tn * C::BN * P.Kp;
+        t.src = wave_src<C>(P.Asl + (int64_t)s * P.Mp * P.Kp + (int64_t)t.tm * C::BM * P.Kp + (int64_t)t.k0 * C::STEP,
+                            P.Bsl + (int64_t)s * P.Np * P.Kp + (int64_t)t.tn * C::BN * P.Kp + (int64_t)t.k0 * C::STEP, P.Kp,
+                            wave);
         const int64_t plane = P.Mp * P.Np;
         t.plane = (j == 0 ? P.dg : P.dgp + (int64_t)(j - 1) * P.S * plane) + (int64_t)s * plane;
         const auto& cs = as_constant(g.crt)->set[P.S - 1];
@@ -160,27 +159,26 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
         t.bias = cs.bias[s];
         return t;
     };
-    Item cur = decode(w);
-    auto own_of = [&](const Item& t) {
-        return [&t](int i) { return StageSrc{t.a, t.b, t.Kp, (t.k0 + i) * C::BK}; };
+    auto stage = [](const Item& t, int i) {  // stage i of an item; its last one past that
+        const int64_t o = (int64_t)min(i, t.KT - 1) * C::STEP;
+        return StageSrc{t.src.a + o, t.src.b + o};
     };
-    chain_start<C>(smem, 0, cur.KT, own_of(cur));  // later items' stages arrive through the chain
+    auto step = [](StageSrc& c) {
+        c.a += C::STEP;
+        c.b += C::STEP;
+    };
+    Item cur = decode(w);
+    chain_start<C>(smem, 0, cur.KT, stage(cur, 0), stage(cur, 1));  // later items' stages arrive through the chain
     int base = 0;  // ring slot of the current item's stage 0
     for (;;) {
         const int64_t w2 = w + gridDim.x;
         const bool more = w2 < g.n;
         Item nxt = cur;
         if (more) nxt = decode(w2);
-        // Source of the next item's stage j; past its stages (or with no next item) a refetch of
-        // the current item's last stage.
-        auto tail = [&](int j) {
-            const bool real = more && j < nxt.KT;
-            return StageSrc{real ? nxt.a : cur.a, real ? nxt.b : cur.b, real ? nxt.Kp : cur.Kp,
-                            (real ? nxt.k0 + j : cur.k0 + cur.KT - 1) * C::BK};
-        };
         v16i acc[C::FM][C::FN];
         fill_acc<C>(acc, (int)cur.bias);
-        mainloop_chain<C>(acc, smem, base, cur.KT, own_of(cur), tail, [] {});
+        mainloop_chain<C>(acc, smem, base, cur.KT, stage(cur, 2), step,
+                          [&] { return NextSrc{stage(nxt, 0), stage(nxt, 1)}; });
         store_digits<C, true, true>(acc, cur.plane, cur.Np, (int64_t)cur.tm * C::BM + wm * C::WTM,
                                     (int64_t)cur.tn * C::BN + wn * C::WTN, cur.M, cur.N, cur.m, cur.minv, lane);
         if (!more) break;

@@ -49,36 +49,41 @@ struct S2Args {
     int tm0;               // first tile row: the launch covers tile rows [tm0, tm0 + tiles_m)
     void* out;             // digits or int32 planes
     const CrtSet* crt;     // device copy (m, minv, bias used)
-    int split, kts;        // K parts and K steps per part (SPLIT only)
+    // SPLIT only: items [0, whole) run whole, the `tail` others in `parts` parts of kts K steps
+    int64_t whole, tail;
+    int parts, kts;
+    uint8_t* part;         // partial tiles of parts 1..
 };
 
 // Work items (modulus, tile) in logical order l = 0..total-1: modulus-major; inside a modulus,
-// tiles in groups of GM tile rows.  SPLIT: items (part j, modulus, tile), part-major, part j over
-// K steps [j kts, min((j + 1) kts, KT)), its digits into plane set j of the output.
+// tiles in groups of GM tile rows.  SPLIT: the whole items first, then the others' parts, part-major, part
+// j over K steps [j kts, min((j + 1) kts, KT)).
 template <class C, bool DIGITS, bool SPLIT = false>
 __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
     __shared__ __attribute__((aligned(1024))) int8_t smem[C::LDS_BYTES];
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n, total = tiles * p.S;
-    const int64_t items = SPLIT ? total * p.split : total;
+    const int64_t items = SPLIT ? p.whole + p.tail * p.parts : total;
     int64_t w = blockIdx.x;
     if (w >= items) return;  // whole workgroup leaves together
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / C::NWN, wn = wave % C::NWN;
     struct Item {
         int s, tm, tn, j, k0, KT;
-        const int8_t* a;
-        const int8_t* b;
+        int64_t l;
+        StageSrc src;  // this wave's blocks of stage 0
         uint32_t m, minv, bias;
     };
     auto decode = [&](int64_t wi) {
         Item t;
-        int64_t l = xcd_remap(wi, items);
+        int64_t l = SPLIT && wi >= p.whole ? p.whole + xcd_remap(wi - p.whole, items - p.whole)
+                                           : xcd_remap(wi, SPLIT ? p.whole : items);
         t.j = 0;
         t.k0 = 0;
         t.KT = p.KT;
-        if (SPLIT) {
-            t.j = (int)(l / total);
-            l -= (int64_t)t.j * total;
+        t.l = l;
+        if (SPLIT && l >= p.whole) {
+            t.j = (int)((l - p.whole) / p.tail);
+            t.l = l -= (int64_t)t.j * p.tail;
             t.k0 = t.j * p.kts;
             t.KT = min(p.kts, p.KT - t.k0);
         }
@@ -86,19 +91,25 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         grouped_tile<C>(l - (int64_t)t.s * tiles, p.tiles_m, p.tiles_n, t.tm, t.tn);
         t.tm += p.tm0;
         // tile (tm, tn) starts at block-row tm*BM/32 of the fragment-tiled planes (BM*Kp bytes)
-        t.a = p.A + (int64_t)t.s * p.Mp * p.Kp + (int64_t)t.tm * C::BM * p.Kp;
-        t.b = p.B + (int64_t)t.s * p.Np * p.Kp + (int64_t)t.tn * C::BN * p.Kp;
+        t.src = wave_src<C>(p.A + (int64_t)t.s * p.Mp * p.Kp + (int64_t)t.tm * C::BM * p.Kp + (int64_t)t.k0 * C::STEP,
+                            p.B + (int64_t)t.s * p.Np * p.Kp + (int64_t)t.tn * C::BN * p.Kp + (int64_t)t.k0 * C::STEP, p.Kp,
+                            wave);
         // scalar loads: counted by lgkmcnt, so the epilogue does not wait for the direct loads
         t.m = as_constant(p.crt)->m[t.s];
         t.minv = as_constant(p.crt)->minv[t.s];
         t.bias = as_constant(p.crt)->bias[t.s];
         return t;
     };
-    Item cur = decode(w);
-    auto own_of = [&](const Item& t) {
-        return [&t, &p](int i) { return StageSrc{t.a, t.b, p.Kp, (t.k0 + i) * C::BK}; };
+    auto stage = [](const Item& t, int i) {  // stage i of an item; its last one past that
+        const int64_t o = (int64_t)min(i, t.KT - 1) * C::STEP;
+        return StageSrc{t.src.a + o, t.src.b + o};
     };
-    chain_start<C>(smem, 0, cur.KT, own_of(cur));
+    auto step = [](StageSrc& c) {
+        c.a += C::STEP;
+        c.b += C::STEP;
+    };
+    Item cur = decode(w);
+    chain_start<C>(smem, 0, cur.KT, stage(cur, 0), stage(cur, 1));
     int base = 0;  // ring slot of the current item's stage 0
     for (;;) {
         w += gridDim.x;
@@ -106,23 +117,20 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         Item nxt = cur;
         auto entry = [&] {
             if (more) nxt = decode(w);
-        };
-        // The next item's stage j; past its stages, or with no next item, a refetch of this item's
-        // last stage.
-        auto tail = [&](int j) {
-            const bool real = more && j < nxt.KT;
-            return StageSrc{real ? nxt.a : cur.a, real ? nxt.b : cur.b, p.Kp,
-                            (real ? nxt.k0 + j : cur.k0 + cur.KT - 1) * C::BK};
+            return NextSrc{stage(nxt, 0), stage(nxt, 1)};
         };
         v16i acc[C::FM][C::FN];
         if (DIGITS) fill_acc<C>(acc, (int)cur.bias);
         else zero_acc<C>(acc);
-        mainloop_chain<C>(acc, smem, base, cur.KT, own_of(cur), tail, entry);
+        mainloop_chain<C>(acc, smem, base, cur.KT, stage(cur, 2), step, entry);
         const int s = cur.s, tm = cur.tm, tn = cur.tn;
         if (DIGITS) {
-            uint8_t* plane = reinterpret_cast<uint8_t*>(p.out) + ((int64_t)cur.j * p.S + s) * p.Mp * p.Np;
-            store_digits<C, false>(acc, plane, p.Np, (int64_t)tm * C::BM + wm * C::WTM, (int64_t)tn * C::BN + wn * C::WTN,
-                                   p.M, p.N, cur.m, cur.minv, lane);
+            const bool part = SPLIT && cur.j > 0;  // a partial tile: the blocks of one tile, row-major
+            uint8_t* plane = part ? p.part + ((cur.j - 1) * p.tail + cur.l - p.whole) * kTileBytes
+                                  : reinterpret_cast<uint8_t*>(p.out) + (int64_t)s * p.Mp * p.Np;
+            const int64_t row0 = (part ? 0 : (int64_t)tm * C::BM) + wm * C::WTM;
+            const int64_t col0 = (part ? 0 : (int64_t)tn * C::BN) + wn * C::WTN;
+            store_digits<C, false>(acc, plane, part ? C::BN : p.Np, row0, col0, p.M, p.N, cur.m, cur.minv, lane);
         } else {
             int32_t* o = reinterpret_cast<int32_t*>(p.out) + (int64_t)s * p.M * p.N;
 #pragma unroll
@@ -142,16 +150,6 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         cur = nxt;
     }
     wait_vmcnt<0>();  // no direct load in flight into LDS when the workgroup leaves
-}
-
-// Split-K digit reduction of a single call: 4 KiB of the S digit planes per workgroup (Mp * Np is a
-// multiple of 65536, so a workgroup's bytes lie in one plane), partial sets after set 0.
-__global__ void __launch_bounds__(256) k_digits_reduce(uint8_t* dg, int64_t plane, int S, int split,
-                                                       const CrtSet* crt) {
-    const int64_t off = (int64_t)blockIdx.x * 4096 + threadIdx.x * 16;
-    const int s = (int)(off / plane);
-    const int64_t stride = (int64_t)S * plane;
-    reduce_digits16(dg, dg + stride, stride, split - 1, crt->m[s], off);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -177,7 +175,7 @@ __device__ __forceinline__ Claims first_claims(unsigned* queue, int xcd, unsigne
         c.w1 = s_pos[1];
     } else {
         c.w = blockIdx.x;
-        c.w1 = c.w + gridDim.x;
+        c.w1 = 2 * (int64_t)gridDim.x - 1 - c.w;
     }
     return c;
 }
@@ -197,25 +195,54 @@ struct S1Args {
     const int8_t* B;
     int64_t M, N, Mp, Np, Kp;
     int S, KT, tiles_m, tiles_n, beta;
-    uint64_t kt_div;         // ceil(2^32 / KT): i / KT = (i * kt_div) >> 32 for the stage indices here
     int tm0;                 // blocked form: the launch covers tile rows [tm0, tm0 + tiles_m)
-    int32_t* T;              // group products: int32 [S][M][N], or blocked [S][Mp][Np]
+    int32_t* T;              // group products: int32 [S][M][N], or blocked [planes][Mp][Np]
     unsigned* queue;         // 8 work counters, zero at launch (dynamic order), or null (static order)
 };
 
-// Stage i of the item of group g (pairs s = 1..g-1, t = g - s, in the reference's ascending-s
-// order, KT stages each) of the tile whose operand tiles start at abase / bbase.
-// i / KT by a multiply with ceil(2^32 / KT) (kt_div): exact while i * KT < 2^32 (the error
-// i * (ceil(2^32/KT) KT - 2^32) / (KT 2^32) stays below 1/KT); here i < 21 KT and KT <= 2148
-// (K <= 137438 in 64-byte steps), so i * KT < 10^8.  A division by a runtime KT would put a long
-// scalar sequence at the head of every iteration.
-__device__ __forceinline__ StageSrc s1_stage(const int8_t* abase, const int8_t* bbase, int64_t planeA,
-                                             int64_t planeB, int g, int KT, uint64_t kt_div, int64_t Kp, int BK, int i) {
-    const int pr = (int)(((uint64_t)(uint32_t)i * kt_div) >> 32), kt = i - pr * KT;
-    return StageSrc{abase + (int64_t)pr * planeA,             // s = pr + 1
-                    bbase + (int64_t)(g - pr - 2) * planeB,   // t = g - s
-                    Kp, kt * BK};
-}
+// A wave's place in the stages of group g of a tile (pairs s = 1..g-1, t = g - s, in the reference's
+// ascending-s order, KT stages each), moved on stage by stage: the next K step, or the next pair's first.
+struct S1Cursor {
+    const int8_t* a;
+    const int8_t* b;
+    int kt;
+};
+template <class C>
+struct S1Walk {
+    int64_t wrapA, wrapB;  // from a pair's last stage to the next pair's first
+    int KT;
+    __device__ __forceinline__ S1Walk(const S1Args& p)
+        : wrapA(p.Mp * p.Kp - (int64_t)(p.KT - 1) * C::STEP), wrapB(-p.Np * p.Kp - (int64_t)(p.KT - 1) * C::STEP), KT(p.KT) {}
+    // Stage i of group g; abase, bbase: the wave's blocks of the tile in slice 1's planes.
+    __device__ __forceinline__ S1Cursor at(const StageSrc& base, const S1Args& p, int g, int i) const {
+        const int pr = i / KT, kt = i - pr * KT;  // s = pr + 1, t = g - s
+        return S1Cursor{base.a + pr * p.Mp * p.Kp + (int64_t)kt * C::STEP,
+                        base.b + (g - pr - 2) * p.Np * p.Kp + (int64_t)kt * C::STEP, kt};
+    }
+    __device__ __forceinline__ void operator()(S1Cursor& c) const {
+        const bool wrap = c.kt + 1 == KT;
+        c.a += wrap ? wrapA : (int64_t)C::STEP;
+        c.b += wrap ? wrapB : (int64_t)C::STEP;
+        c.kt = wrap ? 0 : c.kt + 1;
+    }
+    __device__ __forceinline__ NextSrc next(const StageSrc& base, const S1Args& p, int g, int i0, int nit) const {
+        const S1Cursor s0 = at(base, p, g, i0);
+        S1Cursor s1 = s0;
+        if (nit >= 2) (*this)(s1);
+        return NextSrc{{s0.a, s0.b}, {s1.a, s1.b}};
+    }
+};
+
+// The items of one tile in the blocked form, longest first: stages [i0, i0 + nit) of group g into plane
+// `plane`.
+struct S1Entry {
+    uint8_t g, plane;
+    uint16_t i0, nit;
+};
+struct S1List {
+    int n;
+    S1Entry e[kMaxS1Planes];
+};
 
 // Scheme I group products in the reference's planar layout (the stage entry point): one
 // workgroup per tile; its items are the groups g = s + t = 2..S+1 in ascending order
@@ -227,26 +254,22 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1(S1Args p) {
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
     int tm, tn;
     grouped_tile<C>(xcd_remap(blockIdx.x, tiles), p.tiles_m, p.tiles_n, tm, tn);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / C::NWN, wn = wave % C::NWN;
-    const int64_t planeA = p.Mp * p.Kp, planeB = p.Np * p.Kp;
-    const int8_t* abase = p.A + (int64_t)tm * C::BM * p.Kp;
-    const int8_t* bbase = p.B + (int64_t)tn * C::BN * p.Kp;
-    auto own_of = [&](int g) {
-        return [=](int i) { return s1_stage(abase, bbase, planeA, planeB, g, p.KT, p.kt_div, p.Kp, C::BK, i); };
-    };
-    chain_start<C>(smem, 0, p.KT, own_of(2));
+    const StageSrc src =
+        wave_src<C>(p.A + (int64_t)tm * C::BM * p.Kp, p.B + (int64_t)tn * C::BN * p.Kp, p.Kp, wave);
+    const S1Walk<C> walk(p);
+    const NextSrc first = walk.next(src, p, 2, 0, p.KT);
+    chain_start<C>(smem, 0, p.KT, first.s0, first.s1);
     int base = 0;
     for (int g = 2; g <= p.S + 1; ++g) {
         const int nit = (g - 1) * p.KT;
-        const bool more = g < p.S + 1;
-        auto tail = [&](int j) {  // the next group's stage j, or a refetch of this group's last stage
-            return more ? s1_stage(abase, bbase, planeA, planeB, g + 1, p.KT, p.kt_div, p.Kp, C::BK, j)
-                        : s1_stage(abase, bbase, planeA, planeB, g, p.KT, p.kt_div, p.Kp, C::BK, nit - 1);
+        auto entry = [&] {  // the next group, or this one again (a refetch)
+            return g <= p.S ? walk.next(src, p, g + 1, 0, nit + p.KT) : walk.next(src, p, g, 0, nit);
         };
         v16i acc[C::FM][C::FN];
         zero_acc<C>(acc);
-        mainloop_chain<C>(acc, smem, base, nit, own_of(g), tail, [] {});
+        mainloop_chain<C>(acc, smem, base, nit, walk.at(src, p, g, min(2, nit - 1)), walk, entry);
         int32_t* o = p.T + (int64_t)(g - 2) * p.M * p.N;
 #pragma unroll
         for (int fm = 0; fm < C::FM; ++fm)
@@ -268,68 +291,67 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1(S1Args p) {
 // tile); the pairs s = 1..g-1 (t = g - s) of the group accumulate in INT32 through one pass of
 // the chained mainloop, and T_g is stored as a blocked INT32 plane (store_i32_blocked).  The
 // FP64 sum over groups is step 4 (k_recon_s1_blocked).
-// Work order: items differ in length (g - 1 pairs), so the XCDs split the tiles, not the items:
-// XCD x (workgroups b with b % 8 == x) owns the tiles [x*T/8, (x+1)*T/8) of the grouped tile order
-// in every group, and walks its items largest group first, then tile -- every XCD gets the same
-// mix of work and its CUs share A and B panels in L2.  The workgroups of XCD x take the positions
-// of its sequence in the order they ask for them (counter queue[x]).  Without counters, or with a
-// grid that is not a multiple of 8 (fewer items than CUs), workgroup b walks the whole item list,
-// largest group first, at b, b + gridDim.x, ...
+// A group may run in parts (S1List), each over its own stages into its own plane; step 4 adds them.
+// Work order: items differ in length, so the XCDs split the tiles, not the items: XCD x (workgroups b
+// with b % 8 == x) owns the tiles [x*T/8, (x+1)*T/8) of the grouped tile order in every list entry, and
+// walks its items longest entry first, then tile -- every XCD gets the same mix of work and its CUs share
+// A and B panels in L2.  The workgroups of XCD x take the positions of its sequence in the order they ask
+// for them (counter queue[x]).  Without counters (few tiles, whose shares would be uneven, or few items,
+// see the launcher) the workgroups walk one list over all tiles, longest first, back and forth: round r
+// takes position r * G + b of G workgroups, or (r + 1) * G - 1 - b when r is odd, so that a workgroup with
+// a long item gets a short one next.  (Runs of 32 consecutive positions per XCD instead, whose tiles share
+// panels in its L2, were slower: 1500^3, S = 8 199 against 186 us.)
 template <class C>
-__global__ void __launch_bounds__(C::NT) k_igemm_s1g(S1Args p) {
+__global__ void __launch_bounds__(C::NT) k_igemm_s1g(S1Args p, S1List list) {
     __shared__ __attribute__((aligned(1024))) int8_t smem[C::LDS_BYTES];
     __shared__ unsigned s_pos[2];
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
-    const bool dyn = (gridDim.x & 7) == 0 && p.queue != nullptr;
+    const bool dyn = p.queue != nullptr;
     const int xcd = blockIdx.x & 7;
     const int64_t t0 = dyn ? tiles * xcd / 8 : 0, ntile = dyn ? tiles * (xcd + 1) / 8 - t0 : tiles;
-    const int64_t nwork = ntile * p.S;
-    Claims c = first_claims(dyn ? p.queue : nullptr, xcd, s_pos);
+    const int64_t nwork = ntile * list.n;
+    Claims c = first_claims(p.queue, xcd, s_pos);
     if (c.w >= nwork) return;  // whole workgroup leaves together
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / C::NWN, wn = wave % C::NWN;
-    const int64_t planeA = p.Mp * p.Kp, planeB = p.Np * p.Kp;
     struct Item {
-        int g, tm, tn, nit;
-        const int8_t* abase;
-        const int8_t* bbase;
+        int g, tm, tn, i0, nit, plane;
+        StageSrc src;
     };
     auto decode = [&](int64_t k) {
         Item t;
-        const int gi = (int)(k / ntile);
-        t.g = p.S + 1 - gi;  // S + 1 down to 2
-        t.nit = (t.g - 1) * p.KT;
-        grouped_tile<C>(t0 + (k - (int64_t)gi * ntile), p.tiles_m, p.tiles_n, t.tm, t.tn);
+        const int e = (int)(k / ntile);
+        t.g = list.e[e].g;
+        t.plane = list.e[e].plane;
+        t.i0 = list.e[e].i0;
+        t.nit = list.e[e].nit;
+        grouped_tile<C>(t0 + (k - (int64_t)e * ntile), p.tiles_m, p.tiles_n, t.tm, t.tn);
         t.tm += p.tm0;
-        t.abase = p.A + (int64_t)t.tm * C::BM * p.Kp;
-        t.bbase = p.B + (int64_t)t.tn * C::BN * p.Kp;
+        t.src = wave_src<C>(p.A + (int64_t)t.tm * C::BM * p.Kp, p.B + (int64_t)t.tn * C::BN * p.Kp, p.Kp, wave);
         return t;
     };
+    const S1Walk<C> walk(p);
     Item cur = decode(c.w);
-    auto own_of = [&](const Item& t) {
-        return [&t, &p, planeA, planeB](int i) {
-            return s1_stage(t.abase, t.bbase, planeA, planeB, t.g, p.KT, p.kt_div, p.Kp, C::BK, i);
-        };
-    };
-    chain_start<C>(smem, 0, cur.nit, own_of(cur));
+    const NextSrc first = walk.next(cur.src, p, cur.g, cur.i0, cur.nit);
+    chain_start<C>(smem, 0, cur.nit, first.s0, first.s1);
     int base = 0;
     for (;;) {
         const bool more = c.w1 < nwork;
-        const Item nxt = more ? decode(c.w1) : cur;
-        auto tail = [&](int j) {  // the next item's stage j, or a refetch of this item's last stage
-            const bool real = more && j < nxt.nit;
-            return real ? s1_stage(nxt.abase, nxt.bbase, planeA, planeB, nxt.g, p.KT, p.kt_div, p.Kp, C::BK, j)
-                        : s1_stage(cur.abase, cur.bbase, planeA, planeB, cur.g, p.KT, p.kt_div, p.Kp, C::BK, cur.nit - 1);
+        Item nxt = cur;
+        auto entry = [&] {
+            if (more) nxt = decode(c.w1);
+            return walk.next(nxt.src, p, nxt.g, nxt.i0, nxt.nit);
         };
         v16i acc[C::FM][C::FN];
         zero_acc<C>(acc);
-        mainloop_chain<C>(acc, smem, base, cur.nit, own_of(cur), tail, [] {});
-        unsigned ticket;  // the item after next (dynamic order); thread 0's only, as in k_igemm_s2
+        mainloop_chain<C>(acc, smem, base, cur.nit, walk.at(cur.src, p, cur.g, cur.i0 + min(2, cur.nit - 1)), walk, entry);
+        unsigned ticket;  // the item after next (dynamic order); thread 0's only: a value merged from both
+        // paths would be copied, and so waited for behind the next item's loads, as soon as it returns
         if (dyn && more && threadIdx.x == 0) ticket = atomicAdd(&p.queue[xcd], 1u);
-        store_i32_blocked<C>(acc, p.T + (int64_t)(cur.g - 2) * p.Mp * p.Np, p.Np,
+        store_i32_blocked<C>(acc, p.T + (int64_t)cur.plane * p.Mp * p.Np, p.Np,
                              (int64_t)cur.tm * C::BM + wm * C::WTM, (int64_t)cur.tn * C::BN + wn * C::WTN, lane);
         if (!more) break;
-        const int64_t w2 = dyn ? publish_claim(ticket, s_pos) : c.w1 + gridDim.x;
+        const int64_t w2 = dyn ? publish_claim(ticket, s_pos) : c.w + 2 * (int64_t)gridDim.x;
         base = (base + cur.nit) & 1;
         c.w = c.w1;
         c.w1 = w2;
@@ -356,8 +378,9 @@ using CfgS2 = IgemmCfgS2;
 using CfgS1 = IgemmCfgS1;
 
 hipError_t launch_igemm_s2(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, S2Out mode, void* out,
-                           const CrtSet* crt_dev, hipStream_t st, int tm0, int tms, int split) {
-    if (split < 1 || (split > 1 && mode != S2Out::Digits)) return hipErrorInvalidValue;
+                           const CrtSet* crt_dev, hipStream_t st, int tm0, int tms, const S2Plan* plan) {
+    const bool split = plan && plan->parts > 1;
+    if (split && (mode != S2Out::Digits || tm0 != 0 || tms >= 0)) return hipErrorInvalidValue;
     S2Args p;
     p.A = A_sl;
     p.B = B_sl;
@@ -375,13 +398,17 @@ hipError_t launch_igemm_s2(const Dims& d, const int8_t* A_sl, const int8_t* B_sl
     p.tiles_n = (int)((d.N + CfgS2::BN - 1) / CfgS2::BN);
     p.out = out;
     p.crt = crt_dev;
-    p.kts = (p.KT + split - 1) / split;
-    p.split = (p.KT + p.kts - 1) / p.kts;  // non-empty parts only
-    const int64_t total = (int64_t)p.tiles_m * p.tiles_n * d.S * p.split;
+    int64_t total = (int64_t)p.tiles_m * p.tiles_n * d.S;
+    p.whole = split ? plan->whole : total;
+    p.tail = total - p.whole;
+    p.parts = split ? plan->parts : 1;
+    p.kts = split ? plan->kts : p.KT;
+    p.part = static_cast<uint8_t*>(out) + (int64_t)d.S * d.Mp * d.Np;
+    if (split) total = p.whole + p.tail * p.parts;
     if (total == 0) return hipSuccess;
     unsigned grid = 0;
     if (hipError_t e = persistent_grid(total, grid)) return e;
-    if (mode == S2Out::Digits && p.split > 1)
+    if (split)
         k_igemm_s2<CfgS2, true, true><<<grid, CfgS2::NT, 0, st>>>(p);
     else if (mode == S2Out::Digits)
         k_igemm_s2<CfgS2, true><<<grid, CfgS2::NT, 0, st>>>(p);
@@ -389,19 +416,6 @@ hipError_t launch_igemm_s2(const Dims& d, const int8_t* A_sl, const int8_t* B_sl
         k_igemm_s2<CfgS2, false><<<grid, CfgS2::NT, 0, st>>>(p);
     return hipGetLastError();
 }
-
-hipError_t launch_digits_reduce(const Dims& d, uint8_t* digits, int split, const CrtSet* crt_dev, hipStream_t st) {
-    const int KT = (int)(d.Kp / CfgS2::BK);
-    const int kts = (KT + split - 1) / split;
-    split = (KT + kts - 1) / kts;  // the parts launch_igemm_s2 ran
-    if (split < 2 || d.M == 0 || d.N == 0) return hipSuccess;
-    const int64_t plane = d.Mp * d.Np;
-    k_digits_reduce<<<(unsigned)(d.S * plane / 4096), 256, 0, st>>>(digits, plane, d.S, split, crt_dev);
-    return hipGetLastError();
-}
-
-// ceil(2^32 / KT), the multiplier of s1_stage's division (KT >= 1).
-static uint64_t kt_divisor(int KT) { return ((1ull << 32) + (uint64_t)KT - 1) / (uint64_t)KT; }
 
 static S1Args make_s1(const Dims& d, int beta, const int8_t* A_sl, const int8_t* B_sl) {
     S1Args p;
@@ -414,7 +428,6 @@ static S1Args make_s1(const Dims& d, int beta, const int8_t* A_sl, const int8_t*
     p.Kp = d.Kp;
     p.S = d.S;
     p.KT = (int)(d.Kp / CfgS1::BK);
-    p.kt_div = kt_divisor(p.KT);
     p.tiles_m = (int)((d.M + CfgS1::BM - 1) / CfgS1::BM);
     p.tiles_n = (int)((d.N + CfgS1::BN - 1) / CfgS1::BN);
     p.beta = beta;
@@ -425,25 +438,37 @@ static S1Args make_s1(const Dims& d, int beta, const int8_t* A_sl, const int8_t*
 }
 
 hipError_t launch_igemm_s1_blocked(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, int32_t* T, hipStream_t st,
-                                   unsigned* queue, int tm0, int tms) {
+                                   const S1Plan& plan, unsigned* queue, int tm0, int tms) {
     S1Args p = make_s1(d, 7, A_sl, B_sl);
     p.KT = (int)(d.Kp / CfgS2::BK);
-    p.kt_div = kt_divisor(p.KT);
     const int tiles_m = (int)((d.M + CfgS2::BM - 1) / CfgS2::BM);
     if (tm0 < 0 || tm0 > tiles_m) return hipErrorInvalidValue;
     p.tm0 = tm0;
     p.tiles_m = tms < 0 ? tiles_m - tm0 : std::min(tms, tiles_m - tm0);
     p.tiles_n = (int)((d.N + CfgS2::BN - 1) / CfgS2::BN);
     p.T = T;
-    const int64_t total = (int64_t)p.tiles_m * p.tiles_n * d.S;
+    S1List list;
+    list.n = 0;
+    for (int g = 0, extra = d.S; g < d.S; ++g) {
+        const int stages = (g + 1) * p.KT, parts = plan.parts[g];
+        for (int j = 0; j < parts; ++j) {
+            if (list.n == kMaxS1Planes) return hipErrorInvalidValue;
+            const int i0 = (int)((int64_t)stages * j / parts), i1 = (int)((int64_t)stages * (j + 1) / parts);
+            list.e[list.n++] = S1Entry{(uint8_t)(g + 2), (uint8_t)(j == 0 ? g : extra++), (uint16_t)i0, (uint16_t)(i1 - i0)};
+        }
+    }
+    std::stable_sort(list.e, list.e + list.n, [](const S1Entry& a, const S1Entry& b) {
+        return a.nit != b.nit ? a.nit > b.nit : a.g > b.g;
+    });
+    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n, total = tiles * list.n;
     if (total == 0) return hipSuccess;
     unsigned grid = 0;
     if (hipError_t e = persistent_grid(total, grid)) return e;
     // A workgroup of the dynamic order claims two positions before it starts, so with fewer than two
-    // items per workgroup the first claimants would take them all and the others none: below that,
-    // the static order (every workgroup its own positions) is the balanced one.
-    p.queue = queue && grid % 8 == 0 && total >= 2 * (int64_t)grid ? queue : nullptr;  // counters zeroed by the caller
-    k_igemm_s1g<CfgS2><<<grid, CfgS2::NT, 0, st>>>(p);
+    // items per workgroup the first claimants would take them all and the others none; and with few
+    // tiles the XCDs' shares of them are uneven (30 tiles: three or four each).
+    p.queue = queue && grid % 8 == 0 && total >= 2 * (int64_t)grid && tiles >= 64 ? queue : nullptr;  // zeroed by the caller
+    k_igemm_s1g<CfgS2><<<grid, CfgS2::NT, 0, st>>>(p, list);
     return hipGetLastError();
 }
 

@@ -24,11 +24,14 @@ struct IgemmCfg {
     static constexpr int KB = BK / 32;             // fragment blocks along K per stage
     static constexpr int ABLK = BM * BK / 1024;    // 1 KiB blocks (one wave-wide direct load) per stage
     static constexpr int BBLK = BN * BK / 1024;
+    static constexpr int LPA = ABLK / NWAVES, LPB = BBLK / NWAVES;  // per wave: consecutive along K
+    static constexpr int STEP = KB * 1024;         // bytes of a plane from one stage to the next
     static constexpr int LPS = (ABLK + BBLK) / NWAVES;  // direct loads per thread per stage
     static constexpr int STAGE_BYTES = (BM + BN) * BK;
     static constexpr int LDS_BYTES = STAGES * STAGE_BYTES;
     static_assert(WTM % 32 == 0 && WTN % 32 == 0, "wave tile must be a multiple of 32");
     static_assert(ABLK % NWAVES == 0 && BBLK % NWAVES == 0, "stage must split evenly over waves");
+    static_assert(KB % LPA == 0 && KB % LPB == 0 && LPA <= 4 && LPB <= 4, "a wave's blocks lie in one block-row");
     static_assert(BK % 32 == 0, "BK must be a multiple of the MFMA K (32)");
     static_assert(256 % BM == 0 && 256 % BN == 0, "tile must divide the 256-row padding");
     static_assert(128 % BK == 0, "BK must divide the 128-byte K padding");

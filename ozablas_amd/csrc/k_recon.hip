@@ -15,6 +15,7 @@
 // (k_recon_s1_blocked) or from the reference's planar [S][M][N] planes (stage entry point).
 #include <algorithm>
 
+#include "k_igemm_cfg.hpp"
 #include "recon_core.hpp"
 
 namespace oza {
@@ -25,15 +26,16 @@ using namespace core;
 // ---------------------------------------------------------------- from GEMM digits
 // Workgroup = one 32 x 32 element block of C at a time: blocks [0, nblk) of the block rows from
 // R0 on, block b = (R0 + b / ceil(N/32), b % ceil(N/32)), walked with a grid stride.
-template <int S, bool PLAIN>
+template <int S, bool PLAIN, bool PARTS>
 __global__ void __launch_bounds__(256)
-    k_recon_digits(const uint8_t* __restrict__ dg, const int32_t* __restrict__ shA, const int32_t* __restrict__ shB,
+    k_recon_digits(uint8_t* dg, const int32_t* __restrict__ shA, const int32_t* __restrict__ shB,
                    int64_t M, int64_t N, int64_t Mp, int64_t Np, const CrtSet* __restrict__ cs, OutC c, int64_t R0,
-                   int64_t nblk) {
+                   int64_t nblk, DigitParts parts) {
     const int64_t qn = (N + 31) >> 5;
     for (int64_t b = blockIdx.x; b < nblk; b += gridDim.x) {
         const int64_t r = b / qn, Q = b - r * qn;
-        recon_digits_block<S, PLAIN>(dg, Mp * Np, Np, shA, shB, M, N, cs, c.p, c.ldc, c.alpha, c.beta, R0 + r, Q);
+        recon_digits_block<S, PLAIN, PARTS>(dg, Mp * Np, Np, shA, shB, M, N, cs, c.p, c.ldc, c.alpha, c.beta, R0 + r, Q,
+                                            &parts);
     }
 }
 
@@ -74,35 +76,53 @@ __global__ void __launch_bounds__(256)
 
 // ---------------------------------------------------------------- Scheme I from blocked INT32 planes
 // One 32 x 32 element block (R, Q); thread t reads int4 t of the block in every plane (4
-// elements of one column).  C = 0, then C = fma(T_g, 2^(2 beta - beta g) u_i v_j, C) for
-// g = 2..S+1 (step4_reconstruction.hpp:21-49, pipeline.hip:80, ascending g).  The planes are read
-// four at a time ahead of their FMAs.
-__device__ __forceinline__ void recon_s1_block(const int32_t* __restrict__ T, const int32_t* __restrict__ shA,
+// elements of one column).  T_g is the sum of its parts' planes; C = 0, then
+// C = fma(T_g, 2^(2 beta - beta g) u_i v_j, C) for g = 2..S+1 (step4_reconstruction.hpp:21-49,
+// pipeline.hip:80, ascending g).  The planes are read four at a time ahead of their use.
+struct S1Parts {
+    uint8_t plane[kMaxS1Planes];  // in order of use: group after group
+    uint8_t last[kMaxS1Planes];   // group g whose last plane this is, else 0
+    uint8_t parts[kMaxSlices + 2];  // of group g
+    int planes;
+};
+
+__device__ __forceinline__ void recon_s1_block(int32_t* T, const int32_t* __restrict__ shA,
                                                const int32_t* __restrict__ shB, int64_t M, int64_t N, int64_t Mp,
-                                               int64_t Np, int S, int beta, const OutC& c, int64_t R, int64_t Q) {
+                                               int64_t Np, const S1Parts& parts, int beta, const OutC& c, int64_t R,
+                                               int64_t Q) {
     const int t = threadIdx.x;
     const int lane = t >> 2, wd = t & 3;
     const int64_t col = Q * 32 + (lane & 31);
     const int64_t row0 = R * 32 + 8 * wd + 4 * (lane >> 5);
     if (col >= N || row0 >= M) return;
-    const int32_t* base = T + ((R * (Np >> 5) + Q) << 10) + t * 4;
+    int32_t* base = T + ((R * (Np >> 5) + Q) << 10) + t * 4;
     const int64_t plane = Mp * Np;
     const double v = ldexp(1.0, -shB[col] + 1 - beta);
     double u[4], acc[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int b = 0; b < 4; ++b) u[b] = row0 + b < M ? ldexp(1.0, -shA[row0 + b] + 1 - beta) : 0.0;
-    for (int g0 = 2; g0 <= S + 1; g0 += 4) {
+    int sum[4] = {0, 0, 0, 0};
+    for (int p0 = 0; p0 < parts.planes; p0 += 4) {
         int4 x[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)  // planes past S + 1 read the last one again and are not used
-            x[i] = *reinterpret_cast<const int4*>(base + (int64_t)(min(g0 + i, S + 1) - 2) * plane);
+        for (int i = 0; i < 4; ++i)  // planes past the last one read it again and are not used
+            x[i] = *reinterpret_cast<const int4*>(base + (int64_t)parts.plane[min(p0 + i, parts.planes - 1)] * plane);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int g = g0 + i;
-            if (g > S + 1) break;
+            if (p0 + i >= parts.planes) break;
             const int xs[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
 #pragma unroll
-            for (int b = 0; b < 4; ++b) acc[b] = fma((double)xs[b], ldexp(u[b] * v, -beta * g + 2 * beta), acc[b]);
+            for (int b = 0; b < 4; ++b) sum[b] += xs[b];
+            const int g = parts.last[p0 + i];
+            if (g) {
+                if (parts.parts[g] > 1)
+                    *reinterpret_cast<int4*>(base + (int64_t)(g - 2) * plane) = make_int4(sum[0], sum[1], sum[2], sum[3]);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    acc[b] = fma((double)sum[b], ldexp(u[b] * v, -beta * g + 2 * beta), acc[b]);
+                    sum[b] = 0;
+                }
+            }
         }
     }
 #pragma unroll
@@ -112,13 +132,13 @@ __device__ __forceinline__ void recon_s1_block(const int32_t* __restrict__ T, co
 
 // Blocks [0, nblk) of the block rows from R0 on, walked with a grid stride (as k_recon_digits).
 __global__ void __launch_bounds__(256)
-    k_recon_s1_blocked(const int32_t* __restrict__ T, const int32_t* __restrict__ shA,
-                       const int32_t* __restrict__ shB, int64_t M, int64_t N, int64_t Mp, int64_t Np, int S,
+    k_recon_s1_blocked(int32_t* T, const int32_t* __restrict__ shA,
+                       const int32_t* __restrict__ shB, int64_t M, int64_t N, int64_t Mp, int64_t Np, S1Parts parts,
                        int beta, OutC c, int64_t R0, int64_t nblk) {
     const int64_t qn = (N + 31) >> 5;
     for (int64_t b = blockIdx.x; b < nblk; b += gridDim.x) {
         const int64_t r = b / qn, Q = b - r * qn;
-        recon_s1_block(T, shA, shB, M, N, Mp, Np, S, beta, c, R0 + r, Q);
+        recon_s1_block(T, shA, shB, M, N, Mp, Np, parts, beta, c, R0 + r, Q);
     }
 }
 
@@ -171,15 +191,28 @@ __global__ void __launch_bounds__(256)
 }
 
 template <int S>
-hipError_t recon_digits_S(const Dims& d, const uint8_t* dg, const int32_t* shA, const int32_t* shB,
-                          const CrtSet* cs, const OutC& c, hipStream_t st, int64_t R0, int64_t nR, unsigned grid) {
+hipError_t recon_digits_S(const Dims& d, uint8_t* dg, const int32_t* shA, const int32_t* shB,
+                          const CrtSet* cs, const OutC& c, hipStream_t st, int64_t R0, int64_t nR, unsigned grid,
+                          const S2Plan* plan) {
     const int64_t nblk = nR * ((d.N + 31) >> 5);
     if (nblk == 0) return hipSuccess;
     if (grid == 0 || grid > nblk) grid = (unsigned)nblk;
-    if (c.alpha == 1.0 && c.beta == 0.0)
-        k_recon_digits<S, true><<<grid, 256, 0, st>>>(dg, shA, shB, d.M, d.N, d.Mp, d.Np, cs, c, R0, nblk);
-    else
-        k_recon_digits<S, false><<<grid, 256, 0, st>>>(dg, shA, shB, d.M, d.N, d.Mp, d.Np, cs, c, R0, nblk);
+    const bool plain = c.alpha == 1.0 && c.beta == 0.0;
+    DigitParts p = {};
+    if (plan && plan->parts > 1) {
+        p.tiles_m = (int)((d.M + kS2TileRows - 1) / kS2TileRows);
+        p.tiles_n = (int)((d.N + kS2TileRows - 1) / kS2TileRows);
+        p.gm = IgemmCfgS2::GM;
+        p.parts = plan->parts;
+        p.whole = plan->whole;
+        p.tail = (int64_t)p.tiles_m * p.tiles_n * S - plan->whole;
+        p.part = dg + (int64_t)S * d.Mp * d.Np;
+        if (plain) k_recon_digits<S, true, true><<<grid, 256, 0, st>>>(dg, shA, shB, d.M, d.N, d.Mp, d.Np, cs, c, R0, nblk, p);
+        else k_recon_digits<S, false, true><<<grid, 256, 0, st>>>(dg, shA, shB, d.M, d.N, d.Mp, d.Np, cs, c, R0, nblk, p);
+    } else {
+        if (plain) k_recon_digits<S, true, false><<<grid, 256, 0, st>>>(dg, shA, shB, d.M, d.N, d.Mp, d.Np, cs, c, R0, nblk, p);
+        else k_recon_digits<S, false, false><<<grid, 256, 0, st>>>(dg, shA, shB, d.M, d.N, d.Mp, d.Np, cs, c, R0, nblk, p);
+    }
     return hipGetLastError();
 }
 
@@ -208,9 +241,9 @@ hipError_t recon_int32_S(const Dims& d, const int32_t* Ct, const int32_t* shA, c
 
 }  // namespace
 
-hipError_t launch_recon_s2_digits(const Dims& d, const uint8_t* digits, const int32_t* shift_A,
+hipError_t launch_recon_s2_digits(const Dims& d, uint8_t* digits, const int32_t* shift_A,
                                   const int32_t* shift_B, const CrtSet* crt_dev, const OutC& c, hipStream_t st,
-                                  int64_t row0, int64_t rows, bool narrow) {
+                                  int64_t row0, int64_t rows, bool narrow, const S2Plan* plan) {
     if (d.M == 0 || d.N == 0) return hipSuccess;
     if (row0 < 0 || row0 > d.M || (row0 & 31)) return hipErrorInvalidValue;
     const int64_t end = rows < 0 ? d.M : std::min<int64_t>(d.M, row0 + rows);
@@ -223,7 +256,7 @@ hipError_t launch_recon_s2_digits(const Dims& d, const uint8_t* digits, const in
         if (e != hipSuccess) return e;
         grid = (unsigned)std::max(cus, 1);
     }
-    OZA_S_CASES(recon_digits_S, d, digits, shift_A, shift_B, crt_dev, c, st, R0, nR, grid)
+    OZA_S_CASES(recon_digits_S, d, digits, shift_A, shift_B, crt_dev, c, st, R0, nR, grid, plan)
 }
 
 hipError_t launch_recon_s2_int32(const Dims& d, const int32_t* C_tc, const int32_t* shift_A,
@@ -256,10 +289,17 @@ hipError_t launch_digits_pack(const Dims& d, const uint8_t* planar, const CrtSet
     return hipGetLastError();
 }
 
-hipError_t launch_recon_s1_blocked(const Dims& d, int beta, const int32_t* T, const int32_t* shift_A,
-                                   const int32_t* shift_B, const OutC& c, hipStream_t st, int64_t row0, int64_t rows,
-                                   bool narrow) {
+hipError_t launch_recon_s1_blocked(const Dims& d, int beta, int32_t* T, const int32_t* shift_A,
+                                   const int32_t* shift_B, const OutC& c, hipStream_t st, const S1Plan& plan,
+                                   int64_t row0, int64_t rows, bool narrow) {
     if (d.M == 0 || d.N == 0) return hipSuccess;
+    if (plan.planes < 1 || plan.planes > kMaxS1Planes) return hipErrorInvalidValue;
+    S1Parts parts = {};
+    for (int g = 0, extra = d.S; g < d.S; ++g) {
+        for (int j = 0; j < plan.parts[g]; ++j) parts.plane[parts.planes++] = (uint8_t)(j == 0 ? g : extra++);
+        parts.last[parts.planes - 1] = (uint8_t)(g + 2);
+        parts.parts[g + 2] = (uint8_t)plan.parts[g];
+    }
     if (row0 < 0 || row0 > d.M || (row0 & 31)) return hipErrorInvalidValue;
     const int64_t end = rows < 0 ? d.M : std::min<int64_t>(d.M, row0 + rows);
     const int64_t nblk = ((end - row0 + 31) >> 5) * ((d.N + 31) >> 5);
@@ -272,7 +312,7 @@ hipError_t launch_recon_s1_blocked(const Dims& d, int beta, const int32_t* T, co
         if (e != hipSuccess) return e;
         grid = (unsigned)std::min<int64_t>(nblk, std::max(cus, 1));
     }
-    k_recon_s1_blocked<<<grid, 256, 0, st>>>(T, shift_A, shift_B, d.M, d.N, d.Mp, d.Np, d.S, beta, c, row0 >> 5,
+    k_recon_s1_blocked<<<grid, 256, 0, st>>>(T, shift_A, shift_B, d.M, d.N, d.Mp, d.Np, parts, beta, c, row0 >> 5,
                                              nblk);
     return hipGetLastError();
 }

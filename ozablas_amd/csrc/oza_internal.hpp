@@ -5,9 +5,11 @@
 //   shift_B   int32[N]                   column shifts
 //   A_slices  int8 [S][Mp][Kp]           A residues/slices, K contiguous, fragment-tiled (frag_off16)
 //   B_slices  int8 [S][Np][Kp]           B residues/slices TRANSPOSED (column n is a K-contiguous row)
-//   C_tc      Scheme II: uint8 [S][Mp][Np] stored digits of C_s (stored_digit) in 32 x 32 element blocks
-//             Scheme I : int32 [S][Mp][Np] group products T_g in 32 x 32 element blocks (the stage
-//                        entry point writes the reference's planar int32 [S][M][N] instead)
+//   C_tc      Scheme II: uint8 [S][Mp][Np] stored digits of C_s (stored_digit) in 32 x 32 element blocks,
+//                        then the partial tiles of items that ran in K parts (S2Plan)
+//             Scheme I : int32 [S][Mp][Np] group products T_g in 32 x 32 element blocks, then the planes of
+//                        groups that ran in parts (S1Plan) (the stage entry point writes the reference's
+//                        planar int32 [S][M][N] instead)
 // with Mp = roundup(M, 256), Np = roundup(N, 256), Kp = roundup(K, 128).
 #pragma once
 
@@ -151,36 +153,58 @@ hipError_t launch_one_pass(int scheme, const Dims& d, int offset, const Operand&
 hipError_t launch_unpack_A(const Dims& d, const int8_t* A_sl, int8_t* out, hipStream_t st);
 hipError_t launch_unpack_B(const Dims& d, const int8_t* B_sl, int8_t* out, hipStream_t st);
 
+// How a single call's GEMM is cut into items (plan_host.cpp).
+constexpr int kS2TileRows = 256;
+constexpr int kTileBytes = kS2TileRows * kS2TileRows;  // digits of one tile
+constexpr int kMaxParts = 32;
+constexpr int kMaxS1Planes = 128;
+// Scheme II: items l (modulus-major, then tile) below `whole` run whole, the others in `parts` parts of
+// `kts` K steps (the last one may be shorter).
+struct S2Plan {
+    int parts = 1, kts = 0;
+    int64_t whole = 0;
+};
+S2Plan scheme2_plan(const Dims& d);
+// Digit tiles that a plan writes (65536 bytes each).
+int64_t s2_plan_tiles(const Dims& d, const S2Plan& p);
+// Scheme I: group g + 2 (g + 1 pairs) runs in parts[g] equal runs of its stages; the first part's INT32
+// plane is plane g, the other parts' follow the S planes, group after group.
+struct S1Plan {
+    int parts[kMaxSlices] = {};
+    int planes = 0;
+};
+S1Plan scheme1_plan(const Dims& d);
+// C_tc tiles (of digits, of INT32) that hold the plan of this shape and of every smaller one.
+int64_t s2_most_tiles(const Dims& d);
+int64_t s1_most_tiles(const Dims& d);
+
 // Step 3 (+ fused epilogues).
 enum class S2Out { Digits, Int32 };
 // Tile rows [tm0, tm0 + tms) of BM = 256 rows (tms < 0: to the last tile row).
-// split > 1 (Digits only): the K steps run in `split` parts of ceil(KT / split) steps (every part
-// non-empty), part j writing the digits of its partial product to plane set j of `out`
-// ([split][S][Mp][Np]); launch_digits_reduce then adds sets 1.. into set 0.
+// plan (Digits only, or null: every item whole): items past plan->whole run in plan->parts parts of
+// plan->kts K steps; part 0 writes the digits of its partial product to the S digit planes, part j > 0
+// to the partial tiles behind them, tile (j - 1) * tail + (item - whole) in the blocked layout of one tile.
 hipError_t launch_igemm_s2(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, S2Out mode, void* out,
-                           const CrtSet* crt_dev, hipStream_t st, int tm0 = 0, int tms = -1, int split = 1);
-// Digit planes [split][S][Mp][Np]: set 0 += sets 1..split-1, mod m_s.
-hipError_t launch_digits_reduce(const Dims& d, uint8_t* digits, int split, const CrtSet* crt_dev, hipStream_t st);
-constexpr int kS2TileRows = 256;
-// K split of a single Scheme II call (1: none): the grouped planner's choice for the problem alone,
-// on a fixed description of an MI355X (256 CUs, the default tile cost model) and the 256-wide tile
-// of the single-call GEMM, so that the workspace size and the call agree on it.
-int scheme2_single_split(size_t M, size_t N, size_t K, int S);
-// Scheme I: group products T_g, g = 2..S+1, into blocked INT32 planes [S][Mp][Np] (32 x 32 blocks).
+                           const CrtSet* crt_dev, hipStream_t st, int tm0 = 0, int tms = -1,
+                           const S2Plan* plan = nullptr);
+// Scheme I: group products T_g, g = 2..S+1, into blocked INT32 planes (32 x 32 blocks), one per group,
+// or per part of a group with a plan: [planes][Mp][Np].
 // Tile rows [tm0, tm0 + tms) of 256 rows (tms < 0: to the last tile row).  queue: 8 device counters for
 // the dynamic work order, zero when the launch starts, or null (static order).
 hipError_t launch_igemm_s1_blocked(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, int32_t* T, hipStream_t st,
-                                   unsigned* queue = nullptr, int tm0 = 0, int tms = -1);
+                                   const S1Plan& plan, unsigned* queue = nullptr, int tm0 = 0, int tms = -1);
 // Scheme I: group products T_g only, int32 [S][M][N] (reference C_tc semantics per group).
 hipError_t launch_igemm_s1_groups(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, int32_t* T,
                                   hipStream_t st);
 
 // Step 4.
 // Rows [row0, row0 + rows) of C (row0 a multiple of 32; rows < 0: to the last row).  narrow: one
-// workgroup per CU walks the blocks, leaving room on each CU for a concurrent step-3 workgroup.
-hipError_t launch_recon_s2_digits(const Dims& d, const uint8_t* digits, const int32_t* shift_A,
+// workgroup per CU walks the blocks, leaving room on each CU for a concurrent step-3 workgroup.  plan:
+// launch_igemm_s2's; the parts' digits are added modulo m_s first, in place.
+hipError_t launch_recon_s2_digits(const Dims& d, uint8_t* digits, const int32_t* shift_A,
                                   const int32_t* shift_B, const CrtSet* crt_dev, const OutC& C, hipStream_t st,
-                                  int64_t row0 = 0, int64_t rows = -1, bool narrow = false);
+                                  int64_t row0 = 0, int64_t rows = -1, bool narrow = false,
+                                  const S2Plan* plan = nullptr);
 hipError_t launch_recon_s2_int32(const Dims& d, const int32_t* C_tc, const int32_t* shift_A,
                                  const int32_t* shift_B, const CrtSet* crt_dev, double* C, hipStream_t st);
 // Blocked digit planes <-> planar [s][M][N] digits in [0, m_s) (pack reduces its input mod m_s).
@@ -188,10 +212,11 @@ hipError_t launch_digits_unpack(const Dims& d, const uint8_t* digits, const CrtS
                                 hipStream_t st);
 hipError_t launch_digits_pack(const Dims& d, const uint8_t* planar, const CrtSet* crt_dev, uint8_t* digits,
                               hipStream_t st);
-// Scheme I step 4 from blocked planes: C = fma(T_g, scale_g, C) for g ascending, then the output rule.
-hipError_t launch_recon_s1_blocked(const Dims& d, int beta, const int32_t* T, const int32_t* shift_A,
-                                   const int32_t* shift_B, const OutC& C, hipStream_t st, int64_t row0 = 0,
-                                   int64_t rows = -1, bool narrow = false);
+// Scheme I step 4 from blocked planes: T_g = the sum of its parts' planes (left in the first of them),
+// C = fma(T_g, scale_g, C) for g ascending, then the output rule.
+hipError_t launch_recon_s1_blocked(const Dims& d, int beta, int32_t* T, const int32_t* shift_A,
+                                   const int32_t* shift_B, const OutC& C, hipStream_t st, const S1Plan& plan,
+                                   int64_t row0 = 0, int64_t rows = -1, bool narrow = false);
 hipError_t launch_recon_s1_groups(const Dims& d, int beta, const int32_t* T, const int32_t* shift_A,
                                   const int32_t* shift_B, double* C, hipStream_t st);
 

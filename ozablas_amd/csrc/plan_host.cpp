@@ -1,0 +1,141 @@
+// plan_host.cpp — how a single call's GEMM is cut into work items (host only).
+//
+// The persistent GEMMs run one 256 x 256 tile per CU at a time.  Where the items do not fill whole
+// rounds of the CUs (Scheme II), or the longest item outlasts the rest (Scheme I), items are split along
+// K: their parts are exact integer sums (digits add modulo m_s, group products in INT32), so the result
+// does not depend on the split.  The plans are fixed functions of the shape, for an MI355X's 256 CUs and
+// the measured item time below, so that workspace sizes and calls agree on them.
+#include <algorithm>
+
+#include "oza_internal.hpp"
+
+namespace oza {
+
+namespace {
+
+constexpr int64_t kPlanCus = 256;
+// An item lasts about 3.5 us plus 1.52 us per 128-byte K step (4096^2, S = 8, K = 128, 512, 1024, 2048: 5.0,
+// 9.8, 16.0, 28.0 us per round).
+constexpr double kItemUs = 3.5, kStepUs = 1.52;
+// A Scheme I item stores INT32, four times the bytes of digits.
+constexpr double kS1ItemUs = 9.0;
+// The reconstruction of split items: their extra bytes, and its longer chain of loads.
+constexpr double kBytesPerUs = 4.0e6, kPartsUs = 2.0;
+
+double item_us(int64_t steps) { return kItemUs + kStepUs * (double)steps; }
+int64_t div_up(int64_t a, int64_t b) { return (a + b - 1) / b; }
+// Calls with this many items or more are not split; a split call adds at most this many partial tiles.
+constexpr int64_t kS2Items = 16 * kPlanCus, kS2Extra = 2 * kPlanCus;
+constexpr int64_t kS1Items = 8 * kPlanCus, kS1Extra = kPlanCus;
+constexpr int64_t kS1MinStages = 4;  // per part
+int64_t tiles_of(const Dims& d) { return div_up(d.M, kS2TileRows) * div_up(d.N, kS2TileRows); }
+
+}  // namespace
+
+// Candidates: every item in p parts, or only those past the last full round of the CUs (2048^3, S = 6:
+// 384 items are 1.5 rounds; the last 128 in halves take 1 + 0.5: 95.4 -> 92.7 us for the call; 1500 x 900 x
+// 3000, S = 12, 288 items: 124 -> 112 us; 777 x 1501 x 1003, S = 14: 55.7 -> 54.2 us).  From 16 rounds on row
+// bands may run instead and the last round matters little.
+S2Plan scheme2_plan(const Dims& d) {
+    S2Plan best;  // unsplit
+    const int64_t KT = d.Kp / 128, items = tiles_of(d) * d.S;
+    best.kts = (int)KT;
+    best.whole = items;
+    if (items == 0 || items >= kS2Items) return best;
+    const int64_t full = items / kPlanCus * kPlanCus;
+    double best_us = 0.97 * (double)div_up(items, kPlanCus) * item_us(KT);  // a split has to pay
+    for (const int64_t whole : {full, (int64_t)0}) {
+        const int64_t tail = items - whole;
+        if (tail == 0) continue;
+        for (int64_t p = 2; p <= kMaxParts && 2 * p <= KT; ++p) {
+            const int64_t kts = div_up(KT, p);
+            if (div_up(KT, kts) != p) continue;  // some part would be empty
+            if ((p - 1) * tail > kS2Extra) break;
+            const double us = (double)(whole / kPlanCus) * item_us(KT) + (double)div_up(tail * p, kPlanCus) * item_us(kts) +
+                              (double)((p - 1) * tail * kTileBytes) / kBytesPerUs + kPartsUs;
+            if (us < best_us) {
+                best_us = 0.98 * us;  // more parts only where they pay clearly
+                best.parts = (int)p;
+                best.kts = (int)kts;
+                best.whole = whole;
+            }
+        }
+        if (full == 0) break;
+    }
+    return best;
+}
+
+int64_t s2_plan_tiles(const Dims& d, const S2Plan& p) {
+    const int64_t items = tiles_of(d) * d.S;
+    return p.parts > 1 ? items + (p.parts - 1) * (items - p.whole) : items;
+}
+
+// At least every plan's tiles, and growing with each of M, N, K and S, so that buffers made for the
+// largest of a program's shapes hold the smaller ones (whose plans may have more parts).
+static int64_t most_tiles(int64_t items, int64_t most_parted, int64_t split_items, int64_t extra) {
+    return std::max(items, std::min({most_parted, items + extra, split_items + extra}));
+}
+int64_t s2_most_tiles(const Dims& d) {
+    const int64_t items = tiles_of(d) * d.S;
+    return most_tiles(items, items * std::clamp<int64_t>(d.Kp / 256, 1, kMaxParts), kS2Items, kS2Extra);
+}
+int64_t s1_most_tiles(const Dims& d) {
+    int64_t parts = 0;
+    for (int g = 0; g < d.S; ++g) parts += div_up((g + 1) * (d.Kp / 128), kS1MinStages);
+    return most_tiles(tiles_of(d) * d.S, tiles_of(d) * std::min<int64_t>(parts, kMaxS1Planes), kS1Items, kS1Extra);
+}
+
+// Groups of at most `limit` stages per item, the limit with the least modelled time: the longest load of
+// a workgroup in the launch's order (one list, longest item first, back and forth over the CUs; sampled
+// workgroups), plus the extra planes' bytes.  Calls, us, whole / with this plan: 184 x 499 x 10597, S = 6
+// 622 / 122; 700^2 x 3000, S = 6 208 / 88; 1200^3, S = 6 102 / 86; 1499 x 1200 x 1801, S = 8 199 / 191;
+// 1500^3, S = 8 stays whole (179, in two parts 187), as does 2000^2 x 1000, S = 6 (136, 174).
+S1Plan scheme1_plan(const Dims& d) {
+    S1Plan best;
+    const int64_t KT = d.Kp / 128, tiles = tiles_of(d);
+    auto plan_us = [&](int64_t limit, S1Plan& p) -> double {
+        double len[kMaxS1Planes];  // entries of `tiles` items each
+        p.planes = 0;
+        for (int g = 0; g < d.S; ++g) {  // g + 1 pairs
+            const int64_t stages = (g + 1) * KT;
+            p.parts[g] = (int)div_up(stages, limit);
+            if (p.planes + p.parts[g] > kMaxS1Planes) return 1e30;
+            for (int j = 0; j < p.parts[g]; ++j) len[p.planes++] = kS1ItemUs + kStepUs * (double)div_up(stages, p.parts[g]);
+        }
+        std::sort(len, len + p.planes, [](double a, double b) { return a > b; });
+        const int64_t items = tiles * p.planes;
+        double longest = 0.0;
+        for (int64_t b = 0; b < kPlanCus; b += 15) {
+            double load = 0.0;
+            for (int64_t r = 0; r * kPlanCus < items; ++r) {
+                const int64_t k = r & 1 ? (r + 1) * kPlanCus - 1 - b : r * kPlanCus + b;
+                if (k < items) load += len[k / tiles];
+            }
+            longest = std::max(longest, load);
+        }
+        const int extra = p.planes - d.S;
+        return longest + (extra ? (double)(extra * tiles) * 8.0 * kTileBytes / kBytesPerUs + kPartsUs : 0.0);
+    };
+    const int64_t most = (int64_t)d.S * KT;
+    if (tiles == 0 || tiles * d.S >= kS1Items) {  // enough items to balance
+        best.planes = d.S;
+        std::fill(best.parts, best.parts + d.S, 1);
+        return best;
+    }
+    double best_us = 0.95 * plan_us(most, best);
+    int64_t last = most;
+    for (const int p : {2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32}) {
+        const int64_t limit = std::max(kS1MinStages, div_up(most, p));
+        if (limit == last) continue;
+        last = limit;
+        S1Plan cand;
+        const double us = plan_us(limit, cand);
+        if (us < best_us && (cand.planes - d.S) * tiles <= kS1Extra) {
+            best_us = 0.96 * us;
+            best = cand;
+        }
+    }
+    return best;
+}
+
+}  // namespace oza

@@ -104,16 +104,67 @@ __device__ __forceinline__ void store_c(double* __restrict__ C, int64_t idx, dou
     else C[idx] = fma(alpha, x, beta * C[idx]);
 }
 
+// Partial digits of a call whose items past `whole` ran in parts (S2Plan): part j > 0 of item l at partial
+// tile (j - 1) * tail + (l - whole).
+struct DigitParts {
+    const uint8_t* part;
+    int64_t whole, tail;
+    int parts, tiles_m, tiles_n, gm;  // gm: tile rows per group of the GEMM's tile order
+};
+
+// Four digits each of two words, added modulo m byte by byte (digits below m).
+__device__ __forceinline__ uint32_t add_digits(uint32_t a, uint32_t b, uint32_t m) {
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    const u16x2 mm = {(unsigned short)m, (unsigned short)m};
+    auto add = [&](uint32_t x, uint32_t y) {
+        const u16x2 s = __builtin_bit_cast(u16x2, x) + __builtin_bit_cast(u16x2, y);
+        return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(s, s - mm));  // s - m wraps above s when s < m
+    };
+    const uint32_t lo = add(a & 0x00ff00ffu, b & 0x00ff00ffu);
+    const uint32_t hi = add((a >> 8) & 0x00ff00ffu, (b >> 8) & 0x00ff00ffu);
+    return lo | (hi << 8);
+}
+
+// Adds the parts' digits of element block (R, Q), byte offset `off` in the block, to w and to the digit
+// planes, where w[s] came from dg + s * plane.
+template <int S>
+__device__ __forceinline__ void add_parts(uint32_t (&w)[S], const DigitParts& d, const CrtSet* __restrict__ cs,
+                                          int64_t R, int64_t Q, int off, uint8_t* dg, int64_t plane) {
+    // The block's tile in the GEMM's order: groups of gm tile rows, column by column.  (Inverse of
+    // grouped_tile.)
+    const int tm = (int)(R >> 3), tn = (int)(Q >> 3);
+    const int first = tm / d.gm * d.gm, rows = min(d.tiles_m - first, d.gm);
+    const int64_t t = (int64_t)first * d.tiles_n + (int64_t)tn * rows + (tm - first);
+    const int64_t tiles = (int64_t)d.tiles_m * d.tiles_n;
+    const int s0 = d.whole > t ? (int)((d.whole - t + tiles - 1) / tiles) : 0;  // the moduli that ran in parts
+    if (s0 >= S) return;
+    const uint8_t* base = d.part + (t - d.whole) * kTileBytes + ((((R & 7) << 3) + (Q & 7)) << 10) + off;
+    for (int j = 1; j < d.parts; ++j, base += d.tail * kTileBytes) {
+        uint32_t x[S];
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            x[s] = 0;
+            if (s >= s0) x[s] = *reinterpret_cast<const uint32_t*>(base + s * tiles * kTileBytes);
+        }
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            if (s >= s0) w[s] = add_digits(w[s], x[s], cs->m[s]);
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+        if (s >= s0) *reinterpret_cast<uint32_t*>(dg + s * plane) = w[s];
+}
+
 // One 32 x 32 element block (R, Q) of C from blocked digit planes (layout of store_digits:
 // block (R, Q) at byte (R * Np/32 + Q) * 1024 of each plane, MFMA 32x32 order inside).
 // 256 threads; thread t reads dword t of the block in every plane (4 elements of one column).
-// PLAIN: alpha = 1, beta = 0 (C = X), compiled without the output rule.
-template <int S, bool PLAIN = true>
+// PLAIN: alpha = 1, beta = 0 (C = X), compiled without the output rule.  PARTS: some items ran in parts.
+template <int S, bool PLAIN = true, bool PARTS = false>
 __device__ __forceinline__ void recon_digits_block(const uint8_t* __restrict__ dg, int64_t plane, int64_t Np,
                                                    const int32_t* __restrict__ shA, const int32_t* __restrict__ shB,
                                                    int64_t M, int64_t N, const CrtSet* __restrict__ cs,
                                                    double* __restrict__ Cout, int64_t ldc, double alpha, double beta,
-                                                   int64_t R, int64_t Q) {
+                                                   int64_t R, int64_t Q, const DigitParts* parts = nullptr) {
     const int t = threadIdx.x;
     const int lane = t >> 2, wd = t & 3;
     const int64_t col = Q * 32 + (lane & 31);
@@ -124,6 +175,7 @@ __device__ __forceinline__ void recon_digits_block(const uint8_t* __restrict__ d
 #pragma unroll
     for (int s = 0; s < S; ++s) w[s] = *reinterpret_cast<const uint32_t*>(base + s * plane);
     const int32_t sb = shB[col];
+    if (PARTS) add_parts<S>(w, *parts, cs, R, Q, t * 4, const_cast<uint8_t*>(base), plane);
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
         const int64_t row = row0 + b;
