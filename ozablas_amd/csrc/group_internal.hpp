@@ -33,7 +33,8 @@ struct GroupProblem {
     int32_t split, kbs;           // K splits of the GEMM (1: none), 128-byte K blocks per split
     int64_t chunksA, nblkA, colblkB, nblkB;  // step-1 blocks of A and B
     int64_t slA, slB;                        // step-2 blocks of A and B
-    int64_t nfA;  // blocks of A with steps 1 and 2 fused (Kp <= core::kFuseMaxKp; nblkA = slA = 0 then)
+    // Kp <= core::kPassMaxKp: blocks of A and of B with steps 1 and 2 in one pass (nblk*, sl* = 0 then)
+    int64_t psA, psB;
 };
 
 struct GroupPtrs {
@@ -47,7 +48,7 @@ struct GItem {
     int32_t local;
 };
 
-enum GroupStage { kGStats, kGFinalize, kGFuseA, kGSlice, kGGemm256, kGGemm128, kGGemm64, kGReduce, kGRecon, kGStages };
+enum GroupStage { kGStats, kGFinalize, kGPass, kGSlice, kGGemm256, kGGemm128, kGGemm64, kGReduce, kGRecon, kGStages };
 
 struct GroupLaunch {
     const GroupProblem* probs;

@@ -23,6 +23,19 @@ using GCfg256 = IgemmCfgS2;
 using GCfg128 = IgemmCfg<128, 128, 64, 2, 2, 2, 4>;
 using GCfg64 = IgemmCfg<64, 64, 128, 2, 2, 2, 4>;
 
+// Physical block -> item.  Workgroups are dealt round-robin to the 8 XCDs; this deals runs of
+// kRun consecutive items instead, so each XCD works through its runs in list order (the list is
+// longest-first, and every XCD gets an even share of long and short items) while the tiles of a
+// run, which share operand panels, meet in one L2.  A bijection on [0, n): blocks of the last
+// partial set of 8 runs map to themselves.
+constexpr int64_t kRun = 16;
+__device__ __forceinline__ int64_t xcd_runs(int64_t b, int64_t n) {
+    const int64_t full = n / (8 * kRun) * (8 * kRun);
+    if (b >= full) return b;
+    const int64_t i = b >> 3, x = b & 7;
+    return ((i / kRun) * 8 + x) * kRun + i % kRun;
+}
+
 __global__ void __launch_bounds__(256) k_group_zero(uint32_t* __restrict__ keys, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i < n) keys[i] = 0;
@@ -50,29 +63,43 @@ __global__ void __launch_bounds__(256) k_group_finalize(GroupLaunch g) {
     const GroupProblem& P = g.probs[it.prob];
     const int64_t i = (int64_t)it.local * 256 + threadIdx.x;
     if (i < P.M) {
-        if (!P.nfA) key_to_shift(reinterpret_cast<uint32_t*>(P.shA) + i, P.kparam);  // fused: written as shifts
+        key_to_shift(reinterpret_cast<uint32_t*>(P.shA) + i, P.kparam);
     } else if (i - P.M < P.N) {
         key_to_shift(reinterpret_cast<uint32_t*>(P.shB) + (i - P.M), P.kparam);
     }
 }
 
-// Steps 1 and 2 of A in one pass for problems with short K (fused_s2_A_block).
+// Steps 1 and 2 of both operands in one pass for problems with short K (pass_block).  Neighbouring blocks of
+// a row-contiguous operand share lines: runs of them go to one XCD (xcd_runs).
 template <int ND>
-__device__ __forceinline__ void group_fuse_a(const GroupProblem& P, const double* A, const ResidueConsts& rc,
-                                             int64_t blk, uint32_t* s_key, int32_t* s_shift) {
-    fused_s2_A_block<ND>(A, P.K, P.M, P.K, P.Mp, P.Kp, P.kparam, P.S, rc, P.shA, P.Asl, blk, s_key, s_shift);
+__device__ __forceinline__ void group_pass(const GroupProblem& P, const GroupPtrs& q, const ResidueConsts& rc, int64_t blk,
+                                           uint32_t* s_key, int32_t* s_shift) {
+    PassArgs g;
+    g.K = P.K;
+    g.Kp = P.Kp;
+    g.S = P.S;
+    g.R = group_pass_rows(P.Kp);
+    g.parts = 1;
+    g.offset = P.kparam;
+    if (blk < P.psA) {
+        const PassOp o{q.A, P.M, P.Mp, P.K, 1, P.shA, P.Asl, P.psA};
+        pass_block<ND, kGroupPassThreads, kGroupPassUnits, true, true>(o, g, rc, blk, 0, s_key, s_shift);
+    } else {
+        const PassOp o{q.B, P.N, P.Np, P.N, 0, P.shB, P.Bsl, P.psB};
+        pass_block<ND, kGroupPassThreads, kGroupPassUnits, false, true>(o, g, rc, blk - P.psA, 0, s_key, s_shift);
+    }
 }
 
-__global__ void __launch_bounds__(kFuseThreads) k_group_fuse_a(GroupLaunch g) {
-    __shared__ uint32_t s_key[kFuseThreads];
-    __shared__ int32_t s_shift[128];
-    const GItem it = g.items[blockIdx.x];
+__global__ void __launch_bounds__(kGroupPassThreads) k_group_pass(GroupLaunch g) {
+    __shared__ uint32_t s_key[kGroupPassThreads];
+    __shared__ int32_t s_shift[64];
+    const GItem it = g.items[xcd_runs(blockIdx.x, g.n)];
     const GroupProblem& P = g.probs[it.prob];
     const GroupPtrs q = g.ptrs[it.prob];
     switch (P.words) {  // uniform per workgroup
-        case 1: group_fuse_a<1>(P, q.A, g.rc, it.local, s_key, s_shift); break;
-        case 2: group_fuse_a<2>(P, q.A, g.rc, it.local, s_key, s_shift); break;
-        default: group_fuse_a<3>(P, q.A, g.rc, it.local, s_key, s_shift); break;
+        case 1: group_pass<1>(P, q, g.rc, it.local, s_key, s_shift); break;
+        case 2: group_pass<2>(P, q, g.rc, it.local, s_key, s_shift); break;
+        default: group_pass<3>(P, q, g.rc, it.local, s_key, s_shift); break;
     }
 }
 
@@ -96,19 +123,6 @@ __global__ void __launch_bounds__(kSliceThreads) k_group_slice(GroupLaunch g) {
         case 2: group_slice<2>(P, q, g.rc, it.local); break;
         default: group_slice<3>(P, q, g.rc, it.local); break;
     }
-}
-
-// Physical block -> item.  Workgroups are dealt round-robin to the 8 XCDs; this deals runs of
-// kRun consecutive items instead, so each XCD works through its runs in list order (the list is
-// longest-first, and every XCD gets an even share of long and short items) while the tiles of a
-// run, which share operand panels, meet in one L2.  A bijection on [0, n): blocks of the last
-// partial set of 8 runs map to themselves.
-constexpr int64_t kRun = 16;
-__device__ __forceinline__ int64_t xcd_runs(int64_t b, int64_t n) {
-    const int64_t full = n / (8 * kRun) * (8 * kRun);
-    if (b >= full) return b;
-    const int64_t i = b >> 3, x = b & 7;
-    return ((i / kRun) * 8 + x) * kRun + i % kRun;
 }
 
 // Persistent: workgroup b walks items b, b + gridDim.x, ... (the resident workgroups fill the
@@ -279,7 +293,7 @@ hipError_t launch_group_stage(int stage, const GroupLaunch& g, hipStream_t st) {
     switch (stage) {
         case kGStats: k_group_stats<<<grid, kStatThreads, 0, st>>>(g); break;
         case kGFinalize: k_group_finalize<<<grid, 256, 0, st>>>(g); break;
-        case kGFuseA: k_group_fuse_a<<<grid, kFuseThreads, 0, st>>>(g); break;
+        case kGPass: k_group_pass<<<grid, kGroupPassThreads, 0, st>>>(g); break;
         case kGSlice: k_group_slice<<<grid, kSliceThreads, 0, st>>>(g); break;
         case kGGemm256: {
             unsigned gg = 0;

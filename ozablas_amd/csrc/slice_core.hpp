@@ -139,79 +139,6 @@ __device__ __forceinline__ void slice_s2_A_block(const double* __restrict__ A, i
     for (int s = 0; s < S; ++s) store_unit16<NT>(o + s * plane, residues16(t, rc, s));
 }
 
-// ---------------------------------------------------------------- Scheme II, steps 1 and 2 fused
-// Short K-contiguous rows (Kp <= kFuseMaxKp): a block holds R whole rows (R = fuse_rows(Kp)) in
-// registers, so a row's exponent maximum and its residues come from one read of the row instead
-// of one read for step 1 and another for step 2.  Same results as stats_A_block + key_to_shift +
-// slice_s2_A_block: the maximum is order-free, and every element goes through the same residue
-// arithmetic.  Unit u = (row u % R, 16-byte K chunk u / R) of the block; thread t takes units
-// t, t + 256, ... (at most 4), all of row t % R, so 8 consecutive lanes write one whole 128-byte
-// line of a fragment block.  Rows from M to roundup(M, 32) get zero residues (as in
-// slice_s2_A_block); shift[row] is written for rows < M.
-constexpr int64_t kFuseMaxKp = 2048;
-constexpr int kFuseThreads = 256;
-
-// Rows per fused block: the largest power of two R <= 128 with R * Kp/16 <= 1024 units (R >= 8
-// for Kp <= kFuseMaxKp).
-__host__ __device__ inline int fuse_rows(int64_t Kp) {
-    const int64_t units = Kp / 16;
-    int r = 128;
-    while (r > 8 && (int64_t)r * units > 4 * kFuseThreads) r >>= 1;
-    return r;
-}
-
-// s_key: kFuseThreads words of LDS, s_shift: 128 words.
-template <int ND>
-__device__ __forceinline__ void fused_s2_A_block(const double* __restrict__ A, int64_t lda, int64_t M, int64_t K,
-                                                 int64_t Mp, int64_t Kp, int32_t kparam, int S,
-                                                 const ResidueConsts& rc, int32_t* __restrict__ shift,
-                                                 int8_t* __restrict__ out, int64_t blk, uint32_t* s_key,
-                                                 int32_t* s_shift) {
-    const int R = fuse_rows(Kp);
-    const int64_t U = Kp / 16;  // units per row
-    const int t = threadIdx.x;
-    const int rl = t % R;
-    const int64_t row = blk * R + rl;
-    const int64_t rows_out = (M + 31) / 32 * 32;
-    const int64_t nunits = (int64_t)R * U;
-    double a[4][16];
-    uint32_t key = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int64_t u = t + (int64_t)kFuseThreads * i;
-        if (u < nunits && row < M) {
-            load_row16(A, lda, row, (u / R) * 16, K, a[i]);
-            key = max(key, max_key(a[i]));
-            drop_non_finite(a[i]);
-        } else {
-#pragma unroll
-            for (int j = 0; j < 16; ++j) a[i][j] = 0.0;
-        }
-    }
-    s_key[t] = key;
-    __syncthreads();
-    if (t < R) {
-        uint32_t k = 0;
-        for (int j = t; j < kFuseThreads; j += R) k = max(k, s_key[j]);
-        const int32_t sh = kparam - exp_from_key(k);  // key_to_shift
-        s_shift[t] = sh;
-        if (row < M) shift[row] = sh;
-    }
-    __syncthreads();
-    const int sh = s_shift[rl];
-    if (row >= rows_out) return;  // past the rows the planes hold for this operand
-    const int64_t plane = Mp * Kp;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int64_t u = t + (int64_t)kFuseThreads * i;
-        if (u >= nunits) break;
-        Words16<ND> v;
-        scaled_words16(a[i], sh, v);
-        int8_t* o = out + frag_off16(row, u / R, Kp);
-        for (int s = 0; s < S; ++s) store_unit16<true>(o + s * plane, residues16(v, rc, s));
-    }
-}
-
 // ---------------------------------------------------------------- Scheme II, row-contiguous columns
 // Operand element (col, k) at B[k * ldb + col] (the reference's B; also op(A) = A^T stored K x M).
 // Block = 64 columns x 4 groups of 32 K rows; thread = one column, 32 consecutive k.
@@ -402,7 +329,8 @@ struct PassArgs {
 };
 
 // ND: words per value (Scheme II), or 0 for Scheme I.
-template <int ND, int T, int NU, bool KC>
+// NT: nontemporal plane stores (store_unit16).
+template <int ND, int T, int NU, bool KC, bool NT = false>
 __device__ __forceinline__ void pass_block(const PassOp& o, const PassArgs& g, const ResidueConsts& rc, int64_t rb,
                                            int part, uint32_t* s_key, int32_t* s_shift) {
     const int R = g.R;
@@ -465,9 +393,21 @@ __device__ __forceinline__ void pass_block(const PassOp& o, const PassArgs& g, c
         } else {
             Words16<ND> v;
             scaled_words16(a[i], sh, v);
-            for (int s = s0; s < s1; ++s) store_unit16<false>(out + s * plane, residues16(v, rc, s));
+            for (int s = s0; s < s1; ++s) store_unit16<NT>(out + s * plane, residues16(v, rc, s));
         }
     }
+}
+
+// Grouped problems with Kp <= kPassMaxKp: blocks of 512 threads with up to two units each, any K.  A group's
+// launch is bound by memory, not by latency, and two such blocks share a CU, so that one reads while the
+// other computes and writes.  Two units in 1024 threads, one in 512 and four in 512 or 256 were slower (the
+// whole group of 512 problems, M, N, K log-uniform on [64, 2048]: 5.07, 5.15, 5.12 ms; two in 512 4.96 ms for
+// B, 4.92 ms for both operands; before, with B read by step 1 and again by step 2, 5.17 ms).
+constexpr int kGroupPassThreads = 512, kGroupPassUnits = 2;
+__host__ __device__ inline int group_pass_rows(int64_t Kp) {
+    int r = 64;
+    while (r > 8 && r * (Kp / 16) > kGroupPassThreads * kGroupPassUnits) r >>= 1;
+    return r;
 }
 
 }  // namespace core
