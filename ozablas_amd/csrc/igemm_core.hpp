@@ -65,6 +65,23 @@ __device__ __forceinline__ void issue_stage(int8_t* stage, const int8_t* __restr
     load(b, sb, std::make_integer_sequence<int, C::LPB>{});
 }
 
+struct WavePart {
+    int m, n;
+};
+// A wave's part of the tile.  At the product's edges the parts with nothing to compute leave their SIMD to
+// others (for_part), so the order spreads the rest over the four SIMDs (a workgroup's wave w runs on SIMD
+// w % 4): of 4 x 2 parts the first two rows, or the first column, lie on different SIMDs; of 2 x 2 parts
+// the workgroups of a CU (one per 256 blocks) each take another order.
+template <class C>
+__device__ __forceinline__ WavePart wave_part(int wave) {
+    if (C::NWM == 4 && C::NWN == 2) {
+        const int n = wave >> 2;
+        return {(wave & 3) ^ (n << 1), n};
+    }
+    if (C::NWM == 2 && C::NWN == 2) wave ^= (blockIdx.x >> 8) & 3;
+    return {wave / C::NWN, wave % C::NWN};
+}
+
 // Sources of one K stage for one wave.
 struct StageSrc {
     const int8_t* a;
@@ -72,13 +89,16 @@ struct StageSrc {
 };
 
 // The wave's blocks of stage 0 of the operand tiles at a and b (fragment-tiled planes, ldk K-bytes per
-// row); stage i lies i * C::STEP bytes further.
+// row); stage i lies i * C::STEP bytes further.  A block-row past last_a / last_b, the last that holds a row
+// of the operand, is read as that one: nothing uses it, and it is at hand (the plane's memory there would
+// come from HBM: groups 0.7 to 2.3 % slower).
 template <class C>
-__device__ __forceinline__ StageSrc wave_src(const int8_t* a, const int8_t* b, int64_t ldk, int wave) {
+__device__ __forceinline__ StageSrc wave_src(const int8_t* a, const int8_t* b, int64_t ldk, int wave,
+                                             int last_a = C::BM / 32 - 1, int last_b = C::BN / 32 - 1) {
     const int64_t kblocks = ldk >> 5;  // fragment blocks per block-row of a plane
     constexpr int KB = C::KB;
-    return StageSrc{a + (((wave * C::LPA / KB) * kblocks + wave * C::LPA % KB) << 10),
-                    b + (((wave * C::LPB / KB) * kblocks + wave * C::LPB % KB) << 10)};
+    return StageSrc{a + ((min(wave * C::LPA / KB, last_a) * kblocks + wave * C::LPA % KB) << 10),
+                    b + ((min(wave * C::LPB / KB, last_b) * kblocks + wave * C::LPB % KB) << 10)};
 }
 
 // What a wave loads after its current item's stages: the next item's stages 0 and 1 (any valid source
@@ -99,10 +119,10 @@ __device__ __forceinline__ void load_frags(Frags<C>& f, const int8_t* stage, int
     const int8_t* sb = stage + C::BM * C::BK;
 #pragma unroll
     for (int fm = 0; fm < C::FM; ++fm)
-        f.a[fm] = *reinterpret_cast<const v4i*>(stage + (((wm * C::FM + fm) * C::KB + kk) << 10) + lane * 16);
+        f.a[fm] = *reinterpret_cast<const v4i*>(stage + (((wm * (C::WTM / 32) + fm) * C::KB + kk) << 10) + lane * 16);
 #pragma unroll
     for (int fn = 0; fn < C::FN; ++fn)
-        f.b[fn] = *reinterpret_cast<const v4i*>(sb + (((wn * C::FN + fn) * C::KB + kk) << 10) + lane * 16);
+        f.b[fn] = *reinterpret_cast<const v4i*>(sb + (((wn * (C::WTN / 32) + fn) * C::KB + kk) << 10) + lane * 16);
 }
 
 template <class C>
@@ -199,7 +219,7 @@ __device__ __forceinline__ void mainloop_chain(v16i (&acc)[C::FM][C::FN], int8_t
     constexpr int KSTEPS = C::BK / 32;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave / C::NWN, wn = wave % C::NWN;
+    const int wm = wave_part<C>(wave).m, wn = wave_part<C>(wave).n;
     auto slot = [&](int i) { return smem + ((base + i) & 1) * C::STAGE_BYTES; };
     auto lds_barrier = [] {
         wait_lgkmcnt0();  // this wave's LDS reads are done
@@ -254,6 +274,58 @@ __device__ __forceinline__ void mainloop_chain(v16i (&acc)[C::FM][C::FN], int8_t
         issue_stage<C>(slot(nit + 1), nx.s1.a, nx.s1.b, wave, lane);
         mma_frags<C>(acc, f[(KSTEPS - 1) & 1]);
         __builtin_amdgcn_s_setprio(0);
+    }
+}
+
+// mainloop_chain for a wave whose part of the tile holds no element of the product: its loads, waits and
+// barriers, without fragments.
+template <class C, class Cur, class Step, class Entry>
+__device__ __forceinline__ void mainloop_idle(int8_t* smem, int base, int nit, Cur cur, Step step, Entry entry) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    auto slot = [&](int i) { return smem + ((base + i) & 1) * C::STAGE_BYTES; };
+    if (nit >= 2) wait_vmcnt<C::LPS>();
+    else wait_vmcnt<0>();
+    block_sync_lds();
+    const NextSrc nx = entry();
+    if (nit == 1) issue_stage<C>(slot(1), nx.s0.a, nx.s0.b, wave, lane);
+    for (int it = 0; it + 1 < nit; ++it) {
+        const bool own = it + 2 < nit;
+        const int8_t* pa = own ? cur.a : nx.s0.a;
+        const int8_t* pb = own ? cur.b : nx.s0.b;
+        step(cur);
+        wait_vmcnt<0>();
+        block_sync_lds();
+        issue_stage<C>(slot(it + 2), pa, pb, wave, lane);
+    }
+    block_sync_lds();
+    issue_stage<C>(slot(nit + 1), nx.s1.a, nx.s1.b, wave, lane);
+}
+
+// Edge tiles.  A wave that computes only the first FM_ x FN_ fragments of its part: the padding's products
+// cost time and, in a kernel that is bound by power, the other waves' clock.  Groups of 64, M, N, K log-uniform
+// on [64, 700]: 194 -> 187 us per call, 512 on [64, 2048] 4.95 -> 4.84 ms (4.87 with whole parts only); single
+// calls 300 x 5000 x 3000, S = 12 187 -> 178 us, 100 x 100 x 20000, S = 10 85 -> 74 us; 8192^3 unchanged.
+template <class C, int FM_, int FN_>
+struct PartCfg : C {
+    static constexpr int FM = FM_, FN = FN_;
+};
+
+// Runs full.operator()<P>() with the least of C, its half in either direction and its quarter that covers
+// the `rows` x `cols` elements from the wave's first on that belong to the product, or idle() where
+// none does.
+template <class C, class Full, class Idle>
+__device__ __forceinline__ void for_part(int64_t rows, int64_t cols, Full full, Idle idle) {
+    constexpr int HM = (C::FM + 1) / 2, HN = (C::FN + 1) / 2;
+    if (rows <= 0 || cols <= 0) {
+        idle();
+    } else if (C::FM > HM && rows <= HM * 32) {
+        if (C::FN > HN && cols <= HN * 32) full.template operator()<PartCfg<C, HM, HN>>();
+        else full.template operator()<PartCfg<C, HM, C::FN>>();
+    } else if (C::FN > HN && cols <= HN * 32) {
+        full.template operator()<PartCfg<C, C::FM, HN>>();
+    } else {
+        full.template operator()<C>();
     }
 }
 

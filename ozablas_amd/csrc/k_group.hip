@@ -137,7 +137,7 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
     int64_t w = blockIdx.x;
     if (w >= g.n) return;  // whole workgroup leaves together
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave / C::NWN, wn = wave % C::NWN;
+    const int wm = wave_part<C>(wave).m, wn = wave_part<C>(wave).n;
     struct Item {
         StageSrc src;    // this wave's blocks of stage 0
         uint8_t* plane;  // digit plane of modulus s (a partial plane for splits j > 0)
@@ -164,7 +164,7 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
         t.KT = min(P.kbs * kSteps128, (int)(P.Kp / C::BK) - t.k0);
         t.src = wave_src<C>(P.Asl + (int64_t)s * P.Mp * P.Kp + (int64_t)t.tm * C::BM * P.Kp + (int64_t)t.k0 * C::STEP,
                             P.Bsl + (int64_t)s * P.Np * P.Kp + (int64_t)t.tn * C::BN * P.Kp + (int64_t)t.k0 * C::STEP, P.Kp,
-                            wave);
+                            wave, (int)((P.M - (int64_t)t.tm * C::BM - 1) >> 5), (int)((P.N - (int64_t)t.tn * C::BN - 1) >> 5));
         const int64_t plane = P.Mp * P.Np;
         t.plane = (j == 0 ? P.dg : P.dgp + (int64_t)(j - 1) * P.S * plane) + (int64_t)s * plane;
         const auto& cs = as_constant(g.crt)->set[P.S - 1];
@@ -189,12 +189,17 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
         const bool more = w2 < g.n;
         Item nxt = cur;
         if (more) nxt = decode(w2);
-        v16i acc[C::FM][C::FN];
-        fill_acc<C>(acc, (int)cur.bias);
-        mainloop_chain<C>(acc, smem, base, cur.KT, stage(cur, 2), step,
-                          [&] { return NextSrc{stage(nxt, 0), stage(nxt, 1)}; });
-        store_digits<C, true, true>(acc, cur.plane, cur.Np, (int64_t)cur.tm * C::BM + wm * C::WTM,
-                                    (int64_t)cur.tn * C::BN + wn * C::WTN, cur.M, cur.N, cur.m, cur.minv, lane);
+        auto entry = [&] { return NextSrc{stage(nxt, 0), stage(nxt, 1)}; };
+        const int64_t row0 = (int64_t)cur.tm * C::BM + wm * C::WTM, col0 = (int64_t)cur.tn * C::BN + wn * C::WTN;
+        for_part<C>(
+            cur.M - row0, cur.N - col0,
+            [&]<class P>() {
+                v16i acc[P::FM][P::FN];
+                fill_acc<P>(acc, (int)cur.bias);
+                mainloop_chain<P>(acc, smem, base, cur.KT, stage(cur, 2), step, entry);
+                store_digits<P, true, true>(acc, cur.plane, cur.Np, row0, col0, cur.M, cur.N, cur.m, cur.minv, lane);
+            },
+            [&] { mainloop_idle<C>(smem, base, cur.KT, stage(cur, 2), step, entry); });
         if (!more) break;
         base = (base + cur.KT) & 1;
         w = w2;

@@ -66,7 +66,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
     int64_t w = blockIdx.x;
     if (w >= items) return;  // whole workgroup leaves together
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave / C::NWN, wn = wave % C::NWN;
+    const int wm = wave_part<C>(wave).m, wn = wave_part<C>(wave).n;
     struct Item {
         int s, tm, tn, j, k0, KT;
         int64_t l;
@@ -93,7 +93,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         // tile (tm, tn) starts at block-row tm*BM/32 of the fragment-tiled planes (BM*Kp bytes)
         t.src = wave_src<C>(p.A + (int64_t)t.s * p.Mp * p.Kp + (int64_t)t.tm * C::BM * p.Kp + (int64_t)t.k0 * C::STEP,
                             p.B + (int64_t)t.s * p.Np * p.Kp + (int64_t)t.tn * C::BN * p.Kp + (int64_t)t.k0 * C::STEP, p.Kp,
-                            wave);
+                            wave, (int)((p.M - (int64_t)t.tm * C::BM - 1) >> 5), (int)((p.N - (int64_t)t.tn * C::BN - 1) >> 5));
         // scalar loads: counted by lgkmcnt, so the epilogue does not wait for the direct loads
         t.m = as_constant(p.crt)->m[t.s];
         t.minv = as_constant(p.crt)->minv[t.s];
@@ -119,32 +119,37 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
             if (more) nxt = decode(w);
             return NextSrc{stage(nxt, 0), stage(nxt, 1)};
         };
-        v16i acc[C::FM][C::FN];
-        if (DIGITS) fill_acc<C>(acc, (int)cur.bias);
-        else zero_acc<C>(acc);
-        mainloop_chain<C>(acc, smem, base, cur.KT, stage(cur, 2), step, entry);
-        const int s = cur.s, tm = cur.tm, tn = cur.tn;
-        if (DIGITS) {
-            const bool part = SPLIT && cur.j > 0;  // a partial tile: the blocks of one tile, row-major
-            uint8_t* plane = part ? p.part + ((cur.j - 1) * p.tail + cur.l - p.whole) * kTileBytes
-                                  : reinterpret_cast<uint8_t*>(p.out) + (int64_t)s * p.Mp * p.Np;
-            const int64_t row0 = (part ? 0 : (int64_t)tm * C::BM) + wm * C::WTM;
-            const int64_t col0 = (part ? 0 : (int64_t)tn * C::BN) + wn * C::WTN;
-            store_digits<C, false>(acc, plane, part ? C::BN : p.Np, row0, col0, p.M, p.N, cur.m, cur.minv, lane);
-        } else {
-            int32_t* o = reinterpret_cast<int32_t*>(p.out) + (int64_t)s * p.M * p.N;
+        const int s = cur.s;
+        const int64_t row0 = (int64_t)cur.tm * C::BM + wm * C::WTM, col0 = (int64_t)cur.tn * C::BN + wn * C::WTN;
+        for_part<C>(
+            p.M - row0, p.N - col0,
+            [&]<class P>() {
+                v16i acc[P::FM][P::FN];
+                if (DIGITS) fill_acc<P>(acc, (int)cur.bias);
+                else zero_acc<P>(acc);
+                mainloop_chain<P>(acc, smem, base, cur.KT, stage(cur, 2), step, entry);
+                if (DIGITS) {
+                    const bool part = SPLIT && cur.j > 0;  // a partial tile: the blocks of one tile, row-major
+                    uint8_t* plane = part ? p.part + ((cur.j - 1) * p.tail + cur.l - p.whole) * kTileBytes
+                                          : reinterpret_cast<uint8_t*>(p.out) + (int64_t)s * p.Mp * p.Np;
+                    store_digits<P, false>(acc, plane, part ? C::BN : p.Np, part ? wm * C::WTM : row0,
+                                           part ? wn * C::WTN : col0, p.M, p.N, cur.m, cur.minv, lane);
+                } else {
+                    int32_t* o = reinterpret_cast<int32_t*>(p.out) + (int64_t)s * p.M * p.N;
 #pragma unroll
-            for (int fm = 0; fm < C::FM; ++fm)
+                    for (int fm = 0; fm < P::FM; ++fm)
 #pragma unroll
-                for (int fn = 0; fn < C::FN; ++fn) {
-                    const int64_t col = (int64_t)tn * C::BN + wn * C::WTN + fn * 32 + (lane & 31);
+                        for (int fn = 0; fn < P::FN; ++fn) {
+                            const int64_t col = col0 + fn * 32 + (lane & 31);
 #pragma unroll
-                    for (int j = 0; j < 16; ++j) {
-                        const int64_t row = (int64_t)tm * C::BM + wm * C::WTM + fm * 32 + frag_row(j, lane);
-                        if (row < p.M && col < p.N) o[row * p.N + col] = acc[fm][fn][j];
-                    }
+                            for (int j = 0; j < 16; ++j) {
+                                const int64_t row = row0 + fm * 32 + frag_row(j, lane);
+                                if (row < p.M && col < p.N) o[row * p.N + col] = acc[fm][fn][j];
+                            }
+                        }
                 }
-        }
+            },
+            [&] { mainloop_idle<C>(smem, base, cur.KT, stage(cur, 2), step, entry); });
         if (!more) break;
         base = (base + cur.KT) & 1;
         cur = nxt;
@@ -255,7 +260,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1(S1Args p) {
     int tm, tn;
     grouped_tile<C>(xcd_remap(blockIdx.x, tiles), p.tiles_m, p.tiles_n, tm, tn);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave / C::NWN, wn = wave % C::NWN;
+    const int wm = wave_part<C>(wave).m, wn = wave_part<C>(wave).n;
     const StageSrc src =
         wave_src<C>(p.A + (int64_t)tm * C::BM * p.Kp, p.B + (int64_t)tn * C::BN * p.Kp, p.Kp, wave);
     const S1Walk<C> walk(p);
@@ -313,7 +318,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1g(S1Args p, S1List list) {
     Claims c = first_claims(p.queue, xcd, s_pos);
     if (c.w >= nwork) return;  // whole workgroup leaves together
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave / C::NWN, wn = wave % C::NWN;
+    const int wm = wave_part<C>(wave).m, wn = wave_part<C>(wave).n;
     struct Item {
         int g, tm, tn, i0, nit, plane;
         StageSrc src;
@@ -327,7 +332,8 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1g(S1Args p, S1List list) {
         t.nit = list.e[e].nit;
         grouped_tile<C>(t0 + (k - (int64_t)e * ntile), p.tiles_m, p.tiles_n, t.tm, t.tn);
         t.tm += p.tm0;
-        t.src = wave_src<C>(p.A + (int64_t)t.tm * C::BM * p.Kp, p.B + (int64_t)t.tn * C::BN * p.Kp, p.Kp, wave);
+        t.src = wave_src<C>(p.A + (int64_t)t.tm * C::BM * p.Kp, p.B + (int64_t)t.tn * C::BN * p.Kp, p.Kp, wave,
+                            (int)((p.M - (int64_t)t.tm * C::BM - 1) >> 5), (int)((p.N - (int64_t)t.tn * C::BN - 1) >> 5));
         return t;
     };
     const S1Walk<C> walk(p);
@@ -342,14 +348,23 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1g(S1Args p, S1List list) {
             if (more) nxt = decode(c.w1);
             return walk.next(nxt.src, p, nxt.g, nxt.i0, nxt.nit);
         };
-        v16i acc[C::FM][C::FN];
-        zero_acc<C>(acc);
-        mainloop_chain<C>(acc, smem, base, cur.nit, walk.at(cur.src, p, cur.g, cur.i0 + min(2, cur.nit - 1)), walk, entry);
         unsigned ticket;  // the item after next (dynamic order); thread 0's only: a value merged from both
         // paths would be copied, and so waited for behind the next item's loads, as soon as it returns
-        if (dyn && more && threadIdx.x == 0) ticket = atomicAdd(&p.queue[xcd], 1u);
-        store_i32_blocked<C>(acc, p.T + (int64_t)cur.plane * p.Mp * p.Np, p.Np,
-                             (int64_t)cur.tm * C::BM + wm * C::WTM, (int64_t)cur.tn * C::BN + wn * C::WTN, lane);
+        auto claim = [&] {
+            if (dyn && more && threadIdx.x == 0) ticket = atomicAdd(&p.queue[xcd], 1u);
+        };
+        const int64_t row0 = (int64_t)cur.tm * C::BM + wm * C::WTM, col0 = (int64_t)cur.tn * C::BN + wn * C::WTN;
+        const S1Cursor stage2 = walk.at(cur.src, p, cur.g, cur.i0 + min(2, cur.nit - 1));
+        for_part<C>(
+            p.M - row0, p.N - col0,
+            [&]<class P>() {
+                v16i acc[P::FM][P::FN];
+                zero_acc<P>(acc);
+                mainloop_chain<P>(acc, smem, base, cur.nit, stage2, walk, entry);
+                claim();
+                store_i32_blocked<P>(acc, p.T + (int64_t)cur.plane * p.Mp * p.Np, p.Np, row0, col0, lane);
+            },
+            [&] { mainloop_idle<C>(smem, base, cur.nit, stage2, walk, entry); });  // never thread 0's wave: part (0, 0)
         if (!more) break;
         const int64_t w2 = dyn ? publish_claim(ticket, s_pos) : c.w + 2 * (int64_t)gridDim.x;
         base = (base + cur.nit) & 1;
