@@ -367,6 +367,11 @@ int build_plan(const GroupModel& model, int n, const size_t* M, const size_t* N,
         P.Np = (int64_t)round_up((size_t)P.N, (size_t)P.tile);
         P.tiles_m = (int32_t)(P.Mp / P.tile);
         P.tiles_n = (int32_t)(P.Np / P.tile);
+        P.order = tile_order(P.tiles_m, P.tiles_n, group_gm(P.tile));
+        P.by_S = fast_div(P.S);
+        P.planeA = P.Mp * P.Kp;
+        P.planeB = P.Np * P.Kp;
+        P.planeD = P.Mp * P.Np;
         fixed[i] = splits && splits[i] ? 1 : 0;
         split_shape(P.Kp / 128, fixed[i] ? splits[i] : 1, P.split, P.kbs);
     }

@@ -30,6 +30,9 @@ struct GroupProblem {
     uint8_t* dgp;                 // [split - 1][S][Mp][Np] partial digits of splits 1.. (split > 1)
     int32_t S, kparam, words, tile;  // words: 32-bit words per scaled value (residue_words)
     int32_t tiles_m, tiles_n;
+    TileOrder order;              // of the GEMM's tiles
+    FastDiv by_S;
+    int64_t planeA, planeB, planeD;  // bytes of a plane of Asl, Bsl, dg
     int32_t split, kbs;           // K splits of the GEMM (1: none), 128-byte K blocks per split
     int64_t chunksA, nblkA, colblkB, nblkB;  // step-1 blocks of A and B
     int64_t slA, slB;                        // step-2 blocks of A and B
@@ -62,6 +65,7 @@ struct GroupLaunch {
 
 // Tile edges of the three GEMM shapes, in the order of kGGemm256.. .
 constexpr int kGroupTiles[3] = {256, 128, 64};
+constexpr int group_gm(int tile) { return tile == 256 ? 8 : 4; }  // tile rows per group of the tile order
 // The tile cost model measured once on an MI355X (the contexts' default until oza_group_autotune).
 constexpr double kDefaultGroupCost[6] = {6.3, 1.58, 1.5, 0.48, 0.66, 0.25};
 // Largest K split the planner picks by itself, and the largest a caller may ask for.

@@ -363,25 +363,36 @@ __device__ __forceinline__ int frag_row(int j, int lane) { return 8 * (j >> 2) +
 // Work index -> (s, tm, tn).  Consecutive workgroups are dealt round-robin to the 8 XCDs; the
 // remap gives each XCD a contiguous run of work items so that neighbouring tiles (which share
 // A rows and B columns) meet in the same L2.
-__device__ __forceinline__ int64_t xcd_remap(int64_t id, int64_t total) {
-    const int64_t per = total / 8;
-    if (per == 0) return id;
-    if (id >= per * 8) return id;
-    return (id % 8) * per + id / 8;
+__device__ __forceinline__ uint32_t xcd_remap(uint32_t id, uint32_t total) {
+    const uint32_t per = total / 8;
+    return id >= per * 8 ? id : (id % 8) * per + id / 8;
+}
+
+// n / f.d and n % f.d.
+__device__ __forceinline__ uint32_t div_fast(uint32_t n, const FastDiv& f, uint32_t& rem) {
+    uint32_t q = __umulhi(n, f.inv);
+    rem = n - q * f.d;
+    if (rem >= f.d) {
+        ++q;
+        rem -= f.d;
+    }
+    return q;
 }
 
 // Tile index t in [0, tiles_m*tiles_n) -> (tm, tn), GM tile-rows at a time.
 template <class C>
-__device__ __forceinline__ void grouped_tile(int64_t t, int tiles_m, int tiles_n, int& tm, int& tn) {
-    const int64_t per_group = (int64_t)C::GM * tiles_n;
-    const int g = (int)(t / per_group);
-    const int first = g * C::GM;
-    const int gsz = min(tiles_m - first, C::GM);
-    const int r = (int)(t - g * per_group);
-    tm = first + r % gsz;
-    tn = r / gsz;
+__device__ __forceinline__ void grouped_tile(uint32_t t, const TileOrder& o, int& tm, int& tn) {
+    static_assert((C::GM & (C::GM - 1)) == 0, "full groups divide by a shift");
+    uint32_t r, row;
+    const int first = (int)div_fast(t, o.group, r) * C::GM;
+    if (o.tiles_m - first >= C::GM) {
+        row = r % C::GM;
+        tn = (int)(r / C::GM);
+    } else {
+        tn = (int)div_fast(r, o.last, row);
+    }
+    tm = first + (int)row;
 }
-
 
 // CRT-digit epilogue of one tile: the stored digit of C_s per accumulator element (the accumulators
 // started from the modulus' bias), one 16-byte store per fragment and lane.  Digit planes are blocked in 32 x 32 element blocks: block

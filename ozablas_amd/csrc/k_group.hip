@@ -22,17 +22,18 @@ using GCfg256 = IgemmCfgS2;
 // each other's short-K fill and epilogue (grouped GEMM step -4.5 % against 128-byte stages).
 using GCfg128 = IgemmCfg<128, 128, 64, 2, 2, 2, 4>;
 using GCfg64 = IgemmCfg<64, 64, 128, 2, 2, 2, 4>;
+static_assert(group_gm(256) == GCfg256::GM && group_gm(128) == GCfg128::GM && group_gm(64) == GCfg64::GM, "tile order");
 
 // Physical block -> item.  Workgroups are dealt round-robin to the 8 XCDs; this deals runs of
 // kRun consecutive items instead, so each XCD works through its runs in list order (the list is
 // longest-first, and every XCD gets an even share of long and short items) while the tiles of a
 // run, which share operand panels, meet in one L2.  A bijection on [0, n): blocks of the last
 // partial set of 8 runs map to themselves.
-constexpr int64_t kRun = 16;
-__device__ __forceinline__ int64_t xcd_runs(int64_t b, int64_t n) {
-    const int64_t full = n / (8 * kRun) * (8 * kRun);
+constexpr uint32_t kRun = 16;
+__device__ __forceinline__ uint32_t xcd_runs(uint32_t b, uint32_t n) {
+    const uint32_t full = n / (8 * kRun) * (8 * kRun);
     if (b >= full) return b;
-    const int64_t i = b >> 3, x = b & 7;
+    const uint32_t i = b >> 3, x = b & 7;
     return ((i / kRun) * 8 + x) * kRun + i % kRun;
 }
 
@@ -93,7 +94,7 @@ __device__ __forceinline__ void group_pass(const GroupProblem& P, const GroupPtr
 __global__ void __launch_bounds__(kGroupPassThreads) k_group_pass(GroupLaunch g) {
     __shared__ uint32_t s_key[kGroupPassThreads];
     __shared__ int32_t s_shift[64];
-    const GItem it = g.items[xcd_runs(blockIdx.x, g.n)];
+    const GItem it = g.items[xcd_runs(blockIdx.x, (uint32_t)g.n)];
     const GroupProblem& P = g.probs[it.prob];
     const GroupPtrs q = g.ptrs[it.prob];
     switch (P.words) {  // uniform per workgroup
@@ -128,14 +129,15 @@ __global__ void __launch_bounds__(kSliceThreads) k_group_slice(GroupLaunch g) {
 // Persistent: workgroup b walks items b, b + gridDim.x, ... (the resident workgroups fill the
 // chip once).  Its items form one chain through the LDS ring (mainloop_chain): the next item's
 // first two stages are issued during the current item's last two iterations.
-// An item's descriptor (operand and digit addresses, K steps, modulus) takes two dependent reads
-// (item list, problem); the next item's is read before the current mainloop, so those reads
-// overlap the MFMAs instead of delaying the next item's first loads.
+// An item's descriptor takes dependent reads (item list, problem, modulus) and a decode by scalar
+// instructions, of which a CU issues one per cycle for all its waves: the list entry is read an item ahead, the
+// rest after the current item's first barrier, and the divisions use reciprocals from the plan.
 template <class C>
 __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
     __shared__ __attribute__((aligned(1024))) int8_t smem[C::LDS_BYTES];
-    int64_t w = blockIdx.x;
-    if (w >= g.n) return;  // whole workgroup leaves together
+    const uint32_t n = (uint32_t)g.n;  // below 2^31
+    uint32_t w = blockIdx.x;
+    if (w >= n) return;  // whole workgroup leaves together
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave_part<C>(wave).m, wn = wave_part<C>(wave).n;
     struct Item {
@@ -146,27 +148,29 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
         uint32_t m, minv, bias;
     };
     constexpr int kSteps128 = 128 / C::BK;  // K steps per 128-byte K block
-    auto decode = [&](int64_t wi) {
+    auto item = [&](uint32_t wi) {
+        const auto& it = as_constant(g.items)[xcd_runs(wi, n)];
+        return GItem{it.prob, it.local};
+    };
+    auto decode = [&](GItem it) {
         Item t;
-        const auto& it = as_constant(g.items)[xcd_runs(wi, g.n)];
-        const uint32_t local = (uint32_t)it.local;
         const auto& P = as_constant(g.probs)[it.prob];
-        const uint32_t tiles = (uint32_t)P.tiles_m * (uint32_t)P.tiles_n;  // < 2^31: items are int32
-        const uint32_t per_split = (uint32_t)P.S * tiles;
-        const uint32_t j = P.split > 1 ? local / per_split : 0u;
-        const uint32_t rest = local - j * per_split;
-        const int s = (int)(rest / tiles);
-        grouped_tile<C>((int64_t)(rest - (uint32_t)s * tiles), P.tiles_m, P.tiles_n, t.tm, t.tn);
+        uint32_t tile, s;
+        const auto& o = P.order;
+        const FastDiv by_S{P.by_S.d, P.by_S.inv};
+        const TileOrder order{o.tiles_m, o.tiles_n, {o.tiles.d, o.tiles.inv}, {o.group.d, o.group.inv}, {o.last.d, o.last.inv}};
+        const uint32_t j = div_fast(div_fast((uint32_t)it.local, order.tiles, tile), by_S, s);
+        grouped_tile<C>(tile, order, t.tm, t.tn);
         t.Np = P.Np;
         t.M = P.M;
         t.N = P.N;
         t.k0 = (int)j * P.kbs * kSteps128;
         t.KT = min(P.kbs * kSteps128, (int)(P.Kp / C::BK) - t.k0);
-        t.src = wave_src<C>(P.Asl + (int64_t)s * P.Mp * P.Kp + (int64_t)t.tm * C::BM * P.Kp + (int64_t)t.k0 * C::STEP,
-                            P.Bsl + (int64_t)s * P.Np * P.Kp + (int64_t)t.tn * C::BN * P.Kp + (int64_t)t.k0 * C::STEP, P.Kp,
-                            wave, (int)((P.M - (int64_t)t.tm * C::BM - 1) >> 5), (int)((P.N - (int64_t)t.tn * C::BN - 1) >> 5));
-        const int64_t plane = P.Mp * P.Np;
-        t.plane = (j == 0 ? P.dg : P.dgp + (int64_t)(j - 1) * P.S * plane) + (int64_t)s * plane;
+        const int64_t k0 = (int64_t)t.k0 * C::STEP;
+        t.src = wave_src<C>(P.Asl + s * P.planeA + (int64_t)t.tm * C::BM * P.Kp + k0,
+                            P.Bsl + s * P.planeB + (int64_t)t.tn * C::BN * P.Kp + k0, P.Kp, wave,
+                            (int)((P.M - (int64_t)t.tm * C::BM - 1) >> 5), (int)((P.N - (int64_t)t.tn * C::BN - 1) >> 5));
+        t.plane = (j == 0 ? P.dg : P.dgp + (int64_t)(j - 1) * P.S * P.planeD) + s * P.planeD;
         const auto& cs = as_constant(g.crt)->set[P.S - 1];
         t.m = cs.m[s];
         t.minv = cs.minv[s];
@@ -181,15 +185,22 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
         c.a += C::STEP;
         c.b += C::STEP;
     };
-    Item cur = decode(w);
+    Item cur = decode(item(w));
+    w += gridDim.x;
+    GItem ahead = item(min(w, n - 1));
     chain_start<C>(smem, 0, cur.KT, stage(cur, 0), stage(cur, 1));  // later items' stages arrive through the chain
     int base = 0;  // ring slot of the current item's stage 0
     for (;;) {
-        const int64_t w2 = w + gridDim.x;
-        const bool more = w2 < g.n;
+        const bool more = w < n;
         Item nxt = cur;
-        if (more) nxt = decode(w2);
-        auto entry = [&] { return NextSrc{stage(nxt, 0), stage(nxt, 1)}; };
+        auto entry = [&] {
+            if (more) {
+                nxt = decode(ahead);
+                w += gridDim.x;
+                ahead = item(min(w, n - 1));
+            }
+            return NextSrc{stage(nxt, 0), stage(nxt, 1)};
+        };
         const int64_t row0 = (int64_t)cur.tm * C::BM + wm * C::WTM, col0 = (int64_t)cur.tn * C::BN + wn * C::WTN;
         for_part<C>(
             cur.M - row0, cur.N - col0,
@@ -202,7 +213,6 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
             [&] { mainloop_idle<C>(smem, base, cur.KT, stage(cur, 2), step, entry); });
         if (!more) break;
         base = (base + cur.KT) & 1;
-        w = w2;
         cur = nxt;
     }
     wait_vmcnt<0>();  // no direct load in flight into LDS when the workgroup leaves

@@ -45,12 +45,14 @@ struct S2Args {
     const int8_t* A;
     const int8_t* B;
     int64_t M, N, Mp, Np, Kp;
-    int S, KT, tiles_m, tiles_n;
-    int tm0;               // first tile row: the launch covers tile rows [tm0, tm0 + tiles_m)
+    int S, KT;
+    TileOrder order;       // of the tile rows [tm0, tm0 + order.tiles_m)
+    int tm0;
     void* out;             // digits or int32 planes
     const CrtSet* crt;     // device copy (m, minv, bias used)
     // SPLIT only: items [0, whole) run whole, the `tail` others in `parts` parts of kts K steps
-    int64_t whole, tail;
+    uint32_t items, whole, tail;
+    FastDiv by_tail;
     int parts, kts;
     uint8_t* part;         // partial tiles of parts 1..
 };
@@ -61,34 +63,34 @@ struct S2Args {
 template <class C, bool DIGITS, bool SPLIT = false>
 __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
     __shared__ __attribute__((aligned(1024))) int8_t smem[C::LDS_BYTES];
-    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n, total = tiles * p.S;
-    const int64_t items = SPLIT ? p.whole + p.tail * p.parts : total;
-    int64_t w = blockIdx.x;
-    if (w >= items) return;  // whole workgroup leaves together
+    uint32_t w = blockIdx.x;
+    if (w >= p.items) return;  // whole workgroup leaves together
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave_part<C>(wave).m, wn = wave_part<C>(wave).n;
     struct Item {
         int s, tm, tn, j, k0, KT;
-        int64_t l;
+        uint32_t l;
         StageSrc src;  // this wave's blocks of stage 0
         uint32_t m, minv, bias;
     };
-    auto decode = [&](int64_t wi) {
+    auto decode = [&](uint32_t wi) {
         Item t;
-        int64_t l = SPLIT && wi >= p.whole ? p.whole + xcd_remap(wi - p.whole, items - p.whole)
-                                           : xcd_remap(wi, SPLIT ? p.whole : items);
+        uint32_t l = SPLIT && wi >= p.whole ? p.whole + xcd_remap(wi - p.whole, p.items - p.whole)
+                                            : xcd_remap(wi, SPLIT ? p.whole : p.items);
         t.j = 0;
         t.k0 = 0;
         t.KT = p.KT;
-        t.l = l;
         if (SPLIT && l >= p.whole) {
-            t.j = (int)((l - p.whole) / p.tail);
-            t.l = l -= (int64_t)t.j * p.tail;
+            uint32_t item;
+            t.j = (int)div_fast(l - p.whole, p.by_tail, item);
+            l = p.whole + item;
             t.k0 = t.j * p.kts;
             t.KT = min(p.kts, p.KT - t.k0);
         }
-        t.s = (int)(l / tiles);
-        grouped_tile<C>(l - (int64_t)t.s * tiles, p.tiles_m, p.tiles_n, t.tm, t.tn);
+        t.l = l;
+        uint32_t tile;
+        t.s = (int)div_fast(l, p.order.tiles, tile);
+        grouped_tile<C>(tile, p.order, t.tm, t.tn);
         t.tm += p.tm0;
         // tile (tm, tn) starts at block-row tm*BM/32 of the fragment-tiled planes (BM*Kp bytes)
         t.src = wave_src<C>(p.A + (int64_t)t.s * p.Mp * p.Kp + (int64_t)t.tm * C::BM * p.Kp + (int64_t)t.k0 * C::STEP,
@@ -113,7 +115,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
     int base = 0;  // ring slot of the current item's stage 0
     for (;;) {
         w += gridDim.x;
-        const bool more = w < items;
+        const bool more = w < p.items;
         Item nxt = cur;
         auto entry = [&] {
             if (more) nxt = decode(w);
@@ -130,7 +132,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
                 mainloop_chain<P>(acc, smem, base, cur.KT, stage(cur, 2), step, entry);
                 if (DIGITS) {
                     const bool part = SPLIT && cur.j > 0;  // a partial tile: the blocks of one tile, row-major
-                    uint8_t* plane = part ? p.part + ((cur.j - 1) * p.tail + cur.l - p.whole) * kTileBytes
+                    uint8_t* plane = part ? p.part + (int64_t)((cur.j - 1) * p.tail + cur.l - p.whole) * kTileBytes
                                           : reinterpret_cast<uint8_t*>(p.out) + (int64_t)s * p.Mp * p.Np;
                     store_digits<P, false>(acc, plane, part ? C::BN : p.Np, part ? wm * C::WTM : row0,
                                            part ? wn * C::WTN : col0, p.M, p.N, cur.m, cur.minv, lane);
@@ -161,7 +163,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
 // Scheme I
 // ------------------------------------------------------------------------------------------
 struct Claims {
-    int64_t w, w1;  // positions of the current and the next item
+    uint32_t w, w1;  // positions of the current and the next item
 };
 
 // First two positions of a workgroup.  Dynamic order: the first position is the workgroup's index
@@ -180,7 +182,7 @@ __device__ __forceinline__ Claims first_claims(unsigned* queue, int xcd, unsigne
         c.w1 = s_pos[1];
     } else {
         c.w = blockIdx.x;
-        c.w1 = 2 * (int64_t)gridDim.x - 1 - c.w;
+        c.w1 = 2 * gridDim.x - 1 - c.w;
     }
     return c;
 }
@@ -188,7 +190,7 @@ __device__ __forceinline__ Claims first_claims(unsigned* queue, int xcd, unsigne
 // Position of the item after next, from the ticket thread 0 took (dynamic order).  Every wave read
 // s_pos[1] at the previous publication and has passed the current item's barriers since; the
 // barrier here makes the new value visible.
-__device__ __forceinline__ int64_t publish_claim(unsigned ticket, unsigned* s_pos) {
+__device__ __forceinline__ uint32_t publish_claim(unsigned ticket, unsigned* s_pos) {
     if (threadIdx.x == 0) s_pos[1] = (gridDim.x >> 3) + ticket;
     wait_lgkmcnt0();
     block_sync_lds();
@@ -199,8 +201,11 @@ struct S1Args {
     const int8_t* A;
     const int8_t* B;
     int64_t M, N, Mp, Np, Kp;
-    int S, KT, tiles_m, tiles_n, beta;
-    int tm0;                 // blocked form: the launch covers tile rows [tm0, tm0 + tiles_m)
+    int S, KT;
+    TileOrder order;         // of the tile rows [tm0, tm0 + order.tiles_m)
+    int tm0;                 // blocked form only, else 0
+    FastDiv by_KT;
+    FastDiv by_share, by_share1;  // an XCD's share of the tiles, rounded down, and one more (dynamic order)
     int32_t* T;              // group products: int32 [S][M][N], or blocked [planes][Mp][Np]
     unsigned* queue;         // 8 work counters, zero at launch (dynamic order), or null (static order)
 };
@@ -216,11 +221,13 @@ template <class C>
 struct S1Walk {
     int64_t wrapA, wrapB;  // from a pair's last stage to the next pair's first
     int KT;
+    FastDiv by_KT;
     __device__ __forceinline__ S1Walk(const S1Args& p)
-        : wrapA(p.Mp * p.Kp - (int64_t)(p.KT - 1) * C::STEP), wrapB(-p.Np * p.Kp - (int64_t)(p.KT - 1) * C::STEP), KT(p.KT) {}
+        : wrapA(p.Mp * p.Kp - (int64_t)(p.KT - 1) * C::STEP), wrapB(-p.Np * p.Kp - (int64_t)(p.KT - 1) * C::STEP), KT(p.KT), by_KT(p.by_KT) {}
     // Stage i of group g; abase, bbase: the wave's blocks of the tile in slice 1's planes.
     __device__ __forceinline__ S1Cursor at(const StageSrc& base, const S1Args& p, int g, int i) const {
-        const int pr = i / KT, kt = i - pr * KT;  // s = pr + 1, t = g - s
+        uint32_t k;
+        const int pr = (int)div_fast((uint32_t)i, by_KT, k), kt = (int)k;  // s = pr + 1, t = g - s
         return S1Cursor{base.a + pr * p.Mp * p.Kp + (int64_t)kt * C::STEP,
                         base.b + (g - pr - 2) * p.Np * p.Kp + (int64_t)kt * C::STEP, kt};
     }
@@ -256,9 +263,8 @@ struct S1List {
 template <class C>
 __global__ void __launch_bounds__(C::NT) k_igemm_s1(S1Args p) {
     __shared__ __attribute__((aligned(1024))) int8_t smem[C::LDS_BYTES];
-    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
     int tm, tn;
-    grouped_tile<C>(xcd_remap(blockIdx.x, tiles), p.tiles_m, p.tiles_n, tm, tn);
+    grouped_tile<C>(xcd_remap(blockIdx.x, p.order.tiles.d), p.order, tm, tn);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave_part<C>(wave).m, wn = wave_part<C>(wave).n;
     const StageSrc src =
@@ -310,11 +316,12 @@ template <class C>
 __global__ void __launch_bounds__(C::NT) k_igemm_s1g(S1Args p, S1List list) {
     __shared__ __attribute__((aligned(1024))) int8_t smem[C::LDS_BYTES];
     __shared__ unsigned s_pos[2];
-    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
+    const uint32_t tiles = p.order.tiles.d;
     const bool dyn = p.queue != nullptr;
-    const int xcd = blockIdx.x & 7;
-    const int64_t t0 = dyn ? tiles * xcd / 8 : 0, ntile = dyn ? tiles * (xcd + 1) / 8 - t0 : tiles;
-    const int64_t nwork = ntile * list.n;
+    const uint32_t xcd = blockIdx.x & 7;
+    const uint32_t t0 = dyn ? tiles * xcd / 8 : 0, ntile = dyn ? tiles * (xcd + 1) / 8 - t0 : tiles;
+    const FastDiv by_ntile = !dyn ? p.order.tiles : ntile == p.by_share.d ? p.by_share : p.by_share1;
+    const uint32_t nwork = ntile * list.n;
     Claims c = first_claims(p.queue, xcd, s_pos);
     if (c.w >= nwork) return;  // whole workgroup leaves together
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -323,14 +330,15 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1g(S1Args p, S1List list) {
         int g, tm, tn, i0, nit, plane;
         StageSrc src;
     };
-    auto decode = [&](int64_t k) {
+    auto decode = [&](uint32_t k) {
         Item t;
-        const int e = (int)(k / ntile);
+        uint32_t tile;
+        const uint32_t e = div_fast(k, by_ntile, tile);
         t.g = list.e[e].g;
         t.plane = list.e[e].plane;
         t.i0 = list.e[e].i0;
         t.nit = list.e[e].nit;
-        grouped_tile<C>(t0 + (k - (int64_t)e * ntile), p.tiles_m, p.tiles_n, t.tm, t.tn);
+        grouped_tile<C>(t0 + tile, p.order, t.tm, t.tn);
         t.tm += p.tm0;
         t.src = wave_src<C>(p.A + (int64_t)t.tm * C::BM * p.Kp, p.B + (int64_t)t.tn * C::BN * p.Kp, p.Kp, wave,
                             (int)((p.M - (int64_t)t.tm * C::BM - 1) >> 5), (int)((p.N - (int64_t)t.tn * C::BN - 1) >> 5));
@@ -366,7 +374,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1g(S1Args p, S1List list) {
             },
             [&] { mainloop_idle<C>(smem, base, cur.nit, stage2, walk, entry); });  // never thread 0's wave: part (0, 0)
         if (!more) break;
-        const int64_t w2 = dyn ? publish_claim(ticket, s_pos) : c.w + 2 * (int64_t)gridDim.x;
+        const uint32_t w2 = dyn ? publish_claim(ticket, s_pos) : c.w + 2 * gridDim.x;
         base = (base + cur.nit) & 1;
         c.w = c.w1;
         c.w1 = w2;
@@ -409,18 +417,23 @@ hipError_t launch_igemm_s2(const Dims& d, const int8_t* A_sl, const int8_t* B_sl
     const int tiles_m = (int)((d.M + CfgS2::BM - 1) / CfgS2::BM);
     if (tm0 < 0 || tm0 > tiles_m) return hipErrorInvalidValue;
     p.tm0 = tm0;
-    p.tiles_m = tms < 0 ? tiles_m - tm0 : std::min(tms, tiles_m - tm0);
-    p.tiles_n = (int)((d.N + CfgS2::BN - 1) / CfgS2::BN);
+    const int rows = tms < 0 ? tiles_m - tm0 : std::min(tms, tiles_m - tm0);
+    const int tiles_n = (int)((d.N + CfgS2::BN - 1) / CfgS2::BN);
+    p.order = tile_order(rows, tiles_n, CfgS2::GM);
     p.out = out;
     p.crt = crt_dev;
-    int64_t total = (int64_t)p.tiles_m * p.tiles_n * d.S;
-    p.whole = split ? plan->whole : total;
-    p.tail = total - p.whole;
+    int64_t total = (int64_t)rows * tiles_n * d.S;
+    const int64_t whole = split ? plan->whole : total, tail = total - whole;
     p.parts = split ? plan->parts : 1;
     p.kts = split ? plan->kts : p.KT;
     p.part = static_cast<uint8_t*>(out) + (int64_t)d.S * d.Mp * d.Np;
-    if (split) total = p.whole + p.tail * p.parts;
+    if (split) total = whole + tail * p.parts;
     if (total == 0) return hipSuccess;
+    if (total > INT32_MAX) return hipErrorInvalidValue;  // 2^47 bytes of digits
+    p.items = (uint32_t)total;
+    p.whole = (uint32_t)whole;
+    p.tail = (uint32_t)tail;
+    p.by_tail = fast_div(tail);
     unsigned grid = 0;
     if (hipError_t e = persistent_grid(total, grid)) return e;
     if (split)
@@ -432,7 +445,8 @@ hipError_t launch_igemm_s2(const Dims& d, const int8_t* A_sl, const int8_t* B_sl
     return hipGetLastError();
 }
 
-static S1Args make_s1(const Dims& d, int beta, const int8_t* A_sl, const int8_t* B_sl) {
+template <class C>
+static S1Args make_s1(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, int tm0, int rows) {
     S1Args p;
     p.A = A_sl;
     p.B = B_sl;
@@ -442,25 +456,22 @@ static S1Args make_s1(const Dims& d, int beta, const int8_t* A_sl, const int8_t*
     p.Np = d.Np;
     p.Kp = d.Kp;
     p.S = d.S;
-    p.KT = (int)(d.Kp / CfgS1::BK);
-    p.tiles_m = (int)((d.M + CfgS1::BM - 1) / CfgS1::BM);
-    p.tiles_n = (int)((d.N + CfgS1::BN - 1) / CfgS1::BN);
-    p.beta = beta;
+    p.KT = (int)(d.Kp / C::BK);
+    p.order = tile_order(rows, (d.N + C::BN - 1) / C::BN, C::GM);
+    p.tm0 = tm0;
+    p.by_KT = fast_div(p.KT);
+    p.by_share = fast_div(p.order.tiles.d / 8);
+    p.by_share1 = fast_div(p.order.tiles.d / 8 + 1);
     p.T = nullptr;
     p.queue = nullptr;
-    p.tm0 = 0;
     return p;
 }
 
 hipError_t launch_igemm_s1_blocked(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, int32_t* T, hipStream_t st,
                                    const S1Plan& plan, unsigned* queue, int tm0, int tms) {
-    S1Args p = make_s1(d, 7, A_sl, B_sl);
-    p.KT = (int)(d.Kp / CfgS2::BK);
     const int tiles_m = (int)((d.M + CfgS2::BM - 1) / CfgS2::BM);
     if (tm0 < 0 || tm0 > tiles_m) return hipErrorInvalidValue;
-    p.tm0 = tm0;
-    p.tiles_m = tms < 0 ? tiles_m - tm0 : std::min(tms, tiles_m - tm0);
-    p.tiles_n = (int)((d.N + CfgS2::BN - 1) / CfgS2::BN);
+    S1Args p = make_s1<CfgS2>(d, A_sl, B_sl, tm0, tms < 0 ? tiles_m - tm0 : std::min(tms, tiles_m - tm0));
     p.T = T;
     S1List list;
     list.n = 0;
@@ -475,8 +486,9 @@ hipError_t launch_igemm_s1_blocked(const Dims& d, const int8_t* A_sl, const int8
     std::stable_sort(list.e, list.e + list.n, [](const S1Entry& a, const S1Entry& b) {
         return a.nit != b.nit ? a.nit > b.nit : a.g > b.g;
     });
-    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n, total = tiles * list.n;
+    const int64_t tiles = (int64_t)p.order.tiles_m * p.order.tiles_n, total = tiles * list.n;
     if (total == 0) return hipSuccess;
+    if (total > INT32_MAX) return hipErrorInvalidValue;  // 2^49 bytes of products
     unsigned grid = 0;
     if (hipError_t e = persistent_grid(total, grid)) return e;
     // A workgroup of the dynamic order claims two positions before it starts, so with fewer than two
@@ -489,9 +501,9 @@ hipError_t launch_igemm_s1_blocked(const Dims& d, const int8_t* A_sl, const int8
 
 hipError_t launch_igemm_s1_groups(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, int32_t* T,
                                   hipStream_t st) {
-    S1Args p = make_s1(d, 7, A_sl, B_sl);
+    S1Args p = make_s1<CfgS1>(d, A_sl, B_sl, 0, (int)((d.M + CfgS1::BM - 1) / CfgS1::BM));
     p.T = T;
-    const int64_t grid = (int64_t)p.tiles_m * p.tiles_n;
+    const int64_t grid = (int64_t)p.order.tiles_m * p.order.tiles_n;
     if (grid == 0) return hipSuccess;
     k_igemm_s1<CfgS1><<<(unsigned)grid, CfgS1::NT, 0, st>>>(p);
     return hipGetLastError();

@@ -153,6 +153,24 @@ hipError_t launch_one_pass(int scheme, const Dims& d, int offset, const Operand&
 hipError_t launch_unpack_A(const Dims& d, const int8_t* A_sl, int8_t* out, hipStream_t st);
 hipError_t launch_unpack_B(const Dims& d, const int8_t* B_sl, int8_t* out, hipStream_t st);
 
+// Division of 32-bit numbers by d in five scalar instructions (div_fast): inv = floor(2^32 / d), so that
+// mulhi(n, inv) is the quotient or one less (for d = 1, inv = 2^32 - 1 gives n - 1).
+struct FastDiv {
+    uint32_t d, inv;
+};
+inline FastDiv fast_div(int64_t d) {
+    return FastDiv{(uint32_t)d, d > 1 ? (uint32_t)((uint64_t(1) << 32) / (uint64_t)d) : UINT32_MAX};
+}
+// The order of a GEMM's tiles: groups of gm tile rows (IgemmCfg::GM), column by column (grouped_tile).
+struct TileOrder {
+    int32_t tiles_m, tiles_n;
+    FastDiv tiles, group, last;  // all tiles; a group's tiles; the rows of the last, smaller group
+};
+inline TileOrder tile_order(int64_t tiles_m, int64_t tiles_n, int gm) {
+    return TileOrder{(int32_t)tiles_m, (int32_t)tiles_n, fast_div(tiles_m * tiles_n), fast_div(gm * tiles_n),
+                     fast_div(tiles_m % gm ? tiles_m % gm : gm)};
+}
+
 // How a single call's GEMM is cut into items (plan_host.cpp).
 constexpr int kS2TileRows = 256;
 constexpr int kTileBytes = kS2TileRows * kS2TileRows;  // digits of one tile
