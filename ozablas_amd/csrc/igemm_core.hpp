@@ -202,7 +202,22 @@ __device__ __forceinline__ void interleave_hint_last() {
 //   `cur` is this item's stage 2 (if it has one) and step(cur) moves it on by a stage.  entry() runs after
 //   the first barrier and returns the next item's sources.  The source is selected, so no branch
 //   separates the loads from the MFMAs they are interleaved with.
+//
+//   With Q = STAGES > 2 slots every item has at least Q stages; Q stages are issued before an item starts,
+//   stage i + Q when stage i has been read, `cur` starts at stage Q, entry() returns the next item's stage 0,
+//   and the waits leave the Q - 2 (at an item's start Q - 1) later stages outstanding.
 // ------------------------------------------------------------------------------------------
+// More than two slots.
+template <class C, class Cur, class Step>
+__device__ __forceinline__ void chain_start_deep(int8_t* smem, Cur cur, Step step) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int i = 0; i < C::STAGES; ++i) {
+        issue_stage<C>(smem + i * C::STAGE_BYTES, cur.a, cur.b, wave, lane);
+        step(cur);
+    }
+}
+
 template <class C>
 __device__ __forceinline__ void chain_start(int8_t* smem, int base, int nit, const StageSrc& s0, const StageSrc& s1) {
     static_assert(C::STAGES == 2, "the chain keeps two slots");
@@ -212,45 +227,65 @@ __device__ __forceinline__ void chain_start(int8_t* smem, int base, int nit, con
     if (nit >= 2) issue_stage<C>(smem + ((base + 1) & 1) * C::STAGE_BYTES, s1.a, s1.b, wave, lane);
 }
 
+// The source of the next chain stage: this item's at cur, or the next item's at nx; moves it on.
+template <class C, class Cur, class Next, class Step>
+__device__ __forceinline__ void next_stage(bool own, Cur& cur, Next& nx, Step step, const int8_t*& a, const int8_t*& b) {
+    if constexpr (C::STAGES == 2) {
+        a = own ? cur.a : nx.s0.a;
+        b = own ? cur.b : nx.s0.b;
+        step(cur);
+    } else {
+        a = own ? cur.a : nx.a;
+        b = own ? cur.b : nx.b;
+        if (own) step(cur);
+        else step(nx);
+    }
+}
+template <class C, class Next>
+__device__ __forceinline__ auto last_next(const Next& nx) {
+    if constexpr (C::STAGES == 2) return nx.s1;
+    else return nx;
+}
+
 template <class C, class Cur, class Step, class Entry>
 __device__ __forceinline__ void mainloop_chain(v16i (&acc)[C::FM][C::FN], int8_t* smem, int base, int nit, Cur cur,
                                                Step step, Entry entry) {
-    static_assert(C::STAGES == 2, "the chain keeps two slots");
-    constexpr int KSTEPS = C::BK / 32;
+    constexpr int KSTEPS = C::BK / 32, Q = C::STAGES;
+    static_assert((Q & (Q - 1)) == 0, "slots by a mask");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave_part<C>(wave).m, wn = wave_part<C>(wave).n;
-    auto slot = [&](int i) { return smem + ((base + i) & 1) * C::STAGE_BYTES; };
+    auto slot = [&](int i) { return smem + ((base + i) & (Q - 1)) * C::STAGE_BYTES; };
     auto lds_barrier = [] {
         wait_lgkmcnt0();  // this wave's LDS reads are done
         block_sync_lds();
     };
     Frags<C> f[2];
-    // Stage 0 is the oldest of this wave's outstanding operations, and LPS loads of chain stage 1 and the
+    // Stage 0 is the oldest of this wave's outstanding operations; the loads of Q - 1 chain stages and the
     // previous item's stores (if any) follow it.
-    if (nit >= 2) wait_vmcnt<C::LPS>();
+    if (Q > 2 || nit >= 2) wait_vmcnt<(Q - 1) * C::LPS>();
     else wait_vmcnt<0>();
     lds_barrier();
     load_frags<C>(f[0], slot(0), 0, wm, wn, lane);
-    const NextSrc nx = entry();
-    if (nit == 1) issue_stage<C>(slot(1), nx.s0.a, nx.s0.b, wave, lane);
+    auto nx = entry();
+    if constexpr (Q == 2)
+        if (nit == 1) issue_stage<C>(slot(1), nx.s0.a, nx.s0.b, wave, lane);
     for (int it = 0; it + 1 < nit; ++it) {
         const int8_t* now = slot(it);
-        const bool own = it + 2 < nit;  // chain stage it + 2: this item's, or the next item's stage 0
-        const int8_t* pa = own ? cur.a : nx.s0.a;
-        const int8_t* pb = own ? cur.b : nx.s0.b;
-        step(cur);
+        const bool own = it + Q < nit;  // chain stage it + Q: this item's, or the next item's
+        const int8_t *pa, *pb;
+        next_stage<C>(own, cur, nx, step, pa, pb);
 #pragma unroll
         for (int kk = 0; kk + 1 < KSTEPS; ++kk) {
             load_frags<C>(f[(kk + 1) & 1], now, kk + 1, wm, wn, lane);
             mma_frags<C>(acc, f[kk & 1]);
             interleave_hint<C>();
         }
-        wait_vmcnt<0>();  // stage it+1, issued one iteration ago
+        wait_vmcnt<(Q - 2) * C::LPS>();  // stage it+1, issued Q - 1 iterations ago
         lds_barrier();
         load_frags<C>(f[KSTEPS & 1], slot(it + 1), 0, wm, wn, lane);
         __builtin_amdgcn_s_setprio(1);
-        issue_stage<C>(slot(it + 2), pa, pb, wave, lane);
+        issue_stage<C>(slot(it + Q), pa, pb, wave, lane);
         mma_frags<C>(acc, f[(KSTEPS - 1) & 1]);
         interleave_hint_last<C>();
         __builtin_amdgcn_s_setprio(0);
@@ -261,7 +296,7 @@ __device__ __forceinline__ void mainloop_chain(v16i (&acc)[C::FM][C::FN], int8_t
             for (int i = 0; i < C::FN; ++i) f[0].b[i] = f[1].b[i];
         }
     }
-    {  // last iteration: its slot is freed at the barrier for chain stage nit + 1
+    {  // last iteration: its slot is freed at the barrier for chain stage nit + Q - 1
         const int8_t* now = slot(nit - 1);
 #pragma unroll
         for (int kk = 0; kk + 1 < KSTEPS; ++kk) {
@@ -271,7 +306,7 @@ __device__ __forceinline__ void mainloop_chain(v16i (&acc)[C::FM][C::FN], int8_t
         }
         lds_barrier();
         __builtin_amdgcn_s_setprio(1);
-        issue_stage<C>(slot(nit + 1), nx.s1.a, nx.s1.b, wave, lane);
+        issue_stage<C>(slot(nit + Q - 1), last_next<C>(nx).a, last_next<C>(nx).b, wave, lane);
         mma_frags<C>(acc, f[(KSTEPS - 1) & 1]);
         __builtin_amdgcn_s_setprio(0);
     }
@@ -283,23 +318,23 @@ template <class C, class Cur, class Step, class Entry>
 __device__ __forceinline__ void mainloop_idle(int8_t* smem, int base, int nit, Cur cur, Step step, Entry entry) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    auto slot = [&](int i) { return smem + ((base + i) & 1) * C::STAGE_BYTES; };
-    if (nit >= 2) wait_vmcnt<C::LPS>();
+    constexpr int Q = C::STAGES;
+    auto slot = [&](int i) { return smem + ((base + i) & (Q - 1)) * C::STAGE_BYTES; };
+    if (Q > 2 || nit >= 2) wait_vmcnt<(Q - 1) * C::LPS>();
     else wait_vmcnt<0>();
     block_sync_lds();
-    const NextSrc nx = entry();
-    if (nit == 1) issue_stage<C>(slot(1), nx.s0.a, nx.s0.b, wave, lane);
+    auto nx = entry();
+    if constexpr (Q == 2)
+        if (nit == 1) issue_stage<C>(slot(1), nx.s0.a, nx.s0.b, wave, lane);
     for (int it = 0; it + 1 < nit; ++it) {
-        const bool own = it + 2 < nit;
-        const int8_t* pa = own ? cur.a : nx.s0.a;
-        const int8_t* pb = own ? cur.b : nx.s0.b;
-        step(cur);
-        wait_vmcnt<0>();
+        const int8_t *pa, *pb;
+        next_stage<C>(it + Q < nit, cur, nx, step, pa, pb);
+        wait_vmcnt<(Q - 2) * C::LPS>();
         block_sync_lds();
-        issue_stage<C>(slot(it + 2), pa, pb, wave, lane);
+        issue_stage<C>(slot(it + Q), pa, pb, wave, lane);
     }
     block_sync_lds();
-    issue_stage<C>(slot(nit + 1), nx.s1.a, nx.s1.b, wave, lane);
+    issue_stage<C>(slot(nit + Q - 1), last_next<C>(nx).a, last_next<C>(nx).b, wave, lane);
 }
 
 // Edge tiles.  A wave that computes only the first FM_ x FN_ fragments of its part: the padding's products

@@ -111,7 +111,8 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         c.b += C::STEP;
     };
     Item cur = decode(w);
-    chain_start<C>(smem, 0, cur.KT, stage(cur, 0), stage(cur, 1));
+    if constexpr (C::STAGES == 2) chain_start<C>(smem, 0, cur.KT, stage(cur, 0), stage(cur, 1));
+    else chain_start_deep<C>(smem, cur.src, step);
     int base = 0;  // ring slot of the current item's stage 0
     for (;;) {
         w += gridDim.x;
@@ -119,7 +120,8 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         Item nxt = cur;
         auto entry = [&] {
             if (more) nxt = decode(w);
-            return NextSrc{stage(nxt, 0), stage(nxt, 1)};
+            if constexpr (C::STAGES == 2) return NextSrc{stage(nxt, 0), stage(nxt, 1)};
+            else return nxt.src;
         };
         const int s = cur.s;
         const int64_t row0 = (int64_t)cur.tm * C::BM + wm * C::WTM, col0 = (int64_t)cur.tn * C::BN + wn * C::WTN;
@@ -129,7 +131,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
                 v16i acc[P::FM][P::FN];
                 if (DIGITS) fill_acc<P>(acc, (int)cur.bias);
                 else zero_acc<P>(acc);
-                mainloop_chain<P>(acc, smem, base, cur.KT, stage(cur, 2), step, entry);
+                mainloop_chain<P>(acc, smem, base, cur.KT, stage(cur, C::STAGES), step, entry);
                 if (DIGITS) {
                     const bool part = SPLIT && cur.j > 0;  // a partial tile: the blocks of one tile, row-major
                     uint8_t* plane = part ? p.part + (int64_t)((cur.j - 1) * p.tail + cur.l - p.whole) * kTileBytes
@@ -151,9 +153,9 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
                         }
                 }
             },
-            [&] { mainloop_idle<C>(smem, base, cur.KT, stage(cur, 2), step, entry); });
+            [&] { mainloop_idle<C>(smem, base, cur.KT, stage(cur, C::STAGES), step, entry); });
         if (!more) break;
-        base = (base + cur.KT) & 1;
+        base = (base + cur.KT) & (C::STAGES - 1);
         cur = nxt;
     }
     wait_vmcnt<0>();  // no direct load in flight into LDS when the workgroup leaves
@@ -400,6 +402,19 @@ hipError_t persistent_grid(int64_t total, unsigned& grid) {
 using CfgS2 = IgemmCfgS2;
 using CfgS1 = IgemmCfgS1;
 
+// Four slots of 64 K-bytes instead of two of 128: three stages (96 KiB per CU) on their way from memory while
+// one is computed, instead of one of 64 KiB, for twice the barriers.  That pays where the operand planes come
+// from memory (past some 90 MB, that is with K past a few thousand) and each of their bytes meets few products.
+// Calls, us, two slots / four: 600^2 x 16384, S = 12 227 / 206; 512^2 x 32768, S = 14 327 / 317; 1024^2 x 16384,
+// S = 12 390 / 366; 300 x 8000 x 2048, S = 12 189 / 178; 1500^2 x 8192, S = 12 355 / 344.  Beyond the lines:
+// 2048^3, S = 6 93 / 96; 2100^3, S = 15 216 / 220; 8192^3, S = 17 8459 / 8619; 1800^2 x 8192, S = 12 463 / 467;
+// 1200^2 x 3000, S = 12 (86 MB) 109 / 110; 500^2 x 3000, S = 14 (45 MB) 53.9 / 54.5.
+using CfgS2Deep = IgemmCfg<256, 256, 64, 4, 2, 4, 8>;
+constexpr int64_t kDeepBytes = 90000000, kDeepWidth = 800;
+static bool deep_ring(const Dims& d) {
+    return d.S * (d.Mp + d.Np) * d.Kp >= kDeepBytes && d.M * d.N <= kDeepWidth * (d.M + d.N) && d.Kp >= 256;
+}
+
 hipError_t launch_igemm_s2(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, S2Out mode, void* out,
                            const CrtSet* crt_dev, hipStream_t st, int tm0, int tms, const S2Plan* plan) {
     const bool split = plan && plan->parts > 1;
@@ -436,6 +451,14 @@ hipError_t launch_igemm_s2(const Dims& d, const int8_t* A_sl, const int8_t* B_sl
     p.by_tail = fast_div(tail);
     unsigned grid = 0;
     if (hipError_t e = persistent_grid(total, grid)) return e;
+    if (mode == S2Out::Digits && deep_ring(d) && (int64_t)p.parts * p.kts - p.KT <= p.kts - 2) {
+        constexpr int kStages = CfgS2::BK / CfgS2Deep::BK;
+        p.KT *= kStages;
+        p.kts *= kStages;
+        if (split) k_igemm_s2<CfgS2Deep, true, true><<<grid, CfgS2Deep::NT, 0, st>>>(p);
+        else k_igemm_s2<CfgS2Deep, true><<<grid, CfgS2Deep::NT, 0, st>>>(p);
+        return hipGetLastError();
+    }
     if (split)
         k_igemm_s2<CfgS2, true, true><<<grid, CfgS2::NT, 0, st>>>(p);
     else if (mode == S2Out::Digits)
