@@ -399,7 +399,7 @@ int build_plan(const GroupModel& model, int n, const size_t* M, const size_t* N,
         P.slA = ((P.M + 31) / 32) * (P.Kp / 128);  // blocks holding a logical row (see make_slice_op)
         P.slB = ((P.N + 63) / 64) * (P.Kp / 128);
         P.psA = P.psB = 0;
-        if (P.Kp <= core::kPassMaxKp) {  // short K: steps 1 and 2 in one pass (k_group_pass)
+        if (P.Kp <= core::kGroupPassMaxKp) {  // short K: steps 1 and 2 in one pass (k_group_pass)
             P.psA = core::pass_row_blocks(P.M, core::group_pass_rows(P.Kp));
             P.psB = core::pass_row_blocks(P.N, core::group_pass_rows(P.Kp));
             P.nblkA = P.nblkB = 0;

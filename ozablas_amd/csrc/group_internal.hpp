@@ -36,7 +36,7 @@ struct GroupProblem {
     int32_t split, kbs;           // K splits of the GEMM (1: none), 128-byte K blocks per split
     int64_t chunksA, nblkA, colblkB, nblkB;  // step-1 blocks of A and B
     int64_t slA, slB;                        // step-2 blocks of A and B
-    // Kp <= core::kPassMaxKp: blocks of A and of B with steps 1 and 2 in one pass (nblk*, sl* = 0 then)
+    // Kp <= core::kGroupPassMaxKp: blocks of A and of B with steps 1 and 2 in one pass (nblk*, sl* = 0 then)
     int64_t psA, psB;
 };
 

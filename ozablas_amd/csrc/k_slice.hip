@@ -122,10 +122,17 @@ hipError_t launch_slice_s1(const Dims& d, int beta, const Operand& A, const Oper
 // Not when one more round of 1024-thread blocks would hold a few blocks only, which take as long as a full
 // round, unless there are many rounds: 200 x 8000 x 900, S = 16 (514 row blocks) 120 us per call in one
 // pass, 114 us in two kernels; 200 x 7800 x 900 (502) 102 against 109, 200 x 6000 x 900 (389) 88 against 93.
+// Past K = 2048 (8 rows per block) up to one round, or two that are well filled; us per call in one pass and in
+// two kernels: 512^2 x 4096, S = 14 (128 row blocks) 55 and 62; 1000^2 x 3000, S = 12 (250) 73 and 85;
+// 1300 x 700 x 3500, S = 16 (251) 109 and 122; 1500 x 900 x 4000, S = 12 (304) 147 and 144; 1500^2 x 3000, S = 10
+// (376) 131 and 132; 3000 x 1000 x 2050, S = 16 (504) 161 and 173; 2100^2 x 2100, S = 15 (528) 220 and 220; 4096^3,
+// S = 17 (1024) 1261 and 1249; 300 x 8000 x 2304, S = 12 (1040) 228 and 200.  Past K = 4096 blocks of 4 rows would be
+// needed: 512^2 x 8192, S = 14 124 and 98.
 bool one_pass(const Dims& d) {
     if (d.Kp > kPassMaxKp) return false;
     const int R = pass_rows(d.Kp);
     const int64_t n = pass_row_blocks(d.M, R) + pass_row_blocks(d.N, R), over = n % kPassResident;
+    if (d.Kp > 2048) return n <= kPassResident || (n >= kPassResident * 11 / 8 && n <= 2 * kPassResident);
     return !(pass_threads(d.Kp) == 1024 && n > kPassResident && n < 4 * kPassResident && over > 0 &&
              over < kPassResident / 8);
 }

@@ -289,7 +289,9 @@ __device__ __forceinline__ void slice_s1_op_block(const SliceOp& o, int64_t K, i
 // the shifts and then the slices of the values it still holds.  Unit u = (row u % R, 16-byte K chunk u / R)
 // of the block; thread t takes units t + T i, i < NU, all of row t % R.  With R = 16 a wave reads a
 // row-contiguous operand in 128-byte runs and writes 256-byte runs of a fragment block; R grows to 64
-// for short K so that the threads have units.  Values and results are those of the separate kernels.
+// for short K so that the threads have units, and is 8 past K = 2048, whose runs of 64 and 128 bytes are
+// the better choice only where the blocks run at once (one_pass).  Values and results are those of the
+// separate kernels.
 // A block's planes may be dealt to `parts` blocks that each read the rows again (part j stores planes
 // [S j / parts, S (j + 1) / parts), part 0 the shifts): more blocks for small operands, whose second
 // reads come from the XCD's L2 (the parts of a row block are 8 block indices apart, on one XCD).
@@ -298,13 +300,13 @@ __device__ __forceinline__ void slice_s1_op_block(const SliceOp& o, int64_t K, i
 // and many threads, not four units in 256 threads (184 registers, 8 waves per CU instead of 16):
 // 2048^3, S = 6 111 us per call in two kernels, 101 in one pass (37 us for the launch with four units in 512
 // threads); 1024^3, S = 16 54 and 45; 8192^2 x 1024, S = 16 1.551 and 1.523 ms; 256^3, S = 4 24 and 15 us.
-constexpr int64_t kPassMaxKp = 2048;
+constexpr int64_t kPassMaxKp = 4096, kGroupPassMaxKp = 2048;
 
 inline int pass_threads(int64_t Kp) { return Kp <= 256 ? 256 : Kp <= 512 ? 512 : 1024; }
 inline int pass_units(int64_t Kp) { return Kp <= 1024 ? 1 : 2; }
 inline int pass_rows(int64_t Kp) {
     int r = 64;
-    while (r > 16 && r * (Kp / 16) > pass_threads(Kp) * pass_units(Kp)) r >>= 1;
+    while (r > 8 && r * (Kp / 16) > pass_threads(Kp) * pass_units(Kp)) r >>= 1;
     return r;
 }
 
@@ -398,7 +400,7 @@ __device__ __forceinline__ void pass_block(const PassOp& o, const PassArgs& g, c
     }
 }
 
-// Grouped problems with Kp <= kPassMaxKp: blocks of 512 threads with up to two units each, any K.  A group's
+// Grouped problems with Kp <= kGroupPassMaxKp: blocks of 512 threads with up to two units each, any K.  A group's
 // launch is bound by memory, not by latency, and two such blocks share a CU, so that one reads while the
 // other computes and writes.  Two units in 1024 threads, one in 512 and four in 512 or 256 were slower (the
 // whole group of 512 problems, M, N, K log-uniform on [64, 2048]: 5.07, 5.15, 5.12 ms; two in 512 4.96 ms for
