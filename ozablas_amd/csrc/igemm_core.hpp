@@ -209,12 +209,12 @@ __device__ __forceinline__ void interleave_hint_last() {
 // ------------------------------------------------------------------------------------------
 // More than two slots.
 template <class C, class Cur, class Step>
-__device__ __forceinline__ void chain_start_deep(int8_t* smem, Cur cur, Step step) {
+__device__ __forceinline__ void chain_start_deep(int8_t* smem, int nit, Cur cur, Step step) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (int i = 0; i < C::STAGES; ++i) {
         issue_stage<C>(smem + i * C::STAGE_BYTES, cur.a, cur.b, wave, lane);
-        step(cur);
+        if (i + 1 < nit) step(cur);
     }
 }
 

@@ -112,7 +112,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
     };
     Item cur = decode(w);
     if constexpr (C::STAGES == 2) chain_start<C>(smem, 0, cur.KT, stage(cur, 0), stage(cur, 1));
-    else chain_start_deep<C>(smem, cur.src, step);
+    else chain_start_deep<C>(smem, cur.KT, cur.src, step);
     int base = 0;  // ring slot of the current item's stage 0
     for (;;) {
         w += gridDim.x;
@@ -415,10 +415,27 @@ static bool deep_ring(const Dims& d) {
     return d.S * (d.Mp + d.Np) * d.Kp >= kDeepBytes && d.M * d.N <= kDeepWidth * (d.M + d.N) && d.Kp >= 256;
 }
 
+// Small calls (S2Plan::edge): 64 x 64 or 128 x 128 tiles, one item per workgroup, two workgroups per CU, four
+// slots.  Few 256 x 256 tiles leave CUs idle, and one of them alone spends more on its epilogue (128 digits
+// per thread) and on waiting for one stage at a time than on the products.  Lines and figures: scheme2_plan.
+using CfgS2Small64 = IgemmCfg<64, 64, 128, 2, 2, 4, 4>;
+using CfgS2Small128 = IgemmCfg<128, 128, 64, 2, 2, 4, 4>;
+template <class C>
+static hipError_t launch_small(const Dims& d, S2Args p, hipStream_t st) {
+    p.order = tile_order((d.M + C::BM - 1) / C::BM, (d.N + C::BN - 1) / C::BN, C::GM);
+    const int64_t items = (int64_t)p.order.tiles_m * p.order.tiles_n * d.S;
+    if (items > INT32_MAX) return hipErrorInvalidValue;
+    p.items = p.whole = (uint32_t)items;
+    p.KT = p.kts = (int)(d.Kp / C::BK);
+    k_igemm_s2<C, true><<<p.items, C::NT, 0, st>>>(p);
+    return hipGetLastError();
+}
+
 hipError_t launch_igemm_s2(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, S2Out mode, void* out,
                            const CrtSet* crt_dev, hipStream_t st, int tm0, int tms, const S2Plan* plan) {
     const bool split = plan && plan->parts > 1;
-    if (split && (mode != S2Out::Digits || tm0 != 0 || tms >= 0)) return hipErrorInvalidValue;
+    const bool small = plan && plan->edge != CfgS2::BM;
+    if ((split || small) && (mode != S2Out::Digits || tm0 != 0 || tms >= 0)) return hipErrorInvalidValue;
     S2Args p;
     p.A = A_sl;
     p.B = B_sl;
@@ -449,6 +466,7 @@ hipError_t launch_igemm_s2(const Dims& d, const int8_t* A_sl, const int8_t* B_sl
     p.whole = (uint32_t)whole;
     p.tail = (uint32_t)tail;
     p.by_tail = fast_div(tail);
+    if (small) return plan->edge == 64 ? launch_small<CfgS2Small64>(d, p, st) : launch_small<CfgS2Small128>(d, p, st);
     unsigned grid = 0;
     if (hipError_t e = persistent_grid(total, grid)) return e;
     if (mode == S2Out::Digits && deep_ring(d) && (int64_t)p.parts * p.kts - p.KT <= p.kts - 2) {

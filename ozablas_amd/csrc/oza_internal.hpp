@@ -177,9 +177,10 @@ constexpr int kTileBytes = kS2TileRows * kS2TileRows;  // digits of one tile
 constexpr int kMaxParts = 32;
 constexpr int kMaxS1Planes = 128;
 // Scheme II: items l (modulus-major, then tile) below `whole` run whole, the others in `parts` parts of
-// `kts` K steps (the last one may be shorter).
+// `kts` K steps (the last one may be shorter).  edge: 64 or 128 for small calls, whose tiles of that size
+// all run whole.
 struct S2Plan {
-    int parts = 1, kts = 0;
+    int edge = kS2TileRows, parts = 1, kts = 0;
     int64_t whole = 0;
 };
 S2Plan scheme2_plan(const Dims& d);

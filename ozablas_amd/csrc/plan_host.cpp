@@ -32,6 +32,24 @@ int64_t tiles_of(const Dims& d) { return div_up(d.M, kS2TileRows) * div_up(d.N, 
 
 }  // namespace
 
+// Tile edge.  Calls, us, with 256 x 256 tiles (in parts where that is the plan) / 128 x 128 / 64 x 64:
+//   64: at most 512 items (two workgroups per CU), and their stages, one item after the other, not past what
+//   parts along K would take: 256^3, S = 4 15.0 / 14.0 / 13.5; 256^2 x 2048, S = 12 36.2 / 30.3 / 26.3;
+//   512^2 x 2048, S = 8 36.7 / 29.9 / 28.2; 256^2 x 12000, S = 16 105 / 97 / 78; 100^2 x 4000, S = 10 43 / 38 / 30;
+//   beyond: 512^2 x 16384, S = 8 130 / 161 / 152; 64^2 x 20000, S = 15 59 / 98 / 68; 512^2 x 256, S = 20 (1280
+//   items) 21.4 / 19.3 / 21.6.
+//   128: at most 512 items; with K past 2048 not where some CUs have two of them and most one:
+//   512^2 x 1024, S = 14 31.5 / 24.1 / 26.8; 1024^3, S = 8 35.5 / 30.5 / 37.8; 1000^2 x 1500, S = 8 40.5 / 36.6 / 45.6;
+//   512^2 x 4096, S = 14 57 / 50.5 / 58; beyond: 1024^3, S = 16 (1024 items) 44.6 / 46.5 / 61; 768^2 x 4096, S = 8 (288)
+//   58.9 / 62.0 / 69.5; 512^2 x 8192, S = 14 98.7 / 100.5 / 113.7.
+static int small_edge(const Dims& d) {
+    const auto items = [&](int64_t edge) { return div_up(d.M, edge) * div_up(d.N, edge) * d.S; };
+    const int64_t n64 = items(64), n128 = items(128), most = 2 * kPlanCus;
+    if (n64 <= most && d.Kp <= 16384 && n64 * d.Kp <= most * 8192) return 64;
+    if (n128 <= most && (d.Kp <= 2048 || (d.Kp <= 4096 && (n128 <= kPlanCus || n128 >= most * 7 / 8)))) return 128;
+    return kS2TileRows;
+}
+
 // Candidates: every item in p parts, or only those past the last full round of the CUs (2048^3, S = 6:
 // 384 items are 1.5 rounds; the last 128 in halves take 1 + 0.5: 95.4 -> 92.7 us for the call; 1500 x 900 x
 // 3000, S = 12, 288 items: 124 -> 112 us; 777 x 1501 x 1003, S = 14: 55.7 -> 54.2 us).  From 16 rounds on row
@@ -42,6 +60,8 @@ S2Plan scheme2_plan(const Dims& d) {
     best.kts = (int)KT;
     best.whole = items;
     if (items == 0 || items >= kS2Items) return best;
+    best.edge = small_edge(d);
+    if (best.edge != kS2TileRows) return best;
     const int64_t full = items / kPlanCus * kPlanCus;
     double best_us = 0.97 * (double)div_up(items, kPlanCus) * item_us(KT);  // a split has to pay
     for (const int64_t whole : {full, (int64_t)0}) {
