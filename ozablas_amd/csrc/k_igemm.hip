@@ -175,13 +175,14 @@ struct Claims {
 // round (publish_claim adds the same offset).  Two claims from the counter up front would hand the
 // first claimants every other item of the first two rounds and leave the later ones with nothing
 // when the run is short.  Positions only grow, so when the first is past the end so is the second.
+template <bool DYN>
 __device__ __forceinline__ Claims first_claims(unsigned* queue, int xcd, unsigned* s_pos) {
     Claims c;
-    if (queue) {
+    if (DYN) {
         if (threadIdx.x == 0) s_pos[1] = (gridDim.x >> 3) + atomicAdd(&queue[xcd], 1u);
         __syncthreads();
         c.w = blockIdx.x >> 3;
-        c.w1 = s_pos[1];
+        c.w1 = __builtin_amdgcn_readfirstlane(s_pos[1]);
     } else {
         c.w = blockIdx.x;
         c.w1 = 2 * gridDim.x - 1 - c.w;
@@ -196,7 +197,7 @@ __device__ __forceinline__ uint32_t publish_claim(unsigned ticket, unsigned* s_p
     if (threadIdx.x == 0) s_pos[1] = (gridDim.x >> 3) + ticket;
     wait_lgkmcnt0();
     block_sync_lds();
-    return s_pos[1];
+    return __builtin_amdgcn_readfirstlane(s_pos[1]);
 }
 
 struct S1Args {
@@ -248,10 +249,11 @@ struct S1Walk {
 };
 
 // The items of one tile in the blocked form, longest first: stages [i0, i0 + nit) of group g into plane
-// `plane`.
+// `plane`.  32-bit fields: read by scalar loads, while bytes would take vector loads, and a wait for those
+// is one for the ring's loads too.
 struct S1Entry {
-    uint8_t g, plane;
-    uint16_t i0, nit;
+    uint32_t g_plane;  // g | plane << 16
+    uint32_t i0, nit;
 };
 struct S1List {
     int n;
@@ -314,17 +316,18 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1(S1Args p) {
 // takes position r * G + b of G workgroups, or (r + 1) * G - 1 - b when r is odd, so that a workgroup with
 // a long item gets a short one next.  (Runs of 32 consecutive positions per XCD instead, whose tiles share
 // panels in its L2, were slower: 1500^3, S = 8 199 against 186 us.)
-template <class C>
+template <class C, bool DYN>
 __global__ void __launch_bounds__(C::NT) k_igemm_s1g(S1Args p, S1List list) {
-    __shared__ __attribute__((aligned(1024))) int8_t smem[C::LDS_BYTES];
-    __shared__ unsigned s_pos[2];
+    // The claim words lie behind the ring in one array: with a second LDS variable the compiler tells the
+    // direct loads' LDS writes apart and waits for all of them before each read of the ring that may alias.
+    __shared__ __attribute__((aligned(1024))) int8_t smem[C::LDS_BYTES + (DYN ? 16 : 0)];
+    unsigned* s_pos = reinterpret_cast<unsigned*>(smem + (DYN ? C::LDS_BYTES : 0));
     const uint32_t tiles = p.order.tiles.d;
-    const bool dyn = p.queue != nullptr;
     const uint32_t xcd = blockIdx.x & 7;
-    const uint32_t t0 = dyn ? tiles * xcd / 8 : 0, ntile = dyn ? tiles * (xcd + 1) / 8 - t0 : tiles;
-    const FastDiv by_ntile = !dyn ? p.order.tiles : ntile == p.by_share.d ? p.by_share : p.by_share1;
+    const uint32_t t0 = DYN ? tiles * xcd / 8 : 0, ntile = DYN ? tiles * (xcd + 1) / 8 - t0 : tiles;
+    const FastDiv by_ntile = !DYN ? p.order.tiles : ntile == p.by_share.d ? p.by_share : p.by_share1;
     const uint32_t nwork = ntile * list.n;
-    Claims c = first_claims(p.queue, xcd, s_pos);
+    Claims c = first_claims<DYN>(p.queue, xcd, s_pos);
     if (c.w >= nwork) return;  // whole workgroup leaves together
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave_part<C>(wave).m, wn = wave_part<C>(wave).n;
@@ -336,10 +339,10 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1g(S1Args p, S1List list) {
         Item t;
         uint32_t tile;
         const uint32_t e = div_fast(k, by_ntile, tile);
-        t.g = list.e[e].g;
-        t.plane = list.e[e].plane;
-        t.i0 = list.e[e].i0;
-        t.nit = list.e[e].nit;
+        t.g = (int)(list.e[e].g_plane & 0xffffu);
+        t.plane = (int)(list.e[e].g_plane >> 16);
+        t.i0 = (int)list.e[e].i0;
+        t.nit = (int)list.e[e].nit;
         grouped_tile<C>(t0 + tile, p.order, t.tm, t.tn);
         t.tm += p.tm0;
         t.src = wave_src<C>(p.A + (int64_t)t.tm * C::BM * p.Kp, p.B + (int64_t)t.tn * C::BN * p.Kp, p.Kp, wave,
@@ -348,23 +351,28 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1g(S1Args p, S1List list) {
     };
     const S1Walk<C> walk(p);
     Item cur = decode(c.w);
-    const NextSrc first = walk.next(cur.src, p, cur.g, cur.i0, cur.nit);
-    chain_start<C>(smem, 0, cur.nit, first.s0, first.s1);
+    if constexpr (C::STAGES == 2) {
+        const NextSrc first = walk.next(cur.src, p, cur.g, cur.i0, cur.nit);
+        chain_start<C>(smem, 0, cur.nit, first.s0, first.s1);
+    } else {
+        chain_start_deep<C>(smem, cur.nit, walk.at(cur.src, p, cur.g, cur.i0), walk);
+    }
     int base = 0;
     for (;;) {
         const bool more = c.w1 < nwork;
         Item nxt = cur;
         auto entry = [&] {
             if (more) nxt = decode(c.w1);
-            return walk.next(nxt.src, p, nxt.g, nxt.i0, nxt.nit);
+            if constexpr (C::STAGES == 2) return walk.next(nxt.src, p, nxt.g, nxt.i0, nxt.nit);
+            else return walk.at(nxt.src, p, nxt.g, nxt.i0);
         };
         unsigned ticket;  // the item after next (dynamic order); thread 0's only: a value merged from both
         // paths would be copied, and so waited for behind the next item's loads, as soon as it returns
         auto claim = [&] {
-            if (dyn && more && threadIdx.x == 0) ticket = atomicAdd(&p.queue[xcd], 1u);
+            if (DYN && more && threadIdx.x == 0) ticket = atomicAdd(&p.queue[xcd], 1u);
         };
         const int64_t row0 = (int64_t)cur.tm * C::BM + wm * C::WTM, col0 = (int64_t)cur.tn * C::BN + wn * C::WTN;
-        const S1Cursor stage2 = walk.at(cur.src, p, cur.g, cur.i0 + min(2, cur.nit - 1));
+        const S1Cursor stage2 = walk.at(cur.src, p, cur.g, cur.i0 + min(C::STAGES, cur.nit - 1));
         for_part<C>(
             p.M - row0, p.N - col0,
             [&]<class P>() {
@@ -376,8 +384,8 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s1g(S1Args p, S1List list) {
             },
             [&] { mainloop_idle<C>(smem, base, cur.nit, stage2, walk, entry); });  // never thread 0's wave: part (0, 0)
         if (!more) break;
-        const uint32_t w2 = dyn ? publish_claim(ticket, s_pos) : c.w + 2 * gridDim.x;
-        base = (base + cur.nit) & 1;
+        const uint32_t w2 = DYN ? publish_claim(ticket, s_pos) : c.w + 2 * gridDim.x;
+        base = (base + cur.nit) & (C::STAGES - 1);
         c.w = c.w1;
         c.w1 = w2;
         cur = nxt;
@@ -508,25 +516,51 @@ static S1Args make_s1(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, int
     return p;
 }
 
+// The items of one tile, with kt stages per pair.
+static bool make_s1_list(const S1Plan& plan, int S, int kt, S1List& list) {
+    list.n = 0;
+    for (int g = 0, extra = S; g < S; ++g) {
+        const int stages = (g + 1) * kt, parts = plan.parts[g];
+        for (int j = 0; j < parts; ++j) {
+            if (list.n == kMaxS1Planes) return false;
+            const int i0 = (int)((int64_t)stages * j / parts), i1 = (int)((int64_t)stages * (j + 1) / parts);
+            list.e[list.n++] = S1Entry{(uint32_t)(g + 2) | (uint32_t)(j == 0 ? g : extra++) << 16, (uint32_t)i0, (uint32_t)(i1 - i0)};
+        }
+    }
+    std::stable_sort(list.e, list.e + list.n, [](const S1Entry& a, const S1Entry& b) {
+        return a.nit != b.nit ? a.nit > b.nit : (a.g_plane & 0xffffu) > (b.g_plane & 0xffffu);
+    });
+    return true;
+}
+
+// S1Plan::edge = 64 or 128: as launch_small.
+template <class C>
+static hipError_t launch_s1_small(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, int32_t* T, hipStream_t st,
+                                  const S1Plan& plan) {
+    S1Args p = make_s1<C>(d, A_sl, B_sl, 0, (int)((d.M + C::BM - 1) / C::BM));
+    p.T = T;
+    S1List list;
+    if (!make_s1_list(plan, d.S, p.KT, list)) return hipErrorInvalidValue;
+    const int64_t total = (int64_t)p.order.tiles_m * p.order.tiles_n * list.n;
+    if (total == 0) return hipSuccess;
+    if (total > INT32_MAX) return hipErrorInvalidValue;
+    k_igemm_s1g<C, false><<<(unsigned)total, C::NT, 0, st>>>(p, list);
+    return hipGetLastError();
+}
+
 hipError_t launch_igemm_s1_blocked(const Dims& d, const int8_t* A_sl, const int8_t* B_sl, int32_t* T, hipStream_t st,
                                    const S1Plan& plan, unsigned* queue, int tm0, int tms) {
     const int tiles_m = (int)((d.M + CfgS2::BM - 1) / CfgS2::BM);
     if (tm0 < 0 || tm0 > tiles_m) return hipErrorInvalidValue;
+    if (plan.edge != CfgS2::BM) {
+        if (tm0 != 0 || tms >= 0) return hipErrorInvalidValue;
+        return plan.edge == 64 ? launch_s1_small<CfgS2Small64>(d, A_sl, B_sl, T, st, plan)
+                               : launch_s1_small<CfgS2Small128>(d, A_sl, B_sl, T, st, plan);
+    }
     S1Args p = make_s1<CfgS2>(d, A_sl, B_sl, tm0, tms < 0 ? tiles_m - tm0 : std::min(tms, tiles_m - tm0));
     p.T = T;
     S1List list;
-    list.n = 0;
-    for (int g = 0, extra = d.S; g < d.S; ++g) {
-        const int stages = (g + 1) * p.KT, parts = plan.parts[g];
-        for (int j = 0; j < parts; ++j) {
-            if (list.n == kMaxS1Planes) return hipErrorInvalidValue;
-            const int i0 = (int)((int64_t)stages * j / parts), i1 = (int)((int64_t)stages * (j + 1) / parts);
-            list.e[list.n++] = S1Entry{(uint8_t)(g + 2), (uint8_t)(j == 0 ? g : extra++), (uint16_t)i0, (uint16_t)(i1 - i0)};
-        }
-    }
-    std::stable_sort(list.e, list.e + list.n, [](const S1Entry& a, const S1Entry& b) {
-        return a.nit != b.nit ? a.nit > b.nit : a.g > b.g;
-    });
+    if (!make_s1_list(plan, d.S, p.KT, list)) return hipErrorInvalidValue;
     const int64_t tiles = (int64_t)p.order.tiles_m * p.order.tiles_n, total = tiles * list.n;
     if (total == 0) return hipSuccess;
     if (total > INT32_MAX) return hipErrorInvalidValue;  // 2^49 bytes of products
@@ -536,7 +570,8 @@ hipError_t launch_igemm_s1_blocked(const Dims& d, const int8_t* A_sl, const int8
     // items per workgroup the first claimants would take them all and the others none; and with few
     // tiles the XCDs' shares of them are uneven (30 tiles: three or four each).
     p.queue = queue && grid % 8 == 0 && total >= 2 * (int64_t)grid && tiles >= 64 ? queue : nullptr;  // zeroed by the caller
-    k_igemm_s1g<CfgS2><<<grid, CfgS2::NT, 0, st>>>(p, list);
+    if (p.queue) k_igemm_s1g<CfgS2, true><<<grid, CfgS2::NT, 0, st>>>(p, list);
+    else k_igemm_s1g<CfgS2, false><<<grid, CfgS2::NT, 0, st>>>(p, list);
     return hipGetLastError();
 }
 

@@ -187,8 +187,9 @@ S2Plan scheme2_plan(const Dims& d);
 // Digit tiles that a plan writes (65536 bytes each).
 int64_t s2_plan_tiles(const Dims& d, const S2Plan& p);
 // Scheme I: group g + 2 (g + 1 pairs) runs in parts[g] equal runs of its stages; the first part's INT32
-// plane is plane g, the other parts' follow the S planes, group after group.
+// plane is plane g, the other parts' follow the S planes, group after group.  edge: as in S2Plan.
 struct S1Plan {
+    int edge = kS2TileRows;
     int parts[kMaxSlices] = {};
     int planes = 0;
 };

@@ -105,6 +105,20 @@ int64_t s1_most_tiles(const Dims& d) {
     return most_tiles(tiles_of(d) * d.S, tiles_of(d) * std::min<int64_t>(parts, kMaxS1Planes), kS1Items, kS1Extra);
 }
 
+// Tile edge, by the items and the 128-byte K steps of the longest.  Calls, us, 256 x 256 (in parts) / 128 x 128 /
+// 64 x 64: 256^3, S = 4 (64 items of 64 x 64, longest 8) 24.8 / 18.4 / 15.0; 512^3, S = 8 (512, 32) 40.9 / 36.5 / 27.6;
+// 300^2 x 2000, S = 6 (150, 96) 58 / 78 / 50; 100^2 x 4000, S = 7 (28, 224) 52 / 145 / 80; 768^3, S = 6 (864, 36) 49 / 42 / 39;
+// 1000^2 x 300, S = 4 (1024, 12; 256 of 128 x 128) 38.6 / 28.5 / 30.8; 1024^2 x 256, S = 6 (1536, 12; 384) 41.7 / 31.8 /
+// 36.9; 1000^2 x 500, S = 9 (2304, 36; 576) 66 / 56 / 73; 1200^3, S = 6 (2166, 60; 600) 85 / 81 / 102; 2000^2 x 1000, S = 6
+// (1536 of 128 x 128) 137 / 153 / 203.
+static int small_edge_s1(const Dims& d) {
+    const auto items = [&](int64_t edge) { return div_up(d.M, edge) * div_up(d.N, edge) * d.S; };
+    const int64_t n64 = items(64), n128 = items(128), most = 2 * kPlanCus, longest = d.S * d.Kp / 128;
+    if (longest <= 100 && (n64 <= most || (n64 <= 2 * most && longest > 32))) return 64;
+    if (longest <= 64 && n128 <= 600) return 128;  // the third workgroups of a few CUs are short ones
+    return kS2TileRows;
+}
+
 // Groups of at most `limit` stages per item, the limit with the least modelled time: the longest load of
 // a workgroup in the launch's order (one list, longest item first, back and forth over the CUs; sampled
 // workgroups), plus the extra planes' bytes.  Calls, us, whole / with this plan: 184 x 499 x 10597, S = 6
@@ -137,7 +151,8 @@ S1Plan scheme1_plan(const Dims& d) {
         return longest + (extra ? (double)(extra * tiles) * 8.0 * kTileBytes / kBytesPerUs + kPartsUs : 0.0);
     };
     const int64_t most = (int64_t)d.S * KT;
-    if (tiles == 0 || tiles * d.S >= kS1Items) {  // enough items to balance
+    best.edge = small_edge_s1(d);
+    if (tiles == 0 || tiles * d.S >= kS1Items || best.edge != kS2TileRows) {  // enough items to balance, or small ones
         best.planes = d.S;
         std::fill(best.parts, best.parts + d.S, 1);
         return best;
