@@ -25,7 +25,9 @@ constexpr double kBytesPerUs = 4.0e6, kPartsUs = 2.0;
 double item_us(int64_t steps) { return kItemUs + kStepUs * (double)steps; }
 int64_t div_up(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // Calls with this many items or more are not split; a split call adds at most this many partial tiles.
-constexpr int64_t kS2Items = 16 * kPlanCus, kS2Extra = 2 * kPlanCus;
+// With K below kS2LongKp the parts fill one round at most (more rounds of shorter parts pay for long K only:
+// 192 items in fours are 3 rounds of a quarter).
+constexpr int64_t kS2Items = 16 * kPlanCus, kS2Extra = 2 * kPlanCus, kS2LongKp = 4096;
 constexpr int64_t kS1Items = 8 * kPlanCus, kS1Extra = kPlanCus;
 constexpr int64_t kS1MinStages = 4;  // per part
 int64_t tiles_of(const Dims& d) { return div_up(d.M, kS2TileRows) * div_up(d.N, kS2TileRows); }
@@ -70,7 +72,7 @@ S2Plan scheme2_plan(const Dims& d) {
         for (int64_t p = 2; p <= kMaxParts && 2 * p <= KT; ++p) {
             const int64_t kts = div_up(KT, p);
             if (div_up(KT, kts) != p) continue;  // some part would be empty
-            if ((p - 1) * tail > kS2Extra) break;
+            if (d.Kp < kS2LongKp ? p * tail > kPlanCus : (p - 1) * tail > kS2Extra) break;
             const double us = (double)(whole / kPlanCus) * item_us(KT) + (double)div_up(tail * p, kPlanCus) * item_us(kts) +
                               (double)((p - 1) * tail * kTileBytes) / kBytesPerUs + kPartsUs;
             if (us < best_us) {
@@ -96,8 +98,9 @@ static int64_t most_tiles(int64_t items, int64_t most_parted, int64_t split_item
     return std::max(items, std::min({most_parted, items + extra, split_items + extra}));
 }
 int64_t s2_most_tiles(const Dims& d) {
-    const int64_t items = tiles_of(d) * d.S;
-    return most_tiles(items, items * std::clamp<int64_t>(d.Kp / 256, 1, kMaxParts), kS2Items, kS2Extra);
+    const int64_t items = tiles_of(d) * d.S, parted = items * std::clamp<int64_t>(d.Kp / 256, 1, kMaxParts);
+    if (d.Kp >= kS2LongKp) return most_tiles(items, parted, kS2Items, kS2Extra);
+    return items >= kS2Items ? items : std::min(parted, div_up(items, kPlanCus) * kPlanCus);
 }
 int64_t s1_most_tiles(const Dims& d) {
     int64_t parts = 0;
