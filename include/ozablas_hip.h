@@ -94,8 +94,8 @@ int oza_ctx_event_times(oza_ctx ctx, double sums[5], int* count);
  * scheme is 1 or 2.  bytes[5] = {shift_A, shift_B, A_slices, B_slices, C_tc}.  Layouts:
  *   shift_A int32[M], shift_B int32[N]          (reference semantics)
  *   A_slices int8 [S][Mp][Kp], B_slices int8 [S][Np][Kp] (B transposed: K contiguous)
- *   C_tc   Scheme II: S planes of uint8 CRT digits (-2^-32 C_s mod m_s), Mp x Np each in 32 x 32 element
- *          blocks (oza_unpack_digits gives C_s mod m_s in planar layout); Scheme I: S planes of int32 group
+ *   C_tc   Scheme II: S planes of uint8 CRT digits C_s mod m_s, Mp x Np each in 32 x 32 element
+ *          blocks (oza_unpack_digits gives the planar view); Scheme I: S planes of int32 group
  *          products T_g, Mp x Np each in 32 x 32 element blocks (the stage entry points write the
  *          reference's planar int32 [S][M][N] there); then room for the partial sums of tiles whose
  *          products run in several parts along K, for shapes with few tiles

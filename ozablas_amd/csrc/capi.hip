@@ -670,7 +670,7 @@ int oza_unpack_digits(oza_ctx ctx, size_t M, size_t N, int S, const void* Ctc, u
     const size_t K = 1;
     OZA_STAGE_PROLOGUE(2)
     if (!Ctc || !planar) return fail(OZA_INVALID_ARGUMENT, "OzaBLAS: null digits pointer.");
-    OZA_HIP(launch_digits_unpack(d, static_cast<const uint8_t*>(Ctc), crt_for(ctx, S), planar, st), "unpack");
+    OZA_HIP(launch_digits_unpack(d, static_cast<const uint8_t*>(Ctc), planar, st), "unpack");
     return OZA_SUCCESS;
 }
 

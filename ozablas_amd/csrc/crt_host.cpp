@@ -84,14 +84,19 @@ CrtTables build_tables() {
                 const uint64_t m = kModuli[s], e = P / m;
                 Big q, qq;
                 div_small(M, m, q);
-                // w = -2^32 ((M/m_s) mod m_s)^-1 mod m_s, combined over the group by the CRT mod P
-                const uint64_t a = inverse_mod(div_small(q, m, qq), m) * (m - (uint64_t(1) << 32) % m) % m;
+                // w = ((M/m_s) mod m_s)^-1 mod m_s, combined over the group by the CRT mod P
+                const uint64_t a = inverse_mod(div_small(q, m, qq), m);
                 w = (w + a * inverse_mod(e % m, m) % m * e) % P;
                 cs.E[s] = (uint32_t)e;
                 cs.m[s] = (uint32_t)m;
                 uint32_t inv = 1;  // Newton: correct bits of m^-1 mod 2^32 double each time (m is odd)
                 for (int i = 0; i < 6; ++i) inv *= 2u - (uint32_t)m * inv;
                 cs.minv[s] = inv;
+                uint64_t p = (uint64_t(1) << 32) % m;  // 2^32 2^(8 k) mod m
+                for (int k = 0; k < 4; ++k) {
+                    cs.wt[s] |= (uint32_t)((m - p) % m) << (8 * k);
+                    p = p * 256 % m;
+                }
                 cs.bias[s] = (uint32_t)(((uint64_t(1) << 31) + m - 1) / m * m);
                 err += (m - 1) * e;
             }

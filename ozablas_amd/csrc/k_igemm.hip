@@ -7,7 +7,7 @@
 //
 //   Scheme II (reference: rocblas_gemm_strided_batched_ex, src/hip/pipeline.hip:237-245):
 //     one launch covers every (tile, modulus); the epilogue reduces C_s to its CRT digit
-//     modulo m_s (stored_digit) and stores it as one byte (layout below), or stores
+//     modulo m_s (product_digit) and stores it as one byte (layout below), or stores
 //     the raw INT32 C_s planes in the reference's [s][M][N] layout.
 //   Scheme I (reference: rocblas_gemm_ex loop, pipeline.hip:110-135): one launch covers every
 //     (group g, tile); the pairs of group g = s + t accumulate into one INT32 fragment set and
@@ -49,7 +49,7 @@ struct S2Args {
     TileOrder order;       // of the tile rows [tm0, tm0 + order.tiles_m)
     int tm0;
     void* out;             // digits or int32 planes
-    const CrtSet* crt;     // device copy (m, minv, bias used)
+    const CrtSet* crt;     // device copy (m, minv, wt, bias used)
     // SPLIT only: items [0, whole) run whole, the `tail` others in `parts` parts of kts K steps
     uint32_t items, whole, tail;
     FastDiv by_tail;
@@ -71,7 +71,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         int s, tm, tn, j, k0, KT;
         uint32_t l;
         StageSrc src;  // this wave's blocks of stage 0
-        uint32_t m, minv, bias;
+        uint32_t m, minv, wt, bias;
     };
     auto decode = [&](uint32_t wi) {
         Item t;
@@ -99,6 +99,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         // scalar loads: counted by lgkmcnt, so the epilogue does not wait for the direct loads
         t.m = as_constant(p.crt)->m[t.s];
         t.minv = as_constant(p.crt)->minv[t.s];
+        t.wt = as_constant(p.crt)->wt[t.s];
         t.bias = as_constant(p.crt)->bias[t.s];
         return t;
     };
@@ -137,7 +138,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
                     uint8_t* plane = part ? p.part + (int64_t)((cur.j - 1) * p.tail + cur.l - p.whole) * kTileBytes
                                           : reinterpret_cast<uint8_t*>(p.out) + (int64_t)s * p.Mp * p.Np;
                     store_digits<P, false>(acc, plane, part ? C::BN : p.Np, part ? wm * C::WTM : row0,
-                                           part ? wn * C::WTN : col0, p.M, p.N, cur.m, cur.minv, lane);
+                                           part ? wn * C::WTN : col0, p.M, p.N, cur.wt, cur.m, cur.minv, lane);
                 } else {
                     int32_t* o = reinterpret_cast<int32_t*>(p.out) + (int64_t)s * p.M * p.N;
 #pragma unroll

@@ -4,7 +4,7 @@
 // The reference sums c_s * (M/m_s) modulo M, c_s = (C_s mod m_s) * (M/m_s)^-1 mod m_s, in u64
 // (S <= 7) or four u64 limbs (S > 7), maps acc >= floor(M/2) to -(M - acc), converts limb by limb
 // (to_double_256) and scales by 2^-(shift_A[i] + shift_B[j]).  The value it converts is the fixed
-// integer C mod M, so any exact method gives the same double.  Here the stored digits of the C_s are
+// integer C mod M, so any exact method gives the same double.  Here the digits of the C_s are
 // combined in groups of three moduli into X = C (mod M) in 32-bit words, the quotient
 // q = floor(X/M + 1/2) comes from a 32-bit fixed-point sum of the same groups, Y = X - q*M in one
 // carry pass, an exact range check only when q was ambiguous, then the reference's limb-wise
@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(256)
     uint32_t c[S];
 #pragma unroll
     for (int s = 0; s < S; ++s)
-        c[s] = stored_digit((uint32_t)Ct[s * MN + idx] + cs->bias[s], cs->m[s], cs->minv[s]);
+        c[s] = product_digit((uint32_t)Ct[s * MN + idx] + cs->bias[s], cs->wt[s], cs->m[s], cs->minv[s]);
     const double f = crt_value<S>(c, 0, cs);
     Cout[idx] = ldexp(f, -(shA[row] + shB[col]));
 }
@@ -165,20 +165,20 @@ __device__ __forceinline__ void digit_position(int64_t idx, int64_t plane, int64
     col = Q * 32 + (lane & 31);
 }
 
-// Blocked digit planes -> planar [s][M][N] residues C_s mod m_s (for inspection and parity tests).
+// Blocked digit planes -> planar [s][M][N] (for inspection and parity tests).
 __global__ void __launch_bounds__(256)
     k_digits_unpack(const uint8_t* __restrict__ dg, int64_t M, int64_t N, int64_t Mp, int64_t Np, int S,
-                    const CrtSet* __restrict__ cs, uint8_t* __restrict__ out) {
+                    uint8_t* __restrict__ out) {
     const int64_t plane = Mp * Np;
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= plane * S) return;
     int64_t s, row, col;
     digit_position(idx, plane, Np, s, row, col);
-    if (row < M && col < N) out[(s * M + row) * N + col] = (uint8_t)plain_digit(dg[idx], cs->m[s]);
+    if (row < M && col < N) out[(s * M + row) * N + col] = dg[idx];
 }
 
-// Planar [s][M][N] residues -> blocked digit planes (the inverse of k_digits_unpack for residues in
-// [0, m_s); padding positions get 0).
+// Planar [s][M][N] digits -> blocked digit planes, reduced mod m_s (the inverse of
+// k_digits_unpack for digits in [0, m_s); padding positions get 0).
 __global__ void __launch_bounds__(256)
     k_digits_pack(const uint8_t* __restrict__ in, int64_t M, int64_t N, int64_t Mp, int64_t Np, int S,
                   const CrtSet* __restrict__ cs, uint8_t* __restrict__ dg) {
@@ -187,7 +187,7 @@ __global__ void __launch_bounds__(256)
     if (idx >= plane * S) return;
     int64_t s, row, col;
     digit_position(idx, plane, Np, s, row, col);
-    dg[idx] = row < M && col < N ? (uint8_t)stored_digit(in[(s * M + row) * N + col], cs->m[s], cs->minv[s]) : 0;
+    dg[idx] = row < M && col < N ? (uint8_t)(in[(s * M + row) * N + col] % cs->m[s]) : 0;
 }
 
 template <int S>
@@ -272,12 +272,10 @@ hipError_t launch_scale_c(const OutC& c, int64_t M, int64_t N, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t launch_digits_unpack(const Dims& d, const uint8_t* digits, const CrtSet* crt_dev, uint8_t* out,
-                                hipStream_t st) {
+hipError_t launch_digits_unpack(const Dims& d, const uint8_t* digits, uint8_t* out, hipStream_t st) {
     const int64_t n = d.Mp * d.Np * d.S;
     if (n == 0) return hipSuccess;
-    k_digits_unpack<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(digits, d.M, d.N, d.Mp, d.Np, d.S, crt_dev,
-                                                                      out);
+    k_digits_unpack<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(digits, d.M, d.N, d.Mp, d.Np, d.S, out);
     return hipGetLastError();
 }
 

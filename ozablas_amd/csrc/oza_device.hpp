@@ -100,18 +100,14 @@ __device__ __forceinline__ int sym_residue(const uint32_t (&w)[ND], const uint32
     return __mulhi((int)(d * minv), (int)m);
 }
 
-// Stored digit of an INT32 product v (K 125^2 < 2^31): d = -2^-32 v mod m, in [0, m).  u = v + bias, with
-// bias the least multiple of m that is at least 2^31, lies in [0, 2^32) and is congruent to v; with
-// p = u m^-1 mod 2^32 the product p m is congruent to u modulo 2^32, so p m = d 2^32 + u for
-// d = floor(p m / 2^32) < m, and d 2^32 = -u modulo m (Montgomery's reduction).  Two 32-bit
-// multiplies (full rate, four cycles per wave like every instruction here) against five FP64
-// operations for the plain residue, and bias costs nothing: the accumulators start from it.  The
-// factor -2^-32 is undone by the CRT constants of the reconstruction; sums of digits of partial
-// products, reduced modulo m, are the digits of the whole.  With the FP64 form the epilogue of a
-// 128 x 128 tile took 450 vector instructions per wave beside 80 MFMAs at K = 640; 512-GEMM batch
-// 5.40 -> 5.29 ms, 4096^3 at S = 17 1.33 -> 1.32 ms.
-__device__ __forceinline__ uint32_t stored_digit(uint32_t u, uint32_t m, uint32_t minv) {
-    return __umulhi(u * minv, m);
+// CRT digit v mod m of an INT32 product v (K 125^2 < 2^31), in [0, m), from u = v + bias, where bias, the
+// least multiple of m that is at least 2^31, brings u into [0, 2^32) and costs nothing: the accumulators
+// start from it.  As in sym_residue: d, the sum of u's four bytes times wt (byte k = -2^32 2^(8k) mod m), is
+// congruent to -2^32 u and below 2^18; with p = d m^-1 mod 2^32 the product p m = r 2^32 + d for
+// r = floor(p m / 2^32) < m, so r is congruent to u.  Three 32-bit instructions (full rate, four cycles per wave
+// like every instruction here) against five in FP64 (crt_digit).
+__device__ __forceinline__ uint32_t product_digit(uint32_t u, uint32_t wt, uint32_t m, uint32_t minv) {
+    return __umulhi(__builtin_amdgcn_udot4(u, wt, 0u, false) * minv, m);
 }
 
 // CRT digit of an INT32 product: the Euclidean residue c = v mod m in [0, m) -- the reference's
@@ -128,12 +124,6 @@ __device__ __forceinline__ int crt_digit(int v, double m, double rcp) {
     constexpr double kBias = 2147483648.0 + 0x1p-10;  // 2^31 + 2^-10, exact
     const double x = fma((double)v, rcp, kBias);
     return (int)fma(__builtin_amdgcn_fract(x), m, 0.5);
-}
-
-// The plain residue v mod m of a stored digit of v.
-__device__ __forceinline__ uint32_t plain_digit(uint32_t d, uint32_t m) {
-    const uint32_t f = m - (uint32_t)((1ull << 32) % m);  // -2^32 mod m
-    return (uint32_t)crt_digit((int)(d * f), (double)m, 1.0 / (double)m);
 }
 
 // ---- MFMA-fragment-tiled operand planes -------------------------------------------------------

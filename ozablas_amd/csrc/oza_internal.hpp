@@ -5,7 +5,7 @@
 //   shift_B   int32[N]                   column shifts
 //   A_slices  int8 [S][Mp][Kp]           A residues/slices, K contiguous, fragment-tiled (frag_off16)
 //   B_slices  int8 [S][Np][Kp]           B residues/slices TRANSPOSED (column n is a K-contiguous row)
-//   C_tc      Scheme II: uint8 [S][Mp][Np] stored digits of C_s (stored_digit) in 32 x 32 element blocks,
+//   C_tc      Scheme II: uint8 [S][Mp][Np] digits C_s mod m_s in 32 x 32 element blocks,
 //                        then the partial tiles of items that ran in K parts (S2Plan)
 //             Scheme I : int32 [S][Mp][Np] group products T_g in 32 x 32 element blocks, then the planes of
 //                        groups that ran in parts (S1Plan) (the stage entry point writes the reference's
@@ -57,9 +57,8 @@ static_assert(bitlen_M(8) == 63 && bitlen_M(16) == 124 && bitlen_M(20) == 153, "
 // The moduli s = 0..S-1 are taken in groups of three, g = s / 3 (the last one may be shorter), with
 // P_g the product of a group's moduli (< 2^24).  With the group sums
 //   u_g = sum_{s in g} c_s (P_g / m_s)            (24-bit operands, u_g < 3 * 2^24)
-// and the constants R_g = w_g (M / P_g), w_g < P_g with w_g (M / m_s) = -2^32 mod m_s for every s in g,
-//   X = sum_g u_g R_g = C (mod M)   whenever   c_s = -2^-32 C mod m_s for all s
-// (the digits as the pipeline stores them, see stored_digit; the factor is part of w_g).
+// and the constants R_g = w_g (M / P_g), w_g < P_g with w_g (M / m_s) = 1 mod m_s for every s in g,
+//   X = sum_g u_g R_g = C (mod M)   whenever   c_s = C mod m_s for all s.
 constexpr int kWords = 5;                          // 160 bits: M < 2^153 and a sign
 constexpr int kGroups = (kMaxSlices + 2) / 3;
 struct CrtSet {
@@ -70,8 +69,8 @@ struct CrtSet {
     uint32_t R[kGroups][kWords];
     uint32_t Mneg[kWords];            // 2^160 - M
     uint32_t M32[kWords], Mhalf32[kWords];  // M and floor(M/2)
-    // stored_digit: m_s, m_s^-1 mod 2^32 and the least multiple of m_s that is at least 2^31
-    uint32_t m[kMaxSlices], minv[kMaxSlices], bias[kMaxSlices];
+    // product_digit: m_s, m_s^-1 mod 2^32, the byte weights and the least multiple of m_s that is at least 2^31
+    uint32_t m[kMaxSlices], minv[kMaxSlices], wt[kMaxSlices], bias[kMaxSlices];
     uint64_t M64[4];                  // M in 64-bit words
 };
 
@@ -228,8 +227,7 @@ hipError_t launch_recon_s2_digits(const Dims& d, uint8_t* digits, const int32_t*
 hipError_t launch_recon_s2_int32(const Dims& d, const int32_t* C_tc, const int32_t* shift_A,
                                  const int32_t* shift_B, const CrtSet* crt_dev, double* C, hipStream_t st);
 // Blocked digit planes <-> planar [s][M][N] digits in [0, m_s) (pack reduces its input mod m_s).
-hipError_t launch_digits_unpack(const Dims& d, const uint8_t* digits, const CrtSet* crt_dev, uint8_t* out,
-                                hipStream_t st);
+hipError_t launch_digits_unpack(const Dims& d, const uint8_t* digits, uint8_t* out, hipStream_t st);
 hipError_t launch_digits_pack(const Dims& d, const uint8_t* planar, const CrtSet* crt_dev, uint8_t* digits,
                               hipStream_t st);
 // Scheme I step 4 from blocked planes: T_g = the sum of its parts' planes (left in the first of them),

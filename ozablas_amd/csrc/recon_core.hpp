@@ -29,7 +29,7 @@ __device__ __forceinline__ void add_words(uint32_t (&y)[L], const uint32_t* __re
     for (int l = 0; l < L; ++l) y[l] = __builtin_addc(y[l], SUB ? ~v[l] : v[l], carry, &carry);
 }
 
-// Signed reconstruction of one element from its stored digits, byte b of w[s] = c_s, as the reference's
+// Signed reconstruction of one element from its digits, byte b of w[s] = c_s, as the reference's
 // double.  With the groups of CrtSet:
 //   X = sum_g u_g R_g in LR 64-bit columns (u_g < 2^25.4, at most 7 groups: every column < 2^61);
 //   q estimates floor(X/M + 1/2) from h = 2^31 + sum_g u_g F_g, which is short of 2^32 (X/M + 1/2)
