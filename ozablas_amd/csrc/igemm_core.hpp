@@ -374,7 +374,7 @@ __device__ __forceinline__ void zero_acc(v16i (&acc)[C::FM][C::FN]) {
             for (int j = 0; j < 16; ++j) acc[fm][fn][j] = 0;
 }
 
-// Every accumulator element starts from the uniform value v (product_digit's bias; the MFMA adds
+// Every accumulator element starts from the uniform value v (kProductBias; the MFMA adds
 // modulo 2^32).  One move per element in asm: from plain assignments the compiler keeps one copy of
 // the 16 values alive through the mainloop to start the first fragments from (+60 registers, spills).
 // The mainloop's barrier lies between these moves and the first MFMA that reads them.
@@ -430,7 +430,7 @@ __device__ __forceinline__ void grouped_tile(uint32_t t, const TileOrder& o, int
 }
 
 // CRT-digit epilogue of one tile: the digit of C_s per accumulator element (product_digit; the accumulators
-// started from the modulus' bias), one 16-byte store per fragment and lane.  Digit planes are blocked in
+// started from kProductBias), one 16-byte store per fragment and lane.  Digit planes are blocked in
 // 32 x 32 element blocks: block (R, Q) of a plane with Np columns starts at byte (R * (Np/32) + Q) * 1024, and inside it lane
 // l's 16 bytes j = 0..15 sit at l*16 + j, holding element (row 8*(j/4) + 4*(l/32) + j%4,
 // column l%32) of the block, i.e. the MFMA 32x32 output layout.  The layout does not depend on
@@ -442,8 +442,12 @@ __device__ __forceinline__ void grouped_tile(uint32_t t, const TileOrder& o, int
 template <class C, bool SKIP_PAD, bool NT = false>
 __device__ __forceinline__ void store_digits(const v16i (&acc)[C::FM][C::FN], uint8_t* plane, int64_t Np,
                                              int64_t row0, int64_t col0, int64_t M, int64_t N, uint32_t wt,
-                                             uint32_t m, uint32_t minv, int lane) {
+                                             uint32_t init, uint32_t m, uint32_t minv, int lane) {
     const int64_t qn = Np >> 5;
+    // An instruction takes one scalar register.  From a plain use of a second one the compiler moved the whole
+    // item descriptor to vector registers (185 -> 205 of them).
+    uint32_t vinit;
+    asm("v_mov_b32 %0, %1" : "=v"(vinit) : "s"(init));
     // row0 and col0 are the same for the whole wave
     const int64_t fm_end = (M - (int64_t)__builtin_amdgcn_readfirstlane((int)(row0 >> 5)) * 32 + 31) >> 5;
     const int64_t fn_end = (N - (int64_t)__builtin_amdgcn_readfirstlane((int)(col0 >> 5)) * 32 + 31) >> 5;
@@ -454,7 +458,7 @@ __device__ __forceinline__ void store_digits(const v16i (&acc)[C::FM][C::FN], ui
             if (SKIP_PAD && (fm >= fm_end || fn >= fn_end)) continue;
             uint32_t d[16];
 #pragma unroll
-            for (int j = 0; j < 16; ++j) d[j] = product_digit((uint32_t)acc[fm][fn][j], wt, m, minv);
+            for (int j = 0; j < 16; ++j) d[j] = product_digit((uint32_t)acc[fm][fn][j], wt, vinit, m, minv);
             const int64_t blk = ((row0 >> 5) + fm) * qn + (col0 >> 5) + fn;
             store_global16<NT>(plane + (blk << 10) + lane * 16, pack4u(d[0], d[1], d[2], d[3]),
                            pack4u(d[4], d[5], d[6], d[7]), pack4u(d[8], d[9], d[10], d[11]),

@@ -145,7 +145,7 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
         uint8_t* plane;  // digit plane of modulus s (a partial plane for splits j > 0)
         int64_t Np, M, N;
         int tm, tn, k0, KT;  // K steps [k0, k0 + KT) of BK bytes
-        uint32_t m, minv, wt, bias;
+        uint32_t m, minv, wt, init;
     };
     constexpr int kSteps128 = 128 / C::BK;  // K steps per 128-byte K block
     auto item = [&](uint32_t wi) {
@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
         t.m = cs.m[s];
         t.minv = cs.minv[s];
         t.wt = cs.wt[s];
-        t.bias = cs.bias[s];
+        t.init = cs.init[s];
         return t;
     };
     auto stage = [](const Item& t, int i) {  // stage i of an item; its last one past that
@@ -207,10 +207,10 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
             cur.M - row0, cur.N - col0,
             [&]<class P>() {
                 v16i acc[P::FM][P::FN];
-                fill_acc<P>(acc, (int)cur.bias);
+                fill_acc<P>(acc, (int)kProductBias);
                 mainloop_chain<P>(acc, smem, base, cur.KT, stage(cur, 2), step, entry);
-                store_digits<P, true, true>(acc, cur.plane, cur.Np, row0, col0, cur.M, cur.N, cur.wt, cur.m, cur.minv,
-                                              lane);
+                store_digits<P, true, true>(acc, cur.plane, cur.Np, row0, col0, cur.M, cur.N, cur.wt, cur.init, cur.m,
+                                              cur.minv, lane);
             },
             [&] { mainloop_idle<C>(smem, base, cur.KT, stage(cur, 2), step, entry); });
         if (!more) break;

@@ -49,7 +49,7 @@ struct S2Args {
     TileOrder order;       // of the tile rows [tm0, tm0 + order.tiles_m)
     int tm0;
     void* out;             // digits or int32 planes
-    const CrtSet* crt;     // device copy (m, minv, wt, bias used)
+    const CrtSet* crt;     // device copy (m, minv, wt, init used)
     // SPLIT only: items [0, whole) run whole, the `tail` others in `parts` parts of kts K steps
     uint32_t items, whole, tail;
     FastDiv by_tail;
@@ -71,7 +71,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         int s, tm, tn, j, k0, KT;
         uint32_t l;
         StageSrc src;  // this wave's blocks of stage 0
-        uint32_t m, minv, wt, bias;
+        uint32_t m, minv, wt, init;
     };
     auto decode = [&](uint32_t wi) {
         Item t;
@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         t.m = as_constant(p.crt)->m[t.s];
         t.minv = as_constant(p.crt)->minv[t.s];
         t.wt = as_constant(p.crt)->wt[t.s];
-        t.bias = as_constant(p.crt)->bias[t.s];
+        t.init = as_constant(p.crt)->init[t.s];
         return t;
     };
     auto stage = [](const Item& t, int i) {  // stage i of an item; its last one past that
@@ -130,7 +130,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
             p.M - row0, p.N - col0,
             [&]<class P>() {
                 v16i acc[P::FM][P::FN];
-                if (DIGITS) fill_acc<P>(acc, (int)cur.bias);
+                if (DIGITS) fill_acc<P>(acc, (int)kProductBias);
                 else zero_acc<P>(acc);
                 mainloop_chain<P>(acc, smem, base, cur.KT, stage(cur, C::STAGES), step, entry);
                 if (DIGITS) {
@@ -138,7 +138,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
                     uint8_t* plane = part ? p.part + (int64_t)((cur.j - 1) * p.tail + cur.l - p.whole) * kTileBytes
                                           : reinterpret_cast<uint8_t*>(p.out) + (int64_t)s * p.Mp * p.Np;
                     store_digits<P, false>(acc, plane, part ? C::BN : p.Np, part ? wm * C::WTM : row0,
-                                           part ? wn * C::WTN : col0, p.M, p.N, cur.wt, cur.m, cur.minv, lane);
+                                           part ? wn * C::WTN : col0, p.M, p.N, cur.wt, cur.init, cur.m, cur.minv, lane);
                 } else {
                     int32_t* o = reinterpret_cast<int32_t*>(p.out) + (int64_t)s * p.M * p.N;
 #pragma unroll

@@ -100,14 +100,16 @@ __device__ __forceinline__ int sym_residue(const uint32_t (&w)[ND], const uint32
     return __mulhi((int)(d * minv), (int)m);
 }
 
-// CRT digit v mod m of an INT32 product v (K 125^2 < 2^31), in [0, m), from u = v + bias, where bias, the
-// least multiple of m that is at least 2^31, brings u into [0, 2^32) and costs nothing: the accumulators
-// start from it.  As in sym_residue: d, the sum of u's four bytes times wt (byte k = -2^32 2^(8k) mod m), is
-// congruent to -2^32 u and below 2^18; with p = d m^-1 mod 2^32 the product p m = r 2^32 + d for
-// r = floor(p m / 2^32) < m, so r is congruent to u.  Three 32-bit instructions (full rate, four cycles per wave
-// like every instruction here) against five in FP64 (crt_digit).
-__device__ __forceinline__ uint32_t product_digit(uint32_t u, uint32_t wt, uint32_t m, uint32_t minv) {
-    return __umulhi(__builtin_amdgcn_udot4(u, wt, 0u, false) * minv, m);
+// CRT digit v mod m of any INT32 product v, in [0, m), from u = v + 2^31 in [0, 2^32); the addition costs
+// nothing, the accumulators start from it (kProductBias).  As in sym_residue: d, the sum of u's four bytes times wt
+// (byte k = -2^32 2^(8k) mod m) plus init = 2^32 2^31 mod m, is congruent to -2^32 v and below 2^18 + 2^8; with
+// p = d m^-1 mod 2^32 the product p m = r 2^32 + d for r = floor(p m / 2^32) < m, so r is congruent to v.
+// Three 32-bit instructions (full rate, four cycles per wave like every instruction here) against five in
+// FP64 (crt_digit).  With a multiple of m for the 2^31 there would be no init, but the products past
+// 2^32 minus it, up to 250 of them, would wrap.
+constexpr uint32_t kProductBias = 0x80000000u;
+__device__ __forceinline__ uint32_t product_digit(uint32_t u, uint32_t wt, uint32_t init, uint32_t m, uint32_t minv) {
+    return __umulhi(__builtin_amdgcn_udot4(u, wt, init, false) * minv, m);
 }
 
 // CRT digit of an INT32 product: the Euclidean residue c = v mod m in [0, m) -- the reference's

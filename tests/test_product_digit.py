@@ -8,27 +8,26 @@ import pytest
 from test_crt_groups import tables, value
 
 
-def digit(v, m, bias):
-    minv, p, d = pow(m, -1, 1 << 32), (1 << 32) % m, 0
-    u = v + bias
+def digit(v, m):
+    minv, p, d = pow(m, -1, 1 << 32), (1 << 32) % m, (1 << 63) % m
+    u = v + 2 ** 31
     assert 0 <= u < 1 << 32
     for k in range(4):
         wt = (m - p) % m
         assert wt < 256
         d += (u >> (8 * k) & 0xff) * wt
         p = p * 256 % m
-    assert d < 1 << 18
+    assert d < (1 << 18) + 256
     return (d * minv % (1 << 32)) * m >> 32
 
 
 def test_product_digit(orc):
-    top = 137438 * 125 ** 2  # the largest |C_s| of an accepted K
+    top = 2 ** 31 - 1
     rng = random.Random(7)
     for m in (int(m) for m in orc.moduli()):
-        bias = -(-2 ** 31 // m) * m
-        vs = [0, 1, -1, m, -m, top, -top, top - m, m - top] + [rng.randint(-top, top) for _ in range(3000)]
+        vs = [0, 1, -1, m, -m] + [e + k for e in (top, -top) for k in range(-300, 301)] + [-2 ** 31] + [rng.randint(-top, top) for _ in range(3000)]
         for v in vs:
-            assert digit(v, m, bias) == v % m, (m, v)
+            assert not -2 ** 31 <= v < 2 ** 31 or digit(v, m) == v % m, (m, v)
 
 
 @pytest.mark.parametrize("S", range(1, 21))
