@@ -115,6 +115,12 @@ int oza_workspace_bytes(int scheme, size_t M, size_t N, size_t K, int slices, si
 int oza_scheme1_gemm(oza_ctx ctx, size_t M, size_t N, size_t K, int slices, const double* A, const double* B,
                      double* C, int32_t* shift_A, int32_t* shift_B, int8_t* A_slices, int8_t* B_slices,
                      void* C_tc, oza_timings* timings);
+/* oza_scheme1_gemm for a C_tc of C_tc_bytes.  Few tiles with many stages run in parts whose partial sums lie
+ * behind the S planes, where C_tc holds them (oza_workspace_bytes does); oza_scheme1_gemm, which does not know
+ * the size, writes the S planes only.  The same result either way; fails if C_tc does not hold the planes. */
+int oza_scheme1_gemm_sized(oza_ctx ctx, size_t M, size_t N, size_t K, int slices, const double* A, const double* B,
+                           double* C, int32_t* shift_A, int32_t* shift_B, int8_t* A_slices, int8_t* B_slices,
+                           void* C_tc, size_t C_tc_bytes, oza_timings* timings);
 int oza_scheme2_gemm(oza_ctx ctx, size_t M, size_t N, size_t K, int slices, const double* A, const double* B,
                      double* C, int32_t* shift_A, int32_t* shift_B, int8_t* A_slices, int8_t* B_slices,
                      void* C_tc, oza_timings* timings);

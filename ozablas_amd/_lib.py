@@ -52,6 +52,7 @@ _PROTOS = {
     "oza_ctx_event_times": [_P, C.POINTER(_D), C.POINTER(_I)],
     "oza_workspace_bytes": [_I, _SZ, _SZ, _SZ, _I, C.POINTER(_SZ)],
     "oza_scheme1_gemm": [_P, _SZ, _SZ, _SZ, _I, _P, _P, _P, _P, _P, _P, _P, _P, C.POINTER(oza_timings)],
+    "oza_scheme1_gemm_sized": [_P, _SZ, _SZ, _SZ, _I, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, C.POINTER(oza_timings)],
     "oza_scheme2_gemm": [_P, _SZ, _SZ, _SZ, _I, _P, _P, _P, _P, _P, _P, _P, _P, C.POINTER(oza_timings)],
     "oza_stage1_shifts": [_P, _I, _SZ, _SZ, _SZ, _I, _P, _P, _P, _P],
     "oza_stage2_slices": [_P, _I, _SZ, _SZ, _SZ, _I, _P, _P, _P, _P, _P, _P],
@@ -320,9 +321,9 @@ class WorkspaceScheme2(_Workspace):
     scheme = 2
 
 
-def _gemm(fn, ws, A, B, C_out, timings):
+def _gemm(fn, ws, A, B, C_out, timings, *sizes):
     t = oza_timings()
-    check(fn(ws.ex.ctx, ws.M, ws.N, ws.K, ws.slices, A.ptr, B.ptr, C_out.ptr, *ws.buffers(),
+    check(fn(ws.ex.ctx, ws.M, ws.N, ws.K, ws.slices, A.ptr, B.ptr, C_out.ptr, *ws.buffers(), *sizes,
              C.byref(t) if timings is not None else None))
     if timings is not None:
         timings._fill(t)
@@ -330,7 +331,7 @@ def _gemm(fn, ws, A, B, C_out, timings):
 
 def ozaki_scheme1_gemm(ws: WorkspaceScheme1, A: DeviceBuffer, B: DeviceBuffer, C_out: DeviceBuffer,
                        timings: OzaTimings | None = None) -> None:
-    _gemm(lib.oza_scheme1_gemm, ws, A, B, C_out, timings)
+    _gemm(lib.oza_scheme1_gemm_sized, ws, A, B, C_out, timings, ws.C_tc.nbytes)
 
 
 def ozaki_scheme2_gemm(ws: WorkspaceScheme2, A: DeviceBuffer, B: DeviceBuffer, C_out: DeviceBuffer,

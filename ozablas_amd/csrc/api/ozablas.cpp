@@ -31,9 +31,11 @@ void fill(OzaTimings* t, const oza_timings& ct) {
 void ozaki_scheme1_gemm(WorkspaceScheme1& ws, const double* A, const double* B, double* C, OzaTimings* timings) {
     const HipExecutor& hip = backend_of(ws.get_executor());
     oza_timings ct{};
-    detail::check(oza_scheme1_gemm(hip.context(), ws.get_M(), ws.get_N(), ws.get_K(), ws.get_slices(), A, B, C,
-                                   ws.get_shift_A(), ws.get_shift_B(), ws.get_A_slices(), ws.get_B_slices(),
-                                   ws.get_C_tc(), timings ? &ct : nullptr));
+    size_t b[5];  // as the workspace's constructor allocated them
+    detail::check(oza_workspace_bytes(1, ws.get_M(), ws.get_N(), ws.get_K(), ws.get_slices(), b));
+    detail::check(oza_scheme1_gemm_sized(hip.context(), ws.get_M(), ws.get_N(), ws.get_K(), ws.get_slices(), A, B, C,
+                                         ws.get_shift_A(), ws.get_shift_B(), ws.get_A_slices(), ws.get_B_slices(),
+                                         ws.get_C_tc(), b[4], timings ? &ct : nullptr));
     fill(timings, ct);
 }
 

@@ -418,7 +418,7 @@ static int enqueue_pipeline(int scheme, oza_ctx ctx, const Dims& d, const CallPl
 
 static int run_pipeline(int scheme, oza_ctx ctx, size_t M, size_t N, size_t K, int S, const double* A,
                         const double* B, double* C, int32_t* shA, int32_t* shB, int8_t* Asl, int8_t* Bsl,
-                        void* Ctc, oza_timings* t) {
+                        void* Ctc, oza_timings* t, const size_t* ctc_bytes = nullptr) {
     if (int r = check_ctx(ctx)) return r;
     if (int r = check_problem(scheme, M, N, K, S)) return r;
     if (M == 0 || N == 0) return OZA_SUCCESS;
@@ -426,13 +426,29 @@ static int run_pipeline(int scheme, oza_ctx ctx, size_t M, size_t N, size_t K, i
         return fail(OZA_INVALID_ARGUMENT, "OzaBLAS: null matrix or workspace pointer.");
     DeviceGuard g(ctx->device);
     const Dims d = make_dims(M, N, K, S);
-    return enqueue_pipeline(scheme, ctx, d, call_plan(scheme, d), Operand{A, (int64_t)K, true},
+    CallPlan plan = call_plan(scheme, d);
+    size_t b[5];
+    ws_bytes(scheme, M, N, d, &plan, b);
+    // Where the size is not given, Scheme I's callers may have sized C_tc by the layout of its S planes.
+    if (ctc_bytes ? *ctc_bytes < b[4] : scheme == 1 && plan.s1.planes > S) {  // the same result without partial sums
+        plan = call_plan(scheme, d, false);
+        ws_bytes(scheme, M, N, d, &plan, b);
+        if (ctc_bytes && *ctc_bytes < b[4])
+            return fail(OZA_INVALID_ARGUMENT, "OzaBLAS: C_tc smaller than the call's planes.");
+    }
+    return enqueue_pipeline(scheme, ctx, d, plan, Operand{A, (int64_t)K, true},
                             Operand{B, (int64_t)N, false}, OutC{C, (int64_t)N, 1.0, 0.0}, shA, shB, Asl, Bsl, Ctc, t);
 }
 
 int oza_scheme1_gemm(oza_ctx ctx, size_t M, size_t N, size_t K, int S, const double* A, const double* B, double* C,
                      int32_t* shA, int32_t* shB, int8_t* Asl, int8_t* Bsl, void* Ctc, oza_timings* t) {
     return run_pipeline(1, ctx, M, N, K, S, A, B, C, shA, shB, Asl, Bsl, Ctc, t);
+}
+
+int oza_scheme1_gemm_sized(oza_ctx ctx, size_t M, size_t N, size_t K, int S, const double* A, const double* B,
+                           double* C, int32_t* shA, int32_t* shB, int8_t* Asl, int8_t* Bsl, void* Ctc,
+                           size_t ctc_bytes, oza_timings* t) {
+    return run_pipeline(1, ctx, M, N, K, S, A, B, C, shA, shB, Asl, Bsl, Ctc, t, &ctc_bytes);
 }
 
 int oza_scheme2_gemm(oza_ctx ctx, size_t M, size_t N, size_t K, int S, const double* A, const double* B, double* C,
