@@ -552,21 +552,24 @@ int oza_gemm(oza_ctx ctx, int scheme, int S, int layout, int transA, int transB,
     if (!A || !B) return fail(OZA_INVALID_ARGUMENT, "OzaBLAS: null matrix pointer.");
     size_t b[5];
     const Dims d = make_dims(M, N, K, S);
-    CallPlan plan = call_plan(scheme, d);
-    ws_bytes(scheme, M, N, d, &plan, b);
-    size_t need = ws_total(b);
-    auto unsplit = [&] {  // the same result without partial tiles
-        plan = call_plan(scheme, d, false);
+    CallPlan plan;
+    size_t need = 0;
+    auto set_plan = [&](bool split) {  // the same result without partial tiles
+        plan = call_plan(scheme, d, split);
         ws_bytes(scheme, M, N, d, &plan, b);
         need = ws_total(b);
     };
+    set_plan(true);
     char* ws = static_cast<char*>(workspace);
     if (ws) {
-        if (workspace_bytes < need) unsplit();
+        if (workspace_bytes < need) set_plan(false);
         if (workspace_bytes < need)
             return fail(OZA_INVALID_ARGUMENT, "OzaBLAS: workspace smaller than oza_gemm_workspace_bytes.");
     } else {  // the context's own workspace, grown on demand and kept for later calls
         std::lock_guard<std::mutex> lk(ctx->ws_mu);
+        // Partial sums alone do not make it grow: the call may be captured, and graphs that were captured
+        // before hold its address.
+        if (ctx->ws_bytes < need) set_plan(false);
         if (ctx->ws_bytes < need) {
             if (ctx->ws) {
                 OZA_HIP(hipStreamSynchronize(ctx->stream), "HIP: workspace resize");
@@ -577,9 +580,10 @@ int oza_gemm(oza_ctx ctx, int scheme, int S, int layout, int transA, int transB,
             size_t most[5];  // what oza_gemm_workspace_bytes says: smaller shapes then fit too
             ws_bytes(scheme, M, N, d, nullptr, most);
             size_t size = ws_total(most);
+            set_plan(true);
             if (hipMalloc(&ctx->ws, size) != hipSuccess) {
                 (void)hipGetLastError();
-                unsplit();
+                set_plan(false);
                 size = need;
                 if (hipMalloc(&ctx->ws, size) != hipSuccess) {
                     (void)hipGetLastError();
