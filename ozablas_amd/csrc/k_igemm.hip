@@ -411,18 +411,8 @@ hipError_t persistent_grid(int64_t total, unsigned& grid) {
 using CfgS2 = IgemmCfgS2;
 using CfgS1 = IgemmCfgS1;
 
-// Four slots of 64 K-bytes instead of two of 128: three stages (96 KiB per CU) on their way from memory while
-// one is computed, instead of one of 64 KiB, for twice the barriers.  That pays where the operand planes come
-// from memory (past some 90 MB, that is with K past a few thousand) and each of their bytes meets few products.
-// Calls, us, two slots / four: 600^2 x 16384, S = 12 227 / 206; 512^2 x 32768, S = 14 327 / 317; 1024^2 x 16384,
-// S = 12 390 / 366; 300 x 8000 x 2048, S = 12 189 / 178; 1500^2 x 8192, S = 12 355 / 344.  Beyond the lines:
-// 2048^3, S = 6 93 / 96; 2100^3, S = 15 216 / 220; 8192^3, S = 17 8459 / 8619; 1800^2 x 8192, S = 12 463 / 467;
-// 1200^2 x 3000, S = 12 (86 MB) 109 / 110; 500^2 x 3000, S = 14 (45 MB) 53.9 / 54.5.
+// Four slots of 64 K-bytes instead of two of 128, where s2_deep_ring says.
 using CfgS2Deep = IgemmCfg<256, 256, 64, 4, 2, 4, 8>;
-constexpr int64_t kDeepBytes = 90000000, kDeepWidth = 800;
-static bool deep_ring(const Dims& d) {
-    return d.S * (d.Mp + d.Np) * d.Kp >= kDeepBytes && d.M * d.N <= kDeepWidth * (d.M + d.N) && d.Kp >= 256;
-}
 
 // Small calls (S2Plan::edge): 64 x 64 or 128 x 128 tiles, one item per workgroup, two workgroups per CU, four
 // slots.  Few 256 x 256 tiles leave CUs idle, and one of them alone spends more on its epilogue (128 digits
@@ -478,7 +468,7 @@ hipError_t launch_igemm_s2(const Dims& d, const int8_t* A_sl, const int8_t* B_sl
     if (small) return plan->edge == 64 ? launch_small<CfgS2Small64>(d, p, st) : launch_small<CfgS2Small128>(d, p, st);
     unsigned grid = 0;
     if (hipError_t e = persistent_grid(total, grid)) return e;
-    if (mode == S2Out::Digits && deep_ring(d) && (int64_t)p.parts * p.kts - p.KT <= p.kts - 2) {
+    if (mode == S2Out::Digits && s2_deep_ring(d, split ? *plan : S2Plan{})) {
         constexpr int kStages = CfgS2::BK / CfgS2Deep::BK;
         p.KT *= kStages;
         p.kts *= kStages;

@@ -183,6 +183,8 @@ struct S2Plan {
     int64_t whole = 0;
 };
 S2Plan scheme2_plan(const Dims& d);
+// Whether the 256 x 256 tiles of a plan (or of none: S2Plan{}) run on a ring of four slots.
+bool s2_deep_ring(const Dims& d, const S2Plan& p);
 // Digit tiles that a plan writes (65536 bytes each).
 int64_t s2_plan_tiles(const Dims& d, const S2Plan& p);
 // Scheme I: group g + 2 (g + 1 pairs) runs in parts[g] equal runs of its stages; the first part's INT32

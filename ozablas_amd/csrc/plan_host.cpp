@@ -87,6 +87,21 @@ S2Plan scheme2_plan(const Dims& d) {
     return best;
 }
 
+// Four slots of 64 K-bytes instead of two of 128: three stages (96 KiB per CU) on their way from memory while
+// one is computed, instead of one of 64 KiB, for twice the barriers.  That pays where the operand planes come
+// from memory (past some 90 MB, that is with K past a few thousand) and each of their bytes meets few products.
+// Calls, us, two slots / four: 600^2 x 16384, S = 12 227 / 206; 512^2 x 32768, S = 14 327 / 317; 1024^2 x 16384,
+// S = 12 390 / 366; 300 x 8000 x 2048, S = 12 189 / 178; 1500^2 x 8192, S = 12 355 / 344.  Beyond the lines:
+// 2048^3, S = 6 93 / 96; 2100^3, S = 15 216 / 220; 8192^3, S = 17 8459 / 8619; 1800^2 x 8192, S = 12 463 / 467;
+// 1200^2 x 3000, S = 12 (86 MB) 109 / 110; 500^2 x 3000, S = 14 (45 MB) 53.9 / 54.5.
+// (p.parts * p.kts - KT: what the last part is short of kts K steps; it needs two of them for its four stages.)
+bool s2_deep_ring(const Dims& d, const S2Plan& p) {
+    constexpr int64_t kDeepBytes = 90000000, kDeepWidth = 800;
+    const bool pays = d.S * (d.Mp + d.Np) * d.Kp >= kDeepBytes && d.M * d.N <= kDeepWidth * (d.M + d.N);
+    return pays && p.edge == kS2TileRows && d.Kp >= 256 &&
+           (p.parts == 1 || (int64_t)p.parts * p.kts - d.Kp / 128 <= p.kts - 2);
+}
+
 int64_t s2_plan_tiles(const Dims& d, const S2Plan& p) {
     const int64_t items = tiles_of(d) * d.S;
     return p.parts > 1 ? items + (p.parts - 1) * (items - p.whole) : items;
