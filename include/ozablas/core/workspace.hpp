@@ -112,7 +112,8 @@ private:
     int32_t* C_tc_ = nullptr;
 };
 
-// Stage times in milliseconds.  Large calls overlap step 4 with step 3 in row bands: then
+// Stage times in milliseconds.  Steps 1 and 2 of short K (up to 2048 for most shapes, up to 4096 for
+// some) are one launch: step2_ms then holds both and step1_ms is next to nothing.  Large calls overlap step 4 with step 3 in row bands: then
 // step3_ms runs from the end of step 2 to the end of the last band's products (it includes the
 // earlier bands' reconstruction beside them) and step4_ms is the last band's reconstruction.
 struct OzaTimings {

@@ -33,7 +33,9 @@ typedef enum oza_status {
 } oza_status;
 
 /* Per-call stage times in milliseconds; mirrors struct OzaTimings
- * (include/ozablas/core/workspace.hpp:97-103). */
+ * (include/ozablas/core/workspace.hpp:97-103).  Steps 1 and 2 of short K (up to 2048 for most shapes, up to
+ * 4096 for some) are one launch: step2_ms then holds both and step1_ms is next to nothing.  The same goes for
+ * oza_ctx_event_times and, where every problem is that short, for a group. */
 typedef struct oza_timings {
     float step1_ms, step2_ms, step3_ms, step4_ms, total_ms;
 } oza_timings;

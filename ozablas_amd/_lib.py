@@ -175,7 +175,8 @@ def generate_matrix(rows: int, cols: int, phi: float, seed: int) -> np.ndarray:
 
 
 class OzaTimings:
-    """Mirror of struct OzaTimings (stage times in ms)."""
+    """Mirror of struct OzaTimings (stage times in ms).  Where steps 1 and 2 are one launch (short K), step2_ms
+    holds both and step1_ms is next to nothing."""
 
     __slots__ = ("step1_ms", "step2_ms", "step3_ms", "step4_ms", "total_ms")
 
