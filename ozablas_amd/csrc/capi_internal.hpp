@@ -25,8 +25,8 @@ struct oza_context {
     hipEvent_t band_ev[kMaxBands] = {};
     hipEvent_t join_ev = nullptr;
     double* stats_dev = nullptr;   // 4 doubles for oza_error_stats
-    // Work counters of the step-3 GEMMs: 8 per row band (kMaxBands sets), cleared by each call's
-    // step-1 key-clearing launch.
+    // Work counters of Scheme I's step-3 GEMM: 8 per row band (kMaxBands sets), cleared by each call's
+    // first launch.
     unsigned* queue_dev = nullptr;
     rocblas_handle blas = nullptr;
     std::mutex blas_mu;

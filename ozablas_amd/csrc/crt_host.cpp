@@ -191,7 +191,6 @@ Dims make_dims(size_t M, size_t N, size_t K, int S) {
     d.Mp = (int64_t)round_up(M, kPadMN);
     d.Np = (int64_t)round_up(N, kPadMN);
     d.Kp = (int64_t)round_up(K, kPadK);
-    d.Nd = (int64_t)round_up(N, kPadDigits);
     return d;
 }
 

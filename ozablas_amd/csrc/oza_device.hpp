@@ -104,28 +104,12 @@ __device__ __forceinline__ int sym_residue(const uint32_t (&w)[ND], const uint32
 // nothing, the accumulators start from it (kProductBias).  As in sym_residue: d, the sum of u's four bytes times wt
 // (byte k = -2^32 2^(8k) mod m) plus init = 2^32 2^31 mod m, is congruent to -2^32 v and below 2^18 + 2^8; with
 // p = d m^-1 mod 2^32 the product p m = r 2^32 + d for r = floor(p m / 2^32) < m, so r is congruent to v.
-// Three 32-bit instructions (full rate, four cycles per wave like every instruction here) against five in
-// FP64 (crt_digit).  With a multiple of m for the 2^31 there would be no init, but the products past
+// Three 32-bit instructions (full rate, four cycles per wave like every instruction here) against five for
+// an FP64 quotient.  With a multiple of m for the 2^31 there would be no init, but the products past
 // 2^32 minus it, up to 250 of them, would wrap.
 constexpr uint32_t kProductBias = 0x80000000u;
 __device__ __forceinline__ uint32_t product_digit(uint32_t u, uint32_t wt, uint32_t init, uint32_t m, uint32_t minv) {
     return __umulhi(__builtin_amdgcn_udot4(u, wt, init, false) * minv, m);
-}
-
-// CRT digit of an INT32 product: the Euclidean residue c = v mod m in [0, m) -- the reference's
-// `rem` (step4_reconstruction.hpp:92-94) -- for any int32 v and modulus 3 <= m < 512, with
-// rcp = RN(1/m), in five FP64 operations.
-//   x = fma(v, rcp, 2^31 + 2^-10).  |v/m| < 2^31/3, so 2^30 < x < 2^32 and x is rounded to a
-//   multiple of at most 2^-21 (error <= 2^-22); |v rcp - v/m| <= |v|/m 2^-53 < 2^-23.  With
-//   v = q m + c, x = (q + 2^31) + c/m + 2^-10 + e, |e| < 2^-21.
-//   fract(x) = c/m + 2^-10 + e exactly (in (0, 1) since c <= m - 1 and m < 1024), and
-//   fma(fract(x), m, 0.5) = c + 0.5 + m (2^-10 + e) lies strictly between c + 0.5 and c + 1 for
-//   m < 512 (the product and sum are exact: fract(x) is a multiple of 2^-22 below 1), so the
-//   truncating conversion returns c.
-__device__ __forceinline__ int crt_digit(int v, double m, double rcp) {
-    constexpr double kBias = 2147483648.0 + 0x1p-10;  // 2^31 + 2^-10, exact
-    const double x = fma((double)v, rcp, kBias);
-    return (int)fma(__builtin_amdgcn_fract(x), m, 0.5);
 }
 
 // ---- MFMA-fragment-tiled operand planes -------------------------------------------------------

@@ -23,7 +23,6 @@ namespace oza {
 constexpr int kMaxSlices = 20;
 constexpr int kPadMN = 256;  // row padding of the operand planes (largest GEMM tile edge)
 constexpr int kPadK = 128;   // K padding of the operand planes (largest K stage)
-constexpr int kPadDigits = 16;
 
 inline size_t round_up(size_t x, size_t m) { return (x + m - 1) / m * m; }
 
@@ -92,7 +91,7 @@ int scheme2_slices_for_accuracy(size_t K, double digits, double spread);
 // ------------------------------------------------------------------------------------------
 struct Dims {
     int64_t M, N, K;
-    int64_t Mp, Np, Kp, Nd;
+    int64_t Mp, Np, Kp;
     int S;
 };
 Dims make_dims(size_t M, size_t N, size_t K, int S);

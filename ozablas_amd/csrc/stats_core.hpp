@@ -133,7 +133,7 @@ struct StatOp {
     uint32_t* keys;
 };
 
-// Blocks the column reader aims for in a single-problem launch.  With kColRows-row blocks a small
+// Blocks the column reader aims for in the stage entry point's launch.  With kColRows-row blocks a small
 // operand gives few blocks (1024 x 1024: 16), whose threads each wait for kColRows / kStatUnroll =
 // 16 rounds of loads in turn (15 us for the launch); shorter blocks, down to two rounds, spread the
 // same reads over more CUs at the cost of more atomic maxima per column.

@@ -4,7 +4,7 @@ import ctypes as C
 
 
 class Dims(C.Structure):
-    _fields_ = [(n, C.c_int64) for n in ("M", "N", "K", "Mp", "Np", "Kp", "Nd")] + [("S", C.c_int)]
+    _fields_ = [(n, C.c_int64) for n in ("M", "N", "K", "Mp", "Np", "Kp")] + [("S", C.c_int)]
 
 
 class S2Plan(C.Structure):
