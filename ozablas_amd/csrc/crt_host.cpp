@@ -97,7 +97,7 @@ CrtTables build_tables() {
                     cs.wt[s] |= (uint32_t)((m - p) % m) << (8 * k);
                     p = p * 256 % m;
                 }
-                cs.init[s] = (uint32_t)((uint64_t(1) << 63) % m);
+                cs.m_init[s] = (uint32_t)(m | ((uint64_t(1) << 63) % m) << 8);
                 err += (m - 1) * e;
             }
             Big R = MP;

@@ -442,12 +442,13 @@ __device__ __forceinline__ void grouped_tile(uint32_t t, const TileOrder& o, int
 template <class C, bool SKIP_PAD, bool NT = false>
 __device__ __forceinline__ void store_digits(const v16i (&acc)[C::FM][C::FN], uint8_t* plane, int64_t Np,
                                              int64_t row0, int64_t col0, int64_t M, int64_t N, uint32_t wt,
-                                             uint32_t init, uint32_t m, uint32_t minv, int lane) {
+                                             uint32_t m_init, uint32_t minv, int lane) {
     const int64_t qn = Np >> 5;
     // An instruction takes one scalar register.  From a plain use of a second one the compiler moved the whole
     // item descriptor to vector registers (185 -> 205 of them).
     uint32_t vinit;
-    asm("v_mov_b32 %0, %1" : "=v"(vinit) : "s"(init));
+    asm("v_mov_b32 %0, %1" : "=v"(vinit) : "s"(m_init >> 8));
+    const uint32_t m = m_init & 0xffu;
     // row0 and col0 are the same for the whole wave
     const int64_t fm_end = (M - (int64_t)__builtin_amdgcn_readfirstlane((int)(row0 >> 5)) * 32 + 31) >> 5;
     const int64_t fn_end = (N - (int64_t)__builtin_amdgcn_readfirstlane((int)(col0 >> 5)) * 32 + 31) >> 5;
@@ -456,13 +457,13 @@ __device__ __forceinline__ void store_digits(const v16i (&acc)[C::FM][C::FN], ui
 #pragma unroll
         for (int fn = 0; fn < C::FN; ++fn) {
             if (SKIP_PAD && (fm >= fm_end || fn >= fn_end)) continue;
-            uint32_t d[16];
+            int d[16];
 #pragma unroll
-            for (int j = 0; j < 16; ++j) d[j] = product_digit((uint32_t)acc[fm][fn][j], wt, vinit, m, minv);
+            for (int j = 0; j < 16; ++j) d[j] = (int)product_digit((uint32_t)acc[fm][fn][j], wt, vinit, m, minv);
             const int64_t blk = ((row0 >> 5) + fm) * qn + (col0 >> 5) + fn;
-            store_global16<NT>(plane + (blk << 10) + lane * 16, pack4u(d[0], d[1], d[2], d[3]),
-                           pack4u(d[4], d[5], d[6], d[7]), pack4u(d[8], d[9], d[10], d[11]),
-                           pack4u(d[12], d[13], d[14], d[15]));
+            store_global16<NT>(plane + (blk << 10) + lane * 16, pack4_lo(d[0], d[1], d[2], d[3]),
+                               pack4_lo(d[4], d[5], d[6], d[7]), pack4_lo(d[8], d[9], d[10], d[11]),
+                               pack4_lo(d[12], d[13], d[14], d[15]));
         }
 }
 

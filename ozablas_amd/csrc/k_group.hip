@@ -145,7 +145,7 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
         uint8_t* plane;  // digit plane of modulus s (a partial plane for splits j > 0)
         int64_t Np, M, N;
         int tm, tn, k0, KT;  // K steps [k0, k0 + KT) of BK bytes
-        uint32_t m, minv, wt, init;
+        uint32_t m_init, minv, wt;
     };
     constexpr int kSteps128 = 128 / C::BK;  // K steps per 128-byte K block
     auto item = [&](uint32_t wi) {
@@ -172,10 +172,9 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
                             (int)((P.M - (int64_t)t.tm * C::BM - 1) >> 5), (int)((P.N - (int64_t)t.tn * C::BN - 1) >> 5));
         t.plane = (j == 0 ? P.dg : P.dgp + (int64_t)(j - 1) * P.S * P.planeD) + s * P.planeD;
         const auto& cs = as_constant(g.crt)->set[P.S - 1];
-        t.m = cs.m[s];
+        t.m_init = cs.m_init[s];
         t.minv = cs.minv[s];
         t.wt = cs.wt[s];
-        t.init = cs.init[s];
         return t;
     };
     auto stage = [](const Item& t, int i) {  // stage i of an item; its last one past that
@@ -209,7 +208,7 @@ __global__ void __launch_bounds__(C::NT) k_group_gemm(GroupLaunch g) {
                 v16i acc[P::FM][P::FN];
                 fill_acc<P>(acc, (int)kProductBias);
                 mainloop_chain<P>(acc, smem, base, cur.KT, stage(cur, 2), step, entry);
-                store_digits<P, true, true>(acc, cur.plane, cur.Np, row0, col0, cur.M, cur.N, cur.wt, cur.init, cur.m,
+                store_digits<P, true, true>(acc, cur.plane, cur.Np, row0, col0, cur.M, cur.N, cur.wt, cur.m_init,
                                               cur.minv, lane);
             },
             [&] { mainloop_idle<C>(smem, base, cur.KT, stage(cur, 2), step, entry); });

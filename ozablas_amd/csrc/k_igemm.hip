@@ -49,7 +49,7 @@ struct S2Args {
     TileOrder order;       // of the tile rows [tm0, tm0 + order.tiles_m)
     int tm0;
     void* out;             // digits or int32 planes
-    const CrtSet* crt;     // device copy (m, minv, wt, init used)
+    const CrtSet* crt;     // device copy (m_init, minv, wt used)
     // SPLIT only: items [0, whole) run whole, the `tail` others in `parts` parts of kts K steps
     uint32_t items, whole, tail;
     FastDiv by_tail;
@@ -71,7 +71,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
         int s, tm, tn, j, k0, KT;
         uint32_t l;
         StageSrc src;  // this wave's blocks of stage 0
-        uint32_t m, minv, wt, init;
+        uint32_t m_init, minv, wt;
     };
     auto decode = [&](uint32_t wi) {
         Item t;
@@ -97,10 +97,9 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
                             p.B + (int64_t)t.s * p.Np * p.Kp + (int64_t)t.tn * C::BN * p.Kp + (int64_t)t.k0 * C::STEP, p.Kp,
                             wave, (int)((p.M - (int64_t)t.tm * C::BM - 1) >> 5), (int)((p.N - (int64_t)t.tn * C::BN - 1) >> 5));
         // scalar loads: counted by lgkmcnt, so the epilogue does not wait for the direct loads
-        t.m = as_constant(p.crt)->m[t.s];
+        t.m_init = as_constant(p.crt)->m_init[t.s];
         t.minv = as_constant(p.crt)->minv[t.s];
         t.wt = as_constant(p.crt)->wt[t.s];
-        t.init = as_constant(p.crt)->init[t.s];
         return t;
     };
     auto stage = [](const Item& t, int i) {  // stage i of an item; its last one past that
@@ -138,7 +137,7 @@ __global__ void __launch_bounds__(C::NT) k_igemm_s2(S2Args p) {
                     uint8_t* plane = part ? p.part + (int64_t)((cur.j - 1) * p.tail + cur.l - p.whole) * kTileBytes
                                           : reinterpret_cast<uint8_t*>(p.out) + (int64_t)s * p.Mp * p.Np;
                     store_digits<P, false>(acc, plane, part ? C::BN : p.Np, part ? wm * C::WTM : row0,
-                                           part ? wn * C::WTN : col0, p.M, p.N, cur.wt, cur.init, cur.m, cur.minv, lane);
+                                           part ? wn * C::WTN : col0, p.M, p.N, cur.wt, cur.m_init, cur.minv, lane);
                 } else {
                     int32_t* o = reinterpret_cast<int32_t*>(p.out) + (int64_t)s * p.M * p.N;
 #pragma unroll

@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(256)
     uint32_t c[S];
 #pragma unroll
     for (int s = 0; s < S; ++s)
-        c[s] = product_digit((uint32_t)Ct[s * MN + idx] + kProductBias, cs->wt[s], cs->init[s], cs->m[s], cs->minv[s]);
+        c[s] = product_digit((uint32_t)Ct[s * MN + idx] + kProductBias, cs->wt[s], cs->m_init[s] >> 8, cs->m[s], cs->minv[s]);
     const double f = crt_value<S>(c, 0, cs);
     Cout[idx] = ldexp(f, -(shA[row] + shB[col]));
 }

@@ -168,11 +168,6 @@ __device__ __forceinline__ void store_unit16(void* p, uint4 v) {
 }
 
 // ---- byte packing ---------------------------------------------------------------------------------
-// Four values already in [0, 255] into one word (byte 0 = a).
-__device__ __forceinline__ uint32_t pack4u(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
-    return a | (b << 8) | (c << 16) | (d << 24);
-}
-
 // Low bytes of four values (any sign) into one word (byte 0 = a): v_perm_b32 picks byte 0 of each
 // source (selector 0-3: second source, 4-7: first source, 0x0c: zero).
 __device__ __forceinline__ uint32_t pack4_lo(int a, int b, int c, int d) {

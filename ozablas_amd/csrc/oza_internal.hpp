@@ -68,8 +68,8 @@ struct CrtSet {
     uint32_t R[kGroups][kWords];
     uint32_t Mneg[kWords];            // 2^160 - M
     uint32_t M32[kWords], Mhalf32[kWords];  // M and floor(M/2)
-    // product_digit: m_s, m_s^-1 mod 2^32, the byte weights and 2^63 mod m_s
-    uint32_t m[kMaxSlices], minv[kMaxSlices], wt[kMaxSlices], init[kMaxSlices];
+    // product_digit: m_s, m_s^-1 mod 2^32, the byte weights, and m_s + 2^8 (2^63 mod m_s) in one word
+    uint32_t m[kMaxSlices], minv[kMaxSlices], wt[kMaxSlices], m_init[kMaxSlices];
     uint64_t M64[4];                  // M in 64-bit words
 };
 
