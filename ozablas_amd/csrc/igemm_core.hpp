@@ -438,7 +438,9 @@ __device__ __forceinline__ void grouped_tile(uint32_t t, const TileOrder& o, int
 // blocks that hold no element of the M x N product (tile padding) are neither computed nor stored
 // (the reconstruction never reads them); the grouped GEMM, whose small problems pad much, uses it,
 // while the single-problem GEMM keeps the branch-free epilogue (0.3 % faster at 8192^3).  NT
-// makes the stores nontemporal (store_unit16).
+// makes the stores nontemporal (store_unit16).  Four digits are packed by byte selects (three instructions;
+// shifts and ors took seven, since the compiler does not know that a digit is below 256: 2048^3, S = 6 96.8 and
+// 95.5 us, 512 grouped products 4881 and 4828 us).
 template <class C, bool SKIP_PAD, bool NT = false>
 __device__ __forceinline__ void store_digits(const v16i (&acc)[C::FM][C::FN], uint8_t* plane, int64_t Np,
                                              int64_t row0, int64_t col0, int64_t M, int64_t N, uint32_t wt,

@@ -33,7 +33,7 @@ using namespace core;
 // workgroup b takes positions b, b + gridDim.x, ... of the item list through xcd_remap, so that each XCD
 // (workgroup b runs on XCD b % 8) works through a contiguous run and its tiles in flight share their
 // operand panels in L2.  Taking positions from per-XCD counters instead, to keep them neighbours when
-// CUs drift apart, fetches less (13.4 against 19.1 GB at 8192^3 unbanded) in the same time, and the
+// CUs drift apart, fetched 13.4 GB at 8192^3 unbanded (13.8 in this order), and the
 // claim's wait costs 0.6 % (8192^3, S = 17: 8.715 against 8.667 ms; 4096^2 x 1024, S = 16: 415 against
 // 410 us).  Scheme I's items differ in length and do take them from counters (Claims below).
 // ------------------------------------------------------------------------------------------

@@ -94,6 +94,9 @@ S2Plan scheme2_plan(const Dims& d) {
 // S = 12 390 / 366; 300 x 8000 x 2048, S = 12 189 / 178; 1500^2 x 8192, S = 12 355 / 344.  Beyond the lines:
 // 2048^3, S = 6 93 / 96; 2100^3, S = 15 216 / 220; 8192^3, S = 17 8459 / 8619; 1800^2 x 8192, S = 12 463 / 467;
 // 1200^2 x 3000, S = 12 (86 MB) 109 / 110; 500^2 x 3000, S = 14 (45 MB) 53.9 / 54.5.
+// The bytes are counted with rows padded to 256, although only 32-row blocks that hold a row are read: few rows by
+// a long K gain as well (64^2 x 20000, S = 15, 39 of 154 MB read, 61.3 / 59.5; 30 x 40 x 60000, S = 6, 35 of 184, 76.3 / 72.7;
+// 96 x 13 x 30000, S = 10, 39 of 154, 65.1 / 62.9; 128^2 x 20000, S = 14, 72 of 144, 79.2 / 78.9).
 // (p.parts * p.kts - KT: what the last part is short of kts K steps; it needs two of them for its four stages.)
 bool s2_deep_ring(const Dims& d, const S2Plan& p) {
     constexpr int64_t kDeepBytes = 90000000, kDeepWidth = 800;
